@@ -32,7 +32,8 @@ _vp = C.c_void_p
 def build() -> None:
     """Compile liboracle.so (and oracle/_ref when the reference is present)."""
     subprocess.run(["make", "-s", "-C", _HERE], check=True)
-    if os.path.isdir(os.environ.get("MFP_REFERENCE", "/root/reference")):
+    ref = os.environ.get("MFP_REFERENCE", "/root/reference")
+    if os.path.isfile(os.path.join(ref, "common", "measurement_class.cpp")):
         subprocess.run(["make", "-s", "-C", _HERE, "ref"], check=True)
 
 
