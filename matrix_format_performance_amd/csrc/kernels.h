@@ -31,7 +31,7 @@ uint32_t adaptive_vectors_per_lane(int dtype, uint32_t nnz_per_wg);
 
 int launch_csr_scalar(int dtype, uint32_t rows, const uint32_t *rp, const uint32_t *ci,
                       const void *a, const void *x, void *y, hipStream_t s);
-int launch_csr_vector(int dtype, uint32_t lanes, uint32_t rows, const uint32_t *rp,
+int launch_csr_vector(int dtype, uint32_t lanes, uint32_t rows, uint64_t nnz, const uint32_t *rp,
                       const uint32_t *ci, const void *a, const void *x, void *y, hipStream_t s);
 int launch_csr_adaptive(int dtype, const adaptive_args &g, const void *a, const void *x, void *y,
                         hipStream_t s);

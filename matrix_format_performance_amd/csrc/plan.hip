@@ -696,7 +696,7 @@ static int plan_spmv(mfp_plan p, const void *x, void *y, hipStream_t s, void *pa
   case MFP_CSR_SCALAR:
     return launch_csr_scalar(dt, m->rows, m->row_ptr, m->columns, m->values, x, y, s);
   case MFP_CSR_VECTOR:
-    return launch_csr_vector(dt, p->t.lanes, m->rows, m->row_ptr, m->columns, m->values, x, y, s);
+    return launch_csr_vector(dt, p->t.lanes, m->rows, m->nnz, m->row_ptr, m->columns, m->values, x, y, s);
   case MFP_CSR_ADAPTIVE: {
     adaptive_args g;
     g.rows = m->rows;

@@ -241,7 +241,7 @@ int mfp_gpu_csr_vector_spmv(int dtype, const mfp_host_csr *A, mfp_buffer Ad, mfp
   MFP_CHECK(upload_csr(dtype, A, Ad, cd, rd, xd, yd, 24.0));
   double sec = 0;
   MFP_CHECK(run_timed([&] {
-    return launch_csr_vector(dtype, REFERENCE_VECTOR_LANES, A->rows, (const uint32_t *)mfp_buffer_ptr(rd),
+    return launch_csr_vector(dtype, REFERENCE_VECTOR_LANES, A->rows, A->nnz, (const uint32_t *)mfp_buffer_ptr(rd),
                              (const uint32_t *)mfp_buffer_ptr(cd), mfp_buffer_ptr(Ad),
                              mfp_buffer_ptr(xd), mfp_buffer_ptr(yd), nullptr);
   }, &sec));

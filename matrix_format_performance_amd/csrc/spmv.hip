@@ -139,68 +139,227 @@ __global__ __launch_bounds__(64) void k_csr_scalar(uint32_t rows, const uint32_t
 // offsets, so no load is predicated) before the x entries of the current
 // eight are gathered and summed, so a long row waits for one memory latency
 // per eight elements instead of two per four.
+//
+// Elements i, i + G, ... of one row (below e) onto the lane's sum.
+template <typename T, int G>
+__device__ __forceinline__ T csr_vector_rest(uint32_t i, uint32_t e, const uint32_t *__restrict__ ci,
+                                             const T *__restrict__ a, const T *__restrict__ x, T dot)
+{
+  constexpr uint32_t U = 8;
+  if (i + (U - 1) * G < e) {
+    T an[U];
+    uint32_t cn[U];
+#pragma unroll
+    for (uint32_t u = 0; u < U; u++) {
+      an[u] = ldg_stream(a + i + u * G);
+      cn[u] = ldg_stream(ci + i + u * G);
+    }
+    for (;;) {
+      T ac[U];
+      uint32_t cc[U];
+#pragma unroll
+      for (uint32_t u = 0; u < U; u++) {
+        ac[u] = an[u];
+        cc[u] = cn[u];
+      }
+      const uint32_t inext = i + U * G;
+      const bool more = inext + (U - 1) * G < e;
+#pragma unroll
+      for (uint32_t u = 0; u < U; u++) {
+        const uint32_t j = min(inext + u * G, e - 1u); // e > i: in range
+        an[u] = ldg_stream(a + j);
+        cn[u] = ldg_stream(ci + j);
+      }
+      T xv[U];
+#pragma unroll
+      for (uint32_t u = 0; u < U; u++) xv[u] = x[cc[u]];
+#pragma unroll
+      for (uint32_t u = 0; u < U; u++) dot = fma_t(ac[u], xv[u], dot);
+      i = inext;
+      if (!more) break;
+    }
+  }
+  for (; i + 3u * G < e; i += 4u * G) {
+    const T a0 = ldg_stream(a + i), a1 = ldg_stream(a + i + G);
+    const T a2 = ldg_stream(a + i + 2 * G), a3 = ldg_stream(a + i + 3 * G);
+    const uint32_t c0 = ldg_stream(ci + i), c1 = ldg_stream(ci + i + G);
+    const uint32_t c2 = ldg_stream(ci + i + 2 * G), c3 = ldg_stream(ci + i + 3 * G);
+    const T x0 = x[c0], x1 = x[c1], x2 = x[c2], x3 = x[c3];
+    dot = fma_t(a0, x0, dot);
+    dot = fma_t(a1, x1, dot);
+    dot = fma_t(a2, x2, dot);
+    dot = fma_t(a3, x3, dot);
+  }
+  for (; i < e; i += G) dot = fma_t(ldg_stream(a + i), x[ldg_stream(ci + i)], dot);
+  return dot;
+}
+
 template <typename T, int G>
 __global__ __launch_bounds__(256) void k_csr_vector(uint32_t rows, const uint32_t *__restrict__ rp,
                                                     const uint32_t *__restrict__ ci,
                                                     const T *__restrict__ a, const T *__restrict__ x,
                                                     T *__restrict__ y)
 {
-  constexpr uint32_t U = 8;
   const uint32_t blk = xcd_block(blockIdx.x, gridDim.x);
   const uint32_t row = (blk * 256u + threadIdx.x) / G;
   const uint32_t lane = threadIdx.x % G;
   T dot = 0;
   if (row < rows) {
     const uint32_t b = rp[row], e = rp[row + 1];
-    uint32_t i = b + lane;
-    if (i + (U - 1) * G < e) {
-      T an[U];
-      uint32_t cn[U];
-#pragma unroll
-      for (uint32_t u = 0; u < U; u++) {
-        an[u] = ldg_stream(a + i + u * G);
-        cn[u] = ldg_stream(ci + i + u * G);
-      }
-      for (;;) {
-        T ac[U];
-        uint32_t cc[U];
-#pragma unroll
-        for (uint32_t u = 0; u < U; u++) {
-          ac[u] = an[u];
-          cc[u] = cn[u];
-        }
-        const uint32_t inext = i + U * G;
-        const bool more = inext + (U - 1) * G < e;
-#pragma unroll
-        for (uint32_t u = 0; u < U; u++) {
-          const uint32_t j = min(inext + u * G, e - 1u); // e > i: in range
-          an[u] = ldg_stream(a + j);
-          cn[u] = ldg_stream(ci + j);
-        }
-        T xv[U];
-#pragma unroll
-        for (uint32_t u = 0; u < U; u++) xv[u] = x[cc[u]];
-#pragma unroll
-        for (uint32_t u = 0; u < U; u++) dot = fma_t(ac[u], xv[u], dot);
-        i = inext;
-        if (!more) break;
-      }
-    }
-    for (; i + 3u * G < e; i += 4u * G) {
-      const T a0 = ldg_stream(a + i), a1 = ldg_stream(a + i + G);
-      const T a2 = ldg_stream(a + i + 2 * G), a3 = ldg_stream(a + i + 3 * G);
-      const uint32_t c0 = ldg_stream(ci + i), c1 = ldg_stream(ci + i + G);
-      const uint32_t c2 = ldg_stream(ci + i + 2 * G), c3 = ldg_stream(ci + i + 3 * G);
-      const T x0 = x[c0], x1 = x[c1], x2 = x[c2], x3 = x[c3];
-      dot = fma_t(a0, x0, dot);
-      dot = fma_t(a1, x1, dot);
-      dot = fma_t(a2, x2, dot);
-      dot = fma_t(a3, x3, dot);
-    }
-    for (; i < e; i += G) dot = fma_t(ldg_stream(a + i), x[ldg_stream(ci + i)], dot);
+    dot = csr_vector_rest<T, G>(b + lane, e, ci, a, x, dot);
   }
   dot = group_reduce<G>(dot);
   if (lane == 0 && row < rows) y[row] = dot;
+}
+
+// The same sums from LDS.  A workgroup takes RB consecutive rows and stages
+// as many whole ones as fit (a values and gathered x entries, CVL_K 16-byte
+// vectors per lane, every load in flight before the first wait), then each
+// group of G lanes sums its rows from there.  A longer row goes through LDS
+// in chunks, the first group carrying its lanes' sums from one to the next.
+//
+// What bounds the kernel above is waiting: a wave of G = 64 lanes issues one
+// load of values, one of columns and one of x entries per row of 34 entries,
+// each after the last, and a row's 136 bytes are read in 4-byte loads.  Here
+// a workgroup's loads are independent of its row lengths: 16 bytes per lane,
+// two vectors of values and of columns, then their 8 (FP64: 4) gathers.
+// Eight workgroups share a CU (16 KB of LDS, 44 to 56 VGPRs).  FP32, lanes
+// from the mean, before -> now: 27-point stencil of 100^3 121.7 -> 53.7 us,
+// 5-point stencil of 1400^2 56.8 -> 25.6, 300,007 rows of 4 to 64 random
+// entries 75.4 -> 58 (the gathers alone take 48.5), power-law 1M rows
+// 342 -> 165 (its 50,000-entry row is one wait per 1,984 entries instead of
+// one per 8 per lane).  Larger chunks were slower: three vectors per lane
+// 59.5 and four 70.6 us on the 27-point stencil, against 55.5.
+constexpr uint32_t CVL_K = 2, CVL_U = 2;
+template <typename T>
+struct cvl {
+  static constexpr uint32_t N = vec16<T>::N, K = CVL_K, CAP = 256 * K * N;
+  // chunk of a long row: a multiple of 64 lanes that fits at any alignment
+  static constexpr uint32_t CHUNK = CAP - 64;
+};
+
+// Elements [base, base + n) into LDS at (element - base / N N); n + base % N <= CAP
+template <typename T>
+__device__ __forceinline__ void cvl_stage(uint32_t base, uint32_t n, const uint32_t *__restrict__ ci,
+                                          const T *__restrict__ a, const T *__restrict__ x, T *sa, T *sx)
+{
+  using VT = vec16<T>;
+  constexpr uint32_t N = VT::N, K = cvl<T>::K;
+  const uint32_t v0 = base / N, nv = (uint32_t)(((uint64_t)base + n + N - 1) / N) - v0;
+  const typename VT::V *av = reinterpret_cast<const typename VT::V *>(a) + v0;
+  const typename VT::I *cv = reinterpret_cast<const typename VT::I *>(ci) + v0;
+  typename VT::V va[K], vx[K];
+  typename VT::I vc[K];
+#pragma unroll
+  for (uint32_t k = 0; k < K; k++) {
+    const uint32_t v = min(threadIdx.x + k * 256u, nv - 1u);
+    va[k] = ldg_stream(av + v);
+    vc[k] = ldg_stream(cv + v);
+  }
+  const uint32_t lo = base - v0 * N, hi = lo + n; // the vectors' elements that count
+#pragma unroll
+  for (uint32_t k = 0; k < K; k++)
+#pragma unroll
+    for (uint32_t j = 0; j < N; j++) {
+      const uint32_t e = min(threadIdx.x + k * 256u, nv - 1u) * N + j;
+      vx[k][j] = x[e >= lo && e < hi ? vc[k][j] : 0u];
+    }
+#pragma unroll
+  for (uint32_t k = 0; k < K; k++) {
+    const uint32_t v = threadIdx.x + k * 256u;
+    if (v < nv) {
+      reinterpret_cast<typename VT::V *>(sa)[v] = va[k];
+      reinterpret_cast<typename VT::V *>(sx)[v] = vx[k];
+    }
+  }
+}
+
+template <typename T, int G>
+__global__ __launch_bounds__(256, 8) void k_csr_vector_lds(uint32_t rows, uint32_t RB, const uint32_t *__restrict__ rp,
+                                                        const uint32_t *__restrict__ ci,
+                                                        const T *__restrict__ a, const T *__restrict__ x,
+                                                        T *__restrict__ y)
+{
+  constexpr uint32_t N = cvl<T>::N, CAP = cvl<T>::CAP, CHUNK = cvl<T>::CHUNK;
+  __shared__ __align__(16) T sa[CAP];
+  __shared__ __align__(16) T sx[CAP];
+  __shared__ uint32_t rs[257];
+  const uint32_t r0 = xcd_block(blockIdx.x, gridDim.x) * RB; // RB <= 256
+  const uint32_t nr = min(RB, rows - r0), tid = threadIdx.x;
+  if (tid <= nr) rs[tid] = rp[r0 + tid];
+  if (tid == 0 && nr == 256u) rs[256] = rp[r0 + 256u];
+  __syncthreads();
+  const uint32_t lane = tid % G, grp = tid / G;
+  for (uint32_t cur = 0; cur < nr;) {
+    const uint32_t base = rs[cur], off = base % N;
+    if (rs[cur + 1] - base > CAP - off) {
+      const uint32_t e = rs[cur + 1];
+      T dot = 0;
+      for (uint32_t c0 = base; c0 < e; c0 += CHUNK) {
+        const uint32_t n = min(CHUNK, e - c0);
+        cvl_stage(c0, n, ci, a, x, sa, sx);
+        __syncthreads();
+        if (tid < G) {
+          const uint32_t sh = c0 % N;
+          uint32_t i = lane;
+          for (; i + 7u * G < n; i += 8u * G) {
+            T qa[8], qx[8];
+#pragma unroll
+            for (uint32_t q = 0; q < 8; q++) {
+              qa[q] = sa[sh + i + q * G];
+              qx[q] = sx[sh + i + q * G];
+            }
+#pragma unroll
+            for (uint32_t q = 0; q < 8; q++) dot = fma_t(qa[q], qx[q], dot);
+          }
+          for (; i < n; i += G) dot = fma_t(sa[sh + i], sx[sh + i], dot);
+        }
+        __syncthreads();
+      }
+      if (tid < 64u) { // the first group's wave
+        dot = group_reduce<G>(dot);
+        if (tid == 0) y[r0 + cur] = dot;
+      }
+      cur++;
+      continue;
+    }
+    // whole rows that fit behind base
+    const uint32_t fit = (uint32_t)__syncthreads_count(tid >= cur && tid < nr && rs[tid + 1] - base <= CAP - off);
+    const uint32_t end = cur + fit, n = rs[end] - base;
+    if (n) cvl_stage(base, n, ci, a, x, sa, sx);
+    __syncthreads();
+    const uint32_t org = base - off;
+    // U rows of a group side by side; the wave's groups stay together
+    constexpr uint32_t ST = 256u / G, U = CVL_U;
+    for (uint32_t r = cur + grp; r - grp < end; r += U * ST) {
+      uint32_t b[U], e[U];
+      T dot[U], qa[U], qx[U];
+#pragma unroll
+      for (uint32_t q = 0; q < U; q++) {
+        const uint32_t rr = min(r + q * ST, end - 1u);
+        b[q] = rs[rr] - org + lane;
+        e[q] = rs[rr + 1] - org;
+      }
+#pragma unroll
+      for (uint32_t q = 0; q < U; q++) {
+        const uint32_t i = min(b[q], CAP - 1u);
+        qa[q] = sa[i];
+        qx[q] = sx[i];
+      }
+#pragma unroll
+      for (uint32_t q = 0; q < U; q++) dot[q] = b[q] < e[q] ? fma_t(qa[q], qx[q], (T)0) : (T)0;
+#pragma unroll
+      for (uint32_t q = 0; q < U; q++)
+        for (uint32_t i = b[q] + G; i < e[q]; i += G) dot[q] = fma_t(sa[i], sx[i], dot[q]);
+#pragma unroll
+      for (uint32_t q = 0; q < U; q++) dot[q] = group_reduce<G>(dot[q]);
+#pragma unroll
+      for (uint32_t q = 0; q < U; q++)
+        if (lane == 0 && r + q * ST < end) y[r0 + r + q * ST] = dot[q];
+    }
+    __syncthreads();
+    cur = end;
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1187,19 +1346,41 @@ static int launch_k(void (*kernel)(P...), dim3 grid, dim3 block, uint32_t lds, h
   return launched();
 }
 
+template <typename T, int G>
+static int csr_vector_g(uint32_t rows, uint64_t nnz, const uint32_t *rp, const uint32_t *ci, const T *a, const T *x,
+                        T *y, hipStream_t s)
+{
+  const dim3 b(256);
+  const uint32_t grid = ceil_div_u32((uint64_t)rows * G, 256);
+  // The LDS form for rows of up to CAP / 8 entries on average (256 FP32, 128
+  // FP64: enough rows per chunk for every group of lanes) and for rows of
+  // 2 CAP or more (whole chunks); between them a chunk holds one to seven
+  // rows and most groups idle: rows of about 1,200 took 25 us here against
+  // 27 to 301 from LDS, 64 to 2 lanes.  Below 131,072 entries both are a
+  // launch's latency (3,000 rows of 34: 3.9 us each).
+  const double mean = (double)nnz / rows;
+  const uint32_t cap = cvl<T>::CAP;
+  if (nnz >= (1u << 17) && (mean <= cap / 8 || mean >= 2.0 * cap)) {
+    // rows that fill 85% of a chunk on average, fewer where that would leave
+    // a CU with less than two workgroups
+    const uint32_t fit = (uint32_t)std::min(256.0, std::max(1.0, 0.85 * cap / std::max(mean, 1.0)));
+    const uint32_t rb = std::max(1u, std::min(fit, ceil_div_u32(rows, 2u * (uint32_t)std::max(1, props().cu_count))));
+    return launch_k(k_csr_vector_lds<T, G>, dim3(ceil_div_u32(rows, rb)), b, 0, s, rows, rb, rp, ci, a, x, y);
+  }
+  return launch_k(k_csr_vector<T, G>, dim3(grid), b, 0, s, rows, rp, ci, a, x, y);
+}
+
 template <typename T>
-static int csr_vector_t(uint32_t lanes, uint32_t rows, const uint32_t *rp, const uint32_t *ci,
+static int csr_vector_t(uint32_t lanes, uint32_t rows, uint64_t nnz, const uint32_t *rp, const uint32_t *ci,
                         const T *a, const T *x, T *y, hipStream_t s)
 {
-  const uint32_t grid = ceil_div_u32((uint64_t)rows * lanes, 256);
-  const dim3 g(grid), b(256);
   switch (lanes) {
-  case 2: return launch_k(k_csr_vector<T, 2>, g, b, 0, s, rows, rp, ci, a, x, y);
-  case 4: return launch_k(k_csr_vector<T, 4>, g, b, 0, s, rows, rp, ci, a, x, y);
-  case 8: return launch_k(k_csr_vector<T, 8>, g, b, 0, s, rows, rp, ci, a, x, y);
-  case 16: return launch_k(k_csr_vector<T, 16>, g, b, 0, s, rows, rp, ci, a, x, y);
-  case 32: return launch_k(k_csr_vector<T, 32>, g, b, 0, s, rows, rp, ci, a, x, y);
-  case 64: return launch_k(k_csr_vector<T, 64>, g, b, 0, s, rows, rp, ci, a, x, y);
+  case 2: return csr_vector_g<T, 2>(rows, nnz, rp, ci, a, x, y, s);
+  case 4: return csr_vector_g<T, 4>(rows, nnz, rp, ci, a, x, y, s);
+  case 8: return csr_vector_g<T, 8>(rows, nnz, rp, ci, a, x, y, s);
+  case 16: return csr_vector_g<T, 16>(rows, nnz, rp, ci, a, x, y, s);
+  case 32: return csr_vector_g<T, 32>(rows, nnz, rp, ci, a, x, y, s);
+  case 64: return csr_vector_g<T, 64>(rows, nnz, rp, ci, a, x, y, s);
   default: set_error("lanes must be a power of two in [2, 64]"); return MFP_ERR_ARG;
   }
 }
@@ -1216,13 +1397,13 @@ int launch_csr_scalar(int dtype, uint32_t rows, const uint32_t *rp, const uint32
                   (const double *)x, (double *)y);
 }
 
-int launch_csr_vector(int dtype, uint32_t lanes, uint32_t rows, const uint32_t *rp,
+int launch_csr_vector(int dtype, uint32_t lanes, uint32_t rows, uint64_t nnz, const uint32_t *rp,
                       const uint32_t *ci, const void *a, const void *x, void *y, hipStream_t s)
 {
   if (rows == 0) return MFP_OK;
   if (dtype == MFP_F32)
-    return csr_vector_t<float>(lanes, rows, rp, ci, (const float *)a, (const float *)x, (float *)y, s);
-  return csr_vector_t<double>(lanes, rows, rp, ci, (const double *)a, (const double *)x, (double *)y, s);
+    return csr_vector_t<float>(lanes, rows, nnz, rp, ci, (const float *)a, (const float *)x, (float *)y, s);
+  return csr_vector_t<double>(lanes, rows, nnz, rp, ci, (const double *)a, (const double *)x, (double *)y, s);
 }
 
 // Vectors a lane may need for a block of up to W elements at any alignment.
