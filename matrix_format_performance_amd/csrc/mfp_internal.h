@@ -102,9 +102,12 @@ struct device_props {
 const device_props &props();
 int ensure_init();
 
-// Stream-ordered device allocation helpers (plain hipMalloc; plans own them).
+// Device memory of the library's objects and scratch; freed blocks are kept
+// for the next ones (runtime.hip).  dfree waits for the device, as hipFree.
 int dmalloc(void **p, size_t bytes);
 void dfree(void *p);
+// bytes kept that way now: free memory from the library's point of view
+size_t cached_device_bytes();
 
 // ---- converter entry points used by plans (convert.hip) -------------------
 int row_stats_device(uint32_t rows, const uint32_t *row_ptr_d, mfp_row_stats *out,

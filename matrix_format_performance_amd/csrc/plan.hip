@@ -171,7 +171,7 @@ static uint64_t budget_of(const mfp_tuning &t)
   if (t.budget_bytes) return t.budget_bytes;
   size_t fr = 0, tot = 0;
   if (hipMemGetInfo(&fr, &tot) != hipSuccess) return 0;
-  return (uint64_t)(0.9 * (double)fr);
+  return (uint64_t)(0.9 * (double)(fr + cached_device_bytes()));
 }
 
 static int matrix_stats(mfp_matrix m, mfp_row_stats *out, hipStream_t s);

@@ -7,7 +7,10 @@
 #include <hip/hip_fp16.h>
 
 #include <cstring>
+#include <map>
 #include <mutex>
+#include <unordered_map>
+#include <utility>
 
 namespace mfp {
 
@@ -66,19 +69,151 @@ int ensure_init()
   return init_device(0);
 }
 
+// Device memory of the library's own objects and their scratch.
+//
+// hipMalloc / hipFree map and unmap memory: 30 to 90 us per call for blocks of
+// 16 MB and more, 210 to 250 us to free one while others are held, so that
+// building one plan spent more on its ten or so arrays than on its kernels
+// (nine formats of a 5M-entry matrix: 1.8 ms of kernels in 8.7 to 12.9 ms).
+// Freed blocks of 64 KB to 1 GB are therefore kept and handed out again, in
+// size classes an eighth of a power of two apart.
+//  * A block is kept only once the device is idle (dfree waits for it, as
+//    hipFree does), so whoever gets it next, on any stream or thread, finds
+//    nothing still running on it.
+//  * At most CACHE_BYTES are kept; an allocation that fails gives all of them
+//    back and tries again, and they are given back when the library's last
+//    block is freed.
+//  * mfp_malloc and mfp_free, whose pointers belong to the caller, do not
+//    take part.
+constexpr size_t CACHE_MIN = 64u << 10, CACHE_MAX = 1u << 30, CACHE_BYTES = 4ull << 30;
+
+struct block_cache {
+  std::mutex mutex;
+  std::multimap<size_t, void *> kept;                       // by size, device `device` only
+  std::unordered_map<void *, std::pair<size_t, int>> sizes; // cacheable blocks in use: size, device
+  size_t kept_bytes = 0;
+  size_t in_use = 0; // blocks of any size
+  int device = -1;   // of the kept blocks
+};
+
+static block_cache &cache()
+{
+  static block_cache *c = new block_cache; // never destroyed: objects may outlive static destructors
+  return *c;
+}
+
+// cache().mutex held
+static void cache_release(block_cache &c)
+{
+  for (auto &b : c.kept) (void)hipFree(b.second);
+  c.kept.clear();
+  c.kept_bytes = 0;
+}
+
+size_t cached_device_bytes()
+{
+  block_cache &c = cache();
+  std::lock_guard<std::mutex> lock(c.mutex);
+  return c.kept_bytes;
+}
+
+static size_t cache_class(size_t bytes)
+{
+  size_t step = CACHE_MIN / 8;
+  while (step * 16 <= bytes) step *= 2; // 8 step <= bytes < 16 step
+  return (bytes + step - 1) / step * step;
+}
+
+static hipError_t malloc_or_release(void **p, size_t bytes)
+{
+  hipError_t e = hipMalloc(p, bytes);
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    {
+      block_cache &c = cache();
+      std::lock_guard<std::mutex> lock(c.mutex);
+      cache_release(c);
+    }
+    e = hipMalloc(p, bytes);
+  }
+  return e;
+}
+
 // Every allocation carries 256 bytes of slack past its end: kernels that read
 // 16-byte vectors may touch up to 12 bytes beyond an array's last element.
 int dmalloc(void **p, size_t bytes)
 {
   MFP_CHECK(ensure_init());
   *p = nullptr;
-  MFP_HIP(hipMalloc(p, bytes + 256));
+  bytes += 256;
+  block_cache &c = cache();
+  const bool cacheable = bytes >= CACHE_MIN && bytes <= CACHE_MAX;
+  if (cacheable) {
+    const size_t size = cache_class(bytes);
+    std::lock_guard<std::mutex> lock(c.mutex);
+    if (c.device == g_props.device) {
+      const auto it = c.kept.lower_bound(size);
+      if (it != c.kept.end() && it->first <= size + size / 4) {
+        *p = it->second;
+        c.sizes[*p] = {it->first, c.device};
+        c.kept_bytes -= it->first;
+        c.kept.erase(it);
+        c.in_use++;
+        return MFP_OK;
+      }
+    }
+  }
+  const size_t size = cacheable ? cache_class(bytes) : bytes;
+  hipError_t e = malloc_or_release(p, size);
+  if (e != hipSuccess && size > bytes) { // without the rounding, then
+    (void)hipGetLastError();
+    e = hipMalloc(p, bytes);
+    if (e == hipSuccess) {
+      std::lock_guard<std::mutex> lock(c.mutex);
+      c.in_use++;
+      return MFP_OK;
+    }
+  }
+  MFP_HIP(e);
+  std::lock_guard<std::mutex> lock(c.mutex);
+  c.in_use++;
+  if (cacheable) c.sizes[*p] = {size, g_props.device};
   return MFP_OK;
 }
 
 void dfree(void *p)
 {
-  if (p) (void)hipFree(p);
+  if (!p) return;
+  block_cache &c = cache();
+  size_t size = 0;
+  {
+    std::lock_guard<std::mutex> lock(c.mutex);
+    const auto it = c.sizes.find(p);
+    if (it != c.sizes.end()) {
+      int cur = -1;
+      if (hipGetDevice(&cur) == hipSuccess && cur == it->second.second) size = it->second.first;
+      c.sizes.erase(it);
+    }
+  }
+  if (size && hipDeviceSynchronize() != hipSuccess) {
+    (void)hipGetLastError();
+    size = 0;
+  }
+  void *free_now = p;
+  std::lock_guard<std::mutex> lock(c.mutex);
+  if (size) {
+    if (c.device != g_props.device) {
+      cache_release(c);
+      c.device = g_props.device;
+    }
+    if (c.kept_bytes + size <= CACHE_BYTES) {
+      c.kept.emplace(size, p);
+      c.kept_bytes += size;
+      free_now = nullptr;
+    }
+  }
+  if (free_now) (void)hipFree(free_now);
+  if (--c.in_use == 0) cache_release(c);
 }
 
 // ---- fills ----------------------------------------------------------------
@@ -217,7 +352,7 @@ int mfp_device_query(mfp_device_info *out)
   out->cu_count = g_props.cu_count;
   out->xcd_count = g_props.xcd_count;
   out->lds_per_block = g_props.lds_per_block;
-  out->free_mem = fr;
+  out->free_mem = fr + cached_device_bytes();
   out->total_mem = tot;
   std::strncpy(out->name, g_props.name, sizeof(out->name) - 1);
   std::strncpy(out->arch, g_props.arch, sizeof(out->arch) - 1);
@@ -250,7 +385,10 @@ int mfp_synchronize(void)
 int mfp_malloc(void **p, size_t bytes)
 {
   MFP_ARG(p, "ptr is null");
-  return dmalloc(p, bytes);
+  MFP_CHECK(ensure_init());
+  *p = nullptr;
+  MFP_HIP(malloc_or_release(p, bytes + 256)); // the slack of dmalloc
+  return MFP_OK;
 }
 
 int mfp_free(void *p)
@@ -313,10 +451,10 @@ int mfp_flush_cache(uint64_t bytes, mfp_stream s)
   if (bytes < (64ull << 20)) bytes = 64ull << 20;
   bytes = (bytes + 15) / 16 * 16;
   if (g_flush_bytes < bytes) {
-    dfree(g_flush_buf);
+    (void)mfp_free(g_flush_buf); // held until the process ends: not one of dmalloc's
     g_flush_buf = nullptr;
     g_flush_bytes = 0;
-    MFP_CHECK(dmalloc(&g_flush_buf, bytes));
+    MFP_CHECK(mfp_malloc(&g_flush_buf, bytes));
     MFP_CHECK(launch_fill((uint32_t *)g_flush_buf, bytes / 4, 0x5A5A5A5Au, as_stream(s)));
     g_flush_bytes = bytes;
   }

@@ -64,3 +64,38 @@ def test_csr_vector_from_lds(gpu, rows, lanes, dtype):
     x[0] = np.nan  # slots past a chunk's elements gather x[0]; none may reach a sum
     y = _spmv(gpu, rp, ci, va, x, "csr_vector", lanes=lanes)
     assert np.array_equal(y, oracle.spmv_lanes(rp, ci, va, x, lanes))
+
+
+# ---- device memory kept between objects -----------------------------------------
+
+def test_blocks_from_several_threads(gpu):
+    # four threads build, multiply and destroy plans of sizes that share
+    # memory blocks: none may see another's data
+    import threading
+
+    def work(seed, bad):
+        gpu.init(0)
+        rng = np.random.default_rng(seed)
+        for i in range(6):
+            rp, ci, va = _csr(rng.integers(0, 40, 9000 + 1500 * int(rng.integers(0, 4))), 9001, "float32", seed + i)
+            x = gpu.generate_vector(seed + i, 9001, np.dtype(np.float32))
+            y = _spmv(gpu, rp, ci, va, x, "ell" if i % 2 else "csr_scalar")
+            if not np.array_equal(y, oracle.spmv_seq(rp, ci, va, x)):
+                bad.append((seed, i))
+
+    bad = []
+    threads = [threading.Thread(target=work, args=(100 * s, bad)) for s in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
+
+
+def test_free_memory_counts_kept_blocks(gpu):
+    rp, ci, va = _csr([50] * 200000, 200001, "float32")
+    free = gpu.device_info()["free_mem"]
+    A = gpu.DeviceMatrix.from_csr(rp, ci, va, 200001)
+    gpu.Plan(A, "ell").destroy()
+    A.destroy()
+    assert abs(gpu.device_info()["free_mem"] - free) < 64 << 20
