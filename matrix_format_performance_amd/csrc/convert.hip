@@ -14,208 +14,341 @@
 
 namespace mfp {
 
-// ---------------------------------------------------------------------------
-// Exclusive scan of u32 (hierarchical: tile scan, scan of tile sums, add).
-// ---------------------------------------------------------------------------
-constexpr uint32_t SCAN_T = 256, SCAN_I = 8, SCAN_TILE = SCAN_T * SCAN_I;
-
-__device__ __forceinline__ uint32_t block_exclusive_scan_256(uint32_t v, uint32_t *sh, uint32_t *total)
-{
-  // Hillis-Steele over 256 thread values in LDS.
-  const uint32_t t = threadIdx.x;
-  sh[t] = v;
-  __syncthreads();
-  for (uint32_t off = 1; off < SCAN_T; off <<= 1) {
-    uint32_t add = t >= off ? sh[t - off] : 0u;
-    __syncthreads();
-    sh[t] += add;
-    __syncthreads();
-  }
-  uint32_t incl = sh[t];
-  if (total) *total = sh[SCAN_T - 1];
-  __syncthreads();
-  return incl - v;
-}
-
-__global__ __launch_bounds__(SCAN_T) void k_scan_tiles(const uint32_t *__restrict__ in,
-                                                       uint32_t *__restrict__ out, uint64_t n,
-                                                       uint32_t *__restrict__ sums)
-{
-  __shared__ uint32_t tile[SCAN_TILE];
-  __shared__ uint32_t sh[SCAN_T];
-  const uint64_t base = (uint64_t)blockIdx.x * SCAN_TILE;
-  const uint32_t t = threadIdx.x;
-  for (uint32_t k = 0; k < SCAN_I; k++) {
-    uint64_t i = base + k * SCAN_T + t;
-    tile[k * SCAN_T + t] = i < n ? in[i] : 0u;
-  }
-  __syncthreads();
-  uint32_t loc[SCAN_I];
-  uint32_t acc = 0;
-  for (uint32_t k = 0; k < SCAN_I; k++) {
-    loc[k] = acc;
-    acc += tile[t * SCAN_I + k];
-  }
-  uint32_t total = 0;
-  uint32_t pre = block_exclusive_scan_256(acc, sh, &total);
-  for (uint32_t k = 0; k < SCAN_I; k++) tile[t * SCAN_I + k] = loc[k] + pre;
-  __syncthreads();
-  for (uint32_t k = 0; k < SCAN_I; k++) {
-    uint64_t i = base + k * SCAN_T + t;
-    if (i < n) out[i] = tile[k * SCAN_T + t];
-  }
-  if (t == 0 && sums) sums[blockIdx.x] = total;
-}
-
-__global__ void k_scan_add(uint32_t *__restrict__ out, uint64_t n, const uint32_t *__restrict__ sums)
-{
-  const uint64_t base = (uint64_t)blockIdx.x * SCAN_TILE;
-  const uint32_t add = sums[blockIdx.x];
-  for (uint32_t k = 0; k < SCAN_I; k++) {
-    uint64_t i = base + k * SCAN_T + threadIdx.x;
-    if (i < n) out[i] += add;
-  }
-}
-
-__global__ void k_scan_total(const uint32_t *in, const uint32_t *out, uint64_t n, uint32_t *total)
-{
-  if (threadIdx.x == 0 && blockIdx.x == 0) *total = n ? out[n - 1] + in[n - 1] : 0u;
-}
-
-static int scan_rec(const uint32_t *in, uint32_t *out, uint64_t n, hipStream_t s)
-{
-  if (n == 0) return MFP_OK;
-  const uint64_t tiles = (n + SCAN_TILE - 1) / SCAN_TILE;
-  uint32_t *sums = nullptr;
-  if (tiles > 1) MFP_CHECK(dmalloc((void **)&sums, tiles * 4));
-  k_scan_tiles<<<(uint32_t)tiles, SCAN_T, 0, s>>>(in, out, n, sums);
-  MFP_HIP(hipGetLastError());
-  if (tiles > 1) {
-    int st = scan_rec(sums, sums, tiles, s);
-    if (st == MFP_OK) {
-      k_scan_add<<<(uint32_t)tiles, SCAN_T, 0, s>>>(out, n, sums);
-      st = hipGetLastError() == hipSuccess ? MFP_OK : MFP_ERR_HIP;
-    }
-    MFP_HIP(hipStreamSynchronize(s)); // sums is freed below
-    dfree(sums);
+// Device allocations freed on every return path unless released.
+struct device_temps {
+  std::vector<void *> held;
+  int alloc(void **p, size_t bytes)
+  {
+    const int st = dmalloc(p, bytes);
+    if (st == MFP_OK) held.push_back(*p);
     return st;
   }
-  return MFP_OK;
+  void release(void *p)
+  {
+    for (void *&q : held)
+      if (q == p) q = nullptr;
+  }
+  ~device_temps()
+  {
+    for (void *q : held) dfree(q);
+  }
+};
+
+// ---------------------------------------------------------------------------
+// Exclusive scan of u32: tile sums, one workgroup scans those, then every
+// tile scans itself from its offset (8 bytes read and 4 written per element,
+// three launches; one for a single tile).
+// ---------------------------------------------------------------------------
+constexpr uint32_t SCAN_T = 256, SCAN_I = 16, SCAN_TILE = SCAN_T * SCAN_I;
+
+// Exclusive prefix of v over a workgroup of T lanes; *total (may be null)
+// gets the sum.  sh holds T / 64 words.
+template <uint32_t T>
+__device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t v, uint32_t *sh, uint32_t *total)
+{
+  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+  uint32_t x = v;
+#pragma unroll
+  for (uint32_t d = 1; d < 64; d <<= 1) {
+    const uint32_t y = __shfl_up(x, d, 64);
+    if (lane >= d) x += y;
+  }
+  if (lane == 63) sh[wave] = x;
+  __syncthreads();
+  uint32_t pre = 0, all = 0;
+#pragma unroll
+  for (uint32_t w = 0; w < T / 64; w++) {
+    const uint32_t s = sh[w];
+    if (w < wave) pre += s;
+    all += s;
+  }
+  if (total) *total = all;
+  __syncthreads(); // sh may be written again
+  return pre + x - v;
 }
 
-// In-place (in == out) is allowed.  total_out (host) gets in[0..n) summed.
+__global__ __launch_bounds__(SCAN_T) void k_scan_sums(const uint32_t *__restrict__ in, uint64_t n,
+                                                      uint32_t *__restrict__ sums)
+{
+  __shared__ uint32_t sh[SCAN_T / 64];
+  const uint64_t base = (uint64_t)blockIdx.x * SCAN_TILE;
+  uint32_t acc = 0;
+#pragma unroll
+  for (uint32_t k = 0; k < SCAN_I; k++) {
+    const uint64_t i = base + k * SCAN_T + threadIdx.x;
+    acc += i < n ? in[i] : 0u;
+  }
+  uint32_t total;
+  (void)block_exclusive_scan<SCAN_T>(acc, sh, &total);
+  if (threadIdx.x == 0) sums[blockIdx.x] = total;
+}
+
+// sums[0 .. m) to their exclusive scan, the total to sums[m]; one workgroup
+__global__ __launch_bounds__(1024) void k_scan_offsets(uint32_t *__restrict__ sums, uint64_t m)
+{
+  __shared__ uint32_t sh[16];
+  uint32_t carry = 0;
+  for (uint64_t b = 0; b < m; b += 1024) {
+    const uint64_t i = b + threadIdx.x;
+    const uint32_t v = i < m ? sums[i] : 0u;
+    uint32_t total;
+    const uint32_t pre = block_exclusive_scan<1024>(v, sh, &total);
+    if (i < m) sums[i] = carry + pre;
+    carry += total;
+  }
+  if (threadIdx.x == 0) sums[m] = carry;
+}
+
+// offs: k_scan_offsets' result, or null for a single tile (whose total then
+// goes to *total)
+__global__ __launch_bounds__(SCAN_T) void k_scan_tiles(const uint32_t *in, uint32_t *out, uint64_t n,
+                                                       const uint32_t *__restrict__ offs,
+                                                       uint32_t *__restrict__ total)
+{
+  __shared__ uint32_t tile[SCAN_TILE + SCAN_TILE / 32]; // one word of padding per 32: lanes read SCAN_I apart
+  __shared__ uint32_t sh[SCAN_T / 64];
+  const uint64_t base = (uint64_t)blockIdx.x * SCAN_TILE;
+  const uint32_t t = threadIdx.x;
+#pragma unroll
+  for (uint32_t k = 0; k < SCAN_I; k++) {
+    const uint32_t l = k * SCAN_T + t;
+    tile[l + l / 32] = base + l < n ? in[base + l] : 0u;
+  }
+  __syncthreads();
+  uint32_t loc[SCAN_I], acc = 0;
+#pragma unroll
+  for (uint32_t k = 0; k < SCAN_I; k++) {
+    const uint32_t l = t * SCAN_I + k;
+    loc[k] = acc;
+    acc += tile[l + l / 32];
+  }
+  uint32_t all;
+  const uint32_t pre = block_exclusive_scan<SCAN_T>(acc, sh, &all) + (offs ? offs[blockIdx.x] : 0u);
+#pragma unroll
+  for (uint32_t k = 0; k < SCAN_I; k++) {
+    const uint32_t l = t * SCAN_I + k;
+    tile[l + l / 32] = loc[k] + pre;
+  }
+  __syncthreads();
+#pragma unroll
+  for (uint32_t k = 0; k < SCAN_I; k++) {
+    const uint32_t l = k * SCAN_T + t;
+    if (base + l < n) out[base + l] = tile[l + l / 32];
+  }
+  if (!offs && t == 0) *total = all;
+}
+
+// In-place (in == out) is allowed.  total_out (host) gets in[0..n) summed;
+// the call waits for the stream only when it is given.
 int exclusive_scan_u32(const uint32_t *in, uint32_t *out, uint64_t n, hipStream_t s,
                        uint32_t *total_out)
 {
-  uint32_t last_in = 0;
-  if (total_out && n) MFP_HIP(hipMemcpyAsync(&last_in, in + n - 1, 4, hipMemcpyDeviceToHost, s));
-  if (total_out) MFP_HIP(hipStreamSynchronize(s));
-  MFP_CHECK(scan_rec(in, out, n, s));
-  if (total_out) {
-    uint32_t last_out = 0;
-    if (n) MFP_HIP(hipMemcpyAsync(&last_out, out + n - 1, 4, hipMemcpyDeviceToHost, s));
-    MFP_HIP(hipStreamSynchronize(s));
-    *total_out = n ? last_out + last_in : 0;
+  if (total_out) *total_out = 0;
+  if (n == 0) return MFP_OK;
+  const uint64_t tiles = (n + SCAN_TILE - 1) / SCAN_TILE;
+  device_temps tmp;
+  uint32_t *sums = nullptr;
+  MFP_CHECK(tmp.alloc((void **)&sums, (tiles + 1) * 4));
+  if (tiles > 1) {
+    k_scan_sums<<<(uint32_t)tiles, SCAN_T, 0, s>>>(in, n, sums);
+    k_scan_offsets<<<1, 1024, 0, s>>>(sums, tiles);
+    k_scan_tiles<<<(uint32_t)tiles, SCAN_T, 0, s>>>(in, out, n, sums, nullptr);
+  } else {
+    k_scan_tiles<<<1, SCAN_T, 0, s>>>(in, out, n, nullptr, sums + tiles);
   }
+  MFP_HIP(hipGetLastError());
+  if (total_out) MFP_HIP(hipMemcpyAsync(total_out, sums + tiles, 4, hipMemcpyDeviceToHost, s));
+  MFP_HIP(hipStreamSynchronize(s)); // sums is freed here
   return MFP_OK;
 }
 
 // ---------------------------------------------------------------------------
-// Triplets -> CSR: counts + scan give row_ptr; a stable LSD radix sort of
-// (row, col, input index) by col then row gives the element order.
+// Stable radix sort of (row, column, value) entries by (row, column), least
+// significant digit first.  The values travel with the keys, so nothing is
+// gathered at the end, and as every pass keeps the order of equal digits no
+// input index is carried.  row may be any u32 whose bits above row_shift
+// count (the column-sorted layout sorts by slice).
+//   k_sort_count    digit counts of each tile (SORT_T ITEMS entries)
+//   k_sort_offsets  one workgroup per digit: exclusive scan over the tiles
+//   k_sort_scatter  ranks a tile's entries by digit (ballots inside a wave,
+//                   LDS counts across waves), reorders them in LDS and
+//                   writes each digit's run to its place: 8192 entries make
+//                   runs of 32 on average, so the stores are whole lines
 // ---------------------------------------------------------------------------
-__global__ void k_count_rows(const uint32_t *__restrict__ r, const uint32_t *__restrict__ c,
-                             uint64_t n, uint32_t rows, uint32_t cols,
-                             uint32_t *__restrict__ cnt, uint32_t *__restrict__ bad)
+constexpr uint32_t SORT_T = 512, SORT_W = SORT_T / 64, SORT_BINS = 256;
+
+struct sort_digit {
+  uint32_t row_shift; // row bits below this do not take part
+  uint32_t col_bits;  // columns are below 2^col_bits
+  uint32_t shift, width; // the digit's place in (row >> row_shift) 2^col_bits + column
+};
+
+__device__ __forceinline__ uint32_t digit_of(const sort_digit &d, uint32_t row, uint32_t col)
 {
-  uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-  for (; i < n; i += stride) {
-    uint32_t rr = r[i], cc = c[i];
-    if (rr >= rows || cc >= cols) {
-      atomicOr(bad, 1u);
-      continue;
-    }
-    atomicAdd(cnt + rr, 1u);
-  }
+  const uint64_t key = ((uint64_t)(row >> d.row_shift) << d.col_bits) | col;
+  return (uint32_t)(key >> d.shift) & ((1u << d.width) - 1u);
 }
 
-__global__ void k_iota(uint32_t *__restrict__ p, uint64_t n)
+// CHECK: also sets *bad when a row is not below rows or a column not below cols
+template <uint32_t ITEMS, bool CHECK>
+__global__ __launch_bounds__(SORT_T) void k_sort_count(const uint32_t *__restrict__ row,
+                                                       const uint32_t *__restrict__ col, uint64_t n, sort_digit dg,
+                                                       uint32_t rows, uint32_t cols, uint32_t ntiles,
+                                                       uint32_t *__restrict__ hist, uint32_t *__restrict__ bad)
 {
-  uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-  for (; i < n; i += stride) p[i] = (uint32_t)i;
-}
-
-constexpr uint32_t RX_T = 256, RX_I = 8, RX_TILE = RX_T * RX_I;
-
-__global__ __launch_bounds__(RX_T) void k_radix_hist(const uint32_t *__restrict__ key, uint64_t n,
-                                                     uint32_t shift, uint32_t *__restrict__ hist,
-                                                     uint32_t ntiles)
-{
-  __shared__ uint32_t cnt[256];
+  __shared__ uint32_t cnt[SORT_BINS];
   const uint32_t t = threadIdx.x;
-  cnt[t] = 0;
+  if (t < SORT_BINS) cnt[t] = 0;
   __syncthreads();
-  const uint64_t base = (uint64_t)blockIdx.x * RX_TILE;
-  for (uint32_t k = 0; k < RX_I; k++) {
-    uint64_t i = base + k * RX_T + t;
-    if (i < n) atomicAdd(&cnt[(key[i] >> shift) & 255u], 1u);
+  const uint64_t base = (uint64_t)blockIdx.x * (SORT_T * ITEMS);
+  const bool need_row = CHECK || dg.shift + dg.width > dg.col_bits, need_col = CHECK || dg.shift < dg.col_bits;
+  uint32_t r[ITEMS], c[ITEMS];
+#pragma unroll
+  for (uint32_t k = 0; k < ITEMS; k++) {
+    const uint64_t i = min(base + k * SORT_T + t, n - 1);
+    r[k] = need_row ? row[i] : 0u;
+    c[k] = need_col ? col[i] : 0u;
   }
+  bool out = false;
+#pragma unroll
+  for (uint32_t k = 0; k < ITEMS; k++)
+    if (base + k * SORT_T + t < n) {
+      atomicAdd(&cnt[digit_of(dg, r[k], c[k])], 1u);
+      if (CHECK) out = out || r[k] >= rows || c[k] >= cols;
+    }
+  if (CHECK && out) atomicOr(bad, 1u);
   __syncthreads();
-  hist[(uint64_t)t * ntiles + blockIdx.x] = cnt[t];
+  if (t < (1u << dg.width)) hist[(uint64_t)t * ntiles + blockIdx.x] = cnt[t];
 }
 
-// Stable scatter of three u32 arrays by the 8-bit digit of key.  Elements are
-// ranked in tile order (round k = elements k*256 .. k*256+255, by thread).
-__global__ __launch_bounds__(RX_T) void k_radix_scatter(
-    const uint32_t *__restrict__ key, const uint32_t *__restrict__ a0,
-    const uint32_t *__restrict__ a1, const uint32_t *__restrict__ a2, uint32_t *__restrict__ o0,
-    uint32_t *__restrict__ o1, uint32_t *__restrict__ o2, uint64_t n, uint32_t shift,
-    const uint32_t *__restrict__ offs, uint32_t ntiles)
+// row d of hist to its exclusive scan, its total to totals[d]
+__global__ __launch_bounds__(1024) void k_sort_offsets(uint32_t ntiles, uint32_t *__restrict__ hist,
+                                                       uint32_t *__restrict__ totals)
 {
-  __shared__ uint32_t run[256];
-  __shared__ uint32_t wcnt[RX_T / 64][256];
+  __shared__ uint32_t sh[16];
+  uint32_t *h = hist + (uint64_t)blockIdx.x * ntiles;
+  uint32_t carry = 0;
+  for (uint32_t b = 0; b < ntiles; b += 1024) {
+    const uint32_t i = b + threadIdx.x;
+    const uint32_t v = i < ntiles ? h[i] : 0u;
+    uint32_t total;
+    const uint32_t pre = block_exclusive_scan<1024>(v, sh, &total);
+    if (i < ntiles) h[i] = carry + pre;
+    carry += total;
+  }
+  if (threadIdx.x == 0) totals[blockIdx.x] = carry;
+}
+
+// VI: the values' type as read (the first pass of a triplet sort rounds
+// double values to the matrix's type), V: as moved and written
+template <typename VI, typename V, uint32_t ITEMS>
+__global__ __launch_bounds__(SORT_T, ITEMS > 8 ? 4 : 6) void k_sort_scatter(const uint32_t *__restrict__ row,
+                                                         const uint32_t *__restrict__ col,
+                                                         const VI *__restrict__ val, uint64_t n, sort_digit dg,
+                                                         uint32_t ntiles, const uint32_t *__restrict__ hist,
+                                                         const uint32_t *__restrict__ totals,
+                                                         uint32_t *__restrict__ orow, uint32_t *__restrict__ ocol,
+                                                         V *__restrict__ oval)
+{
+  constexpr uint32_t TILE = SORT_T * ITEMS;
+  __shared__ __align__(16) unsigned char buf_raw[TILE * (sizeof(V) > 4 ? sizeof(V) : 4)];
+  __shared__ uint32_t cnt[SORT_W][SORT_BINS]; // entries of each digit in the waves before
+  __shared__ uint32_t start[SORT_BINS];       // first slot of a digit's run in the tile
+  __shared__ uint32_t glob[SORT_BINS];        // output position of the run, less start
+  __shared__ uint32_t sh[SORT_W];
+  uint32_t *buf = reinterpret_cast<uint32_t *>(buf_raw);
+  V *vbuf = reinterpret_cast<V *>(buf_raw);
   const uint32_t t = threadIdx.x, lane = t & 63u, wave = t >> 6;
-  run[t] = offs[(uint64_t)t * ntiles + blockIdx.x];
-  const uint64_t base = (uint64_t)blockIdx.x * RX_TILE;
-  const uint64_t lt_mask = (lane == 0) ? 0ull : ((1ull << lane) - 1ull);
-  for (uint32_t k = 0; k < RX_I; k++) {
-    for (uint32_t w = 0; w < RX_T / 64; w++) wcnt[w][t] = 0;
-    __syncthreads();
-    const uint64_t i = base + k * RX_T + t;
-    const bool valid = i < n;
-    const uint32_t d = valid ? (key[i] >> shift) & 255u : 0u;
-    uint64_t peers = __ballot(valid);
-    for (uint32_t b = 0; b < 8; b++) {
-      const uint64_t m = __ballot((d >> b) & 1u);
-      peers &= ((d >> b) & 1u) ? m : ~m;
-    }
-    const uint32_t rank = __popcll(peers & lt_mask);
-    if (valid && rank == 0) wcnt[wave][d] = __popcll(peers);
-    __syncthreads();
-    if (valid) {
-      uint32_t pre = 0;
-      for (uint32_t w = 0; w < wave; w++) pre += wcnt[w][d];
-      const uint32_t pos = run[d] + pre + rank;
-      o0[pos] = a0[i];
-      o1[pos] = a1[i];
-      o2[pos] = a2[i];
-    }
-    __syncthreads();
-    uint32_t tot = 0;
-    for (uint32_t w = 0; w < RX_T / 64; w++) tot += wcnt[w][t];
-    run[t] += tot;
+  const uint64_t base = (uint64_t)blockIdx.x * TILE;
+  const uint32_t m = (uint32_t)min((uint64_t)TILE, n - base); // entries of this tile
+  // wave w holds entries w 64 ITEMS .. of the tile, 64 consecutive per item
+  const uint32_t l0 = wave * 64u * ITEMS + lane;
+  uint32_t r[ITEMS], c[ITEMS], pos[ITEMS];
+  V v[ITEMS];
+#pragma unroll
+  for (uint32_t k = 0; k < ITEMS; k++) {
+    const uint64_t i = base + min(l0 + k * 64u, m - 1u);
+    r[k] = row[i];
+    c[k] = col[i];
+    v[k] = (V)val[i];
   }
-}
-
-template <typename T>
-__global__ void k_gather_values(const uint32_t *__restrict__ idx, const double *__restrict__ v,
-                                T *__restrict__ out, uint64_t n)
-{
-  uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-  for (; i < n; i += stride) out[i] = (T)v[idx[i]];
+#pragma unroll
+  for (uint32_t b = 0; b < SORT_BINS / 64; b++) cnt[wave][b * 64u + lane] = 0;
+  // only this wave touches its row of cnt until the barrier below
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  const uint64_t below = lane ? ~0ull >> (64u - lane) : 0ull;
+#pragma unroll
+  for (uint32_t k = 0; k < ITEMS; k++) {
+    const bool valid = l0 + k * 64u < m;
+    const uint32_t d = digit_of(dg, r[k], c[k]);
+    uint64_t peers = __ballot(valid);
+    for (uint32_t b = 0; b < dg.width; b++) {
+      const bool one = (d >> b) & 1u;
+      const uint64_t ones = __ballot(one);
+      peers &= one ? ones : ~ones;
+    }
+    const uint32_t before = cnt[wave][d];
+    pos[k] = before + (uint32_t)__popcll(peers & below);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    if (valid && (peers & below) == 0) cnt[wave][d] = before + (uint32_t)__popcll(peers);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  }
+  __syncthreads();
+  uint32_t mine = 0, tot = 0;
+  if (t < SORT_BINS) {
+#pragma unroll
+    for (uint32_t w = 0; w < SORT_W; w++) {
+      const uint32_t x = cnt[w][t];
+      cnt[w][t] = mine;
+      mine += x;
+    }
+    tot = t < (1u << dg.width) ? totals[t] : 0u;
+  }
+  const uint32_t st = block_exclusive_scan<SORT_T>(mine, sh, nullptr);
+  const uint32_t gt = block_exclusive_scan<SORT_T>(tot, sh, nullptr);
+  if (t < SORT_BINS) {
+    start[t] = st;
+    glob[t] = t < (1u << dg.width) ? gt + hist[(uint64_t)t * ntiles + blockIdx.x] - st : 0u;
+  }
+  __syncthreads();
+#pragma unroll
+  for (uint32_t k = 0; k < ITEMS; k++) {
+    const uint32_t d = digit_of(dg, r[k], c[k]);
+    pos[k] += start[d] + cnt[wave][d];
+  }
+  // slot order: rows, columns, then values through the same LDS
+#pragma unroll
+  for (uint32_t k = 0; k < ITEMS; k++)
+    if (l0 + k * 64u < m) buf[pos[k]] = r[k];
+  __syncthreads();
+#pragma unroll
+  for (uint32_t k = 0; k < ITEMS; k++) r[k] = buf[min(k * SORT_T + t, m - 1u)];
+  __syncthreads();
+#pragma unroll
+  for (uint32_t k = 0; k < ITEMS; k++)
+    if (l0 + k * 64u < m) buf[pos[k]] = c[k];
+  __syncthreads();
+  uint32_t to[ITEMS];
+#pragma unroll
+  for (uint32_t k = 0; k < ITEMS; k++) {
+    const uint32_t j = k * SORT_T + t;
+    c[k] = buf[min(j, m - 1u)];
+    to[k] = glob[digit_of(dg, r[k], c[k])] + j;
+    if (j < m) {
+      orow[to[k]] = r[k];
+      ocol[to[k]] = c[k];
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (uint32_t k = 0; k < ITEMS; k++)
+    if (l0 + k * 64u < m) vbuf[pos[k]] = v[k];
+  __syncthreads();
+#pragma unroll
+  for (uint32_t k = 0; k < ITEMS; k++) {
+    const uint32_t j = k * SORT_T + t;
+    if (j < m) oval[to[k]] = vbuf[j];
+  }
 }
 
 static uint32_t bit_length(uint32_t v)
@@ -233,93 +366,122 @@ static uint32_t grid_for(uint64_t n, uint32_t bs = 256)
   return (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>((n + bs - 1) / bs, 1u << 16));
 }
 
+// The arrays of one side of the sort's ping-pong.
+template <typename V>
+struct sort_arrays {
+  uint32_t *row = nullptr, *col = nullptr;
+  V *val = nullptr;
+};
+
+// Sorts n >= 1 entries into `to`, using `via` between passes; the input is
+// not written.  key_rows / cols bound (row >> row_shift) and the columns.
+// bad (may be null): set when a row is not below rows or a column not below
+// cols; the sort stays in bounds either way.
+template <typename VI, typename V, uint32_t ITEMS>
+static int sort_entries_t(const uint32_t *row, const uint32_t *col, const VI *val, uint64_t n, uint32_t row_shift,
+                          uint64_t key_rows, uint32_t rows, uint32_t cols, const sort_arrays<V> &to,
+                          const sort_arrays<V> &via, uint32_t *bad, hipStream_t s)
+{
+  const uint32_t col_bits = bit_length(cols ? cols - 1 : 0);
+  const uint32_t bits = col_bits + bit_length(key_rows ? (uint32_t)(key_rows - 1) : 0);
+  const uint32_t passes = std::max(1u, (bits + 7) / 8);
+  const uint32_t width = std::max(1u, (bits + passes - 1) / passes); // as even as they come, at most 8
+  const uint32_t ntiles = (uint32_t)((n + SORT_T * ITEMS - 1) / (SORT_T * ITEMS));
+  device_temps tmp;
+  uint32_t *hist = nullptr;
+  MFP_CHECK(tmp.alloc((void **)&hist, ((uint64_t)ntiles + 1) * SORT_BINS * 4));
+  uint32_t *totals = hist + (uint64_t)ntiles * SORT_BINS;
+  for (uint32_t p = 0; p < passes; p++) {
+    const sort_digit dg{row_shift, col_bits, p * width, width};
+    const sort_arrays<V> &o = (passes - 1 - p) % 2 ? via : to; // the last pass lands in `to`
+    const sort_arrays<V> &f = (passes - 1 - p) % 2 ? to : via;
+    const uint32_t *fr = p ? f.row : row, *fc = p ? f.col : col;
+    if (p == 0 && bad)
+      k_sort_count<ITEMS, true><<<ntiles, SORT_T, 0, s>>>(fr, fc, n, dg, rows, cols, ntiles, hist, bad);
+    else
+      k_sort_count<ITEMS, false><<<ntiles, SORT_T, 0, s>>>(fr, fc, n, dg, rows, cols, ntiles, hist, nullptr);
+    k_sort_offsets<<<1u << width, 1024, 0, s>>>(ntiles, hist, totals);
+    if (p)
+      k_sort_scatter<V, V, ITEMS><<<ntiles, SORT_T, 0, s>>>(fr, fc, f.val, n, dg, ntiles, hist, totals, o.row, o.col,
+                                                            o.val);
+    else
+      k_sort_scatter<VI, V, ITEMS><<<ntiles, SORT_T, 0, s>>>(fr, fc, val, n, dg, ntiles, hist, totals, o.row, o.col,
+                                                             o.val);
+    MFP_HIP(hipGetLastError());
+  }
+  MFP_HIP(hipStreamSynchronize(s)); // hist is freed here
+  return MFP_OK;
+}
+
+template <typename VI, typename V>
+static int sort_entries(const uint32_t *row, const uint32_t *col, const VI *val, uint64_t n, uint32_t row_shift,
+                        uint64_t key_rows, uint32_t rows, uint32_t cols, const sort_arrays<V> &to,
+                        const sort_arrays<V> &via, uint32_t *bad, hipStream_t s)
+{
+  // 8192 entries per tile (FP64 values: 4096, 32 KB of LDS either way), 2048
+  // where those would be fewer than two per CU
+  if (n >= (1u << 22))
+    return sort_entries_t<VI, V, sizeof(V) == 8 ? 8 : 16>(row, col, val, n, row_shift, key_rows, rows, cols, to, via, bad, s);
+  return sort_entries_t<VI, V, 4>(row, col, val, n, row_shift, key_rows, rows, cols, to, via, bad, s);
+}
+
+// row_ptr[r] = entries in rows below r, from the entries' sorted rows
+__global__ void k_row_starts(uint32_t rows, uint64_t n, const uint32_t *__restrict__ row, uint32_t *__restrict__ rp)
+{
+  const uint64_t r = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (r > rows) return;
+  uint64_t lo = 0, hi = n;
+  while (lo < hi) {
+    const uint64_t mid = (lo + hi) / 2;
+    if (row[mid] < r)
+      lo = mid + 1;
+    else
+      hi = mid;
+  }
+  rp[r] = (uint32_t)lo;
+}
+
+template <typename V>
+static int csr_from_triplets_t(uint32_t rows, uint32_t cols, uint64_t nnz, const uint32_t *tr_rows,
+                               const uint32_t *tr_cols, const double *tr_vals, uint32_t *row_ptr, uint32_t *columns,
+                               V *values, hipStream_t s)
+{
+  device_temps tmp;
+  uint32_t *bad = nullptr;
+  sort_arrays<V> to, via;
+  to.col = columns;
+  to.val = values;
+  MFP_CHECK(tmp.alloc((void **)&bad, 4));
+  MFP_CHECK(tmp.alloc((void **)&to.row, nnz * 4));
+  MFP_CHECK(tmp.alloc((void **)&via.row, nnz * 4));
+  MFP_CHECK(tmp.alloc((void **)&via.col, nnz * 4));
+  MFP_CHECK(tmp.alloc((void **)&via.val, nnz * sizeof(V)));
+  MFP_CHECK(fill_u32(bad, 0, 1, s));
+  MFP_CHECK(sort_entries(tr_rows, tr_cols, tr_vals, nnz, 0, rows, rows, cols, to, via, bad, s));
+  k_row_starts<<<ceil_div_u32((uint64_t)rows + 1, 256), 256, 0, s>>>(rows, nnz, to.row, row_ptr);
+  MFP_HIP(hipGetLastError());
+  uint32_t hbad = 0;
+  MFP_HIP(hipMemcpyAsync(&hbad, bad, 4, hipMemcpyDeviceToHost, s));
+  MFP_HIP(hipStreamSynchronize(s));
+  if (hbad) {
+    set_error("triplet row/col index out of range");
+    return MFP_ERR_ARG;
+  }
+  return MFP_OK;
+}
+
+// Triplets -> CSR: the sort by (row, column), ties in input order; the row
+// pointers are searched in the sorted rows.
 int csr_from_triplets_device(int dtype, uint32_t rows, uint32_t cols, uint64_t nnz,
                              const uint32_t *tr_rows, const uint32_t *tr_cols,
                              const double *tr_vals, uint32_t *row_ptr, uint32_t *columns,
                              void *values, hipStream_t s)
 {
   MFP_ARG(nnz < (1ull << 32), "nnz must fit in 32 bits");
-  uint32_t *bad = nullptr;
-  MFP_CHECK(dmalloc((void **)&bad, 4));
-  MFP_CHECK(fill_u32(bad, 0, 1, s));
-  MFP_CHECK(fill_u32(row_ptr, 0, (uint64_t)rows + 1, s));
-  if (nnz) {
-    k_count_rows<<<grid_for(nnz), 256, 0, s>>>(tr_rows, tr_cols, nnz, rows, cols, row_ptr, bad);
-    MFP_HIP(hipGetLastError());
-  }
-  uint32_t hbad = 0;
-  MFP_HIP(hipMemcpyAsync(&hbad, bad, 4, hipMemcpyDeviceToHost, s));
-  MFP_HIP(hipStreamSynchronize(s));
-  dfree(bad);
-  if (hbad) {
-    set_error("triplet row/col index out of range");
-    return MFP_ERR_ARG;
-  }
-  MFP_CHECK(exclusive_scan_u32(row_ptr, row_ptr, (uint64_t)rows + 1, s, nullptr));
-  if (nnz == 0) return MFP_OK;
-
-  // ping-pong buffers: (row, col, idx)
-  uint32_t *buf[6] = {};
-  for (int i = 0; i < 6; i++) {
-    int st = dmalloc((void **)&buf[i], nnz * 4);
-    if (st != MFP_OK) {
-      for (int j = 0; j < i; j++) dfree(buf[j]);
-      return st;
-    }
-  }
-  const uint32_t ntiles = (uint32_t)((nnz + RX_TILE - 1) / RX_TILE);
-  uint32_t *hist = nullptr;
-  int st = dmalloc((void **)&hist, (uint64_t)ntiles * 256 * 4);
-  auto cleanup = [&]() {
-    for (int i = 0; i < 6; i++) dfree(buf[i]);
-    dfree(hist);
-  };
-  if (st != MFP_OK) {
-    cleanup();
-    return st;
-  }
-  // own copies of the keys, so the caller's arrays are never written
-  MFP_HIP(hipMemcpyAsync(buf[0], tr_rows, nnz * 4, hipMemcpyDeviceToDevice, s));
-  MFP_HIP(hipMemcpyAsync(buf[1], tr_cols, nnz * 4, hipMemcpyDeviceToDevice, s));
-  k_iota<<<grid_for(nnz), 256, 0, s>>>(buf[2], nnz);
-  uint32_t *cur[3] = {buf[0], buf[1], buf[2]};
-  uint32_t *nxt[3] = {buf[3], buf[4], buf[5]};
-  // passes: col digits (LSD), then row digits
-  std::vector<std::pair<int, uint32_t>> passes;
-  for (uint32_t sh = 0; sh < bit_length(cols ? cols - 1 : 0); sh += 8) passes.push_back({1, sh});
-  for (uint32_t sh = 0; sh < bit_length(rows ? rows - 1 : 0); sh += 8) passes.push_back({0, sh});
-  for (auto [which, sh] : passes) {
-    const uint32_t *key = cur[which];
-    k_radix_hist<<<ntiles, RX_T, 0, s>>>(key, nnz, sh, hist, ntiles);
-    if (hipGetLastError() != hipSuccess) {
-      cleanup();
-      set_error("radix hist launch failed");
-      return MFP_ERR_HIP;
-    }
-    st = exclusive_scan_u32(hist, hist, (uint64_t)ntiles * 256, s, nullptr);
-    if (st != MFP_OK) {
-      cleanup();
-      return st;
-    }
-    k_radix_scatter<<<ntiles, RX_T, 0, s>>>(key, cur[0], cur[1], cur[2], nxt[0], nxt[1], nxt[2],
-                                             nnz, sh, hist, ntiles);
-    if (hipGetLastError() != hipSuccess) {
-      cleanup();
-      set_error("radix scatter launch failed");
-      return MFP_ERR_HIP;
-    }
-    std::swap(cur, nxt);
-  }
-  // cur[1] = sorted columns, cur[2] = source index
-  MFP_HIP(hipMemcpyAsync(columns, cur[1], nnz * 4, hipMemcpyDeviceToDevice, s));
+  if (nnz == 0) return fill_u32(row_ptr, 0, (uint64_t)rows + 1, s);
   if (dtype == MFP_F32)
-    k_gather_values<float><<<grid_for(nnz), 256, 0, s>>>(cur[2], tr_vals, (float *)values, nnz);
-  else
-    k_gather_values<double><<<grid_for(nnz), 256, 0, s>>>(cur[2], tr_vals, (double *)values, nnz);
-  MFP_HIP(hipGetLastError());
-  MFP_HIP(hipStreamSynchronize(s));
-  cleanup();
-  return MFP_OK;
+    return csr_from_triplets_t(rows, cols, nnz, tr_rows, tr_cols, tr_vals, row_ptr, columns, (float *)values, s);
+  return csr_from_triplets_t(rows, cols, nnz, tr_rows, tr_cols, tr_vals, row_ptr, columns, (double *)values, s);
 }
 
 // ---------------------------------------------------------------------------
@@ -425,8 +587,8 @@ int ell_build_device(int dtype, uint32_t rows, const uint32_t *rp, const uint32_
 
 // ---------------------------------------------------------------------------
 // COO (common/matrix_converter.cpp:211-280): CSR order, entries whose in-row
-// offset is >= element_start.  Element-parallel with a binary search for the
-// row of each CSR element.
+// offset is >= element_start.  Element-parallel, the rows of a tile of CSR
+// elements found together.
 // ---------------------------------------------------------------------------
 __global__ void k_tail_counts(uint32_t rows, const uint32_t *__restrict__ rp, uint32_t e0,
                               uint32_t *__restrict__ cnt)
@@ -437,34 +599,119 @@ __global__ void k_tail_counts(uint32_t rows, const uint32_t *__restrict__ rp, ui
   cnt[r] = len > e0 ? len - e0 : 0u;
 }
 
-__device__ __forceinline__ uint32_t row_of(const uint32_t *__restrict__ rp, uint32_t rows, uint32_t e)
+// Rows of a tile of ROWS_TILE consecutive entries.  Two waves find the tile's
+// first and last row with a 64-way search (one load per step where a binary
+// search takes six), each row's number goes to its first entry in LDS, and a
+// running maximum gives every entry its row.  A tile that spans far more rows
+// than entries (long runs of empty rows) searches per entry instead.
+constexpr uint32_t ROWS_T = 256, ROWS_I = 8, ROWS_TILE = ROWS_T * ROWS_I;
+
+// largest r with rp[r] <= e, by one wave (every lane gets it); rp[0] <= e < rp[rows]
+__device__ __forceinline__ uint32_t wave_row_of(const uint32_t *__restrict__ rp, uint32_t rows, uint32_t e)
 {
-  // largest r with rp[r] <= e (and rp[r+1] > e)
-  uint32_t lo = 0, hi = rows; // invariant: rp[lo] <= e < rp[hi]
+  const uint32_t lane = threadIdx.x & 63u;
+  uint32_t lo = 0, hi = rows; // rp[lo] <= e < rp[hi]
   while (hi - lo > 1) {
-    const uint32_t mid = lo + (hi - lo) / 2;
-    if (rp[mid] <= e)
-      lo = mid;
-    else
-      hi = mid;
+    const uint32_t step = (hi - lo + 63u) / 64u; // >= 1
+    const uint64_t at = (uint64_t)lo + (uint64_t)step * lane;
+    const bool below = at < hi && rp[at] <= e; // lane 0: true
+    const uint32_t k = (uint32_t)__popcll(__ballot(below)) - 1u; // a prefix of the lanes
+    const uint32_t next = lo + step * k;
+    hi = (uint32_t)min((uint64_t)hi, (uint64_t)next + step);
+    lo = next;
   }
   return lo;
 }
 
-template <typename T>
-__global__ void k_coo_build(uint32_t rows, uint64_t nnz, const uint32_t *__restrict__ rp,
-                            const uint32_t *__restrict__ ci, const T *__restrict__ a,
-                            uint32_t e0, const uint32_t *__restrict__ toff,
-                            T *__restrict__ cv, uint32_t *__restrict__ cc,
-                            uint32_t *__restrict__ cr)
+// row[k] = the row of entry t0 + ROWS_I threadIdx.x + k (entries at or past
+// t1: the row of entry t1 - 1).  t0 < t1 <= t0 + ROWS_TILE; sh_mark holds
+// ROWS_TILE words and sh 8.
+__device__ __forceinline__ void tile_rows(const uint32_t *__restrict__ rp, uint32_t rows, uint32_t t0, uint64_t t1,
+                                          uint32_t *sh_mark, uint32_t *sh, uint32_t (&row)[ROWS_I])
 {
-  uint64_t e = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-  for (; e < nnz; e += stride) {
-    const uint32_t r = row_of(rp, rows, (uint32_t)e);
-    const uint32_t k = (uint32_t)e - rp[r];
-    if (k < e0) continue;
-    const uint32_t o = toff[r] + (k - e0);
+  const uint32_t t = threadIdx.x, lane = t & 63u, wave = t >> 6;
+  const uint32_t m = (uint32_t)(t1 - t0);
+  if (wave < 2) {
+    const uint32_t r = wave_row_of(rp, rows, wave ? t0 + (m - 1u) : t0);
+    if (lane == 0) sh[4 + wave] = r;
+  }
+#pragma unroll
+  for (uint32_t k = 0; k < ROWS_I; k++) sh_mark[k * ROWS_T + t] = 0;
+  __syncthreads();
+  const uint32_t first = sh[4], last = sh[5];
+  if (last - first > 16u * ROWS_TILE) {
+#pragma unroll
+    for (uint32_t k = 0; k < ROWS_I; k++) {
+      const uint32_t e = t0 + min(t * ROWS_I + k, m - 1u);
+      uint32_t lo = first, hi = last + 1;
+      while (hi - lo > 1) {
+        const uint32_t mid = lo + (hi - lo) / 2;
+        if (rp[mid] <= e)
+          lo = mid;
+        else
+          hi = mid;
+      }
+      row[k] = lo;
+    }
+    return;
+  }
+  // rows first + 1 .. last start inside the tile; of rows that start at the
+  // same entry the last holds it
+  for (uint32_t d = 1 + t; d <= last - first; d += ROWS_T) atomicMax(&sh_mark[rp[first + d] - t0], d);
+  __syncthreads();
+  uint32_t mx = 0;
+#pragma unroll
+  for (uint32_t k = 0; k < ROWS_I; k++) {
+    mx = max(mx, sh_mark[t * ROWS_I + k]);
+    row[k] = mx;
+  }
+  uint32_t x = mx;
+#pragma unroll
+  for (uint32_t d = 1; d < 64; d <<= 1) {
+    const uint32_t y = __shfl_up(x, d, 64);
+    if (lane >= d) x = max(x, y);
+  }
+  if (lane == 63) sh[wave] = x;
+  uint32_t pre = __shfl_up(x, 1, 64);
+  if (lane == 0) pre = 0;
+  __syncthreads();
+  for (uint32_t w = 0; w < wave; w++) pre = max(pre, sh[w]);
+#pragma unroll
+  for (uint32_t k = 0; k < ROWS_I; k++) row[k] = first + max(pre, row[k]);
+}
+
+// COO entries from CSR: entry e of row r with in-row offset k >= e0 to
+// position toff[r] + k - e0 (toff null: e0 = 0, position e)
+template <typename T>
+__global__ __launch_bounds__(ROWS_T) void k_coo_build(uint32_t rows, uint64_t nnz, const uint32_t *__restrict__ rp,
+                                                      const uint32_t *__restrict__ ci, const T *__restrict__ a,
+                                                      uint32_t e0, const uint32_t *__restrict__ toff,
+                                                      T *__restrict__ cv, uint32_t *__restrict__ cc,
+                                                      uint32_t *__restrict__ cr)
+{
+  __shared__ uint32_t mark[ROWS_TILE];
+  __shared__ uint32_t sh[8];
+  const uint32_t t0 = blockIdx.x * ROWS_TILE, t = threadIdx.x;
+  const uint64_t t1 = min(nnz, (uint64_t)t0 + ROWS_TILE);
+  uint32_t row[ROWS_I];
+  tile_rows(rp, rows, t0, t1, mark, sh, row);
+  __syncthreads();
+  // through LDS, so that neighbouring lanes handle neighbouring entries
+#pragma unroll
+  for (uint32_t k = 0; k < ROWS_I; k++) mark[t * ROWS_I + k] = row[k];
+  __syncthreads();
+#pragma unroll
+  for (uint32_t k = 0; k < ROWS_I; k++) {
+    const uint32_t l = k * ROWS_T + t;
+    const uint64_t e = (uint64_t)t0 + l;
+    if (e >= t1) break;
+    const uint32_t r = mark[l];
+    uint64_t o = e;
+    if (toff) {
+      const uint32_t in = (uint32_t)e - rp[r];
+      if (in < e0) continue;
+      o = toff[r] + (in - e0);
+    }
     cv[o] = a[e];
     cc[o] = ci[e];
     cr[o] = r;
@@ -478,38 +725,33 @@ int coo_tail_build_device(int dtype, uint32_t rows, uint64_t nnz, const uint32_t
   *cv = nullptr;
   *cc = nullptr;
   *cr = nullptr;
+  device_temps tmp;
   uint32_t *toff = nullptr;
-  MFP_CHECK(dmalloc((void **)&toff, ((uint64_t)rows + 1) * 4));
-  uint32_t total = 0;
-  if (rows) {
-    k_tail_counts<<<ceil_div_u32(rows, 256), 256, 0, s>>>(rows, rp, e0, toff);
-    MFP_HIP(hipGetLastError());
-  }
-  int st = exclusive_scan_u32(toff, toff, rows, s, &total);
-  if (st != MFP_OK) {
-    dfree(toff);
-    return st;
+  uint32_t total = (uint32_t)nnz;
+  if (e0) { // e0 = 0 takes every entry, in place
+    MFP_CHECK(tmp.alloc((void **)&toff, ((uint64_t)rows + 1) * 4));
+    if (rows) {
+      k_tail_counts<<<ceil_div_u32(rows, 256), 256, 0, s>>>(rows, rp, e0, toff);
+      MFP_HIP(hipGetLastError());
+    }
+    MFP_CHECK(exclusive_scan_u32(toff, toff, rows, s, &total));
   }
   *count = total;
   const size_t vs = dtype_size(dtype);
-  st = dmalloc(cv, (uint64_t)total * vs);
-  if (st == MFP_OK) st = dmalloc((void **)cc, (uint64_t)total * 4);
-  if (st == MFP_OK) st = dmalloc((void **)cr, (uint64_t)total * 4);
-  if (st != MFP_OK) {
-    dfree(toff);
-    return st;
-  }
+  MFP_CHECK(dmalloc(cv, (uint64_t)total * vs));
+  MFP_CHECK(dmalloc((void **)cc, (uint64_t)total * 4));
+  MFP_CHECK(dmalloc((void **)cr, (uint64_t)total * 4));
   if (total) {
+    const uint32_t g = ceil_div_u32(nnz, ROWS_TILE);
     if (dtype == MFP_F32)
-      k_coo_build<float><<<grid_for(nnz), 256, 0, s>>>(rows, nnz, rp, ci, (const float *)val, e0,
-                                                       toff, (float *)*cv, *cc, *cr);
+      k_coo_build<float><<<g, ROWS_T, 0, s>>>(rows, nnz, rp, ci, (const float *)val, e0, toff, (float *)*cv, *cc,
+                                              *cr);
     else
-      k_coo_build<double><<<grid_for(nnz), 256, 0, s>>>(rows, nnz, rp, ci, (const double *)val,
-                                                        e0, toff, (double *)*cv, *cc, *cr);
+      k_coo_build<double><<<g, ROWS_T, 0, s>>>(rows, nnz, rp, ci, (const double *)val, e0, toff, (double *)*cv, *cc,
+                                               *cr);
     MFP_HIP(hipGetLastError());
   }
   MFP_HIP(hipStreamSynchronize(s));
-  dfree(toff);
   return MFP_OK;
 }
 
@@ -569,23 +811,31 @@ __global__ void k_long_mask(uint32_t rows, const uint32_t *__restrict__ flag, ui
   mask[w] = m;
 }
 
-__global__ void k_entry_slice(uint32_t rows, uint64_t nnz, const uint32_t *__restrict__ rp, uint32_t R,
-                              uint32_t rbits, uint32_t S_reg, const uint32_t *__restrict__ flag,
-                              const uint32_t *__restrict__ rank, uint32_t *__restrict__ slice,
-                              uint32_t *__restrict__ lrow)
+// vrow[e] = the slot of entry e's row among S R slice rows: slice R + local
+// row, a long row's in the long-row slices
+__global__ __launch_bounds__(ROWS_T) void k_entry_vrow(uint32_t rows, uint64_t nnz, const uint32_t *__restrict__ rp,
+                                                       uint32_t long0, const uint32_t *__restrict__ mask,
+                                                       const uint32_t *__restrict__ rank, uint32_t *__restrict__ vrow)
 {
-  uint64_t e = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-  for (; e < nnz; e += stride) {
-    const uint32_t r = row_of(rp, rows, (uint32_t)e);
-    if (flag && flag[r]) {
-      const uint32_t j = rank[r];
-      slice[e] = S_reg + (j >> rbits);
-      lrow[e] = j & (R - 1u);
-    } else {
-      slice[e] = r >> rbits;
-      lrow[e] = r & (R - 1u);
-    }
+  __shared__ __align__(16) uint32_t mark[ROWS_TILE];
+  __shared__ uint32_t sh[8];
+  const uint32_t t0 = blockIdx.x * ROWS_TILE, t = threadIdx.x;
+  const uint64_t t1 = min(nnz, (uint64_t)t0 + ROWS_TILE);
+  uint32_t row[ROWS_I];
+  tile_rows(rp, rows, t0, t1, mark, sh, row);
+  if (mask) {
+#pragma unroll
+    for (uint32_t k = 0; k < ROWS_I; k++)
+      if ((mask[row[k] >> 5] >> (row[k] & 31u)) & 1u) row[k] = long0 + rank[row[k]];
+  }
+  __syncthreads();
+#pragma unroll
+  for (uint32_t k = 0; k < ROWS_I; k++) mark[t * ROWS_I + k] = row[k];
+  __syncthreads();
+#pragma unroll
+  for (uint32_t k = 0; k < ROWS_I; k++) {
+    const uint32_t l = k * ROWS_T + t;
+    if (t0 + (uint64_t)l < t1) vrow[t0 + (uint64_t)l] = mark[l];
   }
 }
 
@@ -610,7 +860,7 @@ __global__ void k_band_bounds(uint32_t S, uint32_t nb, uint64_t W, const uint32_
   bb[t] = lo;
 }
 
-__global__ void k_slice_bounds(uint32_t S, uint64_t nnz, const uint32_t *__restrict__ slice_sorted,
+__global__ void k_slice_bounds(uint32_t S, uint64_t nnz, const uint32_t *__restrict__ vrow_sorted, uint32_t rbits,
                                uint32_t *__restrict__ sp)
 {
   const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
@@ -618,7 +868,7 @@ __global__ void k_slice_bounds(uint32_t S, uint64_t nnz, const uint32_t *__restr
   uint64_t lo = 0, hi = nnz;
   while (lo < hi) {
     const uint64_t mid = (lo + hi) / 2;
-    if (slice_sorted[mid] < s)
+    if ((vrow_sorted[mid] >> rbits) < s)
       lo = mid + 1;
     else
       hi = mid;
@@ -650,50 +900,74 @@ __global__ void k_item_base(uint32_t NI, const uint4 *__restrict__ items, const 
   }
 }
 
+// Sorted entries to their words.  A workgroup takes 1024 positions, in order;
+// the item holding its first one is searched once, later ones by advancing.
 template <typename T>
-__global__ void k_cs_scatter(uint64_t nnz, const uint32_t *__restrict__ perm, const uint32_t *__restrict__ col,
-                             const uint32_t *__restrict__ lrow, const T *__restrict__ a, uint32_t NI,
-                             const uint4 *__restrict__ items, const uint32_t *__restrict__ base, uint32_t rbits,
-                             T *__restrict__ ev, uint32_t *__restrict__ ec)
+__global__ __launch_bounds__(256) void k_cs_place(uint64_t nnz, const uint32_t *__restrict__ vrow,
+                                                  const uint32_t *__restrict__ col, const T *__restrict__ a, uint32_t NI,
+                                                  const uint4 *__restrict__ items, const uint32_t *__restrict__ base,
+                                                  uint32_t rbits, T *__restrict__ ev, uint32_t *__restrict__ ec)
 {
-  uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-  for (; i < nnz; i += stride) {
-    const uint32_t src = perm[i];
-    const uint32_t c = col[i];
-    // the item holding sorted position i: last item with e0 <= i (items
-    // are in position order and cover every position)
-    uint32_t lo = 0, hi = NI;
-    while (hi - lo > 1) {
-      const uint32_t mid = lo + (hi - lo) / 2;
-      if (items[mid].y <= i)
-        lo = mid;
-      else
-        hi = mid;
+  const uint64_t p0 = (uint64_t)blockIdx.x * 1024u;
+  // the last item with e0 <= p0 (items are in position order and cover every
+  // position; of empty items at one position the last comes out, and the
+  // position then belongs to it or to a later one)
+  uint32_t lo = 0, hi = NI;
+  while (hi - lo > 1) {
+    const uint32_t mid = lo + (hi - lo) / 2;
+    if (items[mid].y <= p0)
+      lo = mid;
+    else
+      hi = mid;
+  }
+  uint32_t e0 = items[lo].y, e1 = items[lo].z;
+#pragma unroll
+  for (uint32_t k = 0; k < 4; k++) {
+    const uint64_t i = p0 + k * 256u + threadIdx.x;
+    if (i >= nnz) return;
+    while (i >= e1) {
+      lo++;
+      e0 = items[lo].y;
+      e1 = items[lo].z;
     }
+    const uint32_t c = col[i], w = ((c - base[lo]) << rbits) | (vrow[i] & ((1u << rbits) - 1u));
     // inside an aligned block of 256 positions that lies wholly in one
     // item, position 64 j + l goes to word l, slot j: lane l's 16-byte word
     // then holds the block's positions l, 64 + l, 128 + l and 192 + l, so
     // each of the wave's four gathers reads 64 consecutive columns
     const uint64_t b0 = i & ~(uint64_t)255;
-    const bool in_block = b0 >= items[lo].y && b0 + 256 <= items[lo].z;
+    const bool in_block = b0 >= e0 && b0 + 256 <= e1;
     const uint64_t d = in_block ? b0 + 4 * (i & 63) + ((i >> 6) & 3) : i;
     // FP64 values of such a block: slots 0 and 1 of its 64 words first, as
     // 64 consecutive 16-byte pairs, then slots 2 and 3, so that each 16-byte
     // value load of a wave reads 1 KiB contiguous
     const uint64_t dv = sizeof(T) == 8 && in_block ? b0 + (((i >> 7) & 1) << 7) + 2 * (i & 63) + ((i >> 6) & 1) : d;
-    ev[dv] = a[src];
-    ec[d] = ((c - base[lo]) << rbits) | lrow[src];
+    ev[dv] = a[i];
+    ec[d] = w;
   }
 }
 
+// Entries of the CSR matrix sorted by (slice, column), stably: vrow, columns
+// and values into `to`.
 template <typename T>
-static int cs_scatter_t(uint64_t nnz, const uint32_t *perm, const uint32_t *col, const uint32_t *lrow,
-                        const void *a, uint32_t NI, const uint4 *items, const uint32_t *base, uint32_t rbits,
-                        void *ev, uint32_t *ec, hipStream_t s)
+static int cs_sort_t(uint32_t rows, uint32_t cols, uint64_t nnz, const uint32_t *rp, const uint32_t *ci, const void *val,
+                     uint32_t rbits, uint32_t S_reg, uint32_t S, const uint32_t *mask, const uint32_t *rank,
+                     const sort_arrays<T> &to, const sort_arrays<T> &via, hipStream_t s)
 {
-  k_cs_scatter<T><<<grid_for(nnz), 256, 0, s>>>(nnz, perm, col, lrow, (const T *)a, NI, items, base, rbits,
-                                                (T *)ev, ec);
+  // the first pass reads the rows from the side that it does not write
+  const uint32_t bits = (cols ? bit_length(cols - 1) : 0) + (S ? bit_length(S - 1) : 0);
+  uint32_t *vrow = std::max(1u, (bits + 7) / 8) % 2 ? via.row : to.row;
+  k_entry_vrow<<<ceil_div_u32(nnz, ROWS_TILE), ROWS_T, 0, s>>>(rows, nnz, rp, S_reg << rbits, mask, rank, vrow);
+  MFP_HIP(hipGetLastError());
+  return sort_entries(vrow, ci, (const T *)val, nnz, rbits, S, 0, cols, to, via, nullptr, s);
+}
+
+template <typename T>
+static int cs_place_t(uint64_t nnz, const void *sorted_row, const void *sorted_col, const void *sorted_val, uint32_t NI,
+                      const uint4 *items, const uint32_t *base, uint32_t rbits, void *ev, uint32_t *ec, hipStream_t s)
+{
+  k_cs_place<T><<<ceil_div_u32(nnz, 1024), 256, 0, s>>>(nnz, (const uint32_t *)sorted_row, (const uint32_t *)sorted_col,
+                                                        (const T *)sorted_val, NI, items, base, rbits, (T *)ev, ec);
   MFP_HIP(hipGetLastError());
   return MFP_OK;
 }
@@ -739,6 +1013,8 @@ int scoo_cs_build_device(int dtype, uint32_t rows, uint32_t cols, uint64_t nnz, 
     st = exclusive_scan_u32(flag, rank, rows, s, &NL);
     if (st != MFP_OK) return done(st);
   }
+  // the rows of all slices are numbered in 32 bits
+  if (((uint64_t)S_reg + ((uint64_t)NL + R - 1) / R) << rbits > 1ull << 32) NL = 0;
   out->NL = NL;
   out->S_long = (uint32_t)(((uint64_t)NL + R - 1) / R);
   const uint32_t S = S_reg + out->S_long;
@@ -752,40 +1028,28 @@ int scoo_cs_build_device(int dtype, uint32_t rows, uint32_t cols, uint64_t nnz, 
     k_long_mask<<<ceil_div_u32(((uint64_t)rows + 31) / 32, 256), 256, 0, s>>>(rows, flag, out->long_mask);
     if (hipGetLastError() != hipSuccess) return done(MFP_ERR_HIP);
   }
-  // (slice, column, source entry) sorted by column, then stably by slice
-  uint32_t *buf[7] = {};
-  for (int i = 0; i < 7 && st == MFP_OK; i++) st = scratch((void **)&buf[i], nnz * 4);
-  const uint32_t ntiles = (uint32_t)((nnz + RX_TILE - 1) / RX_TILE);
-  uint32_t *hist = nullptr, *span = nullptr;
-  if (st == MFP_OK) st = scratch((void **)&hist, (uint64_t)std::max<uint32_t>(ntiles, 1) * 256 * 4);
+  // the entries sorted by (slice, column), through the plan's own arrays
+  st = dmalloc(&out->ev, std::max<uint64_t>(nnz, 1) * vs);
+  if (st == MFP_OK) st = dmalloc((void **)&out->ec, std::max<uint64_t>(nnz, 1) * 4);
+  uint32_t *span = nullptr, *srow = nullptr, *scol = nullptr, *vrow = nullptr;
+  void *sval = nullptr;
   if (st == MFP_OK) st = scratch((void **)&span, 4);
+  if (st == MFP_OK) st = scratch((void **)&srow, nnz * 4);
+  if (st == MFP_OK) st = scratch((void **)&scol, nnz * 4);
+  if (st == MFP_OK) st = scratch(&sval, nnz * vs);
+  if (st == MFP_OK) st = scratch((void **)&vrow, nnz * 4);
   if (st != MFP_OK) return done(st);
-  uint32_t *lrow = buf[6];
-  uint32_t *cur[3] = {buf[0], buf[1], buf[2]};
-  uint32_t *nxt[3] = {buf[3], buf[4], buf[5]};
   if (nnz) {
-    k_entry_slice<<<grid_for(nnz), 256, 0, s>>>(rows, nnz, rp, R, rbits, S_reg, NL ? flag : nullptr, rank, buf[0],
-                                                 lrow);
-    if (hipGetLastError() != hipSuccess) return done(MFP_ERR_HIP);
-    if (hipMemcpyAsync(buf[1], ci, nnz * 4, hipMemcpyDeviceToDevice, s) != hipSuccess) return done(MFP_ERR_HIP);
-    k_iota<<<grid_for(nnz), 256, 0, s>>>(buf[2], nnz);
-    if (hipGetLastError() != hipSuccess) return done(MFP_ERR_HIP);
-    std::vector<std::pair<int, uint32_t>> passes;
-    for (uint32_t sh = 0; sh < bit_length(cols ? cols - 1 : 0); sh += 8) passes.push_back({1, sh});
-    for (uint32_t sh = 0; sh < bit_length(S ? S - 1 : 0); sh += 8) passes.push_back({0, sh});
-    for (auto [which, sh] : passes) {
-      k_radix_hist<<<ntiles, RX_T, 0, s>>>(cur[which], nnz, sh, hist, ntiles);
-      if (hipGetLastError() != hipSuccess) return done(MFP_ERR_HIP);
-      st = exclusive_scan_u32(hist, hist, (uint64_t)ntiles * 256, s, nullptr);
-      if (st != MFP_OK) return done(st);
-      k_radix_scatter<<<ntiles, RX_T, 0, s>>>(cur[which], cur[0], cur[1], cur[2], nxt[0], nxt[1], nxt[2], nnz, sh,
-                                               hist, ntiles);
-      if (hipGetLastError() != hipSuccess) return done(MFP_ERR_HIP);
-      std::swap(cur, nxt);
-    }
+    auto sort = [&](auto tv) {
+      using T = decltype(tv);
+      return cs_sort_t<T>(rows, cols, nnz, rp, ci, val, rbits, S_reg, S, NL ? out->long_mask : nullptr, rank,
+                          sort_arrays<T>{srow, scol, (T *)sval}, sort_arrays<T>{vrow, out->ec, (T *)out->ev}, s);
+    };
+    st = vs == 2 ? sort(uint16_t()) : vs == 4 ? sort(uint32_t()) : sort(uint64_t());
+    if (st != MFP_OK) return done(st);
   }
   // slice boundaries, then work items on the host
-  k_slice_bounds<<<ceil_div_u32((uint64_t)S + 1, 256), 256, 0, s>>>(S, nnz, cur[0], out->sp);
+  k_slice_bounds<<<ceil_div_u32((uint64_t)S + 1, 256), 256, 0, s>>>(S, nnz, srow, rbits, out->sp);
   if (hipGetLastError() != hipSuccess) return done(MFP_ERR_HIP);
   std::vector<uint32_t> hsp((size_t)S + 1);
   if (hipMemcpyAsync(hsp.data(), out->sp, hsp.size() * 4, hipMemcpyDeviceToHost, s) != hipSuccess ||
@@ -805,9 +1069,9 @@ int scoo_cs_build_device(int dtype, uint32_t rows, uint32_t cols, uint64_t nnz, 
     st = scratch((void **)&bb, hbb.size() * 4);
     if (st == MFP_OK) st = scratch((void **)&sspan, (uint64_t)S * 4);
     if (st != MFP_OK) return done(st);
-    k_band_bounds<<<ceil_div_u32(hbb.size(), 256), 256, 0, s>>>(S, nb, W, out->sp, cur[1], bb);
+    k_band_bounds<<<ceil_div_u32(hbb.size(), 256), 256, 0, s>>>(S, nb, W, out->sp, scol, bb);
     if (hipGetLastError() != hipSuccess) return done(MFP_ERR_HIP);
-    k_slice_span<<<ceil_div_u32(S, 256), 256, 0, s>>>(S, out->sp, cur[1], sspan);
+    k_slice_span<<<ceil_div_u32(S, 256), 256, 0, s>>>(S, out->sp, scol, sspan);
     if (hipGetLastError() != hipSuccess ||
         hipMemcpyAsync(hbb.data(), bb, hbb.size() * 4, hipMemcpyDeviceToHost, s) != hipSuccess ||
         hipMemcpyAsync(slice_span.data(), sspan, (size_t)S * 4, hipMemcpyDeviceToHost, s) != hipSuccess ||
@@ -872,8 +1136,6 @@ int scoo_cs_build_device(int dtype, uint32_t rows, uint32_t cols, uint64_t nnz, 
   if (dtype == MFP_F32 || dtype == MFP_F64)
     while (out->kmax < 16 && (uint64_t)R * out->kmax * 2 * 8 <= 163840) out->kmax *= 2;
   if (st == MFP_OK && slots && own_partials) st = dmalloc(&out->partial, (uint64_t)slots * R * out->kmax * ps);
-  if (st == MFP_OK) st = dmalloc(&out->ev, std::max<uint64_t>(nnz, 1) * vs);
-  if (st == MFP_OK) st = dmalloc((void **)&out->ec, std::max<uint64_t>(nnz, 1) * 4);
   if (st != MFP_OK) return done(st);
   if (!items.empty() &&
       hipMemcpyAsync(out->items, items.data(), items.size() * sizeof(uint4), hipMemcpyHostToDevice, s) != hipSuccess)
@@ -884,7 +1146,7 @@ int scoo_cs_build_device(int dtype, uint32_t rows, uint32_t cols, uint64_t nnz, 
   st = fill_u32(span, 0, 1, s);
   if (st != MFP_OK) return done(st);
   if (out->NI) {
-    k_item_base<<<ceil_div_u32(out->NI, 256), 256, 0, s>>>(out->NI, out->items, cur[1], out->base, span);
+    k_item_base<<<ceil_div_u32(out->NI, 256), 256, 0, s>>>(out->NI, out->items, scol, out->base, span);
     if (hipGetLastError() != hipSuccess) return done(MFP_ERR_HIP);
   }
   uint32_t hspan = 0;
@@ -896,8 +1158,8 @@ int scoo_cs_build_device(int dtype, uint32_t rows, uint32_t cols, uint64_t nnz, 
     return done(MFP_ERR_STATE);
   }
   if (nnz) {
-    st = (dtype == MFP_F32 ? cs_scatter_t<float> : dtype == MFP_F64 ? cs_scatter_t<double> : cs_scatter_t<uint16_t>)(
-        nnz, cur[2], cur[1], lrow, val, out->NI, out->items, out->base, rbits, out->ev, out->ec, s);
+    st = (vs == 2 ? cs_place_t<uint16_t> : vs == 4 ? cs_place_t<uint32_t> : cs_place_t<uint64_t>)(
+        nnz, srow, scol, sval, out->NI, out->items, out->base, rbits, out->ev, out->ec, s);
     if (st != MFP_OK) return done(st);
   }
   if (hipStreamSynchronize(s) != hipSuccess) {
@@ -907,7 +1169,7 @@ int scoo_cs_build_device(int dtype, uint32_t rows, uint32_t cols, uint64_t nnz, 
   // Launch order: piece k of n covers about columns [k/n, (k+1)/n) of its
   // slice, so ordering the items by the centre of that band (then by slice)
   // gives each XCD's contiguous range of items one band of x for its L2.
-  // The scatter above needed the items in entry order; the kernel does not.
+  // The placement above needed the items in entry order; the kernel does not.
   if (out->NI > 1) {
     std::vector<uint32_t> hbase(out->NI);
     if (hipMemcpyAsync(hbase.data(), out->base, (size_t)out->NI * 4, hipMemcpyDeviceToHost, s) != hipSuccess ||
@@ -1050,26 +1312,6 @@ __global__ void k_compact(uint32_t rows, const uint32_t *__restrict__ mark,
 }
 
 __global__ void k_store1(uint32_t *p, uint32_t v) { *p = v; }
-
-// Device allocations freed on every return path unless released.
-struct device_temps {
-  std::vector<void *> held;
-  int alloc(void **p, size_t bytes)
-  {
-    const int st = dmalloc(p, bytes);
-    if (st == MFP_OK) held.push_back(*p);
-    return st;
-  }
-  void release(void *p)
-  {
-    for (void *&q : held)
-      if (q == p) q = nullptr;
-  }
-  ~device_temps()
-  {
-    for (void *q : held) dfree(q);
-  }
-};
 
 int row_blocks_device(uint32_t rows, const uint32_t *rp, uint32_t W, uint32_t **blocks_out,
                       uint32_t *count_out, hipStream_t s)

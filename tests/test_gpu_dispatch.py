@@ -99,3 +99,88 @@ def test_free_memory_counts_kept_blocks(gpu):
     gpu.Plan(A, "ell").destroy()
     A.destroy()
     assert abs(gpu.device_info()["free_mem"] - free) < 64 << 20
+# ---- converters ---------------------------------------------------------------
+# Tiles of the sort hold 2,048 entries below 4,194,304 of them, then 8,192
+# (FP64 4,096); digits have 1 to 8 bits; tiles of entry rows hold 2,048.
+
+def _triplets(rows, cols, n, seed, dup):
+    rng = np.random.default_rng(seed)
+    r = rng.integers(0, rows, n).astype(np.uint32)
+    c = rng.integers(0, cols, n).astype(np.uint32)
+    if dup:  # equal (row, column) pairs keep their input order
+        r, c = r // np.uint32(dup) * np.uint32(dup), c // np.uint32(dup) * np.uint32(dup)
+    return r, c, rng.uniform(-1, 1, n)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("rows,cols,n,dup", [
+    (1, 1, 1, 0), (1, 1, 3000, 0), (3, 2, 2047, 0), (257, 256, 2048, 0), (256, 257, 2049, 0), (65537, 1, 5000, 0),
+    (1, 100000, 6001, 0), (1000003, 1000003, 70001, 0), (4294967295 // 64, 4294967295, 4097, 0),
+    (50000, 50000, (1 << 22) - 1, 50), (50000, 300, 1 << 22, 0), (1 << 20, 1 << 20, (1 << 22) + 8193, 7)])
+def test_triplets_any_size(gpu, rows, cols, n, dup, dtype):
+    announce(f"triplets rows={rows} cols={cols} n={n} dup={dup} dtype={dtype}")
+    r, c, v = _triplets(rows, cols, n, n % 97, dup)
+    A = gpu.DeviceMatrix.from_triplets(rows, cols, r, c, v, np.dtype(dtype))
+    rp, ci, va = A.download()
+    A.destroy()
+    order = np.lexsort((c, r))  # stable: ties in input order
+    assert np.array_equal(rp, np.searchsorted(r[order], np.arange(rows + 1, dtype=np.int64)).astype(np.uint32))
+    assert np.array_equal(ci, c[order])
+    assert np.array_equal(va, v[order].astype(dtype))
+
+
+@pytest.mark.parametrize("where", ["row", "column"])
+def test_triplets_out_of_range_are_refused(gpu, where):
+    r, c, v = _triplets(1000, 1000, 9001, 3, 0)
+    (r if where == "row" else c)[8999] = 1000
+    with pytest.raises(gpu.MfpError):
+        gpu.DeviceMatrix.from_triplets(1000, 1000, r, c, v)
+
+
+ENTRY_ROWS = {
+    "tile edges": [2047, 1, 0, 2048, 0, 0, 2049, 1, 2046] + [3] * 4000,
+    "empty runs": [0] * 40000 + [1] + [0] * 50000 + [1, 2, 3] + [0] * 33000,
+    "one row": [5000],
+    "all ones": [1] * 4099,
+}
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("width", [0, 2])
+@pytest.mark.parametrize("rows", list(ENTRY_ROWS))
+def test_coo_entries_and_tails(gpu, rows, width, dtype):
+    rp, ci, va = _csr(ENTRY_ROWS[rows], 7001, dtype)
+    announce(f"coo build {rows} width={width} dtype={dtype}")
+    A = gpu.DeviceMatrix.from_csr(rp, ci, va, 7001)
+    plan = gpu.Plan(A, "hyb", hyb_width=width) if width else gpu.Plan(A, "coo")
+    row = np.repeat(np.arange(rp.size - 1), np.diff(rp.astype(np.int64)))
+    tail = np.arange(ci.size) - rp[row] >= width
+    from matrix_format_performance_amd import _lib as L
+    assert np.array_equal(plan.array(L.MFP_ARR_COO_ROWS, np.uint32), row[tail])
+    assert np.array_equal(plan.array(L.MFP_ARR_COO_COLS, np.uint32), ci[tail])
+    assert np.array_equal(plan.array(L.MFP_ARR_COO_VALUES, np.dtype(dtype)), va[tail])
+    plan.destroy()
+    A.destroy()
+
+
+@pytest.mark.parametrize("values", ["f32", "f64", "bf16"])
+@pytest.mark.parametrize("rows", list(ENTRY_ROWS))
+def test_column_sorted_build(gpu, rows, values):
+    # slices of 256 rows, long-row slices among them: every entry placed once
+    rp, ci, va = _csr(ENTRY_ROWS[rows], 7001, "float64" if values == "f64" else "float32")
+    va = np.round(va * 64) / 64  # exact in BF16, and their sums exact in FP32
+    x = gpu.generate_vector(5, 7001, va.dtype)
+    x = np.round(x * 64) / 64
+    announce(f"column-sorted build {rows} {values}")
+    from matrix_format_performance_amd import _lib as L
+    A = gpu.DeviceMatrix.from_csr(rp, ci, va.astype(x.dtype), 7001)
+    M = A.convert(values) if values == "bf16" else A
+    plan = gpu.Plan(M, "scoo", flags=L.MFP_TUNE_SCOO_COLSORT, scoo_slice_size=256, scoo_pieces=0)
+    xd, yd = gpu.DeviceArray.from_host(x), gpu.DeviceArray(rp.size - 1, x.dtype)
+    yd.fill(np.nan)
+    plan.spmv(xd, yd)
+    gpu.synchronize()
+    y64, _ = oracle.spmv_f64(rp, ci, va, x)
+    assert np.array_equal(yd.to_host().astype(np.float64), y64)
+    plan.destroy()
+    A.destroy()
