@@ -4,6 +4,7 @@
 // common/scoo_matrix_class.cpp, gpu/csr_adaptive_spmv.cu:180-240).  Here each
 // layout is built by HIP kernels in HBM; the results are bit-identical to the
 // reference's host algorithms (ties in triplets->CSR keep input order).
+#include "entry_rows.h"
 #include "mfp_internal.h"
 #include "wave64.h"
 
@@ -488,63 +489,87 @@ int csr_from_triplets_device(int dtype, uint32_t rows, uint32_t cols, uint64_t n
 // Row statistics (get_rows_statistics, common/matrix_converter.cpp:95-127).
 // min/max/sum exactly; sum of squared deviations from the integer average in
 // u64 (exact; equals the reference's double sum whenever that sum is below
-// 2^53, where every partial double sum is exact).
+// 2^53, where every partial double sum is exact), as sum len^2 - 2 avg sum len
+// + rows avg^2 in the same modular arithmetic.  One pass: a workgroup reduces
+// its rows in registers and LDS and writes one record (300,007 rows: 5 us,
+// where five atomics per lane on one address took 220 + 80 us), the host adds
+// the records.
 // ---------------------------------------------------------------------------
 struct stats_acc {
   uint32_t mn, mx;
   unsigned long long sum, sq;
 };
 
-__global__ void k_row_minmax(const uint32_t *__restrict__ rp, uint32_t rows, stats_acc *acc)
+__device__ __forceinline__ unsigned long long wave_sum_u64(unsigned long long v)
 {
-  uint32_t mn = 0xFFFFFFFFu, mx = 0;
-  unsigned long long sum = 0;
-  uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-  for (; i < rows; i += stride) {
-    uint32_t len = rp[i + 1] - rp[i];
+#pragma unroll
+  for (int d = 32; d >= 1; d >>= 1) v += (unsigned long long)__shfl_xor((long long)v, d, 64);
+  return v;
+}
+
+constexpr uint32_t STATS_GRID = 512;
+
+__global__ __launch_bounds__(256) void k_row_stats(const uint32_t *__restrict__ rp, uint32_t rows,
+                                                   stats_acc *__restrict__ out)
+{
+  __shared__ stats_acc part[4];
+  uint32_t mn = 0xFFFFFFFEu, mx = 0; // min starts at UINT_MAX-1 (:98)
+  unsigned long long sum = 0, sq = 0;
+  const uint64_t stride = (uint64_t)gridDim.x * 256u;
+  for (uint64_t i = (uint64_t)blockIdx.x * 256u + threadIdx.x; i < rows; i += stride) {
+    const uint32_t len = rp[i + 1] - rp[i];
     mn = min(mn, len);
     mx = max(mx, len);
     sum += len;
+    sq += (unsigned long long)len * len;
   }
-  atomicMin(&acc->mn, mn);
-  atomicMax(&acc->mx, mx);
-  atomicAdd(&acc->sum, sum);
-}
-
-__global__ void k_row_sq(const uint32_t *__restrict__ rp, uint32_t rows, stats_acc *acc)
-{
-  const uint32_t avg = rows ? (uint32_t)acc->sum / rows : 0u; // 32-bit sum as the reference
-  unsigned long long sq = 0;
-  uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-  for (; i < rows; i += stride) {
-    long long d = (long long)(rp[i + 1] - rp[i]) - (long long)avg;
-    sq += (unsigned long long)(d * d);
+#pragma unroll
+  for (int d = 32; d >= 1; d >>= 1) {
+    mn = min(mn, (uint32_t)__shfl_xor((int)mn, d, 64));
+    mx = max(mx, (uint32_t)__shfl_xor((int)mx, d, 64));
   }
-  atomicAdd(&acc->sq, sq);
+  sum = wave_sum_u64(sum);
+  sq = wave_sum_u64(sq);
+  if ((threadIdx.x & 63u) == 0) part[threadIdx.x >> 6] = stats_acc{mn, mx, sum, sq};
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    stats_acc a = part[0];
+    for (int w = 1; w < 4; w++) {
+      a.mn = min(a.mn, part[w].mn);
+      a.mx = max(a.mx, part[w].mx);
+      a.sum += part[w].sum;
+      a.sq += part[w].sq;
+    }
+    out[blockIdx.x] = a;
+  }
 }
 
 int row_stats_device(uint32_t rows, const uint32_t *rp, mfp_row_stats *out, hipStream_t s)
 {
-  stats_acc init{0xFFFFFFFFu - 1u, 0u, 0ull, 0ull}; // min starts at UINT_MAX-1 (:98)
-  stats_acc *acc = nullptr;
-  MFP_CHECK(dmalloc((void **)&acc, sizeof(stats_acc)));
-  MFP_HIP(hipMemcpyAsync(acc, &init, sizeof(init), hipMemcpyHostToDevice, s));
-  const uint32_t g = std::min<uint32_t>(grid_for(rows), 2048);
+  stats_acc h{0xFFFFFFFEu, 0u, 0ull, 0ull};
   if (rows) {
-    k_row_minmax<<<g, 256, 0, s>>>(rp, rows, acc);
-    k_row_sq<<<g, 256, 0, s>>>(rp, rows, acc);
+    const uint32_t g = std::min<uint32_t>(ceil_div_u32(rows, 256), STATS_GRID);
+    device_temps tmp;
+    stats_acc *acc = nullptr;
+    MFP_CHECK(tmp.alloc((void **)&acc, STATS_GRID * sizeof(stats_acc)));
+    k_row_stats<<<g, 256, 0, s>>>(rp, rows, acc);
     MFP_HIP(hipGetLastError());
+    std::vector<stats_acc> part(g);
+    MFP_HIP(hipMemcpyAsync(part.data(), acc, g * sizeof(stats_acc), hipMemcpyDeviceToHost, s));
+    MFP_HIP(hipStreamSynchronize(s));
+    for (const stats_acc &p : part) {
+      h.mn = std::min(h.mn, p.mn);
+      h.mx = std::max(h.mx, p.mx);
+      h.sum += p.sum;
+      h.sq += p.sq;
+    }
   }
-  stats_acc h{};
-  MFP_HIP(hipMemcpyAsync(&h, acc, sizeof(h), hipMemcpyDeviceToHost, s));
-  MFP_HIP(hipStreamSynchronize(s));
-  dfree(acc);
+  const uint32_t avg = rows ? (uint32_t)h.sum / rows : 0u; // 32-bit sum as the reference
+  const unsigned long long dev = h.sq - 2ull * avg * h.sum + (unsigned long long)rows * avg * avg;
   out->min_elements_in_rows = h.mn;
   out->max_elements_in_rows = h.mx;
-  out->avg_elements_in_rows = rows ? (uint32_t)h.sum / rows : 0u;
-  out->elements_in_rows_std_deviation = rows ? std::sqrt((double)h.sq / rows) : 0.0;
+  out->avg_elements_in_rows = avg;
+  out->elements_in_rows_std_deviation = rows ? std::sqrt((double)dev / rows) : 0.0;
   return MFP_OK;
 }
 
@@ -552,23 +577,42 @@ int row_stats_device(uint32_t rows, const uint32_t *rp, mfp_row_stats *out, hipS
 // ELL (common/matrix_converter.cpp:139-203): data[row + k*rows], pad (0, 0),
 // rows longer than the width truncated.  Every slot is written.
 // ---------------------------------------------------------------------------
+// A workgroup turns 64 rows x 16 slots around in LDS: 16 lanes read a row's
+// 16 entries, then 64 lanes write one slot of 64 rows (5.1M entries, width
+// 64: 69 us with a lane per row reading along its own row).
+constexpr uint32_t ELLB_R = 64, ELLB_S = 16;
+
 template <typename T>
-__global__ void k_ell_build(uint32_t rows, const uint32_t *__restrict__ rp,
-                            const uint32_t *__restrict__ ci, const T *__restrict__ a,
-                            uint32_t width, T *__restrict__ ev, uint32_t *__restrict__ ec)
+__global__ __launch_bounds__(256) void k_ell_build(uint32_t rows, const uint32_t *__restrict__ rp,
+                                                   const uint32_t *__restrict__ ci, const T *__restrict__ a,
+                                                   uint32_t width, T *__restrict__ ev, uint32_t *__restrict__ ec)
 {
-  const uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= rows) return;
-  const uint32_t s = rp[r], len = rp[r + 1] - s;
-  for (uint32_t k = 0; k < width; k++) {
-    const uint64_t o = (uint64_t)r + (uint64_t)k * rows;
-    if (k < len) {
-      ev[o] = a[s + k];
-      ec[o] = ci[s + k];
-    } else {
-      ev[o] = (T)0;
-      ec[o] = 0u;
+  __shared__ T sv[ELLB_R][ELLB_S + 1];
+  __shared__ uint32_t sc[ELLB_R][ELLB_S + 1];
+  __shared__ uint32_t srp[ELLB_R + 1];
+  const uint32_t r0 = blockIdx.x * ELLB_R, t = threadIdx.x;
+  if (t <= ELLB_R) srp[t] = rp[min((uint64_t)r0 + t, (uint64_t)rows)];
+  __syncthreads();
+  for (uint32_t k0 = blockIdx.y * ELLB_S; k0 < width; k0 += gridDim.y * ELLB_S) {
+#pragma unroll
+    for (uint32_t q = 0; q < ELLB_R * ELLB_S / 256; q++) {
+      const uint32_t lr = q * (256 / ELLB_S) + t / ELLB_S, k = k0 + t % ELLB_S;
+      const uint32_t s = srp[lr], len = srp[lr + 1] - s;
+      const bool in = k < len;
+      sv[lr][t % ELLB_S] = in ? a[s + k] : (T)0;
+      sc[lr][t % ELLB_S] = in ? ci[s + k] : 0u;
     }
+    __syncthreads();
+#pragma unroll
+    for (uint32_t q = 0; q < ELLB_R * ELLB_S / 256; q++) {
+      const uint32_t lk = q * (256 / ELLB_R) + t / ELLB_R, lr = t % ELLB_R;
+      if (k0 + lk < width && r0 + lr < rows) {
+        const uint64_t o = (uint64_t)r0 + lr + (uint64_t)(k0 + lk) * rows;
+        ev[o] = sv[lr][lk];
+        ec[o] = sc[lr][lk];
+      }
+    }
+    __syncthreads();
   }
 }
 
@@ -576,7 +620,7 @@ int ell_build_device(int dtype, uint32_t rows, const uint32_t *rp, const uint32_
                      const void *val, uint32_t width, void *ev, uint32_t *ec, hipStream_t s)
 {
   if (rows == 0 || width == 0) return MFP_OK;
-  const uint32_t g = ceil_div_u32(rows, 256);
+  const dim3 g(ceil_div_u32(rows, ELLB_R), std::min(ceil_div_u32(width, ELLB_S), 1024u));
   if (dtype == MFP_F32)
     k_ell_build<float><<<g, 256, 0, s>>>(rows, rp, ci, (const float *)val, width, (float *)ev, ec);
   else
@@ -597,87 +641,6 @@ __global__ void k_tail_counts(uint32_t rows, const uint32_t *__restrict__ rp, ui
   if (r >= rows) return;
   const uint32_t len = rp[r + 1] - rp[r];
   cnt[r] = len > e0 ? len - e0 : 0u;
-}
-
-// Rows of a tile of ROWS_TILE consecutive entries.  Two waves find the tile's
-// first and last row with a 64-way search (one load per step where a binary
-// search takes six), each row's number goes to its first entry in LDS, and a
-// running maximum gives every entry its row.  A tile that spans far more rows
-// than entries (long runs of empty rows) searches per entry instead.
-constexpr uint32_t ROWS_T = 256, ROWS_I = 8, ROWS_TILE = ROWS_T * ROWS_I;
-
-// largest r with rp[r] <= e, by one wave (every lane gets it); rp[0] <= e < rp[rows]
-__device__ __forceinline__ uint32_t wave_row_of(const uint32_t *__restrict__ rp, uint32_t rows, uint32_t e)
-{
-  const uint32_t lane = threadIdx.x & 63u;
-  uint32_t lo = 0, hi = rows; // rp[lo] <= e < rp[hi]
-  while (hi - lo > 1) {
-    const uint32_t step = (hi - lo + 63u) / 64u; // >= 1
-    const uint64_t at = (uint64_t)lo + (uint64_t)step * lane;
-    const bool below = at < hi && rp[at] <= e; // lane 0: true
-    const uint32_t k = (uint32_t)__popcll(__ballot(below)) - 1u; // a prefix of the lanes
-    const uint32_t next = lo + step * k;
-    hi = (uint32_t)min((uint64_t)hi, (uint64_t)next + step);
-    lo = next;
-  }
-  return lo;
-}
-
-// row[k] = the row of entry t0 + ROWS_I threadIdx.x + k (entries at or past
-// t1: the row of entry t1 - 1).  t0 < t1 <= t0 + ROWS_TILE; sh_mark holds
-// ROWS_TILE words and sh 8.
-__device__ __forceinline__ void tile_rows(const uint32_t *__restrict__ rp, uint32_t rows, uint32_t t0, uint64_t t1,
-                                          uint32_t *sh_mark, uint32_t *sh, uint32_t (&row)[ROWS_I])
-{
-  const uint32_t t = threadIdx.x, lane = t & 63u, wave = t >> 6;
-  const uint32_t m = (uint32_t)(t1 - t0);
-  if (wave < 2) {
-    const uint32_t r = wave_row_of(rp, rows, wave ? t0 + (m - 1u) : t0);
-    if (lane == 0) sh[4 + wave] = r;
-  }
-#pragma unroll
-  for (uint32_t k = 0; k < ROWS_I; k++) sh_mark[k * ROWS_T + t] = 0;
-  __syncthreads();
-  const uint32_t first = sh[4], last = sh[5];
-  if (last - first > 16u * ROWS_TILE) {
-#pragma unroll
-    for (uint32_t k = 0; k < ROWS_I; k++) {
-      const uint32_t e = t0 + min(t * ROWS_I + k, m - 1u);
-      uint32_t lo = first, hi = last + 1;
-      while (hi - lo > 1) {
-        const uint32_t mid = lo + (hi - lo) / 2;
-        if (rp[mid] <= e)
-          lo = mid;
-        else
-          hi = mid;
-      }
-      row[k] = lo;
-    }
-    return;
-  }
-  // rows first + 1 .. last start inside the tile; of rows that start at the
-  // same entry the last holds it
-  for (uint32_t d = 1 + t; d <= last - first; d += ROWS_T) atomicMax(&sh_mark[rp[first + d] - t0], d);
-  __syncthreads();
-  uint32_t mx = 0;
-#pragma unroll
-  for (uint32_t k = 0; k < ROWS_I; k++) {
-    mx = max(mx, sh_mark[t * ROWS_I + k]);
-    row[k] = mx;
-  }
-  uint32_t x = mx;
-#pragma unroll
-  for (uint32_t d = 1; d < 64; d <<= 1) {
-    const uint32_t y = __shfl_up(x, d, 64);
-    if (lane >= d) x = max(x, y);
-  }
-  if (lane == 63) sh[wave] = x;
-  uint32_t pre = __shfl_up(x, 1, 64);
-  if (lane == 0) pre = 0;
-  __syncthreads();
-  for (uint32_t w = 0; w < wave; w++) pre = max(pre, sh[w]);
-#pragma unroll
-  for (uint32_t k = 0; k < ROWS_I; k++) row[k] = first + max(pre, row[k]);
 }
 
 // COO entries from CSR: entry e of row r with in-row offset k >= e0 to
@@ -1255,97 +1218,231 @@ void scoo_cs_free(scoo_cs_layout *l)
 // Row blocks (fill_row_blocks, gpu/csr_adaptive_spmv.cu:180-240) in parallel.
 // The greedy partition is a chain 0 -> close(0) -> ...: close(s) is the row
 // where a block started at s closes (or NONE when the loop ends first), and it
-// depends on s only.  Chain nodes are found by pointer jumping: mark[0] = 1;
-// round k marks J_k(s) for every marked s with J_k = close^(2^k).  Marked
-// nodes in [0, rows] in order, followed by rows, are the reference's output.
+// depends on s only.  The chain's nodes in [0, rows] in order, followed by rows,
+// are the reference's output.
+//   k_close      close(s) of every row, by binary search in the row pointers
+//                (they only grow, so the first row that fills the block can be
+//                searched)
+//   k_seg_exit   a segment of SEG nodes finds, by pointer jumping in LDS,
+//                where a chain from each node leaves the segment
+//   k_seg_chase  one lane follows the chain from segment to segment
+//   k_seg_mark   each segment marks the chain from its entry node, in LDS
+//   k_seg_write  the marked nodes in order
+// Jumping over all nodes in HBM took two launches per doubling, 40 and more
+// in all, and close(s) up to W serial steps per node.
 // ---------------------------------------------------------------------------
-__global__ void k_close(uint32_t rows, const uint32_t *__restrict__ rp, uint32_t W,
-                        uint32_t *__restrict__ J)
+// Segments of 16,384 rows, of 4,096 up to 262,144 rows (more workgroups, and
+// at most 64 steps of the chase).
+constexpr uint32_t SEG_T = 1024;
+constexpr uint32_t NO_NODE = 0xFFFFFFFFu;
+
+// close(s) for s < rows, always above s; rows also where the loop ends first
+__device__ __forceinline__ uint32_t close_of(uint32_t s, uint32_t rows, const uint32_t *__restrict__ rp, uint32_t W)
 {
-  const uint64_t s = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (s > (uint64_t)rows + 1) return;
-  const uint32_t NONE = rows + 1;
-  if (s >= rows) {
-    J[s] = NONE;
-    return;
+  const uint32_t b = rp[s];
+  const uint64_t end = min((uint64_t)rows, (uint64_t)s + W + 1u);
+  uint64_t lo = s, hi = end + 1; // rp[lo] - b < W; hi: first row known to reach W, or end + 1
+  while (hi - lo > 1) {
+    const uint64_t mid = lo + (hi - lo) / 2;
+    if (rp[mid] - b >= W)
+      hi = mid;
+    else
+      lo = mid;
   }
-  uint32_t sum = 0;
-  uint32_t res = NONE;
-  for (uint64_t i = s + 1; i <= rows; i++) {
-    sum += rp[i] - rp[i - 1];
-    if (sum == W) {
-      res = (uint32_t)i;
-      break;
-    }
-    if (sum > W) {
-      res = (i - s > 1) ? (uint32_t)(i - 1) : (uint32_t)i;
-      break;
-    }
-    if (i - s > W) {
-      res = (uint32_t)i;
-      break;
+  // full at row hi: closes there when exactly full or when it holds one row,
+  // else before it; not full: closes at end, after W + 1 rows or with the matrix
+  if (hi <= end) return (uint32_t)(rp[hi] - b == W || hi - s == 1 ? hi : hi - 1);
+  return (uint32_t)end;
+}
+
+__global__ __launch_bounds__(256) void k_close(uint32_t rows, const uint32_t *__restrict__ rp, uint32_t W,
+                                               uint32_t *__restrict__ J)
+{
+  const uint64_t s = (uint64_t)blockIdx.x * 256u + threadIdx.x;
+  if (s < rows) J[s] = close_of((uint32_t)s, rows, rp, W);
+}
+
+// exit[s] = first node of s's chain outside its segment
+template <uint32_t SEG>
+__global__ __launch_bounds__(SEG_T) void k_seg_exit(uint32_t rows, const uint32_t *__restrict__ J,
+                                                    uint32_t *__restrict__ exit, uint32_t *__restrict__ entry)
+{
+  constexpr uint32_t SEG_I = SEG / SEG_T;
+  extern __shared__ uint32_t nxt[]; // SEG
+  const uint32_t s0 = blockIdx.x * SEG, n = min(SEG, rows - s0), t = threadIdx.x;
+  uint32_t v[SEG_I];
+#pragma unroll
+  for (uint32_t k = 0; k < SEG_I; k++) {
+    const uint32_t l = k * SEG_T + t;
+    v[k] = l < n ? J[s0 + l] : NO_NODE;
+    nxt[l] = v[k];
+  }
+  if (t == 0) entry[blockIdx.x] = NO_NODE;
+  for (;;) {
+    __syncthreads();
+    bool moved = false;
+#pragma unroll
+    for (uint32_t k = 0; k < SEG_I; k++)
+      if (v[k] - s0 < n) { // still inside (nodes only grow)
+        v[k] = nxt[v[k] - s0];
+        moved = true;
+      }
+    if (!__syncthreads_or(moved)) break;
+#pragma unroll
+    for (uint32_t k = 0; k < SEG_I; k++) nxt[k * SEG_T + t] = v[k];
+  }
+#pragma unroll
+  for (uint32_t k = 0; k < SEG_I; k++) {
+    const uint32_t l = k * SEG_T + t;
+    if (l < n) exit[s0 + l] = v[k];
+  }
+}
+
+// entry[segment] = the chain's first node in it
+__global__ void k_seg_chase(uint32_t rows, uint32_t seg, const uint32_t *__restrict__ exit, uint32_t *__restrict__ entry)
+{
+  uint32_t node = 0;
+  while (node < rows) {
+    entry[node / seg] = node;
+    node = exit[node]; // a later segment's, or rows
+  }
+}
+
+// bits of the segment's chain nodes (SEG / 32 words per segment) and
+// their count; the chain's last node says whether its block closes at rows
+// (*at_end: node rows is marked too) or the loop ended first
+template <uint32_t SEG>
+__global__ __launch_bounds__(SEG_T) void k_seg_mark(uint32_t rows, const uint32_t *__restrict__ rp, uint32_t W,
+                                                    const uint32_t *__restrict__ J,
+                                                    const uint32_t *__restrict__ entry, uint32_t *__restrict__ bits,
+                                                    uint32_t *__restrict__ count, uint32_t *__restrict__ at_end)
+{
+  constexpr uint32_t SEG_I = SEG / SEG_T;
+  extern __shared__ uint32_t nxt[]; // SEG, then SEG / 32 words of marks
+  uint32_t *mark = nxt + SEG;
+  __shared__ uint32_t sh[SEG_T / 64];
+  const uint32_t s0 = blockIdx.x * SEG, n = min(SEG, rows - s0), t = threadIdx.x;
+  const uint32_t e = entry[blockIdx.x];
+  static_assert(SEG / 32 <= SEG_T, "one word of marks per lane");
+  uint32_t v[SEG_I];
+#pragma unroll
+  for (uint32_t k = 0; k < SEG_I; k++) {
+    const uint32_t l = k * SEG_T + t;
+    v[k] = l < n ? J[s0 + l] : NO_NODE;
+    nxt[l] = v[k];
+  }
+  if (t < SEG / 32) mark[t] = e != NO_NODE && (e - s0) / 32 == t ? 1u << ((e - s0) & 31u) : 0u;
+  if (e != NO_NODE) { // uniform
+    for (;;) {
+      __syncthreads();
+      bool moved = false;
+      // v = 2^k steps from each node: a marked node marks the one it leads to
+#pragma unroll
+      for (uint32_t k = 0; k < SEG_I; k++) {
+        const uint32_t l = k * SEG_T + t, to = v[k] - s0;
+        if (to < n) {
+          if ((mark[l / 32] >> (l & 31u)) & 1u) atomicOr(&mark[to / 32], 1u << (to & 31u));
+          v[k] = nxt[to];
+          moved = true;
+        }
+      }
+      if (!__syncthreads_or(moved)) break;
+#pragma unroll
+      for (uint32_t k = 0; k < SEG_I; k++) nxt[k * SEG_T + t] = v[k];
     }
   }
-  J[s] = res;
+  __syncthreads();
+  const uint32_t w = t < SEG / 32 ? mark[t] : 0u;
+  if (t < SEG / 32) bits[(uint64_t)blockIdx.x * (SEG / 32) + t] = w;
+#pragma unroll
+  for (uint32_t k = 0; k < SEG_I; k++) {
+    const uint32_t l = k * SEG_T + t;
+    if (l < n && ((mark[l / 32] >> (l & 31u)) & 1u) && J[s0 + l] == rows) // one lane of the grid
+      *at_end = rp[rows] - rp[s0 + l] >= W || (uint64_t)rows == (uint64_t)s0 + l + W + 1u ? 1u : 0u;
+  }
+  uint32_t total;
+  (void)block_exclusive_scan<SEG_T>((uint32_t)__popc(w), sh, &total);
+  if (t == 0) count[blockIdx.x] = total;
 }
 
-__global__ void k_mark(uint64_t n, const uint32_t *__restrict__ J, uint32_t *__restrict__ mark)
+// the marked nodes from offs[segment] on; the first workgroup adds node rows
+// when marked, and the closing rows
+template <uint32_t SEG>
+__global__ __launch_bounds__(SEG / 32) void k_seg_write(uint32_t rows, uint32_t nseg,
+                                                             const uint32_t *__restrict__ bits,
+                                                             const uint32_t *__restrict__ offs,
+                                                             const uint32_t *__restrict__ at_end,
+                                                             uint32_t *__restrict__ out)
 {
-  const uint64_t s = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= n) return;
-  if (mark[s]) mark[J[s]] = 1u;
+  __shared__ uint32_t sh[SEG / 32 / 64];
+  uint32_t w = bits[(uint64_t)blockIdx.x * (SEG / 32) + threadIdx.x];
+  uint32_t o = offs[blockIdx.x] + block_exclusive_scan<SEG / 32>((uint32_t)__popc(w), sh, nullptr);
+  uint32_t node = blockIdx.x * SEG + threadIdx.x * 32u;
+  while (w) {
+    const uint32_t b = (uint32_t)__ffs((int)w) - 1u;
+    out[o++] = node + b;
+    w &= w - 1u;
+  }
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    const uint32_t total = offs[nseg];
+    out[total] = rows;
+    if (*at_end) out[total + 1] = rows;
+  }
 }
 
-__global__ void k_jump(uint64_t n, const uint32_t *__restrict__ J, uint32_t *__restrict__ J2)
+template <uint32_t SEG>
+static int row_blocks_t(uint32_t rows, const uint32_t *rp, uint32_t W, uint32_t **blocks_out, uint32_t *count_out,
+                        hipStream_t s)
 {
-  const uint64_t s = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= n) return;
-  J2[s] = J[J[s]];
+  device_temps tmp;
+  uint32_t *out = nullptr;
+  const uint32_t nseg = ceil_div_u32(rows, SEG);
+  uint32_t *J = nullptr, *exit = nullptr, *entry = nullptr, *bits = nullptr, *count = nullptr;
+  MFP_CHECK(tmp.alloc((void **)&J, (uint64_t)rows * 4));
+  MFP_CHECK(tmp.alloc((void **)&exit, (uint64_t)rows * 4));
+  MFP_CHECK(tmp.alloc((void **)&entry, (uint64_t)nseg * 4));
+  MFP_CHECK(tmp.alloc((void **)&bits, (uint64_t)nseg * (SEG / 32) * 4));
+  MFP_CHECK(tmp.alloc((void **)&count, ((uint64_t)nseg + 2) * 4)); // + total, at_end
+  const uint32_t lds = SEG * 4, lds_mark = lds + SEG / 32 * 4;
+  MFP_HIP(hipFuncSetAttribute((const void *)k_seg_exit<SEG>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  MFP_HIP(hipFuncSetAttribute((const void *)k_seg_mark<SEG>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_mark));
+  k_close<<<ceil_div_u32(rows, 256), 256, 0, s>>>(rows, rp, W, J);
+  k_seg_exit<SEG><<<nseg, SEG_T, lds, s>>>(rows, J, exit, entry);
+  k_seg_chase<<<1, 1, 0, s>>>(rows, SEG, exit, entry);
+  k_seg_mark<SEG><<<nseg, SEG_T, lds_mark, s>>>(rows, rp, W, J, entry, bits, count, count + nseg + 1);
+  k_scan_offsets<<<1, 1024, 0, s>>>(count, nseg);
+  MFP_HIP(hipGetLastError());
+  uint32_t h[2] = {0, 0};
+  MFP_HIP(hipMemcpyAsync(h, count + nseg, 8, hipMemcpyDeviceToHost, s));
+  MFP_HIP(hipStreamSynchronize(s));
+  const uint32_t total = h[0] + h[1];
+  MFP_CHECK(tmp.alloc((void **)&out, ((uint64_t)total + 1) * 4));
+  k_seg_write<SEG><<<nseg, SEG / 32, 0, s>>>(rows, nseg, bits, count, count + nseg + 1, out);
+  MFP_HIP(hipGetLastError());
+  MFP_HIP(hipStreamSynchronize(s));
+  tmp.release(out);
+  *blocks_out = out;
+  *count_out = total;
+  return MFP_OK;
 }
-
-__global__ void k_compact(uint32_t rows, const uint32_t *__restrict__ mark,
-                          const uint32_t *__restrict__ pos, uint32_t *__restrict__ out)
-{
-  const uint64_t s = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (s > rows) return;
-  if (mark[s]) out[pos[s]] = (uint32_t)s;
-}
-
-__global__ void k_store1(uint32_t *p, uint32_t v) { *p = v; }
 
 int row_blocks_device(uint32_t rows, const uint32_t *rp, uint32_t W, uint32_t **blocks_out,
                       uint32_t *count_out, hipStream_t s)
 {
   MFP_ARG(W > 0, "nnz_per_wg must be positive");
-  const uint64_t n = (uint64_t)rows + 2; // nodes 0..rows, sentinel rows+1
-  device_temps tmp;
-  uint32_t *J = nullptr, *J2 = nullptr, *mark = nullptr;
-  MFP_CHECK(tmp.alloc((void **)&J, n * 4));
-  MFP_CHECK(tmp.alloc((void **)&J2, n * 4));
-  MFP_CHECK(tmp.alloc((void **)&mark, n * 4));
-  const uint32_t g = ceil_div_u32(n, 256);
-  k_close<<<g, 256, 0, s>>>(rows, rp, W, J);
-  MFP_CHECK(fill_u32(mark, 0, n, s));
-  MFP_CHECK(fill_u32(mark, 1, 1, s));
-  for (uint64_t span = 1; span < 2 * n; span <<= 1) {
-    k_mark<<<g, 256, 0, s>>>(n, J, mark);
-    k_jump<<<g, 256, 0, s>>>(n, J, J2);
-    std::swap(J, J2);
+  if (rows == 0) { // node 0 is node rows: one marked node, then the closing rows
+    device_temps tmp;
+    uint32_t *out = nullptr;
+    MFP_CHECK(tmp.alloc((void **)&out, 2 * 4));
+    MFP_CHECK(fill_u32(out, 0, 2, s));
+    MFP_HIP(hipStreamSynchronize(s));
+    tmp.release(out);
+    *blocks_out = out;
+    *count_out = 1;
+    return MFP_OK;
   }
-  MFP_HIP(hipGetLastError());
-  // count = marked nodes in [0, rows]; positions by exclusive scan
-  uint32_t count = 0;
-  MFP_CHECK(exclusive_scan_u32(mark, J2, (uint64_t)rows + 1, s, &count));
-  uint32_t *out = nullptr;
-  MFP_CHECK(tmp.alloc((void **)&out, ((uint64_t)count + 1) * 4));
-  k_compact<<<ceil_div_u32((uint64_t)rows + 1, 256), 256, 0, s>>>(rows, mark, J2, out);
-  k_store1<<<1, 1, 0, s>>>(out + count, rows);
-  MFP_HIP(hipGetLastError());
-  MFP_HIP(hipStreamSynchronize(s));
-  tmp.release(out);
-  *blocks_out = out;
-  *count_out = count;
-  return MFP_OK;
+  return rows > (1u << 18) ? row_blocks_t<16384>(rows, rp, W, blocks_out, count_out, s)
+                           : row_blocks_t<4096>(rows, rp, W, blocks_out, count_out, s);
 }
 
 } // namespace mfp

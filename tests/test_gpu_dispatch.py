@@ -184,3 +184,55 @@ def test_column_sorted_build(gpu, rows, values):
     assert np.array_equal(yd.to_host().astype(np.float64), y64)
     plan.destroy()
     A.destroy()
+
+
+# Segments of row blocks hold 16,384 rows; a block holds at most W entries (a
+# longer row alone) and W + 1 rows.
+BLOCK_ROWS = {
+    "segment edges": [2] * 16384 * 3,
+    "one short of a segment": [3] * 16383,
+    "one past a segment": [1] * 16385,
+    "empty rows over segments": [0] * 40000 + [5] + [0] * 30000 + [9] * 3 + [0] * 17000,
+    "all empty": [0] * 33000,
+    "long rows": [700, 1, 0, 699, 513, 512, 511, 1] * 9000,
+    "one row": [1],
+    "mixed": [int(v) for v in np.minimum(1 / (1 - np.random.default_rng(8).random(70001)), 5000)],
+}
+
+
+@pytest.mark.parametrize("W", [1, 2, 64, 511, 512, 2040, 40000])
+@pytest.mark.parametrize("rows", list(BLOCK_ROWS))
+def test_row_blocks_any_chain(gpu, rows, W):
+    announce(f"row blocks {rows} W={W}")
+    rp = np.concatenate([[0], np.cumsum(BLOCK_ROWS[rows])]).astype(np.uint32)
+    assert np.array_equal(gpu.fill_row_blocks(rp.size - 1, rp, W), oracle.fill_row_blocks(rp, W))
+
+
+@pytest.mark.parametrize("rows", list(BLOCK_ROWS))
+def test_row_statistics(gpu, rows):
+    lens = np.asarray(BLOCK_ROWS[rows], np.int64)
+    rp = np.concatenate([[0], np.cumsum(lens)]).astype(np.uint32)
+    ci = np.zeros(rp[-1], np.uint32)  # statistics read row lengths only
+    A = gpu.DeviceMatrix.from_csr(rp, ci, np.ones(rp[-1], np.float32), 1)
+    mn, mx, avg, sd = A.row_stats()
+    A.destroy()
+    dev = int(((lens - int(lens.sum()) // lens.size) ** 2).sum())
+    assert (mn, mx, avg) == (lens.min(), lens.max(), lens.sum() // lens.size)
+    assert sd == np.sqrt(np.float64(dev) / lens.size)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("lens", [[1], [0, 0, 17], [16] * 64, [15, 16, 17, 33] * 49, [0] * 63 + [65] + [1] * 64])
+def test_ell_build_tiles(gpu, lens, dtype):
+    from matrix_format_performance_amd import _lib as L
+    rp, ci, va = _csr(lens, 301, dtype)
+    A = gpu.DeviceMatrix.from_csr(rp, ci, va, 301)
+    plan = gpu.Plan(A, "ell")
+    n, w = len(lens), max(lens)
+    ev, ec = np.zeros((w, n), dtype), np.zeros((w, n), np.uint32)
+    for r in range(n):
+        ev[:lens[r], r], ec[:lens[r], r] = va[rp[r]:rp[r + 1]], ci[rp[r]:rp[r + 1]]
+    assert np.array_equal(plan.array(L.MFP_ARR_ELL_VALUES, np.dtype(dtype)), ev.ravel())
+    assert np.array_equal(plan.array(L.MFP_ARR_ELL_COLS, np.uint32), ec.ravel())
+    plan.destroy()
+    A.destroy()
