@@ -657,7 +657,7 @@ __global__ __launch_bounds__(ROWS_T) void k_coo_build(uint32_t rows, uint64_t nn
   const uint32_t t0 = blockIdx.x * ROWS_TILE, t = threadIdx.x;
   const uint64_t t1 = min(nnz, (uint64_t)t0 + ROWS_TILE);
   uint32_t row[ROWS_I];
-  tile_rows(rp, rows, t0, t1, mark, sh, row);
+  tile_rows(rp, rows, block_row_of(rp, rows, t0, sh + 4), t0, t1, mark, sh, row);
   __syncthreads();
   // through LDS, so that neighbouring lanes handle neighbouring entries
 #pragma unroll
@@ -785,7 +785,7 @@ __global__ __launch_bounds__(ROWS_T) void k_entry_vrow(uint32_t rows, uint64_t n
   const uint32_t t0 = blockIdx.x * ROWS_TILE, t = threadIdx.x;
   const uint64_t t1 = min(nnz, (uint64_t)t0 + ROWS_TILE);
   uint32_t row[ROWS_I];
-  tile_rows(rp, rows, t0, t1, mark, sh, row);
+  tile_rows(rp, rows, block_row_of(rp, rows, t0, sh + 4), t0, t1, mark, sh, row);
   if (mask) {
 #pragma unroll
     for (uint32_t k = 0; k < ROWS_I; k++)

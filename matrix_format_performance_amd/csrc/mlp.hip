@@ -59,6 +59,17 @@ __global__ void k_bias_act(float *__restrict__ H, const float *__restrict__ b, i
   H[i] = relu ? fmaxf(v, 0.f) : v;
 }
 
+// q = softmax(z), in the steps of k_softmax_xent
+__device__ __forceinline__ void softmax_row(const float *z, float *__restrict__ q)
+{
+  float mx = -INFINITY;
+  for (int j = 0; j < NO; j++) mx = fmaxf(mx, z[j]);
+  float s = 0.f;
+  for (int j = 0; j < NO; j++) s += expf(z[j] - mx);
+  const float ls = logf(s);
+  for (int j = 0; j < NO; j++) q[j] = expf(z[j] - mx - ls);
+}
+
 // per row: softmax, loss -sum p log q, dZ = (q - p) / n
 __global__ void k_softmax_xent(const float *__restrict__ Z, const float *__restrict__ P, int M,
                                float *__restrict__ dZ, float *__restrict__ Q, double *__restrict__ loss)
@@ -126,37 +137,99 @@ __device__ __forceinline__ short to_bf16(float f)
   return *reinterpret_cast<short *>(&h);
 }
 
-// C[M x N] = A[M x K] W[K x N] (+ bias, ReLU) with A, W rounded to BF16.
-// One wave per 16 x 16 output tile; K in steps of 16.  Operand layout of
-// v_mfma_f32_16x16x16_bf16: lane l holds A[l % 16][4 (l / 16) + j] and
-// W[4 (l / 16) + j][l % 16] (j = 0..3); the result D[4 (l / 16) + j][l % 16].
-__global__ __launch_bounds__(64) void k_mfma_linear(const float *__restrict__ A, const float *__restrict__ W,
-                                                    const float *__restrict__ bias, float *__restrict__ C,
-                                                    int M, int N, int K, int relu)
+// The whole network for 16 rows per workgroup, one wave per 16 hidden units.
+// Activations and weights are rounded to BF16, K goes in steps of 16.  Operand
+// layout of v_mfma_f32_16x16x16_bf16: lane l holds A[l % 16][4 (l / 16) + j]
+// and W[4 (l / 16) + j][l % 16] (j = 0..3); the result D[4 (l / 16) + j][l % 16].
+// A call is three layers of a few products each, so it is bound by waiting:
+// the weights are read once, in 16-byte loads that are all in flight together,
+// and put into LDS in BF16, column by column, where a lane finds its four k in
+// one read; the hidden layers stay in LDS.  One row takes 8 us, a launch per
+// layer took 10 us each.
+constexpr int INF_T = NH / 16 * 64;
+constexpr int W1S = NI + 4, W2S = NH + 4; // strides in LDS: 8-byte aligned, off the same banks
+
+// W (K x N, row-major) to dst[n][k] in BF16, by the whole workgroup
+template <int K, int N, int S>
+__device__ __forceinline__ void stage_weights(short *dst, const f32x4 (&v)[(K * N / 4 + INF_T - 1) / INF_T])
 {
-  const int lane = threadIdx.x;
-  const int tm = blockIdx.y * 16, tn = blockIdx.x * 16;
+#pragma unroll
+  for (int q = 0; q < (K * N / 4 + INF_T - 1) / INF_T; q++) {
+    const int i = q * INF_T + (int)threadIdx.x;
+    if (i < K * N / 4) {
+      const int k = i / (N / 4), n = i % (N / 4) * 4;
+#pragma unroll
+      for (int j = 0; j < 4; j++) dst[(n + j) * S + k] = to_bf16(v[q][j]);
+    }
+  }
+}
+
+template <int K, int N>
+__device__ __forceinline__ void load_weights(const float *__restrict__ W, f32x4 (&v)[(K * N / 4 + INF_T - 1) / INF_T])
+{
+#pragma unroll
+  for (int q = 0; q < (K * N / 4 + INF_T - 1) / INF_T; q++) {
+    const int i = min(q * INF_T + (int)threadIdx.x, K * N / 4 - 1);
+    v[q] = reinterpret_cast<const f32x4 *>(W)[i];
+  }
+}
+
+__global__ __launch_bounds__(INF_T) void k_mlp_infer(const float *__restrict__ X, const float *__restrict__ p, int M,
+                                                     float *__restrict__ Q)
+{
+  static_assert(OFF_W2 % 4 == 0 && OFF_W3 % 4 == 0, "16-byte loads of the weights");
+  __shared__ __align__(16) short w1[NH * W1S], w2[NH * W2S], w3[16 * W2S];
+  __shared__ __align__(16) short x[16 * W1S], h1[16 * W2S], h2[16 * W2S];
+  __shared__ float z[16][NO];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int tm = blockIdx.x * 16, tn = wave * 16;
   const int r = lane % 16, kq = 4 * (lane / 16);
-  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-  for (int k0 = 0; k0 < K; k0 += 16) {
-    bf16x4 a, b;
+  const float b1 = p[OFF_B1 + tn + r], b2 = p[OFF_B2 + tn + r], b3 = p[OFF_B3 + r % NO];
+  {
+    f32x4 v1[NI * NH / 4 / INF_T], v2[NH * NH / 4 / INF_T], v3[1], vx[1];
+    load_weights<NI, NH>(p + OFF_W1, v1);
+    load_weights<NH, NH>(p + OFF_W2, v2);
+    load_weights<NH, NO>(p + OFF_W3, v3);
+    const int xr = (int)threadIdx.x / (NI / 4), xk = (int)threadIdx.x % (NI / 4) * 4; // 16 rows: 256 lanes
+    if (threadIdx.x < 16 * NI / 4) {
+      vx[0] = tm + xr < M ? *reinterpret_cast<const f32x4 *>(X + (size_t)(tm + xr) * NI + xk) : f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-      const int k = k0 + kq + j;
-      const int ar = tm + r, bc = tn + r;
-      a[j] = to_bf16((ar < M && k < K) ? A[(size_t)ar * K + k] : 0.f);
-      b[j] = to_bf16((k < K && bc < N) ? W[(size_t)k * N + bc] : 0.f);
+      for (int j = 0; j < 4; j++) x[xr * W1S + xk + j] = to_bf16(vx[0][j]);
     }
-    acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc, 0, 0, 0);
+    stage_weights<NI, NH, W1S>(w1, v1);
+    stage_weights<NH, NH, W2S>(w2, v2);
+    stage_weights<NH, NO, W2S>(w3, v3);
+    // columns 8..15 of the last layer's tile
+    for (int i = threadIdx.x; i < (16 - NO) * W2S; i += INF_T) w3[NO * W2S + i] = 0;
   }
+  __syncthreads();
+  auto layer = [&](const short *A, int as, const short *W, int ws, int K) {
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int j = 0; j < 4; j++) {
-    const int row = tm + kq + j, col = tn + r;
-    if (row < M && col < N) {
-      float v = acc[j] + bias[col];
-      C[(size_t)row * N + col] = relu ? fmaxf(v, 0.f) : v;
+    for (int k0 = 0; k0 < K; k0 += 16) {
+      const bf16x4 a = *reinterpret_cast<const bf16x4 *>(A + r * as + k0 + kq);
+      const bf16x4 b = *reinterpret_cast<const bf16x4 *>(W + r * ws + k0 + kq);
+      acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc, 0, 0, 0);
+    }
+    return acc;
+  };
+  f32x4 acc = layer(x, W1S, w1 + tn * W1S, W1S, NI);
+#pragma unroll
+  for (int j = 0; j < 4; j++) h1[(kq + j) * W2S + tn + r] = to_bf16(fmaxf(acc[j] + b1, 0.f));
+  __syncthreads();
+  acc = layer(h1, W2S, w2 + tn * W2S, W2S, NH);
+#pragma unroll
+  for (int j = 0; j < 4; j++) h2[(kq + j) * W2S + tn + r] = to_bf16(fmaxf(acc[j] + b2, 0.f));
+  __syncthreads();
+  if (wave == 0) {
+    acc = layer(h2, W2S, w3, W2S, NH);
+    if (r < NO) {
+#pragma unroll
+      for (int j = 0; j < 4; j++) z[kq + j][r] = acc[j] + b3;
     }
   }
+  __syncthreads();
+  if (threadIdx.x < 16 && tm + (int)threadIdx.x < M) softmax_row(z[threadIdx.x], Q + (size_t)(tm + threadIdx.x) * NO);
 }
 
 } // namespace mfp
@@ -344,16 +417,11 @@ int mfp_mlp_predict(mfp_mlp m, const float *X, uint32_t n, int bf16, float *prob
   MFP_CHECK(mlp_reserve(m, n));
   MFP_CHECK(mfp_memcpy_h2d(m->X, X, (size_t)n * NI * 4));
   if (bf16) {
-    const float *p = m->params;
-    const dim3 g1(NH / 16, (n + 15) / 16), g3((NO + 15) / 16, (n + 15) / 16);
-    k_mfma_linear<<<g1, 64>>>(m->X, p + OFF_W1, p + OFF_B1, m->H1, n, NH, NI, 1);
-    k_mfma_linear<<<g1, 64>>>(m->H1, p + OFF_W2, p + OFF_B2, m->H2, n, NH, NH, 1);
-    k_mfma_linear<<<g3, 64>>>(m->H2, p + OFF_W3, p + OFF_B3, m->Z, n, NO, NH, 0);
-    MFP_HIP(hipGetLastError());
+    k_mlp_infer<<<(n + 15) / 16, INF_T>>>(m->X, m->params, (int)n, m->Q);
   } else {
     MFP_CHECK(mlp_forward(m, n));
+    k_softmax_xent<<<ceil_div_u32(n, 256), 256>>>(m->Z, nullptr, n, nullptr, m->Q, nullptr);
   }
-  k_softmax_xent<<<ceil_div_u32(n, 256), 256>>>(m->Z, nullptr, n, nullptr, m->Q, nullptr);
   MFP_HIP(hipGetLastError());
   return mfp_memcpy_d2h(probs, m->Q, (size_t)n * NO * 4);
 }

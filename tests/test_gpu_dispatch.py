@@ -236,3 +236,31 @@ def test_ell_build_tiles(gpu, lens, dtype):
     assert np.array_equal(plan.array(L.MFP_ARR_ELL_COLS, np.uint32), ec.ravel())
     plan.destroy()
     A.destroy()
+
+
+# ---- selector features -------------------------------------------------------------
+# The distance bins come from reciprocals up to rows cols = 2^53, from divisions
+# above; tiles hold 2,048 entries.
+
+@pytest.mark.parametrize("rows,cols", [(1, 1), (10000, 10000), (4096, 10000), (10000, 40000), (65537, 300007),
+                                       (4099, 4294967295), (3000001, 3002399751)])
+def test_features_any_shape(gpu, rows, cols):
+    from matrix_format_performance_amd import selector
+    from oracle import selector as ref
+    announce(f"features rows={rows} cols={cols}")
+    rng = np.random.default_rng(rows % 1000)
+    lens = np.zeros(rows, np.int64)
+    used = rng.choice(rows, min(rows, 3000), replace=False)
+    lens[used] = rng.integers(1, 1 + min(cols, 9), used.size)
+    rp = np.concatenate([[0], np.cumsum(lens)]).astype(np.uint32)
+    row = np.repeat(np.arange(rows), lens)
+    # half of the columns exactly at multiples of 1e-4 cols from the diagonal
+    at = (row * np.float64(cols) / rows).astype(np.int64)
+    off = (rng.integers(0, 4096, row.size) * (cols // 10000)) * rng.choice([-1, 1], row.size)
+    ci = np.where(rng.random(row.size) < 0.5, at + off, rng.integers(0, cols, row.size)) % cols
+    order = np.lexsort((ci, row))
+    ci = ci[order].astype(np.uint32)
+    A = gpu.DeviceMatrix.from_csr(rp, ci, np.ones(ci.size, np.float32), cols)
+    got = selector.features(A)
+    A.destroy()
+    assert np.array_equal(got, ref.features(rp, ci, rows, cols).astype(np.float32))
