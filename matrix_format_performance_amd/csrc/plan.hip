@@ -634,6 +634,12 @@ int mfp_plan_create(mfp_plan *out, mfp_matrix m, int format, const mfp_tuning *t
                                &p->coo_val, &p->coo_col, &p->coo_row, &p->ncoo, s);
     if (st != MFP_OK) return fail(st);
     p->device_bytes = p->ncoo * (vs + 8);
+    if (format == MFP_COO) {
+      mfp_row_stats rs;
+      st = matrix_stats(m, &rs, s);
+      if (st != MFP_OK) return fail(st);
+      p->coo_owner = coo_owner_fits(p->ncoo, rs.max_elements_in_rows);
+    }
     if (format == MFP_SCOO) {
       p->ss = t.scoo_slice_size;
       p->L = t.scoo_lanes;
@@ -717,6 +723,8 @@ static int plan_spmv(mfp_plan p, const void *x, void *y, hipStream_t s, void *pa
       return launch_ell_pk(dt, m->rows, p->ell_w, p->pk_w4, p->pk_base, p->pk_val, p->pk_off, x, y, s);
     return launch_ell(dt, m->rows, p->ell_w, p->ell_col, p->ell_val, x, y, s);
   case MFP_COO:
+    if (p->coo_owner)
+      return launch_coo_owner(dt, m->rows, p->ncoo, m->row_ptr, p->coo_row, p->coo_col, p->coo_val, x, y, s);
     MFP_CHECK(fill_bytes_zero(y, (size_t)m->rows * dtype_size(dt), s));
     mark_kernel_end(); // the zero fill of y is its own interval under mfp_plan_kernel_times
     return launch_coo_add(dt, p->ncoo, p->coo_row, p->coo_col, p->coo_val, x, y, s);

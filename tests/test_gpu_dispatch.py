@@ -264,3 +264,37 @@ def test_features_any_shape(gpu, rows, cols):
     got = selector.features(A)
     A.destroy()
     assert np.array_equal(got, ref.features(rp, ci, rows, cols).astype(np.float32))
+
+
+# ---- COO and hybrids ------------------------------------------------------------
+# A wave takes 256 entries (4 per lane) and looks 64 ahead; rows of at most 64
+# entries are stored by the wave of their first entry, longer ones are added.
+
+COO_ROWS = {
+    "span edges": [255, 1, 256, 257, 0, 3, 252, 4, 0, 0, 320, 321, 319, 63, 64, 65] * 9,
+    "lane edges": [1, 2, 3, 4, 5, 6, 7, 8, 9] * 801,
+    "ones and gaps": [1, 0, 0, 1] * 5001,
+    "longest owned": [64, 0, 64, 1, 63, 7, 62, 64, 64, 3] * 25,
+    "one too long": [65, 3, 0, 64, 64] * 25,
+    "last row long": [2] * 127 + [64],
+    "empty": [0] * 300,
+    "single": [1],
+    "very long": [9000, 0, 1] * 3 + [5] * 777,
+}
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("fmt", ["coo", "hyb", "hyb_atomic"])
+@pytest.mark.parametrize("rows", list(COO_ROWS))
+def test_coo_rows_of_any_length(gpu, rows, fmt, dtype):
+    rp, ci, va = _csr(COO_ROWS[rows], 10007, dtype)
+    x = gpu.generate_vector(3, 10007, np.dtype(dtype))
+    if fmt == "coo":
+        x[0] = np.inf  # no entry reads column 0 (an ELL part's padding multiplies x[0] by zero)
+    y = _spmv(gpu, rp, ci, va, x, fmt, **({} if fmt == "coo" else {"hyb_width": 3}))
+    x[0] = 0
+    y64, absdot = oracle.spmv_f64(rp, ci, va, x)
+    assert not np.isnan(y).any()
+    # any order of n products and sums is within n u of sum |a x| (u: unit roundoff)
+    bound = (max(COO_ROWS[rows]) + 1) * np.finfo(dtype).eps / 2
+    assert oracle.tolerance_check(y, y64, absdot, bound) <= bound
