@@ -298,3 +298,52 @@ def test_coo_rows_of_any_length(gpu, rows, fmt, dtype):
     # any order of n products and sums is within n u of sum |a x| (u: unit roundoff)
     bound = (max(COO_ROWS[rows]) + 1) * np.finfo(dtype).eps / 2
     assert oracle.tolerance_check(y, y64, absdot, bound) <= bound
+
+
+# ---- batch SpMM, slices with aligned rows -----------------------------------------
+# k = 4: 2,048-row slices, 64 rows per workgroup, chunks of 2,048 (FP64 1,024)
+# entries; rows above 128 entries keep a slice in the column-sorted form.
+
+def _band(rows, width, seed, cols=None, gaps=False):
+    """Rows of `width` columns side by side along the diagonal."""
+    cols = cols or rows
+    lens = np.full(rows, min(width, cols))
+    if gaps:
+        lens[5::11] = 0
+        lens[2000 % rows] = 1
+    rp = np.concatenate([[0], np.cumsum(lens)]).astype(np.uint32)
+    r = np.repeat(np.arange(rows), lens)
+    t = np.arange(rp[-1]) - rp[r]
+    ci = (np.minimum(r * cols // rows, cols - min(width, cols)) + t).astype(np.uint32)
+    return rp, ci, np.random.default_rng(seed).uniform(-1, 1, ci.size), cols
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("k", [1, 2, 4, 8])
+def test_batch_aligned_and_random_slices(gpu, k, dtype):
+    announce(f"batch aligned slices k={k} dtype={dtype}")
+    members = [_band(2048, 27, 0), _band(5001, 5, 1), _band(1, 1, 2), _band(4097, 128, 3), _band(2100, 129, 4),
+               _band(3000, 40, 5, cols=9000), _band(6145, 31, 6, gaps=True)]
+    for seed in (7, 8):
+        lens = np.random.default_rng(seed).integers(0, 30, 4500)
+        members.append((*_csr(lens, 4000, "float64", seed), 4000))
+    mats = [gpu.DeviceMatrix.from_csr(rp, ci, va.astype(dtype), cols) for rp, ci, va, cols in members]
+    B = gpu.Batch(mats, lanes=1, flags=4, scoo_slice_size=2048, scoo_pieces=1)
+    X = gpu.generate_vector(11, B.cols * k, np.dtype(dtype))
+    Xd, Yd = gpu.DeviceArray.from_host(X), gpu.DeviceArray(B.rows * k, np.dtype(dtype))
+    Yd.fill(np.nan)
+    B.spmm(k, Xd, Yd)
+    gpu.synchronize()
+    Y = Yd.to_host().reshape(B.rows, k)
+    for i, (rp, ci, va, cols) in enumerate(members):
+        for j in range(k):
+            x = X.reshape(B.cols, k)[B.col_offsets[i]:B.col_offsets[i + 1], j].copy()
+            y64, absdot = oracle.spmv_f64(rp, ci, va.astype(dtype), x)
+            y = Y[B.row_offsets[i]:B.row_offsets[i + 1], j]
+            # sums in double, rounded once (FP64: at most 129 roundings of each kind)
+            bound = 2 * np.finfo(dtype).eps * (1 if dtype == "float32" else 130)
+            assert not np.isnan(y).any()
+            assert oracle.tolerance_check(y, y64, absdot, bound) <= bound, (i, j)
+    B.destroy()
+    for m in mats:
+        m.destroy()
