@@ -266,7 +266,7 @@ typedef struct mfp_graph_s *mfp_graph;
  * column-sorted SCOO SpMM over the assembled matrix (one plan per k, built by
  * the first mfp_batch_spmm or mfp_batch_graph_create with that k: the
  * largest power-of-two slice whose k doubles per row fit in 160 KB of LDS,
- * one work item per slice and column band, 1,024 threads; for k = 2 and 4,
+ * one work item per slice and column band, 1,024 threads;
  * slices whose neighbouring rows have nearly the same columns are summed row
  * by row, in double as well); MFP_BATCH_STREAM
  * for the CSR-stream SpMM: row blocks of whole rows with at most 512 entries

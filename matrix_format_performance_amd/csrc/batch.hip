@@ -603,7 +603,7 @@ int stream_meta_device(uint32_t rows, const uint32_t *rp, uint32_t **meta, uint3
   return MFP_OK;
 }
 
-// ---- slices with aligned rows (column-sorted batch SpMM, k = 2 and 4) -----------------
+// ---- slices with aligned rows (column-sorted batch SpMM) ----------------------------------
 // The column-sorted kernel adds every product into LDS, k double atomics per
 // entry at two to three lanes per clock and CU, to read each X line once per
 // slice.  Where neighbouring rows have nearly the same columns (grids, bands)
@@ -613,7 +613,8 @@ int stream_meta_device(uint32_t rows, const uint32_t *rp, uint32_t **meta, uint3
 // register, in double as the slices do (exact for FP32 values).  The 16 rows
 // of a wave gather neighbouring X rows, so its gathers are two or three lines
 // each, mostly in L1.  64-matrix batch, k = 4, FP32: 20M entries of grids take
-// 64 us here and 99 there, the step 230 -> 190 us; k = 2 179 -> 156.  Measured
+// 64 us here and 99 there, the step 230 -> 190 us; k = 2 179 -> 156, k = 8
+// 417 -> 328, k = 16 875 -> 662.  Measured
 // without gain: 2 or 4 columns per lane with wider gathers (71 to 79 us),
 // workgroups of 2, 4 or 8 row groups with the next group's loads in flight
 // (69 to 82).
@@ -762,7 +763,7 @@ struct mfp_batch_s {
   uint32_t *stream_meta = nullptr; // lanes == MFP_BATCH_STREAM: row blocks of STREAM_W entries, (row, entry) pairs
   uint32_t nstream = 0;
   mfp_plan cs[5] = {};         // lanes == 1: column-sorted SCOO plan for k = 2 << (i - 1)
-  uint32_t *aligned[5] = {};   // k = 2 and 4: its slices with aligned rows, which k_spmm_aligned takes
+  uint32_t *aligned[5] = {};   // its slices with aligned rows, which k_spmm_aligned takes
   uint32_t naligned[5] = {};
 };
 
@@ -779,7 +780,7 @@ static uint32_t log2_k(uint32_t k)
 static int batch_split_aligned(mfp_batch b, uint32_t i, hipStream_t s)
 {
   scoo_cs_layout &l = b->cs[i]->cs;
-  if (l.S_reg == 0 || l.NI == 0 || l.R < AL_T || l.S_long) return MFP_OK;
+  if (l.S_reg == 0 || l.NI == 0 || l.R < AL_T) return MFP_OK;
   uint32_t *flag = nullptr, *list = nullptr;
   MFP_CHECK(dmalloc((void **)&flag, (uint64_t)l.S_reg * 4));
   k_aligned_slices<<<ceil_div_u32(l.S_reg, 4), 256, 0, s>>>(l.S_reg, l.R, b->big->rows, b->big->row_ptr,
@@ -797,7 +798,7 @@ static int batch_split_aligned(mfp_batch b, uint32_t i, hipStream_t s)
   dfree(flag);
   if (st != MFP_OK) return st;
   for (uint32_t q = 0; q < l.NI; q++) {
-    if (items[q].w == CS_DIRECT && hf[items[q].x]) {
+    if (items[q].w == CS_DIRECT && items[q].x < l.S_reg && hf[items[q].x]) {
       al.push_back(items[q].x);
     } else {
       keep.push_back(items[q]);
@@ -835,9 +836,13 @@ static int spmm_aligned_t(const mfp_batch_s *b, uint32_t i, const void *X, void 
 static int launch_spmm_aligned(const mfp_batch_s *b, uint32_t i, const void *X, void *Y, hipStream_t s)
 {
   if (b->naligned[i] == 0) return MFP_OK;
-  if (b->big->dtype == MFP_F32)
-    return i == 1 ? spmm_aligned_t<float, 2>(b, i, X, Y, s) : spmm_aligned_t<float, 4>(b, i, X, Y, s);
-  return i == 1 ? spmm_aligned_t<double, 2>(b, i, X, Y, s) : spmm_aligned_t<double, 4>(b, i, X, Y, s);
+  const bool f32 = b->big->dtype == MFP_F32;
+  switch (i) {
+  case 1: return f32 ? spmm_aligned_t<float, 2>(b, i, X, Y, s) : spmm_aligned_t<double, 2>(b, i, X, Y, s);
+  case 2: return f32 ? spmm_aligned_t<float, 4>(b, i, X, Y, s) : spmm_aligned_t<double, 4>(b, i, X, Y, s);
+  case 3: return f32 ? spmm_aligned_t<float, 8>(b, i, X, Y, s) : spmm_aligned_t<double, 8>(b, i, X, Y, s);
+  default: return f32 ? spmm_aligned_t<float, 16>(b, i, X, Y, s) : spmm_aligned_t<double, 16>(b, i, X, Y, s);
+  }
 }
 
 // lanes == 1: the column-sorted plan for k columns, built on first use (never
@@ -872,7 +877,7 @@ static int batch_cs_plan(mfp_batch b, uint32_t k, mfp_stream sv)
   if (k <= 4) t.flags |= MFP_TUNE_SCOO_WHOLE_SLICES;
   t.scoo_threads = 1024;
   MFP_CHECK(mfp_plan_create(&b->cs[i], b->big, MFP_SCOO, &t, sv));
-  const int st = k <= 4 ? batch_split_aligned(b, i, as_stream(sv)) : MFP_OK;
+  const int st = batch_split_aligned(b, i, as_stream(sv));
   if (st != MFP_OK) {
     mfp_plan_destroy(b->cs[i]);
     b->cs[i] = nullptr;

@@ -319,7 +319,7 @@ def _band(rows, width, seed, cols=None, gaps=False):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
-@pytest.mark.parametrize("k", [1, 2, 4, 8])
+@pytest.mark.parametrize("k", [1, 2, 4, 8, 16])
 def test_batch_aligned_and_random_slices(gpu, k, dtype):
     announce(f"batch aligned slices k={k} dtype={dtype}")
     members = [_band(2048, 27, 0), _band(5001, 5, 1), _band(1, 1, 2), _band(4097, 128, 3), _band(2100, 129, 4),
