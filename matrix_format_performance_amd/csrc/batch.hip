@@ -317,12 +317,13 @@ __device__ __forceinline__ V stream_gather(const T *__restrict__ X, uint32_t c, 
 }
 
 // Workgroups per CU that the register budget is set for: 8 (the wave limit)
-// for every f32 form and the narrow f64 ones; wider f64 X rows hold more
-// registers per gather.
+// where the gathers in flight leave room.  f32 at KV = 16 holds 32 registers
+// of X: at 8 waves they spill (a batch of 64: 466 us), at 7 they do not
+// (373 us).  Wider f64 X rows hold more per gather.
 template <typename T, int KV>
 constexpr int stream_min_wg()
 {
-  return sizeof(T) == 4 || KV <= 4 ? 8 : (KV == 8 ? 5 : 4);
+  return sizeof(T) == 4 && KV == 16 ? 7 : sizeof(T) == 4 || KV <= 4 ? 8 : (KV == 8 ? 5 : 4);
 }
 
 template <typename T, int KV, bool OFF32>
@@ -436,6 +437,20 @@ __global__ __launch_bounds__(STREAM_T, (stream_min_wg<T, KV>())) void k_spmm_str
     s_row[i1] = 0;
   }
   __syncthreads();
+  // The group's X rows, in flight while the entries' rows are found (below):
+  // a block spends its time on the latency of its phases one after another.
+  // A batch of 64 in f32, gathers after the row scan -> before it: k = 4
+  // 256 -> 237 us, k = 8 310 -> 283 us, k = 16 378 -> 373 us; f64, k = 2, 4,
+  // 8, 16: 273 -> 247, 321 -> 299, 414 -> 396, 572 -> 568 us.
+  const uint32_t base = g * EPG;
+  V xv[EPG];
+  {
+    uint32_t cc[EPG];
+    lds_run<EPG>(&s_col[base], cc);
+#pragma unroll
+    for (uint32_t j = 0; j < EPG; j++) // past the block: X row 0, never summed into a row
+      xv[j] = stream_gather<V, LPE, OFF32>(X, base + j < n ? cc[j] : 0u, l);
+  }
   for (uint32_t r = tid; r < nr; r += STREAM_T) {
     const uint32_t b = s_rp[r], z = s_rp[r + 1];
     if (b == z) {
@@ -463,15 +478,6 @@ __global__ __launch_bounds__(STREAM_T, (stream_min_wg<T, KV>())) void k_spmm_str
     *reinterpret_cast<uint2 *>(&s_row[2 * tid]) = make_uint2(max(ex, p.x), max(ex, hi));
   }
   __syncthreads();
-  const uint32_t base = g * EPG;
-  V xv[EPG];
-  {
-    uint32_t cc[EPG];
-    lds_run<EPG>(&s_col[base], cc);
-#pragma unroll
-    for (uint32_t j = 0; j < EPG; j++) // past the block: X row 0, never summed into a row
-      xv[j] = stream_gather<V, LPE, OFF32>(X, base + j < n ? cc[j] : 0u, l);
-  }
   uint32_t rr[EPG];
   T v[EPG];
   lds_run<EPG>(&s_row[base], rr);
