@@ -264,8 +264,12 @@ static int spmm_bins_build(uint32_t rows, const uint32_t *rp_dev, spmm_bins_args
 // then a halving tree over the groups.  Every lane is
 // busy whatever the row lengths, and a group's gathers do not wait on one
 // another, where CSR-vector leaves lanes idle on short rows and each row is
-// one chain of dependent loads.  Blocks are remapped so that each XCD works
-// on one contiguous range of them.
+// one chain of dependent loads.  Of a batch, an XCD takes runs of 64
+// consecutive blocks: a batch of 64 in f32, one range per XCD -> runs: k = 8
+// 283 -> 243 us, k = 16 373 -> 328 us (f64 k = 2 248 -> 233, k = 16 568 ->
+// 554); runs of 8, 16, 32, 128 and 256 blocks are within 2% of 64.  One matrix
+// keeps a range per XCD (300k rows within a band of 1%, k = 16: 58.1 us, 60.7
+// in runs).
 constexpr uint32_t STREAM_T = 256; // STREAM_W (kernels.h): entries per row block
 static_assert(STREAM_W == 2 * STREAM_T, "the row scan gives each lane two entries");
 
@@ -328,7 +332,7 @@ constexpr int stream_min_wg()
 
 template <typename T, int KV, bool OFF32>
 __global__ __launch_bounds__(STREAM_T, (stream_min_wg<T, KV>())) void k_spmm_stream(
-    const uint2 *__restrict__ meta, const uint32_t *__restrict__ rp, const uint32_t *__restrict__ ci,
+    uint32_t run, const uint2 *__restrict__ meta, const uint32_t *__restrict__ rp, const uint32_t *__restrict__ ci,
     const T *__restrict__ a, const T *__restrict__ X, T *__restrict__ Y)
 {
   using V = typename vec16b<T>::V;
@@ -341,7 +345,7 @@ __global__ __launch_bounds__(STREAM_T, (stream_min_wg<T, KV>())) void k_spmm_str
   __shared__ uint32_t s_rp[STREAM_W + 2];
   __shared__ V s_seg[STREAM_T];
   __shared__ uint32_t s_wmax[STREAM_T / 64];
-  const uint32_t bi = xcd_block(blockIdx.x, gridDim.x);
+  const uint32_t bi = xcd_runs(blockIdx.x, gridDim.x, run);
   const uint2 m0 = meta[bi], m1 = meta[bi + 1];
   const uint32_t r0 = m0.x, r1 = m1.x, e0 = m0.y, e1 = m1.y;
   const uint32_t tid = threadIdx.x, g = tid / LPE, l = tid % LPE, lane = tid & 63, wv = tid >> 6;
@@ -523,17 +527,17 @@ __global__ __launch_bounds__(STREAM_T, (stream_min_wg<T, KV>())) void k_spmm_str
 }
 
 template <typename T, int KV>
-static void spmm_stream_launch(uint32_t nblocks, bool off32, const uint2 *meta, const uint32_t *rp,
+static void spmm_stream_launch(uint32_t nblocks, uint32_t run, bool off32, const uint2 *meta, const uint32_t *rp,
                                const uint32_t *ci, const T *a, const T *X, T *Y, hipStream_t s)
 {
   if (off32)
-    k_spmm_stream<T, KV, true><<<nblocks, STREAM_T, 0, s>>>(meta, rp, ci, a, X, Y);
+    k_spmm_stream<T, KV, true><<<nblocks, STREAM_T, 0, s>>>(run, meta, rp, ci, a, X, Y);
   else
-    k_spmm_stream<T, KV, false><<<nblocks, STREAM_T, 0, s>>>(meta, rp, ci, a, X, Y);
+    k_spmm_stream<T, KV, false><<<nblocks, STREAM_T, 0, s>>>(run, meta, rp, ci, a, X, Y);
 }
 
 template <typename T>
-static int spmm_stream_t(uint32_t k, uint32_t cols, uint32_t nblocks, const uint2 *meta, const uint32_t *rp,
+static int spmm_stream_t(uint32_t k, uint32_t cols, uint32_t nblocks, uint32_t run, const uint2 *meta, const uint32_t *rp,
                          const uint32_t *ci, const T *a, const T *X, T *Y, hipStream_t s)
 {
   if (nblocks == 0) return MFP_OK;
@@ -541,21 +545,21 @@ static int spmm_stream_t(uint32_t k, uint32_t cols, uint32_t nblocks, const uint
   switch (k) {
   case 2:
     if constexpr (sizeof(T) == 8) {
-      spmm_stream_launch<T, 2>(nblocks, off32, meta, rp, ci, a, X, Y, s);
+      spmm_stream_launch<T, 2>(nblocks, run, off32, meta, rp, ci, a, X, Y, s);
       break;
     }
     [[fallthrough]];
   case 1: set_error("the CSR-stream SpMM needs k values to fill whole 16-byte pieces (k >= 4 for f32, >= 2 for f64)");
     return MFP_ERR_ARG;
-  case 4: spmm_stream_launch<T, 4>(nblocks, off32, meta, rp, ci, a, X, Y, s); break;
-  case 8: spmm_stream_launch<T, 8>(nblocks, off32, meta, rp, ci, a, X, Y, s); break;
-  case 16: spmm_stream_launch<T, 16>(nblocks, off32, meta, rp, ci, a, X, Y, s); break;
+  case 4: spmm_stream_launch<T, 4>(nblocks, run, off32, meta, rp, ci, a, X, Y, s); break;
+  case 8: spmm_stream_launch<T, 8>(nblocks, run, off32, meta, rp, ci, a, X, Y, s); break;
+  case 16: spmm_stream_launch<T, 16>(nblocks, run, off32, meta, rp, ci, a, X, Y, s); break;
   default: set_error("k must be 1, 2, 4, 8 or 16"); return MFP_ERR_ARG;
   }
   return hipGetLastError() == hipSuccess ? MFP_OK : (set_error("kernel launch failed"), MFP_ERR_HIP);
 }
 
-int launch_spmm_stream(int dtype, uint32_t k, uint32_t cols, uint32_t nblocks, const uint32_t *meta,
+int launch_spmm_stream(int dtype, uint32_t k, uint32_t cols, uint32_t nblocks, uint32_t run, const uint32_t *meta,
                        const uint32_t *rp, const uint32_t *ci, const void *a, const void *X, void *Y, hipStream_t s)
 {
   if (((uintptr_t)X % 16) != 0 || ((uintptr_t)Y % 16) != 0) {
@@ -564,9 +568,9 @@ int launch_spmm_stream(int dtype, uint32_t k, uint32_t cols, uint32_t nblocks, c
   }
   const uint2 *m = reinterpret_cast<const uint2 *>(meta);
   if (dtype == MFP_F32)
-    return spmm_stream_t<float>(k, cols, nblocks, m, rp, ci, (const float *)a, (const float *)X, (float *)Y, s);
+    return spmm_stream_t<float>(k, cols, nblocks, run, m, rp, ci, (const float *)a, (const float *)X, (float *)Y, s);
   if (dtype == MFP_F64)
-    return spmm_stream_t<double>(k, cols, nblocks, m, rp, ci, (const double *)a, (const double *)X, (double *)Y, s);
+    return spmm_stream_t<double>(k, cols, nblocks, run, m, rp, ci, (const double *)a, (const double *)X, (double *)Y, s);
   set_error("SpMM values must be f32 or f64");
   return MFP_ERR_ARG;
 }
@@ -620,10 +624,10 @@ int stream_meta_device(uint32_t rows, const uint32_t *rp, uint32_t **meta, uint3
 // of a wave gather neighbouring X rows, so its gathers are two or three lines
 // each, mostly in L1.  64-matrix batch, k = 4, FP32: 20M entries of grids take
 // 64 us here and 99 there, the step 230 -> 190 us; k = 2 179 -> 156, k = 8
-// 417 -> 328, k = 16 875 -> 662.  Measured
-// without gain: 2 or 4 columns per lane with wider gathers (71 to 79 us),
-// workgroups of 2, 4 or 8 row groups with the next group's loads in flight
-// (69 to 82).
+// 417 -> 328, k = 16 875 -> 662 (with an XCD on one range; in runs of 64
+// workgroups 186, 148, 318 and 643).  Measured without gain: 2 or 4 columns
+// per lane with wider gathers (71 to 79 us), workgroups of 2, 4 or 8 row
+// groups with the next group's loads in flight (69 to 82).
 constexpr uint32_t AL_T = 256, AL_CAP = 2048; // entries per chunk (FP64: half)
 constexpr uint32_t AL_U = 8;                  // gathers of a lane in flight
 constexpr uint32_t AL_MAX_ROW = 128;          // a lane walks its row alone
@@ -641,7 +645,7 @@ __global__ __launch_bounds__(AL_T) void k_spmm_aligned(uint32_t rows, uint32_t R
   __shared__ __align__(16) T sa[CAP];
   __shared__ __align__(16) uint32_t sc[CAP];
   const uint32_t per = R / RB; // workgroups per slice (R and RB are powers of two, RB <= R)
-  const uint32_t b = xcd_block(blockIdx.x, gridDim.x);
+  const uint32_t b = xcd_runs(blockIdx.x, gridDim.x, BATCH_RUN);
   const uint64_t r0 = (uint64_t)slices[b / per] * R + (uint64_t)(b % per) * RB;
   if (r0 >= rows) return;
   const uint32_t tid = threadIdx.x, j = tid % KV;
@@ -921,7 +925,7 @@ static int batch_launch(mfp_batch b, uint32_t k, const void *X, void *Y, hipStre
     return launch_spmm_binned(m->dtype, k, b->bins, b->bin_list, m->rows, m->row_ptr, m->columns, m->values, X,
                               Y, s);
   if (b->lanes == MFP_BATCH_STREAM)
-    return launch_spmm_stream(m->dtype, k, m->cols, b->nstream, b->stream_meta, m->row_ptr, m->columns, m->values, X, Y,
+    return launch_spmm_stream(m->dtype, k, m->cols, b->nstream, BATCH_RUN, b->stream_meta, m->row_ptr, m->columns, m->values, X, Y,
                               s);
   if (b->lanes == 1) {
     const uint32_t i = log2_k(k);
@@ -951,7 +955,7 @@ int mfp_plan_spmm(mfp_plan p, uint32_t k, const void *X, void *Y, mfp_stream sv)
   }
   if (p->format == MFP_CSR_ADAPTIVE && p->stream_meta) {
     const mfp_matrix m = p->m;
-    return launch_spmm_stream(p->dtype, k, m->cols, p->nstream, p->stream_meta, m->row_ptr, m->columns, m->values, X,
+    return launch_spmm_stream(p->dtype, k, m->cols, p->nstream, XCD_ONE_RUN, p->stream_meta, m->row_ptr, m->columns, m->values, X,
                               Y, as_stream(sv));
   }
   MFP_ARG(p->format == MFP_CSR_VECTOR,

@@ -97,6 +97,18 @@ __device__ __forceinline__ uint32_t xcd_block(uint32_t b, uint32_t nb)
   return xcd < rem ? xcd * (q + 1) + idx : rem * (q + 1) + (xcd - rem) * q + idx;
 }
 
+// The same in runs of 1 << run logical blocks: XCD k takes runs k, k + 8, ...
+// Where the cost of a block differs along the range (a batch of matrices of
+// several kinds), one contiguous range per XCD leaves the XCDs with the cheap
+// ones idle at the end; a run still is long enough for its rows to share x.
+constexpr uint32_t XCD_ONE_RUN = 28; // a run no grid exceeds: as xcd_block
+constexpr uint32_t BATCH_RUN = 6;
+__device__ __forceinline__ uint32_t xcd_runs(uint32_t b, uint32_t nb, uint32_t run)
+{
+  const uint32_t w = 8u << run, at = b & ~(w - 1u);
+  return at + xcd_block(b - at, min(w, nb - at));
+}
+
 // A row of X (KV values, aligned to KV * sizeof(T)) with 16-byte loads where
 // the row is a multiple of 16 bytes.
 template <typename T, int KV>

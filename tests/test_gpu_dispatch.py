@@ -347,3 +347,40 @@ def test_batch_aligned_and_random_slices(gpu, k, dtype):
     B.destroy()
     for m in mats:
         m.destroy()
+
+
+# Blocks of a batch go to the XCDs in runs of 64 (512 blocks a round): one
+# block per row of 512 entries (stream, and CSR-Adaptive with 512 per
+# workgroup), one per 64 rows of a band (aligned slices, k = 4).  Whole
+# numbers, so every order gives the same sums.
+@pytest.mark.parametrize("blocks", [31, 511, 512, 513, 543, 544, 1061])
+@pytest.mark.parametrize("form", ["stream", "rows", "aligned"])
+def test_batch_blocks_over_the_xcds(gpu, form, blocks):
+    announce(f"batch blocks over the XCDs form={form} blocks={blocks}")
+    rng = np.random.default_rng(blocks)
+    cut = blocks // 3
+    members = []
+    for n in (cut, blocks - cut):
+        if form == "aligned":
+            rp, ci, va, cols = _band(64 * n, 3, n)
+        else:
+            rp, ci, va = _csr([512] * n, 700, "float32", n)
+            cols = 700
+        members.append((rp, ci, rng.integers(-3, 4, ci.size).astype("float32"), cols))
+    mats = [gpu.DeviceMatrix.from_csr(*m) for m in members]
+    k = 1 if form == "rows" else 4
+    B = {"stream": lambda: gpu.Batch(mats, lanes=3), "rows": lambda: gpu.Batch(mats, lanes=16, nnz_per_wg=512),
+         "aligned": lambda: gpu.Batch(mats, lanes=1, flags=4, scoo_slice_size=2048, scoo_pieces=1)}[form]()
+    X = rng.integers(-5, 6, B.cols * k).astype("float32")
+    Xd, Yd = gpu.DeviceArray.from_host(X), gpu.DeviceArray(B.rows * k, np.dtype("float32"))
+    Yd.fill(np.nan)
+    B.spmm(k, Xd, Yd)
+    gpu.synchronize()
+    Y = Yd.to_host().reshape(B.rows, k)
+    for i, (rp, ci, va, cols) in enumerate(members):
+        xs = X.reshape(B.cols, k)[B.col_offsets[i]:B.col_offsets[i + 1]].astype(np.float64)
+        want = np.add.reduceat(va[:, None] * xs[ci], rp[:-1].astype(np.int64), axis=0)
+        assert np.array_equal(Y[B.row_offsets[i]:B.row_offsets[i + 1]], want), i
+    B.destroy()
+    for m in mats:
+        m.destroy()
