@@ -887,6 +887,7 @@ static int batch_cs_plan(mfp_batch b, uint32_t k, mfp_stream sv)
   if (k <= 4) t.flags |= MFP_TUNE_SCOO_WHOLE_SLICES;
   t.scoo_threads = 1024;
   MFP_CHECK(mfp_plan_create(&b->cs[i], b->big, MFP_SCOO, &t, sv));
+  b->cs[i]->cs.run = BATCH_ITEM_RUN;
   const int st = batch_split_aligned(b, i, as_stream(sv));
   if (st != MFP_OK) {
     mfp_plan_destroy(b->cs[i]);
@@ -1024,6 +1025,7 @@ int mfp_batch_create(mfp_batch *out, const mfp_matrix *ms, uint32_t count, uint3
   if (st == MFP_OK) {
     const int f = k1_tuning && (k1_tuning->flags & MFP_TUNE_SCOO_COLSORT) ? MFP_SCOO : MFP_CSR_ADAPTIVE;
     st = mfp_plan_create(&b->k1, m, f, k1_tuning, sv);
+    if (st == MFP_OK) b->k1->cs.run = BATCH_ITEM_RUN;
   }
   if (st == MFP_OK && lanes == 0) st = spmm_bins_build(m->rows, m->row_ptr, &b->bins, &b->bin_list, s);
   if (st == MFP_OK && lanes == MFP_BATCH_STREAM)

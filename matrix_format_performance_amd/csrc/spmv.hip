@@ -1146,7 +1146,7 @@ struct cs_values {
 };
 
 template <typename T, int DT>
-__global__ void k_scoo_cs(uint32_t rows, uint32_t R, uint32_t rbits, uint32_t S_reg, uint32_t NL,
+__global__ void k_scoo_cs(uint32_t run, uint32_t rows, uint32_t R, uint32_t rbits, uint32_t S_reg, uint32_t NL,
                           const uint4 *__restrict__ items, const uint32_t *__restrict__ ibase,
                           const typename cs_values<T, DT>::V *__restrict__ ev, const uint32_t *__restrict__ ec,
                           const T *__restrict__ x, T *__restrict__ y,
@@ -1156,13 +1156,14 @@ __global__ void k_scoo_cs(uint32_t rows, uint32_t R, uint32_t rbits, uint32_t S_
   using CV = cs_values<T, DT>;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   double *acc = reinterpret_cast<double *>(smem_raw);
-  const uint4 it = items[xcd_block(blockIdx.x, gridDim.x)];
+  const uint32_t item = xcd_runs(blockIdx.x, gridDim.x, run);
+  const uint4 it = items[item];
   const uint32_t sl = it.x, e0 = it.y, e1 = it.z, slot = it.w;
   const uint32_t lim = sl < S_reg ? min(R, rows - sl * R) : min(R, NL - (sl - S_reg) * R);
   const uint32_t bt = blockDim.x, tid = threadIdx.x;
   for (uint32_t i = tid; i < lim; i += bt) acc[i] = 0.0;
   __syncthreads();
-  const uint32_t cbase = ibase[xcd_block(blockIdx.x, gridDim.x)];
+  const uint32_t cbase = ibase[item];
   // head: up to the first multiple of 256 (positions stored in order)
   const uint32_t ea = (uint32_t)min<uint64_t>(e1, ((uint64_t)e0 + 255u) & ~(uint64_t)255);
   for (uint32_t i = e0 + tid; i < ea; i += bt) {
@@ -1332,7 +1333,7 @@ __global__ __launch_bounds__(CS_FIN_ROWS) void k_scoo_cs_finish(uint32_t rows, u
 // entry.  Partial slots hold R KV values, row-major like Y.
 // ---------------------------------------------------------------------------
 template <typename T, int KV>
-__global__ void k_scoo_cs_k(uint32_t rows, uint32_t R, uint32_t rbits, uint32_t S_reg, uint32_t NL,
+__global__ void k_scoo_cs_k(uint32_t run, uint32_t rows, uint32_t R, uint32_t rbits, uint32_t S_reg, uint32_t NL,
                             const uint4 *__restrict__ items, const uint32_t *__restrict__ ibase,
                             const T *__restrict__ ev, const uint32_t *__restrict__ ec, const T *__restrict__ X,
                             T *__restrict__ Y, T *__restrict__ partial, const uint32_t *__restrict__ long_rows,
@@ -1341,13 +1342,14 @@ __global__ void k_scoo_cs_k(uint32_t rows, uint32_t R, uint32_t rbits, uint32_t 
   using CV = cs_values<T, -1>;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   double *acc = reinterpret_cast<double *>(smem_raw);
-  const uint4 it = items[xcd_block(blockIdx.x, gridDim.x)];
+  const uint32_t item = xcd_runs(blockIdx.x, gridDim.x, run);
+  const uint4 it = items[item];
   const uint32_t sl = it.x, e0 = it.y, e1 = it.z, slot = it.w;
   const uint32_t lim = sl < S_reg ? min(R, rows - sl * R) : min(R, NL - (sl - S_reg) * R);
   const uint32_t bt = blockDim.x, tid = threadIdx.x;
   for (uint32_t i = tid; i < R * KV; i += bt) acc[i] = 0.0;
   __syncthreads();
-  const uint32_t cbase = ibase[xcd_block(blockIdx.x, gridDim.x)];
+  const uint32_t cbase = ibase[item];
   auto add_row = [&](uint32_t c, uint32_t lr, double v) {
     T xr[KV];
     load_row<T, KV>(X + (uint64_t)c * KV, xr);
@@ -1732,8 +1734,8 @@ static int scoo_cs_t(uint32_t rows, const scoo_cs_layout &l, uint32_t threads, c
   if (lds > 65536)
     MFP_HIP(hipFuncSetAttribute((const void *)k_scoo_cs<T, DT>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 (int)lds));
-  MFP_CHECK(launch_k(k_scoo_cs<T, DT>, dim3(l.NI), dim3(threads), (uint32_t)lds, s, rows, l.R, l.rbits, l.S_reg,
-                     l.NL, l.items, l.base, (const V *)l.ev, l.ec, (const T *)x, (T *)y, (T *)l.partial,
+  MFP_CHECK(launch_k(k_scoo_cs<T, DT>, dim3(l.NI), dim3(threads), (uint32_t)lds, s, l.run, rows, l.R, l.rbits,
+                     l.S_reg, l.NL, l.items, l.base, (const V *)l.ev, l.ec, (const T *)x, (T *)y, (T *)l.partial,
                      l.long_rows, l.long_mask));
   if (l.NF)
     MFP_CHECK(launch_k(k_scoo_cs_finish<T>, dim3(l.NF), dim3(CS_FIN_ROWS), 0, s, rows, l.R, l.S_reg, l.NL, l.NFR,
@@ -1749,7 +1751,7 @@ static int scoo_cs_k_t(uint32_t rows, const scoo_cs_layout &l, uint32_t threads,
   if (lds > 65536)
     MFP_HIP(hipFuncSetAttribute((const void *)k_scoo_cs_k<T, KV>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 (int)lds));
-  k_scoo_cs_k<T, KV><<<l.NI, threads, lds, s>>>(rows, l.R, l.rbits, l.S_reg, l.NL, l.items, l.base,
+  k_scoo_cs_k<T, KV><<<l.NI, threads, lds, s>>>(l.run, rows, l.R, l.rbits, l.S_reg, l.NL, l.items, l.base,
                                                 (const T *)l.ev, l.ec, (const T *)X, (T *)Y, (T *)l.partial,
                                                 l.long_rows, l.long_mask);
   MFP_CHECK(launched());

@@ -101,8 +101,6 @@ __device__ __forceinline__ uint32_t xcd_block(uint32_t b, uint32_t nb)
 // Where the cost of a block differs along the range (a batch of matrices of
 // several kinds), one contiguous range per XCD leaves the XCDs with the cheap
 // ones idle at the end; a run still is long enough for its rows to share x.
-constexpr uint32_t XCD_ONE_RUN = 28; // a run no grid exceeds: as xcd_block
-constexpr uint32_t BATCH_RUN = 6;
 __device__ __forceinline__ uint32_t xcd_runs(uint32_t b, uint32_t nb, uint32_t run)
 {
   const uint32_t w = 8u << run, at = b & ~(w - 1u);
