@@ -784,6 +784,58 @@ static uint32_t log2_k(uint32_t k)
   return i;
 }
 
+// The items by their number of entries, the largest first (equal ones in their
+// order): item i goes to the place that counts the items before it.
+__global__ __launch_bounds__(256) void k_items_largest_first(uint32_t n, const uint4 *__restrict__ in,
+                                                             const uint32_t *__restrict__ base,
+                                                             uint4 *__restrict__ out, uint32_t *__restrict__ out_base)
+{
+  const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+  if (i >= n) return;
+  const uint4 it = in[i];
+  const uint32_t len = it.z - it.y;
+  uint32_t at = 0;
+  for (uint32_t j = 0; j < n; j++) {
+    const uint32_t o = in[j].z - in[j].y;
+    at += o > len || (o == len && j < i) ? 1u : 0u;
+  }
+  out[at] = it;
+  out_base[at] = base[i];
+}
+
+// The order and the XCDs of a batch's column-sorted items.  Up to four per CU
+// they differ most in what they cost (a slice of a random matrix holds three
+// times one of a power-law matrix) and there is one round of them or two, so
+// the largest go first, XCD after XCD: a batch of 64, k = 2 (266 items) 150 ->
+// 121 us, k = 4 (521) 179 -> 176; of 130, k = 4 (900) 288 -> 276.  With more,
+// those of one matrix side by side share X in the L2 (a batch of 200, k = 4,
+// 1,700 items: 489 us in runs of 8, 532 largest first).
+constexpr uint32_t BATCH_FEW_ITEMS = 4; // per CU
+static int batch_order_items(scoo_cs_layout &l, hipStream_t s)
+{
+  l.run = BATCH_ITEM_RUN;
+  if (l.NI < 2 || l.NI > BATCH_FEW_ITEMS * (uint32_t)std::max(1, props().cu_count)) return MFP_OK;
+  uint4 *items = nullptr;
+  uint32_t *base = nullptr;
+  int st = dmalloc((void **)&items, (uint64_t)l.NI * sizeof(uint4));
+  if (st == MFP_OK) st = dmalloc((void **)&base, (uint64_t)l.NI * 4);
+  if (st == MFP_OK) {
+    k_items_largest_first<<<ceil_div_u32(l.NI, 256), 256, 0, s>>>(l.NI, l.items, l.base, items, base);
+    if (hipGetLastError() != hipSuccess || hipStreamSynchronize(s) != hipSuccess) {
+      set_error("column-sorted items: kernel failed");
+      st = MFP_ERR_HIP;
+    }
+  }
+  if (st == MFP_OK) {
+    std::swap(l.items, items);
+    std::swap(l.base, base);
+    l.run = 0;
+  }
+  dfree(items);
+  dfree(base);
+  return st;
+}
+
 // Takes the slices with aligned rows out of the column-sorted plan's items
 // (those whose single item writes Y directly) and lists them for
 // k_spmm_aligned.
@@ -887,8 +939,8 @@ static int batch_cs_plan(mfp_batch b, uint32_t k, mfp_stream sv)
   if (k <= 4) t.flags |= MFP_TUNE_SCOO_WHOLE_SLICES;
   t.scoo_threads = 1024;
   MFP_CHECK(mfp_plan_create(&b->cs[i], b->big, MFP_SCOO, &t, sv));
-  b->cs[i]->cs.run = BATCH_ITEM_RUN;
-  const int st = batch_split_aligned(b, i, as_stream(sv));
+  int st = batch_split_aligned(b, i, as_stream(sv));
+  if (st == MFP_OK) st = batch_order_items(b->cs[i]->cs, as_stream(sv));
   if (st != MFP_OK) {
     mfp_plan_destroy(b->cs[i]);
     b->cs[i] = nullptr;
@@ -1025,7 +1077,7 @@ int mfp_batch_create(mfp_batch *out, const mfp_matrix *ms, uint32_t count, uint3
   if (st == MFP_OK) {
     const int f = k1_tuning && (k1_tuning->flags & MFP_TUNE_SCOO_COLSORT) ? MFP_SCOO : MFP_CSR_ADAPTIVE;
     st = mfp_plan_create(&b->k1, m, f, k1_tuning, sv);
-    if (st == MFP_OK) b->k1->cs.run = BATCH_ITEM_RUN;
+    if (st == MFP_OK) st = batch_order_items(b->k1->cs, s);
   }
   if (st == MFP_OK && lanes == 0) st = spmm_bins_build(m->rows, m->row_ptr, &b->bins, &b->bin_list, s);
   if (st == MFP_OK && lanes == MFP_BATCH_STREAM)

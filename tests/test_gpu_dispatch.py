@@ -384,3 +384,33 @@ def test_batch_blocks_over_the_xcds(gpu, form, blocks):
     B.destroy()
     for m in mats:
         m.destroy()
+
+
+# Column-sorted items of a batch: largest first up to 4 per CU (256 threads a
+# workgroup rank them), in runs of 8 above.  Whole numbers, as above.
+@pytest.mark.parametrize("slices", [1, 2, 3, 255, 256, 257, 1023, 1024, 1025, 1060])
+def test_batch_column_sorted_items(gpu, slices):
+    announce(f"batch column-sorted items slices={slices}")
+    rng = np.random.default_rng(slices)
+    cut = slices // 2
+    members = []
+    for n in (cut, slices - cut):
+        if n:
+            lens = rng.integers(0, 4, 512 * n) * rng.integers(0, 2, n).repeat(512) + 1  # equal and unequal items
+            rp, ci, _ = _csr(lens, 1500, "float32", n)
+            members.append((rp, ci, rng.integers(-3, 4, ci.size).astype("float32"), 1500))
+    mats = [gpu.DeviceMatrix.from_csr(*m) for m in members]
+    B = gpu.Batch(mats, lanes=1, flags=4, scoo_slice_size=512, scoo_pieces=1)
+    X = rng.integers(-5, 6, B.cols).astype("float32")
+    Xd, Yd = gpu.DeviceArray.from_host(X), gpu.DeviceArray(B.rows, np.dtype("float32"))
+    Yd.fill(np.nan)
+    B.spmm(1, Xd, Yd)
+    gpu.synchronize()
+    Y = Yd.to_host()
+    for i, (rp, ci, va, cols) in enumerate(members):
+        xs = X[B.col_offsets[i]:B.col_offsets[i + 1]].astype(np.float64)
+        want = np.add.reduceat(va * xs[ci], rp[:-1].astype(np.int64))
+        assert np.array_equal(Y[B.row_offsets[i]:B.row_offsets[i + 1]], want), i
+    B.destroy()
+    for m in mats:
+        m.destroy()
