@@ -910,7 +910,8 @@ static int launch_spmm_aligned(const mfp_batch_s *b, uint32_t i, const void *X, 
 // lanes == 1: the column-sorted plan for k columns, built on first use (never
 // inside a graph capture): the largest slice (a power of two, up to 16384
 // rows) whose R k double accumulators fill at most half of the LDS, so that
-// two workgroups share a CU, but never below 1024 rows; 1024 threads.
+// two workgroups share a CU, but never below 1024 rows; smaller where that
+// leaves CUs without a slice; 1024 threads.
 static int batch_cs_plan(mfp_batch b, uint32_t k, mfp_stream sv)
 {
   const uint32_t i = log2_k(k);
@@ -928,6 +929,13 @@ static int batch_cs_plan(mfp_batch b, uint32_t k, mfp_stream sv)
   // 6,787 us).
   t.scoo_slice_size = 16384;
   while (t.scoo_slice_size > 1024 && (uint64_t)t.scoo_slice_size * k * 8 > 81920) t.scoo_slice_size /= 2;
+  // a slice per CU at least, as far as 256 rows: a slice is one workgroup, and
+  // a batch of few rows left most CUs without one.  407k rows (16 matrices),
+  // k = 2, 4: 72 -> 46, 82 -> 74 us (99, 199 -> 397 slices); 197k (6), k = 2, 4,
+  // 8: 65 -> 20, 64 -> 27, 74 -> 46.  Beyond it a smaller slice reads X more
+  // often: 1.3M rows, k = 4, 647 slices 112 us, 1,294 130, 2,588 163.
+  while (t.scoo_slice_size > 256 && b->big->rows / t.scoo_slice_size < (uint32_t)std::max(1, props().cu_count))
+    t.scoo_slice_size /= 2;
   // one piece per slice: a slice of the block-diagonal batch seldom spans
   // more than one column band, so most slices write Y directly and skip the
   // partial round trip of R k values per slot (k = 4: 1.70 against 1.80 ms
