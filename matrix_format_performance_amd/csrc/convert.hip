@@ -173,10 +173,18 @@ int exclusive_scan_u32(const uint32_t *in, uint32_t *out, uint64_t n, hipStream_
 //   k_sort_offsets  one workgroup per digit: exclusive scan over the tiles
 //   k_sort_scatter  ranks a tile's entries by digit (ballots inside a wave,
 //                   LDS counts across waves), reorders them in LDS and
-//                   writes each digit's run to its place: 8192 entries make
-//                   runs of 32 on average, so the stores are whole lines
+//                   writes each digit's run to its place
+// Bound by the writes: 4096 entries make runs of 16 on average, so most lines
+// are written by two tiles or more.  Tiles side by side are on one XCD (runs of
+// 32 tiles) and so complete each other's lines in its L2, which is what lets a
+// tile be this small, with three workgroups per CU to overlap the loads, the
+// ranking and the stores.  11.7M FP32 entries, a pass of 281 MB: tiles dealt
+// round robin 82 us (8192 entries) and 85 (4096), on one XCD 76 and 67; 3072
+// entries 70, 2048 79; the first pass, which reads doubles, 115 -> 78; with
+// runs of 64 tiles the same, of 16 or 256 and one range per XCD 2% slower.
 // ---------------------------------------------------------------------------
 constexpr uint32_t SORT_T = 512, SORT_W = SORT_T / 64, SORT_BINS = 256;
+constexpr uint32_t SORT_RUN = 5; // log2 of the tiles an XCD takes in a row
 
 struct sort_digit {
   uint32_t row_shift; // row bits below this do not take part
@@ -201,7 +209,8 @@ __global__ __launch_bounds__(SORT_T) void k_sort_count(const uint32_t *__restric
   const uint32_t t = threadIdx.x;
   if (t < SORT_BINS) cnt[t] = 0;
   __syncthreads();
-  const uint64_t base = (uint64_t)blockIdx.x * (SORT_T * ITEMS);
+  const uint32_t tile = xcd_runs(blockIdx.x, gridDim.x, SORT_RUN);
+  const uint64_t base = (uint64_t)tile * (SORT_T * ITEMS);
   const bool need_row = CHECK || dg.shift + dg.width > dg.col_bits, need_col = CHECK || dg.shift < dg.col_bits;
   uint32_t r[ITEMS], c[ITEMS];
 #pragma unroll
@@ -219,7 +228,7 @@ __global__ __launch_bounds__(SORT_T) void k_sort_count(const uint32_t *__restric
     }
   if (CHECK && out) atomicOr(bad, 1u);
   __syncthreads();
-  if (t < (1u << dg.width)) hist[(uint64_t)t * ntiles + blockIdx.x] = cnt[t];
+  if (t < (1u << dg.width)) hist[(uint64_t)t * ntiles + tile] = cnt[t];
 }
 
 // row d of hist to its exclusive scan, its total to totals[d]
@@ -243,7 +252,7 @@ __global__ __launch_bounds__(1024) void k_sort_offsets(uint32_t ntiles, uint32_t
 // VI: the values' type as read (the first pass of a triplet sort rounds
 // double values to the matrix's type), V: as moved and written
 template <typename VI, typename V, uint32_t ITEMS>
-__global__ __launch_bounds__(SORT_T, ITEMS > 8 ? 4 : 6) void k_sort_scatter(const uint32_t *__restrict__ row,
+__global__ __launch_bounds__(SORT_T, 6) void k_sort_scatter(const uint32_t *__restrict__ row,
                                                          const uint32_t *__restrict__ col,
                                                          const VI *__restrict__ val, uint64_t n, sort_digit dg,
                                                          uint32_t ntiles, const uint32_t *__restrict__ hist,
@@ -260,7 +269,8 @@ __global__ __launch_bounds__(SORT_T, ITEMS > 8 ? 4 : 6) void k_sort_scatter(cons
   uint32_t *buf = reinterpret_cast<uint32_t *>(buf_raw);
   V *vbuf = reinterpret_cast<V *>(buf_raw);
   const uint32_t t = threadIdx.x, lane = t & 63u, wave = t >> 6;
-  const uint64_t base = (uint64_t)blockIdx.x * TILE;
+  const uint32_t tile = xcd_runs(blockIdx.x, gridDim.x, SORT_RUN);
+  const uint64_t base = (uint64_t)tile * TILE;
   const uint32_t m = (uint32_t)min((uint64_t)TILE, n - base); // entries of this tile
   // wave w holds entries w 64 ITEMS .. of the tile, 64 consecutive per item
   const uint32_t l0 = wave * 64u * ITEMS + lane;
@@ -309,7 +319,7 @@ __global__ __launch_bounds__(SORT_T, ITEMS > 8 ? 4 : 6) void k_sort_scatter(cons
   const uint32_t gt = block_exclusive_scan<SORT_T>(tot, sh, nullptr);
   if (t < SORT_BINS) {
     start[t] = st;
-    glob[t] = t < (1u << dg.width) ? gt + hist[(uint64_t)t * ntiles + blockIdx.x] - st : 0u;
+    glob[t] = t < (1u << dg.width) ? gt + hist[(uint64_t)t * ntiles + tile] - st : 0u;
   }
   __syncthreads();
 #pragma unroll
@@ -419,10 +429,10 @@ static int sort_entries(const uint32_t *row, const uint32_t *col, const VI *val,
                         uint64_t key_rows, uint32_t rows, uint32_t cols, const sort_arrays<V> &to,
                         const sort_arrays<V> &via, uint32_t *bad, hipStream_t s)
 {
-  // 8192 entries per tile (FP64 values: 4096, 32 KB of LDS either way), 2048
-  // where those would be fewer than two per CU
-  if (n >= (1u << 22))
-    return sort_entries_t<VI, V, sizeof(V) == 8 ? 8 : 16>(row, col, val, n, row_shift, key_rows, rows, cols, to, via, bad, s);
+  // 4096 entries per tile, 2048 where those would be fewer than two per CU
+  // (1.2M entries: 147 us against 157; 2M: 155 each)
+  if (n >= (1u << 21))
+    return sort_entries_t<VI, V, 8>(row, col, val, n, row_shift, key_rows, rows, cols, to, via, bad, s);
   return sort_entries_t<VI, V, 4>(row, col, val, n, row_shift, key_rows, rows, cols, to, via, bad, s);
 }
 
