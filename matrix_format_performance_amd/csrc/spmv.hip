@@ -374,6 +374,16 @@ __global__ __launch_bounds__(256, 8) void k_csr_vector_lds(uint32_t rows, uint32
 //     partial a lane carries into the next enters a 256-lane Hillis-Steele
 //     segmented scan; a row ending in lane j that began earlier is
 //     scan[j-1] + lane j's partial.
+//     A block spends its time waiting, phase after phase, so the phases are
+//     kept short and side by side: the row starts are loaded before the
+//     gathers and searched while these are in flight (they came after the
+//     products), gathers are unconditional, products lie where the lanes'
+//     runs read them from different banks, and the scan takes as many steps
+//     as the longest carried row needs, one barrier each (eight steps of two).
+//     27-point grid of 100^3 f32 58.6 -> 52.6 us, f64 93.4 -> 72.3; 300k rows
+//     of 34 f32 60.4 -> 53.0, f64 71.4 -> 57.6 (random gathers alone 48.5 and
+//     57); 1M power-law rows f32 84.4 -> 81.6, f64 139 as before (x of 8 MB is
+//     past an XCD's L2: its gathers alone take 125).
 //   single-row block (CSR-Vector/VectorL): 256 lanes strided with fma, a
 //     64-lane halving tree per wave, then a halving tree over the 4 waves.
 //   rows longer than long_row: split into `chunk`-element pieces, one
@@ -413,12 +423,27 @@ __device__ __forceinline__ T wg_row_sum(const uint32_t *__restrict__ ci, const T
   return r;
 }
 
+// Place of staged product e: lanes read runs of 8 (FP32) or 4 (FP64) side by
+// side, and a gap after each keeps their reads on different banks.
+template <typename T>
+__host__ __device__ constexpr uint32_t adaptive_slot(uint32_t e)
+{
+  return e + (sizeof(T) == 4 ? e >> 3 : e >> 2);
+}
+
+// bytes of the staged products, a multiple of 16
+template <typename T>
+__host__ __device__ constexpr uint32_t adaptive_products(uint32_t W)
+{
+  return (adaptive_slot<T>(W) * (uint32_t)sizeof(T) + 15u) & ~15u;
+}
+
 template <typename T>
 struct adaptive_smem {
-  T *cache;     // staged products (nnz_per_wg)
+  T *cache;     // staged products (nnz_per_wg, by adaptive_slot)
   uint32_t *rs; // block-relative row starts (nnz_per_wg + 2)
-  T *wsum, *sv;
-  uint32_t *sf;
+  T *wsum, *sv; // sv: 2 AD_T
+  uint32_t *wsteps;
 };
 
 // One work item of the launch: hw is the item's dispatch index among grid
@@ -440,7 +465,6 @@ __device__ __forceinline__ void adaptive_item(
   T *cache = sm.cache;
   uint32_t *rs = sm.rs;
   T *wsum = sm.wsum, *sv = sm.sv;
-  uint32_t *sf = sm.sf;
   const uint32_t tid = threadIdx.x;
 
   if (hw < nchunks_pad) {
@@ -482,28 +506,26 @@ __device__ __forceinline__ void adaptive_item(
       vc[k] = ldg_stream(cv + v);
     }
   }
+  // the row starts are on their way before the gathers, which are in flight
+  // while the rows are searched
+  const uint32_t nr = r1 - r0;
+  const uint32_t p0 = tid <= nr ? rp[r0 + tid] : 0u, p1 = tid + AD_T <= nr ? rp[r0 + tid + AD_T] : 0u;
   T xv[K][N];
+  if (n) { // without entries x may be empty
 #pragma unroll
-  for (uint32_t k = 0; k < K; k++) {
-    const uint32_t v = v0 + tid + k * AD_T;
+    for (uint32_t k = 0; k < K; k++) {
+      const uint32_t v = v0 + tid + k * AD_T;
 #pragma unroll
-    for (uint32_t j = 0; j < N; j++) {
-      const uint32_t e = v * N + j;
-      xv[k][j] = (v < v1 && e >= base && e < base + n) ? x[vc[k][j]] : (T)0;
-    }
-  }
-#pragma unroll
-  for (uint32_t k = 0; k < K; k++) {
-    const uint32_t v = v0 + tid + k * AD_T;
-#pragma unroll
-    for (uint32_t j = 0; j < N; j++) {
-      const uint32_t e = v * N + j;
-      if (v < v1 && e >= base && e < base + n) cache[e - base] = va[k][j] * xv[k][j];
+      for (uint32_t j = 0; j < N; j++) {
+        const uint32_t e = v * N + j;
+        xv[k][j] = x[v < v1 && e >= base && e < base + n ? vc[k][j] : 0u]; // outside the block: x[0], not used
+      }
     }
   }
   // block-relative row starts rs[0..nr]
-  const uint32_t nr = r1 - r0;
-  for (uint32_t lr = tid; lr <= nr; lr += AD_T) rs[lr] = rp[r0 + lr] - base;
+  if (tid <= nr) rs[tid] = p0 - base;
+  if (tid + AD_T <= nr) rs[tid + AD_T] = p1 - base;
+  for (uint32_t lr = tid + 2 * AD_T; lr <= nr; lr += AD_T) rs[lr] = rp[r0 + lr] - base;
   __syncthreads();
   for (uint32_t lr = tid; lr < nr; lr += AD_T)
     if (rs[lr] == rs[lr + 1]) y[r0 + lr] = (T)0; // empty rows
@@ -512,20 +534,32 @@ __device__ __forceinline__ void adaptive_item(
   const uint32_t E = (nnz_per_wg + AD_T - 1) / AD_T;
   const uint32_t e0 = tid * E;
   const uint32_t e1 = min(n, e0 + E);
-  T carry_v = 0;       // partial carried into the next lane
-  uint32_t carry_f = 1; // 1: no chain comes in from the left
-  uint32_t frow = 0xFFFFFFFFu;
-  T fval = 0;
+  uint32_t cur = 0;
   if (e0 < e1) {
-    uint32_t lo = 0, hi = nr; // rs[lo] <= e0 < rs[hi]
-    while (hi - lo > 1) {
-      const uint32_t mid = (lo + hi) >> 1;
+    uint32_t hi = nr; // rs[cur] <= e0 < rs[hi]
+    while (hi - cur > 1) {
+      const uint32_t mid = (cur + hi) >> 1;
       if (rs[mid] <= e0)
-        lo = mid;
+        cur = mid;
       else
         hi = mid;
     }
-    uint32_t cur = lo;
+  }
+#pragma unroll
+  for (uint32_t k = 0; k < K; k++) {
+    const uint32_t v = v0 + tid + k * AD_T;
+#pragma unroll
+    for (uint32_t j = 0; j < N; j++) {
+      const uint32_t e = v * N + j;
+      if (v < v1 && e >= base && e < base + n) cache[adaptive_slot<T>(e - base)] = va[k][j] * xv[k][j];
+    }
+  }
+  __syncthreads();
+  T carry_v = 0;     // partial carried into the next lane
+  uint32_t back = 0; // lanes back to the one where the carried row begins
+  uint32_t frow = 0xFFFFFFFFu;
+  T fval = 0;
+  if (e0 < e1) {
     uint32_t cur_start = rs[cur], cur_end = rs[cur + 1];
     uint32_t seg = e0;
     T d = 0;
@@ -545,7 +579,7 @@ __device__ __forceinline__ void adaptive_item(
         cur_start = cur_end;
         cur_end = rs[cur + 1];
       }
-      d = d + cache[e];
+      d = d + cache[adaptive_slot<T>(e)];
     }
     const bool starts = seg == cur_start;
     if (e1 == cur_end) {
@@ -557,39 +591,35 @@ __device__ __forceinline__ void adaptive_item(
       }
     } else {
       carry_v = d;
-      carry_f = starts ? 1u : 0u;
+      if (!starts) back = tid - cur_start / E;
     }
   }
-  // segmented inclusive scan of the carried partials (Hillis-Steele)
+  // segmented inclusive scan of the carried partials (Hillis-Steele), as many
+  // steps as the longest way back takes; the two halves of sv take turns
+  uint32_t steps = 0;
+  while (__ballot(back >= (1u << steps))) steps++;
   sv[tid] = carry_v;
-  sf[tid] = carry_f;
+  if ((tid & 63u) == 0) sm.wsteps[tid >> 6] = steps;
   __syncthreads();
-  for (uint32_t off = 1; off < AD_T; off <<= 1) {
-    const bool take = sf[tid] == 0u && tid >= off;
-    T pv = 0;
-    uint32_t pf = 0;
-    if (take) {
-      pv = sv[tid - off];
-      pf = sf[tid - off];
-    }
-    __syncthreads();
-    if (take) {
-      sv[tid] = pv + sv[tid];
-      sf[tid] = pf;
-    }
+  steps = max(max(sm.wsteps[0], sm.wsteps[1]), max(sm.wsteps[2], sm.wsteps[3]));
+  for (uint32_t i = 0; i < steps; i++) {
+    const uint32_t off = 1u << i, from = (i & 1u) * AD_T + tid;
+    T v = sv[from];
+    if (back >= off) v = sv[from - off] + v;
+    sv[AD_T - (i & 1u) * AD_T + tid] = v;
     __syncthreads();
   }
-  if (frow != 0xFFFFFFFFu) y[r0 + frow] = sv[tid - 1] + fval;
+  if (frow != 0xFFFFFFFFu) y[r0 + frow] = sv[(steps & 1u) * AD_T + tid - 1] + fval;
 }
 
 #define ADAPTIVE_SMEM(T)                                                                       \
   extern __shared__ __align__(16) unsigned char smem_raw[];                                    \
   __shared__ T wsum_[4];                                                                       \
-  __shared__ T sv_[AD_T];                                                                      \
-  __shared__ uint32_t sf_[AD_T];                                                               \
+  __shared__ T sv_[2 * AD_T];                                                                  \
+  __shared__ uint32_t wsteps_[4];                                                              \
   adaptive_smem<T> sm{reinterpret_cast<T *>(smem_raw),                                         \
-                      reinterpret_cast<uint32_t *>(smem_raw + ((nnz_per_wg * sizeof(T) + 15u) & ~15u)), \
-                      wsum_, sv_, sf_};
+                      reinterpret_cast<uint32_t *>(smem_raw + adaptive_products<T>(nnz_per_wg)), \
+                      wsum_, sv_, wsteps_};
 
 template <typename T, uint32_t K>
 __global__ __launch_bounds__(AD_T) void k_csr_adaptive(
@@ -1548,9 +1578,10 @@ static int adaptive_launch_k(const adaptive_args &g, const T *a, const T *x, T *
 }
 
 // Dynamic LDS of k_csr_adaptive: the staged products, then the row starts.
-size_t adaptive_lds_bytes(int dtype, uint32_t W)
+template <typename T>
+static size_t adaptive_lds_bytes(uint32_t W)
 {
-  return ((W * dtype_size(dtype) + 15u) & ~size_t(15)) + ((size_t)W + 2) * 4;
+  return adaptive_products<T>(W) + ((size_t)W + 2) * 4;
 }
 
 template <typename T>
@@ -1559,7 +1590,7 @@ static int adaptive_t(const adaptive_args &g, const T *a, const T *x, T *y, hipS
   // chunk items first; padded to a multiple of 8 so block ids keep their XCD
   const uint32_t nchunks_pad = (g.nchunks + 7u) & ~7u;
   const uint32_t items = g.nblocks ? g.nblocks + nchunks_pad : nchunks_pad;
-  const size_t lds = adaptive_lds_bytes(sizeof(T) == 4 ? MFP_F32 : MFP_F64, g.nnz_per_wg);
+  const size_t lds = adaptive_lds_bytes<T>(g.nnz_per_wg);
   const uint32_t K = adaptive_vectors_per_lane(sizeof(T) == 4 ? MFP_F32 : MFP_F64, g.nnz_per_wg);
   // persistent: 8 workgroups per CU (the LDS/wave occupancy), a multiple of 8
   uint32_t pgrid = 0;

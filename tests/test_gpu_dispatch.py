@@ -116,6 +116,8 @@ def _triplets(rows, cols, n, seed, dup):
 @pytest.mark.parametrize("rows,cols,n,dup", [
     (1, 1, 1, 0), (1, 1, 3000, 0), (3, 2, 2047, 0), (257, 256, 2048, 0), (256, 257, 2049, 0), (65537, 1, 5000, 0),
     (1, 100000, 6001, 0), (1000003, 1000003, 70001, 0), (4294967295 // 64, 4294967295, 4097, 0),
+    (70000, 70000, (1 << 21) - 1, 3), (1023, 5000, 1 << 21, 0), (1024, 100, (1 << 21) + 4097, 0),
+    (5, 3000, 70000, 0), (30, 3000, 2200000, 0), (5000, 30000, 300, 7),
     (50000, 50000, (1 << 22) - 1, 50), (50000, 300, 1 << 22, 0), (1 << 20, 1 << 20, (1 << 22) + 8193, 7)])
 def test_triplets_any_size(gpu, rows, cols, n, dup, dtype):
     announce(f"triplets rows={rows} cols={cols} n={n} dup={dup} dtype={dtype}")
@@ -414,3 +416,26 @@ def test_batch_column_sorted_items(gpu, slices):
     B.destroy()
     for m in mats:
         m.destroy()
+
+
+# CSR-Adaptive row blocks: a lane sums ceil(W / 256) products, a carried row
+# reaches back over up to 255 lanes, the row starts come in 256, 512 and more;
+# block and run edges, empty rows, the smallest and largest W.
+ADAPTIVE_ROWS = {
+    "over many lanes": [2039, 1, 2040, 7, 0, 0, 1021, 1019, 1, 1020, 3, 511, 513, 8, 8, 8, 4, 4, 9] * 3,
+    "more rows than 512": [0] * 700 + [3] + [0] * 600 + [5] * 300 + [0] * 255 + [1] * 3000,
+    "whole runs": [8] * 255 + [16] * 64 + [64] * 33 + [256] * 9 + [0, 1, 2, 3, 4, 5, 6, 7] * 40,
+    "empty": [0] * 1500,
+    "one": [1],
+}
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("W", [1, 5, 255, 257, 1020, 2040, 8190])
+@pytest.mark.parametrize("rows", list(ADAPTIVE_ROWS))
+def test_csr_adaptive_row_blocks(gpu, rows, W, dtype):
+    rp, ci, va = _csr(ADAPTIVE_ROWS[rows], 5003, dtype)
+    x = gpu.generate_vector(5, 5003, np.dtype(dtype))
+    x[0] = np.nan  # vectors past a block's elements gather x[0]; none may reach a sum
+    y = _spmv(gpu, rp, ci, va, x, "csr_adaptive", nnz_per_wg=W, long_row=4096, chunk=4096)
+    assert np.array_equal(y, oracle.spmv_adaptive(rp, ci, va, x, W, 256, 4096, 4096))
