@@ -223,13 +223,17 @@ __global__ __launch_bounds__(256) void k_csr_vector(uint32_t rows, const uint32_
 // each after the last, and a row's 136 bytes are read in 4-byte loads.  Here
 // a workgroup's loads are independent of its row lengths: 16 bytes per lane,
 // two vectors of values and of columns, then their 8 (FP64: 4) gathers.
-// Eight workgroups share a CU (16 KB of LDS, 44 to 56 VGPRs).  FP32, lanes
-// from the mean, before -> now: 27-point stencil of 100^3 121.7 -> 53.7 us,
-// 5-point stencil of 1400^2 56.8 -> 25.6, 300,007 rows of 4 to 64 random
-// entries 75.4 -> 58 (the gathers alone take 48.5), power-law 1M rows
-// 342 -> 165 (its 50,000-entry row is one wait per 1,984 entries instead of
-// one per 8 per lane).  Larger chunks were slower: three vectors per lane
-// 59.5 and four 70.6 us on the 27-point stencil, against 55.5.
+// Eight workgroups share a CU (16 KB of LDS, 44 to 56 VGPRs).  Where the
+// rows fit at once, their values and columns are on the way before the row
+// starts are staged, and the gathers go out together behind that barrier:
+// 300,007 rows of 4 to 64 random entries 58.7 -> 53.1 us (FP64 72.5 -> 61.5);
+// without the barrier between a wave's loads and its gathers 57 to 61 (71 to
+// 72).  FP32, lanes from the mean, row by row -> from LDS: 27-point stencil of
+// 100^3 121.7 -> 54.2 us, 5-point stencil of 1400^2 56.8 -> 22.5, those random
+// rows 75.4 -> 53.1 (the gathers alone take 48.5), power-law 1M rows 342 -> 169
+// (its 50,000-entry row is one wait per 1,984 entries instead of one per 8 per
+// lane).  Larger chunks were slower: three vectors per lane 59.5 and four 70.6
+// us on the 27-point stencil, against 55.5.
 constexpr uint32_t CVL_K = 2, CVL_U = 2;
 template <typename T>
 struct cvl {
@@ -238,10 +242,11 @@ struct cvl {
   static constexpr uint32_t CHUNK = CAP - 64;
 };
 
-// Elements [base, base + n) into LDS at (element - base / N N); n + base % N <= CAP
-template <typename T>
+// Elements [base, base + n) into LDS at (element - base / N N); n + base % N <=
+// CAP.  between() runs after the loads are issued and before the gathers.
+template <typename T, typename F>
 __device__ __forceinline__ void cvl_stage(uint32_t base, uint32_t n, const uint32_t *__restrict__ ci,
-                                          const T *__restrict__ a, const T *__restrict__ x, T *sa, T *sx)
+                                          const T *__restrict__ a, const T *__restrict__ x, T *sa, T *sx, F between)
 {
   using VT = vec16<T>;
   constexpr uint32_t N = VT::N, K = cvl<T>::K;
@@ -256,6 +261,7 @@ __device__ __forceinline__ void cvl_stage(uint32_t base, uint32_t n, const uint3
     va[k] = ldg_stream(av + v);
     vc[k] = ldg_stream(cv + v);
   }
+  between();
   const uint32_t lo = base - v0 * N, hi = lo + n; // the vectors' elements that count
 #pragma unroll
   for (uint32_t k = 0; k < K; k++)
@@ -286,18 +292,28 @@ __global__ __launch_bounds__(256, 8) void k_csr_vector_lds(uint32_t rows, uint32
   __shared__ uint32_t rs[257];
   const uint32_t r0 = xcd_block(blockIdx.x, gridDim.x) * RB; // RB <= 256
   const uint32_t nr = min(RB, rows - r0), tid = threadIdx.x;
-  if (tid <= nr) rs[tid] = rp[r0 + tid];
-  if (tid == 0 && nr == 256u) rs[256] = rp[r0 + 256u];
-  __syncthreads();
+  const uint32_t p = tid <= nr ? rp[r0 + tid] : 0u, first = rp[r0], last = rp[r0 + nr];
+  const bool all = last - first <= CAP - first % N; // the usual case: every row fits at once
+  auto row_starts = [&] {
+    if (tid <= nr) rs[tid] = p;
+    if (tid == 0 && nr == 256u) rs[256] = last;
+    __syncthreads();
+  };
+  if (all && last > first) {
+    cvl_stage(first, last - first, ci, a, x, sa, sx, row_starts);
+    __syncthreads();
+  } else {
+    row_starts();
+  }
   const uint32_t lane = tid % G, grp = tid / G;
   for (uint32_t cur = 0; cur < nr;) {
     const uint32_t base = rs[cur], off = base % N;
-    if (rs[cur + 1] - base > CAP - off) {
+    if (!all && rs[cur + 1] - base > CAP - off) {
       const uint32_t e = rs[cur + 1];
       T dot = 0;
       for (uint32_t c0 = base; c0 < e; c0 += CHUNK) {
         const uint32_t n = min(CHUNK, e - c0);
-        cvl_stage(c0, n, ci, a, x, sa, sx);
+        cvl_stage(c0, n, ci, a, x, sa, sx, [] {});
         __syncthreads();
         if (tid < G) {
           const uint32_t sh = c0 % N;
@@ -324,10 +340,13 @@ __global__ __launch_bounds__(256, 8) void k_csr_vector_lds(uint32_t rows, uint32
       continue;
     }
     // whole rows that fit behind base
-    const uint32_t fit = (uint32_t)__syncthreads_count(tid >= cur && tid < nr && rs[tid + 1] - base <= CAP - off);
-    const uint32_t end = cur + fit, n = rs[end] - base;
-    if (n) cvl_stage(base, n, ci, a, x, sa, sx);
-    __syncthreads();
+    uint32_t end = nr;
+    if (!all) {
+      end = cur + (uint32_t)__syncthreads_count(tid >= cur && tid < nr && rs[tid + 1] - base <= CAP - off);
+      const uint32_t n = rs[end] - base;
+      if (n) cvl_stage(base, n, ci, a, x, sa, sx, [] {});
+      __syncthreads();
+    }
     const uint32_t org = base - off;
     // U rows of a group side by side; the wave's groups stay together
     constexpr uint32_t ST = 256u / G, U = CVL_U;
@@ -357,6 +376,7 @@ __global__ __launch_bounds__(256, 8) void k_csr_vector_lds(uint32_t rows, uint32
       for (uint32_t q = 0; q < U; q++)
         if (lane == 0 && r + q * ST < end) y[r0 + r + q * ST] = dot[q];
     }
+    if (all) return;
     __syncthreads();
     cur = end;
   }
