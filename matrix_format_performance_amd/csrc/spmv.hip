@@ -395,15 +395,17 @@ __global__ __launch_bounds__(256, 8) void k_csr_vector_lds(uint32_t rows, uint32
 //     segmented scan; a row ending in lane j that began earlier is
 //     scan[j-1] + lane j's partial.
 //     A block spends its time waiting, phase after phase, so the phases are
-//     kept short and side by side: the row starts are loaded before the
-//     gathers and searched while these are in flight (they came after the
-//     products), gathers are unconditional, products lie where the lanes'
-//     runs read them from different banks, and the scan takes as many steps
-//     as the longest carried row needs, one barrier each (eight steps of two).
-//     27-point grid of 100^3 f32 58.6 -> 52.6 us, f64 93.4 -> 72.3; 300k rows
-//     of 34 f32 60.4 -> 53.0, f64 71.4 -> 57.6 (random gathers alone 48.5 and
-//     57); 1M power-law rows f32 84.4 -> 81.6, f64 139 as before (x of 8 MB is
-//     past an XCD's L2: its gathers alone take 125).
+//     kept short and side by side: the row starts are loaded beside the
+//     entries (they came after the products), the gathers go out together
+//     behind the barrier that stages them and are in flight while the rows
+//     are searched, products lie where the lanes' runs read them from
+//     different banks, and the scan takes as many steps as the longest
+//     carried row needs, one barrier each (it took eight of two).  27-point
+//     grid of 100^3 f32 58.6 -> 52.5 us, f64 93.4 -> 67.9; 300k rows of 34
+//     random entries f32 60.4 -> 51.2, f64 71.4 -> 54.6; 1M power-law rows f32
+//     84.4 -> 79.0, f64 139 -> 138 (x of 8 MB is past an XCD's L2: its gathers
+//     alone take 125).  Gathers before the barrier: 52.6, 72.0, 52.8, 57.4,
+//     81.6 and 139 us.
 //   single-row block (CSR-Vector/VectorL): 256 lanes strided with fma, a
 //     64-lane halving tree per wave, then a halving tree over the 4 waves.
 //   rows longer than long_row: split into `chunk`-element pieces, one
@@ -526,10 +528,15 @@ __device__ __forceinline__ void adaptive_item(
       vc[k] = ldg_stream(cv + v);
     }
   }
-  // the row starts are on their way before the gathers, which are in flight
-  // while the rows are searched
+  // the row starts are loaded beside the entries; the gathers go out together
+  // behind their barrier and are in flight while the rows are searched
   const uint32_t nr = r1 - r0;
   const uint32_t p0 = tid <= nr ? rp[r0 + tid] : 0u, p1 = tid + AD_T <= nr ? rp[r0 + tid + AD_T] : 0u;
+  // block-relative row starts rs[0..nr]
+  if (tid <= nr) rs[tid] = p0 - base;
+  if (tid + AD_T <= nr) rs[tid + AD_T] = p1 - base;
+  for (uint32_t lr = tid + 2 * AD_T; lr <= nr; lr += AD_T) rs[lr] = rp[r0 + lr] - base;
+  __syncthreads();
   T xv[K][N];
   if (n) { // without entries x may be empty
 #pragma unroll
@@ -542,11 +549,6 @@ __device__ __forceinline__ void adaptive_item(
       }
     }
   }
-  // block-relative row starts rs[0..nr]
-  if (tid <= nr) rs[tid] = p0 - base;
-  if (tid + AD_T <= nr) rs[tid + AD_T] = p1 - base;
-  for (uint32_t lr = tid + 2 * AD_T; lr <= nr; lr += AD_T) rs[lr] = rp[r0 + lr] - base;
-  __syncthreads();
   for (uint32_t lr = tid; lr < nr; lr += AD_T)
     if (rs[lr] == rs[lr + 1]) y[r0 + lr] = (T)0; // empty rows
 
