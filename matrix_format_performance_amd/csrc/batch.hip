@@ -979,7 +979,7 @@ static int batch_launch(mfp_batch b, uint32_t k, const void *X, void *Y, hipStre
     g.nchunks = p->ad.nchunks;
     g.chunk = p->t.chunk;
     g.partials = p->ad.partials;
-    g.persistent = true;
+    g.batch = true;
     return launch_csr_adaptive(m->dtype, g, m->values, X, Y, s);
   }
   if (b->lanes == 0)

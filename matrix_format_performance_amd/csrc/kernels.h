@@ -20,7 +20,7 @@ struct adaptive_args {
   uint32_t nchunks = 0;
   uint32_t chunk = 0;
   void *partials = nullptr; // nchunks values
-  bool persistent = false;  // fixed grid walking the items (batched launches)
+  bool batch = false;       // row blocks in runs per XCD (several matrices)
 };
 
 // CSR-Adaptive defaults: a row block holds up to this many nonzeros, which a

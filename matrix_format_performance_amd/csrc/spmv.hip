@@ -460,33 +460,30 @@ __host__ __device__ constexpr uint32_t adaptive_products(uint32_t W)
   return (adaptive_slot<T>(W) * (uint32_t)sizeof(T) + 15u) & ~15u;
 }
 
-template <typename T>
-struct adaptive_smem {
-  T *cache;     // staged products (nnz_per_wg, by adaptive_slot)
-  uint32_t *rs; // block-relative row starts (nnz_per_wg + 2)
-  T *wsum, *sv; // sv: 2 AD_T
-  uint32_t *wsteps;
-};
-
-// One work item of the launch: hw is the item's dispatch index among grid
-// items (pieces of long rows first, then row blocks in XCD order).  A batch's
-// blocks differ in cost from one member to the next, so there the XCDs take
-// runs of 64: a batch of 64, f32 225 -> 167 us, f64 271 -> 231 us.  One matrix
-// keeps a range per XCD (300k rows within a band of 1%: 28.3 us, 29.3 in runs
-// of 64 and 32 in runs of 16).
+// A workgroup takes one item: the pieces of long rows first, then the row
+// blocks in XCD order.  A batch's blocks differ in cost from one member to the
+// next, so there the XCDs take runs of 64, as workgroups end: 512 matrices,
+// f32, 1,468 us with a range per XCD, 1,341 in runs; 64 257 and 212.  (A fixed
+// grid that walks the items in runs drifts apart and loses x in the L2s: 2,477
+// us for the 512, 228 for the 64.)  One matrix keeps a range per XCD (300k rows
+// within a band of 1%: 28.3 us, 29.3 in runs of 64 and 32 in runs of 16).
 template <typename T, uint32_t K, bool BATCH>
-__device__ __forceinline__ void adaptive_item(
-    uint32_t hw, uint32_t grid, const uint32_t *__restrict__ rp, const uint32_t *__restrict__ ci,
-    const T *__restrict__ a, const T *__restrict__ x, T *__restrict__ y,
-    const uint32_t *__restrict__ blocks, uint32_t nnz_per_wg, uint32_t long_row,
-    const uint4 *__restrict__ chunks, uint32_t nchunks, uint32_t nchunks_pad, uint32_t chunk,
-    T *__restrict__ partials, const adaptive_smem<T> &sm)
+__global__ __launch_bounds__(AD_T) void k_csr_adaptive(
+    const uint32_t *__restrict__ rp, const uint32_t *__restrict__ ci, const T *__restrict__ a,
+    const T *__restrict__ x, T *__restrict__ y, const uint32_t *__restrict__ blocks,
+    uint32_t nnz_per_wg, uint32_t long_row, const uint4 *__restrict__ chunks, uint32_t nchunks,
+    uint32_t nchunks_pad, uint32_t chunk, T *__restrict__ partials)
 {
   using VT = vec16<T>;
   constexpr uint32_t N = VT::N;
-  T *cache = sm.cache;
-  uint32_t *rs = sm.rs;
-  T *wsum = sm.wsum, *sv = sm.sv;
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  T *cache = reinterpret_cast<T *>(smem_raw); // staged products (nnz_per_wg, by adaptive_slot)
+  // block-relative row starts (nnz_per_wg + 2)
+  uint32_t *rs = reinterpret_cast<uint32_t *>(smem_raw + adaptive_products<T>(nnz_per_wg));
+  __shared__ T wsum[4];
+  __shared__ T sv[2 * AD_T];
+  __shared__ uint32_t wsteps[4];
+  const uint32_t hw = blockIdx.x;
   const uint32_t tid = threadIdx.x;
 
   if (hw < nchunks_pad) {
@@ -500,7 +497,7 @@ __device__ __forceinline__ void adaptive_item(
     return;
   }
 
-  const uint32_t b = hw - nchunks_pad, nb = grid - nchunks_pad;
+  const uint32_t b = hw - nchunks_pad, nb = gridDim.x - nchunks_pad;
   const uint32_t item = BATCH ? xcd_runs(b, nb, BATCH_RUN) : xcd_block(b, nb);
   const uint32_t r0 = blocks[item], r1 = blocks[item + 1];
   if (r1 <= r0) return;
@@ -621,9 +618,9 @@ __device__ __forceinline__ void adaptive_item(
   uint32_t steps = 0;
   while (__ballot(back >= (1u << steps))) steps++;
   sv[tid] = carry_v;
-  if ((tid & 63u) == 0) sm.wsteps[tid >> 6] = steps;
+  if ((tid & 63u) == 0) wsteps[tid >> 6] = steps;
   __syncthreads();
-  steps = max(max(sm.wsteps[0], sm.wsteps[1]), max(sm.wsteps[2], sm.wsteps[3]));
+  steps = max(max(wsteps[0], wsteps[1]), max(wsteps[2], wsteps[3]));
   for (uint32_t i = 0; i < steps; i++) {
     const uint32_t off = 1u << i, from = (i & 1u) * AD_T + tid;
     T v = sv[from];
@@ -632,45 +629,6 @@ __device__ __forceinline__ void adaptive_item(
     __syncthreads();
   }
   if (frow != 0xFFFFFFFFu) y[r0 + frow] = sv[(steps & 1u) * AD_T + tid - 1] + fval;
-}
-
-#define ADAPTIVE_SMEM(T)                                                                       \
-  extern __shared__ __align__(16) unsigned char smem_raw[];                                    \
-  __shared__ T wsum_[4];                                                                       \
-  __shared__ T sv_[2 * AD_T];                                                                  \
-  __shared__ uint32_t wsteps_[4];                                                              \
-  adaptive_smem<T> sm{reinterpret_cast<T *>(smem_raw),                                         \
-                      reinterpret_cast<uint32_t *>(smem_raw + adaptive_products<T>(nnz_per_wg)), \
-                      wsum_, sv_, wsteps_};
-
-template <typename T, uint32_t K>
-__global__ __launch_bounds__(AD_T) void k_csr_adaptive(
-    const uint32_t *__restrict__ rp, const uint32_t *__restrict__ ci, const T *__restrict__ a,
-    const T *__restrict__ x, T *__restrict__ y, const uint32_t *__restrict__ blocks,
-    uint32_t nnz_per_wg, uint32_t long_row, const uint4 *__restrict__ chunks, uint32_t nchunks,
-    uint32_t nchunks_pad, uint32_t chunk, T *__restrict__ partials)
-{
-  ADAPTIVE_SMEM(T)
-  adaptive_item<T, K, false>(blockIdx.x, gridDim.x, rp, ci, a, x, y, blocks, nnz_per_wg, long_row, chunks,
-                      nchunks, nchunks_pad, chunk, partials, sm);
-}
-
-// Persistent form: a fixed grid (a multiple of 8, so a workgroup keeps its
-// XCD) walks the items; used for batched launches.
-template <typename T, uint32_t K>
-__global__ __launch_bounds__(AD_T) void k_csr_adaptive_persistent(
-    uint32_t items, const uint32_t *__restrict__ rp, const uint32_t *__restrict__ ci,
-    const T *__restrict__ a, const T *__restrict__ x, T *__restrict__ y,
-    const uint32_t *__restrict__ blocks, uint32_t nnz_per_wg, uint32_t long_row,
-    const uint4 *__restrict__ chunks, uint32_t nchunks, uint32_t nchunks_pad, uint32_t chunk,
-    T *__restrict__ partials)
-{
-  ADAPTIVE_SMEM(T)
-  for (uint32_t hw = blockIdx.x; hw < items; hw += gridDim.x) {
-    adaptive_item<T, K, true>(hw, items, rp, ci, a, x, y, blocks, nnz_per_wg, long_row, chunks, nchunks,
-                        nchunks_pad, chunk, partials, sm);
-    __syncthreads();
-  }
 }
 
 // One lane per long row: add its pieces left to right.
@@ -1595,17 +1553,13 @@ uint32_t adaptive_vectors_per_lane(int dtype, uint32_t W)
 
 template <typename T, uint32_t K>
 static int adaptive_launch_k(const adaptive_args &g, const T *a, const T *x, T *y, hipStream_t s,
-                             size_t lds, uint32_t items, uint32_t nchunks_pad, uint32_t persistent_grid)
+                             size_t lds, uint32_t items, uint32_t nchunks_pad)
 {
-  const void *fn = persistent_grid ? (const void *)k_csr_adaptive_persistent<T, K>
-                                   : (const void *)k_csr_adaptive<T, K>;
-  if (lds > 65536) MFP_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-  if (persistent_grid)
-    return launch_k(k_csr_adaptive_persistent<T, K>, dim3(persistent_grid), dim3(AD_T), (uint32_t)lds, s, items,
-                    g.rp, g.ci, a, x, y, g.blocks, g.nnz_per_wg, g.long_row, g.chunks, g.nchunks, nchunks_pad,
-                    g.chunk, (T *)g.partials);
-  return launch_k(k_csr_adaptive<T, K>, dim3(items), dim3(AD_T), (uint32_t)lds, s, g.rp, g.ci, a, x, y, g.blocks,
-                  g.nnz_per_wg, g.long_row, g.chunks, g.nchunks, nchunks_pad, g.chunk, (T *)g.partials);
+  const auto fn = g.batch ? k_csr_adaptive<T, K, true> : k_csr_adaptive<T, K, false>;
+  if (lds > 65536)
+    MFP_HIP(hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  return launch_k(fn, dim3(items), dim3(AD_T), (uint32_t)lds, s, g.rp, g.ci, a, x, y, g.blocks, g.nnz_per_wg,
+                  g.long_row, g.chunks, g.nchunks, nchunks_pad, g.chunk, (T *)g.partials);
 }
 
 // Dynamic LDS of k_csr_adaptive: the staged products, then the row starts.
@@ -1623,21 +1577,14 @@ static int adaptive_t(const adaptive_args &g, const T *a, const T *x, T *y, hipS
   const uint32_t items = g.nblocks ? g.nblocks + nchunks_pad : nchunks_pad;
   const size_t lds = adaptive_lds_bytes<T>(g.nnz_per_wg);
   const uint32_t K = adaptive_vectors_per_lane(sizeof(T) == 4 ? MFP_F32 : MFP_F64, g.nnz_per_wg);
-  // persistent: 8 workgroups per CU (the LDS/wave occupancy), a multiple of 8
-  uint32_t pgrid = 0;
-  if (g.persistent) {
-    pgrid = std::max<uint32_t>(8, (uint32_t)std::max(1, props().cu_count) * 8u);
-    pgrid = std::min<uint32_t>(pgrid, (items + 7u) & ~7u);
-    pgrid = std::max<uint32_t>(8, pgrid & ~7u);
-  }
   if (items) {
     int st;
     switch (K) {
-    case 1: st = adaptive_launch_k<T, 1>(g, a, x, y, s, lds, items, nchunks_pad, pgrid); break;
-    case 2: st = adaptive_launch_k<T, 2>(g, a, x, y, s, lds, items, nchunks_pad, pgrid); break;
-    case 4: st = adaptive_launch_k<T, 4>(g, a, x, y, s, lds, items, nchunks_pad, pgrid); break;
-    case 8: st = adaptive_launch_k<T, 8>(g, a, x, y, s, lds, items, nchunks_pad, pgrid); break;
-    case 16: st = adaptive_launch_k<T, 16>(g, a, x, y, s, lds, items, nchunks_pad, pgrid); break;
+    case 1: st = adaptive_launch_k<T, 1>(g, a, x, y, s, lds, items, nchunks_pad); break;
+    case 2: st = adaptive_launch_k<T, 2>(g, a, x, y, s, lds, items, nchunks_pad); break;
+    case 4: st = adaptive_launch_k<T, 4>(g, a, x, y, s, lds, items, nchunks_pad); break;
+    case 8: st = adaptive_launch_k<T, 8>(g, a, x, y, s, lds, items, nchunks_pad); break;
+    case 16: st = adaptive_launch_k<T, 16>(g, a, x, y, s, lds, items, nchunks_pad); break;
     default: set_error("nnz_per_wg too large"); return MFP_ERR_ARG;
     }
     MFP_CHECK(st);
