@@ -808,12 +808,14 @@ __global__ __launch_bounds__(256) void k_items_largest_first(uint32_t n, const u
 // times one of a power-law matrix) and there is one round of them or two, so
 // the largest go first, XCD after XCD: a batch of 64, k = 2 (266 items) 150 ->
 // 121 us, k = 4 (521) 179 -> 176; of 130, k = 4 (900) 288 -> 276.  With more,
-// those of one matrix side by side share X in the L2 (a batch of 200, k = 4,
-// 1,700 items: 489 us in runs of 8, 532 largest first).
+// those of one matrix side by side share X in the L2: k = 1 in runs of 8 (512
+// matrices 731 -> 716 us, 200 352 -> 341; 64 of them 114 -> 96), k > 1, whose X
+// is larger, a range per XCD (k = 4, 512 matrices: 1,418 us, 1,581 in runs of
+// 8; 200: 765 and 791, largest first 9% above).
 constexpr uint32_t BATCH_FEW_ITEMS = 4; // per CU
-static int batch_order_items(scoo_cs_layout &l, hipStream_t s)
+static int batch_order_items(scoo_cs_layout &l, uint32_t k, hipStream_t s)
 {
-  l.run = BATCH_ITEM_RUN;
+  l.run = k == 1 ? BATCH_ITEM_RUN : XCD_ONE_RUN;
   if (l.NI < 2 || l.NI > BATCH_FEW_ITEMS * (uint32_t)std::max(1, props().cu_count)) return MFP_OK;
   uint4 *items = nullptr;
   uint32_t *base = nullptr;
@@ -948,7 +950,7 @@ static int batch_cs_plan(mfp_batch b, uint32_t k, mfp_stream sv)
   t.scoo_threads = 1024;
   MFP_CHECK(mfp_plan_create(&b->cs[i], b->big, MFP_SCOO, &t, sv));
   int st = batch_split_aligned(b, i, as_stream(sv));
-  if (st == MFP_OK) st = batch_order_items(b->cs[i]->cs, as_stream(sv));
+  if (st == MFP_OK) st = batch_order_items(b->cs[i]->cs, k, as_stream(sv));
   if (st != MFP_OK) {
     mfp_plan_destroy(b->cs[i]);
     b->cs[i] = nullptr;
@@ -1085,7 +1087,7 @@ int mfp_batch_create(mfp_batch *out, const mfp_matrix *ms, uint32_t count, uint3
   if (st == MFP_OK) {
     const int f = k1_tuning && (k1_tuning->flags & MFP_TUNE_SCOO_COLSORT) ? MFP_SCOO : MFP_CSR_ADAPTIVE;
     st = mfp_plan_create(&b->k1, m, f, k1_tuning, sv);
-    if (st == MFP_OK) st = batch_order_items(b->k1->cs, s);
+    if (st == MFP_OK) st = batch_order_items(b->k1->cs, 1, s);
   }
   if (st == MFP_OK && lanes == 0) st = spmm_bins_build(m->rows, m->row_ptr, &b->bins, &b->bin_list, s);
   if (st == MFP_OK && lanes == MFP_BATCH_STREAM)

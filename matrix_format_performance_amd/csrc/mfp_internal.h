@@ -138,10 +138,8 @@ int exclusive_scan_u32(const uint32_t *in, uint32_t *out, uint64_t n, hipStream_
 constexpr uint32_t CS_DIRECT = 0xFFFFFFFEu, CS_FIN_ROWS = 256, CS_FIN_LONG = CS_FIN_ROWS / 64;
 // Runs of workgroups an XCD takes (wave64.h), as log2: a run that no grid
 // exceeds, which is one contiguous range per XCD; a batch's row blocks; and its
-// column-sorted items.  Those, one range per XCD -> runs of 8, batch of 64:
-// k = 1 114 -> 96 us, f64 177 -> 149, k = 4 185 -> 178, k = 8 318 -> 310, k = 16
-// 643 -> 618, k = 2 the same within 1%; runs of 2, 4 and 16: k = 1 103, 100 and
-// 96, k = 2 150, 150 and 152.
+// column-sorted items at k = 1 (a batch of 64, one range per XCD -> runs of 8:
+// 114 -> 96 us, f64 177 -> 149; runs of 2, 4 and 16: 103, 100 and 96).
 constexpr uint32_t XCD_ONE_RUN = 28, BATCH_RUN = 6, BATCH_ITEM_RUN = 3;
 struct scoo_cs_layout {
   uint32_t run = XCD_ONE_RUN;
