@@ -211,17 +211,19 @@ def log(msg):
     print(msg, file=sys.stderr, flush=True)
 
 
-def kernel_names(fmt, info):
-    """The kernels one SpMV of an FP32/FP64 plan launches, in order."""
+def kernel_names(fmt, info, nk):
+    """The kernels one SpMV of an FP32/FP64 plan launches, in order; nk of them."""
     if fmt == "scoo":
         return ["k_scoo_cs", "k_scoo_cs_finish"] if info["scoo_colsort"] else ["k_scoo"]
     if fmt == "csr_adaptive":
         return ["k_csr_adaptive", "k_adaptive_finish"] if info["chunks"] else ["k_csr_adaptive"]
     if fmt == "ell" and info["column_bytes"] == 2:
         return ["k_ell_pk"]
-    return {"csr_scalar": ["k_csr_scalar"], "csr_vector": ["k_csr_vector"], "ell": ["k_ell"], "coo": ["k_coo"],
+    # CSR-vector: from LDS or row by row, by size; COO: one kernel where no row has more than 64 entries
+    return {"csr_scalar": ["k_csr_scalar"], "csr_vector": ["k_csr_vector_lds or k_csr_vector"], "ell": ["k_ell"],
+            "coo": ["k_coo_owner"] if nk == 1 else ["k_fill", "k_coo"],
             "hyb": ["k_ell", "k_coo"] if info["coo_elements"] else ["k_ell"],
-            "hyb_atomic": ["k_hyb_atomic"]}.get(fmt)
+            "hyb_atomic": ["k_fill", "k_hyb_atomic"]}.get(fmt)
 
 
 def kernel_bytes(fmt, info, nbytes, rows, s_y, nk):
@@ -681,7 +683,7 @@ def main():
     if args.values:
         share_note = "approximate: 16-bit value plans time each kernel from the previous event; " + share_note
     dom_bytes = shares[dom]
-    dom_names = None if args.values else kernel_names(best, pinfo)
+    dom_names = None if args.values else kernel_names(best, pinfo, nk)
     achieved = dom_bytes / (kernel_ms[dom] * 1e-3) / 1e9
 
     traffic = None
