@@ -67,7 +67,7 @@ WORKLOADS = {
 
 
 def run_batch(mfp, args, timer, production=False):
-    """One step = one replay of the captured persistent launch over all 512
+    """One step = one replay of the captured launch over all 512
     matrices (k right-hand sides); value = algorithmic bytes / mean step.
     production: build only the two batches whose forms the full study keeps
     (column-sorted SCOO for k = 1 and 4, CSR-stream SpMM for k = 16; the
@@ -145,7 +145,7 @@ def run_batch(mfp, args, timer, production=False):
         nb = nnz * 8 + (rows + 1) * 4 + k * (cols + rows) * 4
         res[k] = {"ms": round(mean_ms, 5), "GB_per_s": round(nb / (mean_ms * 1e-3) / 1e9, 1),
                   "gflops": round(2 * nnz * k / (mean_ms * 1e-3) / 1e9, 1), "algorithmic_bytes": nb,
-                  "plan": {"adaptive": "persistent CSR-Adaptive",
+                  "plan": {"adaptive": "CSR-Adaptive",
                            "colsort": "column-sorted SCOO" + (", 8192-row slices" if k == 1 else " SpMM"),
                            "mean": f"CSR-vector SpMM, {mean_lanes} lanes",
                            "half": f"CSR-vector SpMM, {mean_lanes // 2} lanes",
@@ -174,7 +174,7 @@ def run_batch(mfp, args, timer, production=False):
         "dtype": "f32", "data": "synthetic",
         "config": {"workload": "batch512", "description": WORKLOADS["batch512"], "matrices": batch.count,
                    "plans": "per k in batch[k].plan (the fastest of those timed in ms_by_plan)",
-                   "rows": rows, "cols": cols, "nnz": nnz, "launch": "one HIP graph replay per step (one persistent SpMM kernel, or the column-sorted SCOO main + finish kernels)",
+                   "rows": rows, "cols": cols, "nnz": nnz, "launch": "one HIP graph replay per step (one SpMM kernel, or the column-sorted SCOO main + finish kernels)",
                    "cache": "Infinity Cache evicted before every step",
                    "measured_copy_GB_per_s": round(copy_gbs, 1)},
         "pct_hbm_roofline": round(100 * value / HBM_PEAK_GBS, 2),
