@@ -1128,40 +1128,40 @@ struct cs_values {
     else
       return (double)lp_val<DT>(ldg_stream(ev + i));
   }
-  // the four values of 16-byte entry word g, as stored and in double
-  typedef double f64x4 __attribute__((ext_vector_type(4)));
-  using W = typename std::conditional<(DT >= 0), u32x2,
-                                      typename std::conditional<sizeof(T) == 4, f32x4, f64x4>::type>::type;
-  __device__ __forceinline__ static W word(const V *__restrict__ ev, uint32_t g)
+  // the four values of 16-byte entry word g
+  __device__ __forceinline__ static void word(const V *__restrict__ ev, uint32_t g, double (&v)[4])
   {
-    if constexpr (DT < 0 && sizeof(T) == 8) {
-      // slots 0, 1 of the block's 64 words, then slots 2, 3 (word g is word
-      // g % 64 of block g / 64)
-      const f64x2 *p = reinterpret_cast<const f64x2 *>(ev) + (g >> 6) * 128u + (g & 63u);
-      const f64x2 d0 = __builtin_nontemporal_load(p), d1 = __builtin_nontemporal_load(p + 64);
-      return W{d0[0], d0[1], d1[0], d1[1]};
+    if constexpr (DT >= 0) {
+      const u32x2 h = __builtin_nontemporal_load(reinterpret_cast<const u32x2 *>(ev) + g);
+      v[0] = (double)lp_val<DT>((uint16_t)(h[0] & 0xFFFFu));
+      v[1] = (double)lp_val<DT>((uint16_t)(h[0] >> 16));
+      v[2] = (double)lp_val<DT>((uint16_t)(h[1] & 0xFFFFu));
+      v[3] = (double)lp_val<DT>((uint16_t)(h[1] >> 16));
+    } else if constexpr (sizeof(T) == 4) {
+      const f32x4 f = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(ev) + g);
+#pragma unroll
+      for (uint32_t j = 0; j < 4; j++) v[j] = (double)f[j];
     } else {
-      return __builtin_nontemporal_load(reinterpret_cast<const W *>(ev) + g);
+      // FP64: slots 0, 1 of the block's 64 words, then slots 2, 3 (word g
+      // is word g % 64 of block g / 64)
+      const f64x2 *p = reinterpret_cast<const f64x2 *>(ev) + (g >> 6) * 128u + (g & 63u);
+      const f64x2 d0 = __builtin_nontemporal_load(p);
+      const f64x2 d1 = __builtin_nontemporal_load(p + 64);
+      v[0] = d0[0];
+      v[1] = d0[1];
+      v[2] = d1[0];
+      v[3] = d1[1];
     }
-  }
-  __device__ __forceinline__ static double at(const W &w, uint32_t j)
-  {
-    if constexpr (DT >= 0)
-      return (double)lp_val<DT>((uint16_t)(w[j / 2] >> (j % 2 * 16)));
-    else
-      return (double)w[j];
   }
 };
 
 template <typename T, int DT>
-__global__ __launch_bounds__(1024) void k_scoo_cs(uint32_t run, uint32_t rows, uint32_t R, uint32_t rbits,
-                                                  uint32_t S_reg, uint32_t NL, const uint4 *__restrict__ items,
-                                                  const uint32_t *__restrict__ ibase,
-                                                  const typename cs_values<T, DT>::V *__restrict__ ev,
-                                                  const uint32_t *__restrict__ ec, const T *__restrict__ x,
-                                                  T *__restrict__ y, T *__restrict__ partial,
-                                                  const uint32_t *__restrict__ long_rows,
-                                                  const uint32_t *__restrict__ long_mask)
+__global__ void k_scoo_cs(uint32_t run, uint32_t rows, uint32_t R, uint32_t rbits, uint32_t S_reg, uint32_t NL,
+                          const uint4 *__restrict__ items, const uint32_t *__restrict__ ibase,
+                          const typename cs_values<T, DT>::V *__restrict__ ev, const uint32_t *__restrict__ ec,
+                          const T *__restrict__ x, T *__restrict__ y,
+                          T *__restrict__ partial, const uint32_t *__restrict__ long_rows,
+                          const uint32_t *__restrict__ long_mask)
 {
   using CV = cs_values<T, DT>;
   extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -1186,48 +1186,38 @@ __global__ __launch_bounds__(1024) void k_scoo_cs(uint32_t run, uint32_t rows, u
   // flight.  The decode does not depend on which positions a word holds.
   const uint32_t g0 = ea >> 2, g1 = max(g0, (e1 & ~255u) >> 2); // words [g0, g1) lie inside [ea, e1)
   uint32_t g = g0 + tid;
-  // The next two words are loaded while the current ones' gathers are in
-  // flight: power-law 1M rows 39.0 -> 38.2 us, 300k random rows 33.3 -> 32.0,
-  // slices of 16384 rows by 512 threads 45.7 -> 42.6.  Not for FP64, whose
-  // words ahead leave one workgroup of 1024 per CU (45.8 -> 50.6 us).
-  constexpr bool AHEAD = sizeof(typename CV::W) <= 16;
-  u32x4 w[2];
-  typename CV::W v[2];
-  auto load = [&](uint32_t at) {
+  for (; g + bt < g1; g += 2 * bt) {
+    u32x4 w[2];
+    double v[2][4];
 #pragma unroll
     for (uint32_t k = 0; k < 2; k++) {
-      w[k] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(ec) + at + k * bt);
-      v[k] = CV::word(ev, at + k * bt);
+      w[k] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(ec) + g + k * bt);
+      CV::word(ev, g + k * bt, v[k]);
     }
-  };
-  if (AHEAD && g + bt < g1) load(g);
-  for (; g + bt < g1; g += 2 * bt) {
-    uint32_t lr[2][4];
+    uint32_t c[2][4], lr[2][4];
     T xv[2][4];
-    if (!AHEAD) load(g);
-    const typename CV::W vv[2] = {v[0], v[1]};
 #pragma unroll
     for (uint32_t k = 0; k < 2; k++)
 #pragma unroll
-      for (uint32_t j = 0; j < 4; j++) {
-        uint32_t c;
-        cs_decode(w[k][j], cbase, rbits, c, lr[k][j]);
-        xv[k][j] = x[c];
-      }
-    if (AHEAD && g + 3 * bt < g1) load(g + 2 * bt);
+      for (uint32_t j = 0; j < 4; j++) cs_decode(w[k][j], cbase, rbits, c[k][j], lr[k][j]);
 #pragma unroll
     for (uint32_t k = 0; k < 2; k++)
 #pragma unroll
-      for (uint32_t j = 0; j < 4; j++) atomicAdd(acc + lr[k][j], CV::at(vv[k], j) * (double)xv[k][j]);
+      for (uint32_t j = 0; j < 4; j++) xv[k][j] = x[c[k][j]];
+#pragma unroll
+    for (uint32_t k = 0; k < 2; k++)
+#pragma unroll
+      for (uint32_t j = 0; j < 4; j++) atomicAdd(acc + lr[k][j], v[k][j] * (double)xv[k][j]);
   }
   for (; g < g1; g += bt) {
     const u32x4 w = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(ec) + g);
-    const typename CV::W v = CV::word(ev, g);
+    double v[4];
+    CV::word(ev, g, v);
 #pragma unroll
     for (uint32_t j = 0; j < 4; j++) {
       uint32_t c, lr;
       cs_decode(w[j], cbase, rbits, c, lr);
-      atomicAdd(acc + lr, CV::at(v, j) * (double)x[c]);
+      atomicAdd(acc + lr, v[j] * (double)x[c]);
     }
   }
   // tail: entries after the last whole group
@@ -1386,7 +1376,8 @@ __global__ void k_scoo_cs_k(uint32_t run, uint32_t rows, uint32_t R, uint32_t rb
   const uint32_t g0 = ea >> 2, g1 = max(g0, (e1 & ~255u) >> 2);
   for (uint32_t g = g0 + tid; g < g1; g += bt) {
     const u32x4 w = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(ec) + g);
-    const typename CV::W v = CV::word(ev, g);
+    double v[4];
+    CV::word(ev, g, v);
     uint32_t c[4], lr[4];
 #pragma unroll
     for (uint32_t j = 0; j < 4; j++) cs_decode(w[j], cbase, rbits, c[j], lr[j]);
@@ -1396,7 +1387,7 @@ __global__ void k_scoo_cs_k(uint32_t run, uint32_t rows, uint32_t R, uint32_t rb
 #pragma unroll
     for (uint32_t j = 0; j < 4; j++)
 #pragma unroll
-      for (int q = 0; q < KV; q++) atomicAdd(acc + q * R + lr[j], CV::at(v, j) * (double)xr[j][q]);
+      for (int q = 0; q < KV; q++) atomicAdd(acc + q * R + lr[j], v[j] * (double)xr[j][q]);
   }
   for (uint32_t i = max(ea, g1 << 2) + tid; i < e1; i += bt) {
     uint32_t c, lr;
