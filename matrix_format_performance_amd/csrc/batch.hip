@@ -803,20 +803,26 @@ __global__ __launch_bounds__(256) void k_items_largest_first(uint32_t n, const u
   out_base[at] = base[i];
 }
 
-// The order and the XCDs of a batch's column-sorted items.  Up to four per CU
-// they differ most in what they cost (a slice of a random matrix holds three
-// times one of a power-law matrix) and there is one round of them or two, so
-// the largest go first, XCD after XCD: a batch of 64, k = 2 (266 items) 150 ->
-// 121 us, k = 4 (521) 179 -> 176; of 130, k = 4 (900) 288 -> 276.  With more,
-// those of one matrix side by side share X in the L2: k = 1 in runs of 8 (512
-// matrices 731 -> 716 us, 200 352 -> 341; 64 of them 114 -> 96), k > 1, whose X
-// is larger, a range per XCD (k = 4, 512 matrices: 1,418 us, 1,581 in runs of
-// 8; 200: 765 and 791, largest first 9% above).
+// The order and the XCDs of a batch's column-sorted items.  Up to one per CU
+// they start together and keep the plan's order, a range per XCD (24 matrices,
+// k = 1, 200 items: 73.7 us, 75.7 largest first; 32: 47.3 and 49.3).  Up to four
+// per CU they differ most in what they cost (a slice of a random matrix holds
+// three times one of a power-law matrix) and there is one round of them or two,
+// so the largest go first, XCD after XCD: a batch of 64, k = 2 (266 items) 150
+// -> 121 us, k = 4 (521) 179 -> 176; of 56, k = 1 (301) 79 -> 65; of 130, k = 4
+// (900) 288 -> 276.  With more, those of one matrix side by side share X in the
+// L2: k = 1 in runs of 8 (512 matrices 731 -> 716 us, 200 352 -> 341), k > 1,
+// whose X is larger, a range per XCD (k = 4, 512 matrices: 1,418 us, 1,581 in
+// runs of 8; 200: 765 and 791, largest first 9% above).
 constexpr uint32_t BATCH_FEW_ITEMS = 4; // per CU
 static int batch_order_items(scoo_cs_layout &l, uint32_t k, hipStream_t s)
 {
-  l.run = k == 1 ? BATCH_ITEM_RUN : XCD_ONE_RUN;
-  if (l.NI < 2 || l.NI > BATCH_FEW_ITEMS * (uint32_t)std::max(1, props().cu_count)) return MFP_OK;
+  const uint32_t cus = (uint32_t)std::max(1, props().cu_count);
+  if (l.NI <= cus) return MFP_OK;
+  if (l.NI > BATCH_FEW_ITEMS * cus) {
+    l.run = k == 1 ? BATCH_ITEM_RUN : XCD_ONE_RUN;
+    return MFP_OK;
+  }
   uint4 *items = nullptr;
   uint32_t *base = nullptr;
   int st = dmalloc((void **)&items, (uint64_t)l.NI * sizeof(uint4));
