@@ -1,0 +1,174 @@
+// Freed device blocks, kept for the library's next allocations.  Host code
+// only; the device calls come from Dev, so that the bookkeeping can be checked
+// without a GPU:
+//   static bool alloc(void **p, size_t bytes)  on the current device
+//   static void release(void *p)               a block of any device
+//   static int current()                       the current device, -1 unknown
+//   static bool idle()                         waits for the current device
+#pragma once
+
+#include <cstddef>
+#include <map>
+#include <mutex>
+#include <new>
+#include <unordered_map>
+#include <utility>
+
+namespace mfp {
+
+// hipMalloc / hipFree map and unmap memory: 30 to 90 us per call for blocks of
+// 16 MB and more, 210 to 250 us to free one while others are held, so that
+// building one plan spent more on its ten or so arrays than on its kernels
+// (nine formats of a 5M-entry matrix: 1.8 ms of kernels in 8.7 to 12.9 ms).
+// Freed blocks of 64 KB to 1 GB are therefore kept and handed out again, in
+// size classes an eighth of a power of two apart.
+//  * A block is kept only once its device is idle (put waits for it, as
+//    hipFree does), so whoever gets it next, on any stream or thread, finds
+//    nothing still running on it.
+//  * A block is filed under the device it was allocated on, whichever device
+//    the freeing thread uses, and handed out on that device only.
+//  * At most CACHE_BYTES are kept; an allocation that fails gives all of them
+//    back and tries again, and they are given back when the library's last
+//    block is freed.
+constexpr size_t CACHE_MIN = 64u << 10, CACHE_MAX = 1u << 30, CACHE_BYTES = 4ull << 30;
+
+template <class Dev>
+class block_cache {
+  using block = std::pair<int, size_t>; // device, size (0: not cacheable)
+  using blocks = std::multimap<block, void *>;
+
+public:
+  // a block of at least bytes on the current device, null when there is none
+  void *get(size_t bytes)
+  {
+    const int device = Dev::current();
+    const bool cacheable = bytes >= CACHE_MIN && bytes <= CACHE_MAX && device >= 0;
+    const size_t size = cacheable ? size_class(bytes) : bytes;
+    if (cacheable) {
+      std::lock_guard<std::mutex> lock(mutex_);
+      const auto it = kept_.lower_bound({device, size});
+      if (it != kept_.end() && it->first.first == device && it->first.second <= size + size / 4) {
+        void *p = it->second;
+        const block b = it->first;
+        kept_bytes_ -= b.second;
+        kept_.erase(it);
+        taken(p, b);
+        return p;
+      }
+    }
+    void *p = nullptr;
+    block b{device, cacheable ? size : 0};
+    if (!alloc(&p, size)) {
+      b.second = 0;
+      if (size == bytes || !Dev::alloc(&p, bytes)) return nullptr; // without the rounding, then
+    }
+    std::lock_guard<std::mutex> lock(mutex_);
+    taken(p, b);
+    return p;
+  }
+
+  // gives back a block of get
+  void put(void *p)
+  {
+    if (!p) return;
+    block b{-1, 0};
+    {
+      std::lock_guard<std::mutex> lock(mutex_);
+      const auto it = sizes_.find(p);
+      if (it != sizes_.end()) {
+        b = it->second;
+        sizes_.erase(it);
+      }
+    }
+    // idle() waits for the current device, so only its blocks are kept
+    const bool keep = b.second && Dev::current() == b.first && Dev::idle();
+    if (!(keep && add(b, p))) Dev::release(p);
+    blocks out;
+    {
+      std::lock_guard<std::mutex> lock(mutex_);
+      if (--in_use_ == 0) take_all(out);
+    }
+    release(out);
+  }
+
+  // an allocation beside the cache's own that may take what it keeps
+  bool alloc(void **p, size_t bytes)
+  {
+    if (Dev::alloc(p, bytes)) return true;
+    trim();
+    return Dev::alloc(p, bytes);
+  }
+
+  // gives back every kept block
+  void trim()
+  {
+    blocks out;
+    {
+      std::lock_guard<std::mutex> lock(mutex_);
+      take_all(out);
+    }
+    release(out);
+  }
+
+  // bytes kept on a device
+  size_t kept_bytes(int device)
+  {
+    std::lock_guard<std::mutex> lock(mutex_);
+    size_t sum = 0;
+    for (auto it = kept_.lower_bound({device, 0}); it != kept_.end() && it->first.first == device; ++it)
+      sum += it->first.second;
+    return sum;
+  }
+
+private:
+  static size_t size_class(size_t bytes)
+  {
+    size_t step = CACHE_MIN / 8;
+    while (step * 16 <= bytes) step *= 2; // 8 step <= bytes < 16 step
+    return (bytes + step - 1) / step * step;
+  }
+
+  // mutex_ held; without memory for the entry the block is not cacheable
+  void taken(void *p, const block &b)
+  {
+    in_use_++;
+    try {
+      if (b.second) sizes_[p] = b;
+    } catch (const std::bad_alloc &) {
+    }
+  }
+
+  bool add(const block &b, void *p)
+  {
+    std::lock_guard<std::mutex> lock(mutex_);
+    if (kept_bytes_ + b.second > CACHE_BYTES) return false;
+    try {
+      kept_.emplace(b, p);
+    } catch (const std::bad_alloc &) {
+      return false;
+    }
+    kept_bytes_ += b.second;
+    return true;
+  }
+
+  // mutex_ held
+  void take_all(blocks &out)
+  {
+    out.swap(kept_);
+    kept_bytes_ = 0;
+  }
+
+  // without the mutex: giving memory back takes its time
+  static void release(const blocks &out)
+  {
+    for (const auto &b : out) Dev::release(b.second);
+  }
+
+  std::mutex mutex_;
+  blocks kept_;
+  std::unordered_map<void *, block> sizes_; // cacheable blocks in use
+  size_t kept_bytes_ = 0;
+  size_t in_use_ = 0; // blocks of any size
+};
+
+} // namespace mfp

@@ -103,7 +103,7 @@ const device_props &props();
 int ensure_init();
 
 // Device memory of the library's objects and scratch; freed blocks are kept
-// for the next ones (runtime.hip).  dfree waits for the device, as hipFree.
+// for the next ones (block_cache.h).  dfree waits for the device, as hipFree.
 int dmalloc(void **p, size_t bytes);
 void dfree(void *p);
 // bytes kept that way now: free memory from the library's point of view

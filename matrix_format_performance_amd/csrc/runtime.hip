@@ -1,5 +1,6 @@
 // Runtime: device selection, memory, grow-only buffers, timers, fills and the
 // Infinity-Cache flush.
+#include "block_cache.h"
 #include "mfp_internal.h"
 #include "wave64.h"
 
@@ -7,10 +8,7 @@
 #include <hip/hip_fp16.h>
 
 #include <cstring>
-#include <map>
 #include <mutex>
-#include <unordered_map>
-#include <utility>
 
 namespace mfp {
 
@@ -69,152 +67,55 @@ int ensure_init()
   return init_device(0);
 }
 
-// Device memory of the library's own objects and their scratch.
-//
-// hipMalloc / hipFree map and unmap memory: 30 to 90 us per call for blocks of
-// 16 MB and more, 210 to 250 us to free one while others are held, so that
-// building one plan spent more on its ten or so arrays than on its kernels
-// (nine formats of a 5M-entry matrix: 1.8 ms of kernels in 8.7 to 12.9 ms).
-// Freed blocks of 64 KB to 1 GB are therefore kept and handed out again, in
-// size classes an eighth of a power of two apart.
-//  * A block is kept only once the device is idle (dfree waits for it, as
-//    hipFree does), so whoever gets it next, on any stream or thread, finds
-//    nothing still running on it.
-//  * At most CACHE_BYTES are kept; an allocation that fails gives all of them
-//    back and tries again, and they are given back when the library's last
-//    block is freed.
-//  * mfp_malloc and mfp_free, whose pointers belong to the caller, do not
-//    take part.
-constexpr size_t CACHE_MIN = 64u << 10, CACHE_MAX = 1u << 30, CACHE_BYTES = 4ull << 30;
-
-struct block_cache {
-  std::mutex mutex;
-  std::multimap<size_t, void *> kept;                       // by size, device `device` only
-  std::unordered_map<void *, std::pair<size_t, int>> sizes; // cacheable blocks in use: size, device
-  size_t kept_bytes = 0;
-  size_t in_use = 0; // blocks of any size
-  int device = -1;   // of the kept blocks
+// Device memory of the library's own objects and their scratch comes from one
+// cache of blocks.  mfp_malloc and mfp_free, whose pointers belong to the
+// caller, do not take part.
+struct hip_memory {
+  static bool alloc(void **p, size_t bytes)
+  {
+    const hipError_t e = hipMalloc(p, bytes);
+    if (e != hipSuccess) {
+      (void)hipGetLastError();
+      set_error(std::string("hipMalloc of ") + std::to_string(bytes) + " bytes: " + hipGetErrorString(e));
+    }
+    return e == hipSuccess;
+  }
+  static void release(void *p) { (void)hipFree(p); }
+  static int current()
+  {
+    int d = -1;
+    if (hipGetDevice(&d) != hipSuccess) {
+      (void)hipGetLastError();
+      return -1;
+    }
+    return d;
+  }
+  static bool idle()
+  {
+    if (hipDeviceSynchronize() == hipSuccess) return true;
+    (void)hipGetLastError();
+    return false;
+  }
 };
 
-static block_cache &cache()
+static block_cache<hip_memory> &cache()
 {
-  static block_cache *c = new block_cache; // never destroyed: objects may outlive static destructors
+  static auto *c = new block_cache<hip_memory>; // never destroyed: objects may outlive static destructors
   return *c;
 }
 
-// cache().mutex held
-static void cache_release(block_cache &c)
-{
-  for (auto &b : c.kept) (void)hipFree(b.second);
-  c.kept.clear();
-  c.kept_bytes = 0;
-}
-
-size_t cached_device_bytes()
-{
-  block_cache &c = cache();
-  std::lock_guard<std::mutex> lock(c.mutex);
-  return c.kept_bytes;
-}
-
-static size_t cache_class(size_t bytes)
-{
-  size_t step = CACHE_MIN / 8;
-  while (step * 16 <= bytes) step *= 2; // 8 step <= bytes < 16 step
-  return (bytes + step - 1) / step * step;
-}
-
-static hipError_t malloc_or_release(void **p, size_t bytes)
-{
-  hipError_t e = hipMalloc(p, bytes);
-  if (e != hipSuccess) {
-    (void)hipGetLastError();
-    {
-      block_cache &c = cache();
-      std::lock_guard<std::mutex> lock(c.mutex);
-      cache_release(c);
-    }
-    e = hipMalloc(p, bytes);
-  }
-  return e;
-}
+size_t cached_device_bytes() { return cache().kept_bytes(g_props.device); }
 
 // Every allocation carries 256 bytes of slack past its end: kernels that read
-// 16-byte vectors may touch up to 12 bytes beyond an array's last element.
+// 16-byte vectors may touch up to 24 bytes beyond an array's last element.
 int dmalloc(void **p, size_t bytes)
 {
   MFP_CHECK(ensure_init());
-  *p = nullptr;
-  bytes += 256;
-  block_cache &c = cache();
-  const bool cacheable = bytes >= CACHE_MIN && bytes <= CACHE_MAX;
-  if (cacheable) {
-    const size_t size = cache_class(bytes);
-    std::lock_guard<std::mutex> lock(c.mutex);
-    if (c.device == g_props.device) {
-      const auto it = c.kept.lower_bound(size);
-      if (it != c.kept.end() && it->first <= size + size / 4) {
-        *p = it->second;
-        c.sizes[*p] = {it->first, c.device};
-        c.kept_bytes -= it->first;
-        c.kept.erase(it);
-        c.in_use++;
-        return MFP_OK;
-      }
-    }
-  }
-  const size_t size = cacheable ? cache_class(bytes) : bytes;
-  hipError_t e = malloc_or_release(p, size);
-  if (e != hipSuccess && size > bytes) { // without the rounding, then
-    (void)hipGetLastError();
-    e = hipMalloc(p, bytes);
-    if (e == hipSuccess) {
-      std::lock_guard<std::mutex> lock(c.mutex);
-      c.in_use++;
-      return MFP_OK;
-    }
-  }
-  MFP_HIP(e);
-  std::lock_guard<std::mutex> lock(c.mutex);
-  c.in_use++;
-  if (cacheable) c.sizes[*p] = {size, g_props.device};
-  return MFP_OK;
+  *p = cache().get(bytes + 256);
+  return *p ? MFP_OK : MFP_ERR_HIP;
 }
 
-void dfree(void *p)
-{
-  if (!p) return;
-  block_cache &c = cache();
-  size_t size = 0;
-  {
-    std::lock_guard<std::mutex> lock(c.mutex);
-    const auto it = c.sizes.find(p);
-    if (it != c.sizes.end()) {
-      int cur = -1;
-      if (hipGetDevice(&cur) == hipSuccess && cur == it->second.second) size = it->second.first;
-      c.sizes.erase(it);
-    }
-  }
-  if (size && hipDeviceSynchronize() != hipSuccess) {
-    (void)hipGetLastError();
-    size = 0;
-  }
-  void *free_now = p;
-  std::lock_guard<std::mutex> lock(c.mutex);
-  if (size) {
-    if (c.device != g_props.device) {
-      cache_release(c);
-      c.device = g_props.device;
-    }
-    if (c.kept_bytes + size <= CACHE_BYTES) {
-      c.kept.emplace(size, p);
-      c.kept_bytes += size;
-      free_now = nullptr;
-    }
-  }
-  if (free_now) (void)hipFree(free_now);
-  if (--c.in_use == 0) cache_release(c);
-}
+void dfree(void *p) { cache().put(p); }
 
 // ---- fills ----------------------------------------------------------------
 
@@ -387,8 +288,7 @@ int mfp_malloc(void **p, size_t bytes)
   MFP_ARG(p, "ptr is null");
   MFP_CHECK(ensure_init());
   *p = nullptr;
-  MFP_HIP(malloc_or_release(p, bytes + 256)); // the slack of dmalloc
-  return MFP_OK;
+  return cache().alloc(p, bytes + 256) ? MFP_OK : MFP_ERR_HIP; // the slack of dmalloc
 }
 
 int mfp_free(void *p)

@@ -1,0 +1,200 @@
+// The bookkeeping of csrc/block_cache.h against a simulated set of devices
+// (CPU only).  Built and run by tests/test_block_cache.py; prints "ALL OK" and
+// exits 0 on success.
+#include "block_cache.h"
+
+#include <cstdint>
+#include <cstdio>
+#include <cstdlib>
+#include <random>
+#include <thread>
+#include <vector>
+
+#define REQUIRE(c)                                                      \
+  do {                                                                  \
+    if (!(c)) {                                                         \
+      std::fprintf(stderr, "FAILED %s at line %d\n", #c, __LINE__);     \
+      std::exit(1);                                                     \
+    }                                                                   \
+  } while (0)
+
+namespace {
+
+// Addresses are handed out by counting and freed ones are not used again
+struct devices {
+  struct block {
+    int device;
+    size_t size;
+    bool busy; // work of the device may still use it
+  };
+  static inline std::mutex mutex;
+  static inline std::map<void *, block> live;
+  static inline size_t bytes = 0, limit = ~size_t(0), next = 4096;
+  static inline bool sync_fails = false;
+  static inline thread_local int now = 0; // a new thread's device is 0
+
+  static bool alloc(void **p, size_t n)
+  {
+    std::lock_guard<std::mutex> lock(mutex);
+    if (bytes + n > limit) return false;
+    *p = reinterpret_cast<void *>(next);
+    next += n + 4096;
+    bytes += n;
+    live[*p] = {now, n, false};
+    return true;
+  }
+  static void release(void *p)
+  {
+    std::lock_guard<std::mutex> lock(mutex);
+    REQUIRE(live.count(p));
+    bytes -= live[p].size;
+    live.erase(p);
+  }
+  static int current() { return now; }
+  static bool idle()
+  {
+    std::lock_guard<std::mutex> lock(mutex);
+    if (sync_fails) return false;
+    for (auto &b : live)
+      if (b.second.device == now) b.second.busy = false;
+    return true;
+  }
+};
+
+using cache_t = mfp::block_cache<devices>;
+
+// a block as an object of the current device gets it
+void *take(cache_t &c, size_t n)
+{
+  void *p = c.get(n);
+  REQUIRE(p);
+  std::lock_guard<std::mutex> lock(devices::mutex);
+  REQUIRE(devices::live.count(p));
+  auto &b = devices::live[p];
+  REQUIRE(b.device == devices::now); // another device's memory is not this one's
+  REQUIRE(b.size >= n);
+  REQUIRE(!b.busy); // nothing runs on it any more
+  b.busy = true;
+  return p;
+}
+
+constexpr size_t MB = 1u << 20;
+
+void reuse()
+{
+  cache_t c;
+  void *hold = take(c, 1000); // keeps the cache from emptying
+  void *p = take(c, 20 * MB);
+  c.put(p);
+  REQUIRE(c.kept_bytes(0) >= 20 * MB && c.kept_bytes(1) == 0);
+  REQUIRE(take(c, 19 * MB) == p);
+  REQUIRE(c.kept_bytes(0) == 0);
+  c.put(p);
+  void *q = take(c, 5 * MB); // a far smaller one does not take it
+  REQUIRE(q != p);
+  c.trim();
+  REQUIRE(c.kept_bytes(0) == 0 && devices::live.size() == 2);
+  c.put(q);
+  c.put(hold);
+  REQUIRE(devices::live.empty()); // the last block gives everything back
+}
+
+// The object of one device is destroyed while the library works on another,
+// from a thread on either
+void two_devices()
+{
+  for (int from = 0; from < 2; from++) {
+    cache_t c;
+    devices::now = 0;
+    void *a = take(c, 20 * MB);
+    devices::now = 1;
+    void *b = take(c, 1000);
+    devices::now = from;
+    c.put(a);
+    REQUIRE(c.kept_bytes(1) == 0);
+    devices::now = 1;
+    void *d = take(c, 20 * MB); // take checks its device
+    REQUIRE(d != a);
+    devices::now = 0;
+    if (from == 0) REQUIRE(take(c, 20 * MB) == a); // kept where it belongs
+    if (from == 0) c.put(a);
+    devices::now = 1;
+    c.put(d);
+    c.put(b);
+    REQUIRE(devices::live.empty());
+  }
+  devices::now = 0;
+}
+
+void limits()
+{
+  cache_t c;
+  void *hold = take(c, 1000);
+  std::vector<void *> many;
+  for (int i = 0; i < 12; i++) many.push_back(take(c, 700 * MB));
+  for (void *p : many) c.put(p);
+  REQUIRE(c.kept_bytes(0) <= mfp::CACHE_BYTES);
+  REQUIRE(c.kept_bytes(0) >= mfp::CACHE_BYTES - 1024 * MB);
+  // an allocation that fails takes back what is kept, the caller's own too
+  devices::limit = devices::bytes + MB;
+  void *big = take(c, 900 * MB);
+  REQUIRE(c.kept_bytes(0) == 0);
+  void *own = nullptr;
+  c.put(big);
+  REQUIRE(c.alloc(&own, 3000 * MB));
+  REQUIRE(c.kept_bytes(0) == 0);
+  devices::release(own);
+  // exactly the last bytes: without the rounding to a class
+  devices::limit = devices::bytes + 70001;
+  void *tight = c.get(70001);
+  REQUIRE(tight && devices::live[tight].size == 70001);
+  REQUIRE(!c.get(70001));
+  c.put(tight);
+  devices::limit = ~size_t(0);
+  // a device that cannot be waited for keeps nothing
+  void *p = take(c, 10 * MB);
+  devices::sync_fails = true;
+  c.put(p);
+  devices::sync_fails = false;
+  REQUIRE(c.kept_bytes(0) == 0 && !devices::live.count(p));
+  c.put(hold);
+  c.put(nullptr);
+  REQUIRE(devices::live.empty());
+}
+
+void threads()
+{
+  cache_t c;
+  std::vector<std::thread> ts;
+  for (int t = 0; t < 8; t++)
+    ts.emplace_back([&c, t] {
+      std::mt19937 rng(t);
+      std::vector<void *> held;
+      for (int i = 0; i < 4000; i++) {
+        devices::now = (int)(rng() % 2);
+        if (held.size() < 6 && rng() % 2) {
+          held.push_back(take(c, 1 + (size_t)(rng() % 4 ? rng() % (2 * MB) : rng() % (80 * MB))));
+        } else if (!held.empty()) {
+          const size_t k = rng() % held.size();
+          c.put(held[k]); // from either device
+          held[k] = held.back();
+          held.pop_back();
+        }
+        if (rng() % 500 == 0) c.trim();
+      }
+      for (void *p : held) c.put(p);
+    });
+  for (auto &t : ts) t.join();
+  REQUIRE(devices::live.empty() && devices::bytes == 0);
+}
+
+} // namespace
+
+int main()
+{
+  reuse();
+  two_devices();
+  limits();
+  threads();
+  std::printf("ALL OK\n");
+}
