@@ -15,6 +15,7 @@
 // COO, SCOO and the hybrids accumulate with atomics (order not fixed).
 #include "kernels.h"
 #include "mfp_internal.h"
+#include "row_chunks.h"
 #include "values16.h"
 #include "wave64.h"
 
@@ -311,8 +312,7 @@ __global__ __launch_bounds__(256, 8) void k_csr_vector_lds(uint32_t rows, uint32
     if (!all && rs[cur + 1] - base > CAP - off) {
       const uint32_t e = rs[cur + 1];
       T dot = 0;
-      for (uint32_t c0 = base; c0 < e; c0 += CHUNK) {
-        const uint32_t n = min(CHUNK, e - c0);
+      for_row_chunks(base, e, CHUNK, [&](uint32_t c0, uint32_t n) {
         cvl_stage(c0, n, ci, a, x, sa, sx, [] {});
         __syncthreads();
         if (tid < G) {
@@ -331,7 +331,7 @@ __global__ __launch_bounds__(256, 8) void k_csr_vector_lds(uint32_t rows, uint32
           for (; i < n; i += G) dot = fma_t(sa[sh + i], sx[sh + i], dot);
         }
         __syncthreads();
-      }
+      });
       if (tid < 64u) { // the first group's wave
         dot = group_reduce<G>(dot);
         if (tid == 0) y[r0 + cur] = dot;
