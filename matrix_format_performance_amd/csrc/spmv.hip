@@ -140,74 +140,68 @@ __global__ __launch_bounds__(64) void k_csr_scalar(uint32_t rows, const uint32_t
 // offsets, so no load is predicated) before the x entries of the current
 // eight are gathered and summed, so a long row waits for one memory latency
 // per eight elements instead of two per four.
-//
-// Elements i, i + G, ... of one row (below e) onto the lane's sum.
-template <typename T, int G>
-__device__ __forceinline__ T csr_vector_rest(uint32_t i, uint32_t e, const uint32_t *__restrict__ ci,
-                                             const T *__restrict__ a, const T *__restrict__ x, T dot)
-{
-  constexpr uint32_t U = 8;
-  if (i + (U - 1) * G < e) {
-    T an[U];
-    uint32_t cn[U];
-#pragma unroll
-    for (uint32_t u = 0; u < U; u++) {
-      an[u] = ldg_stream(a + i + u * G);
-      cn[u] = ldg_stream(ci + i + u * G);
-    }
-    for (;;) {
-      T ac[U];
-      uint32_t cc[U];
-#pragma unroll
-      for (uint32_t u = 0; u < U; u++) {
-        ac[u] = an[u];
-        cc[u] = cn[u];
-      }
-      const uint32_t inext = i + U * G;
-      const bool more = inext + (U - 1) * G < e;
-#pragma unroll
-      for (uint32_t u = 0; u < U; u++) {
-        const uint32_t j = min(inext + u * G, e - 1u); // e > i: in range
-        an[u] = ldg_stream(a + j);
-        cn[u] = ldg_stream(ci + j);
-      }
-      T xv[U];
-#pragma unroll
-      for (uint32_t u = 0; u < U; u++) xv[u] = x[cc[u]];
-#pragma unroll
-      for (uint32_t u = 0; u < U; u++) dot = fma_t(ac[u], xv[u], dot);
-      i = inext;
-      if (!more) break;
-    }
-  }
-  for (; i + 3u * G < e; i += 4u * G) {
-    const T a0 = ldg_stream(a + i), a1 = ldg_stream(a + i + G);
-    const T a2 = ldg_stream(a + i + 2 * G), a3 = ldg_stream(a + i + 3 * G);
-    const uint32_t c0 = ldg_stream(ci + i), c1 = ldg_stream(ci + i + G);
-    const uint32_t c2 = ldg_stream(ci + i + 2 * G), c3 = ldg_stream(ci + i + 3 * G);
-    const T x0 = x[c0], x1 = x[c1], x2 = x[c2], x3 = x[c3];
-    dot = fma_t(a0, x0, dot);
-    dot = fma_t(a1, x1, dot);
-    dot = fma_t(a2, x2, dot);
-    dot = fma_t(a3, x3, dot);
-  }
-  for (; i < e; i += G) dot = fma_t(ldg_stream(a + i), x[ldg_stream(ci + i)], dot);
-  return dot;
-}
-
+// The loops stand in the kernel itself: as a function that is inlined they
+// take 65 VGPRs in FP32 instead of 48 and cost a wave per SIMD (800k entries in
+// rows of 6, 34, 100: 7.3, 7.3, 5.6 us instead of 6.7, 6.8, 4.6).
 template <typename T, int G>
 __global__ __launch_bounds__(256) void k_csr_vector(uint32_t rows, const uint32_t *__restrict__ rp,
                                                     const uint32_t *__restrict__ ci,
                                                     const T *__restrict__ a, const T *__restrict__ x,
                                                     T *__restrict__ y)
 {
+  constexpr uint32_t U = 8;
   const uint32_t blk = xcd_block(blockIdx.x, gridDim.x);
   const uint32_t row = (blk * 256u + threadIdx.x) / G;
   const uint32_t lane = threadIdx.x % G;
   T dot = 0;
   if (row < rows) {
     const uint32_t b = rp[row], e = rp[row + 1];
-    dot = csr_vector_rest<T, G>(b + lane, e, ci, a, x, dot);
+    uint32_t i = b + lane;
+    if (i + (U - 1) * G < e) {
+      T an[U];
+      uint32_t cn[U];
+#pragma unroll
+      for (uint32_t u = 0; u < U; u++) {
+        an[u] = ldg_stream(a + i + u * G);
+        cn[u] = ldg_stream(ci + i + u * G);
+      }
+      for (;;) {
+        T ac[U];
+        uint32_t cc[U];
+#pragma unroll
+        for (uint32_t u = 0; u < U; u++) {
+          ac[u] = an[u];
+          cc[u] = cn[u];
+        }
+        const uint32_t inext = i + U * G;
+        const bool more = inext + (U - 1) * G < e;
+#pragma unroll
+        for (uint32_t u = 0; u < U; u++) {
+          const uint32_t j = min(inext + u * G, e - 1u); // e > i: in range
+          an[u] = ldg_stream(a + j);
+          cn[u] = ldg_stream(ci + j);
+        }
+        T xv[U];
+#pragma unroll
+        for (uint32_t u = 0; u < U; u++) xv[u] = x[cc[u]];
+#pragma unroll
+        for (uint32_t u = 0; u < U; u++) dot = fma_t(ac[u], xv[u], dot);
+        i = inext;
+        if (!more) break;
+      }
+    }
+    for (; i + 3u * G < e; i += 4u * G) {
+      const T a0 = ldg_stream(a + i), a1 = ldg_stream(a + i + G);
+      const T a2 = ldg_stream(a + i + 2 * G), a3 = ldg_stream(a + i + 3 * G);
+      const uint32_t c0 = ldg_stream(ci + i), c1 = ldg_stream(ci + i + G);
+      const uint32_t c2 = ldg_stream(ci + i + 2 * G), c3 = ldg_stream(ci + i + 3 * G);
+      const T x0 = x[c0], x1 = x[c1], x2 = x[c2], x3 = x[c3];
+      dot = fma_t(a0, x0, dot);
+      dot = fma_t(a1, x1, dot);
+      dot = fma_t(a2, x2, dot);
+      dot = fma_t(a3, x3, dot);
+    }
+    for (; i < e; i += G) dot = fma_t(ldg_stream(a + i), x[ldg_stream(ci + i)], dot);
   }
   dot = group_reduce<G>(dot);
   if (lane == 0 && row < rows) y[row] = dot;
