@@ -1465,27 +1465,43 @@ static int launch_k(void (*kernel)(P...), dim3 grid, dim3 block, uint32_t lds, h
   return launched();
 }
 
+// Rows per workgroup of k_csr_vector_lds, 0 where k_csr_vector serves the
+// matrix.  The LDS form for rows of up to CAP / 8 entries on average (256 FP32,
+// 128 FP64: enough rows per chunk for every group of lanes) and for rows of
+// 2 CAP or more (whole chunks); between them a chunk holds one to seven
+// rows and most groups idle: rows of about 1,200 took 25 us here against
+// 27 to 301 from LDS, 64 to 2 lanes.
+// A small matrix is a chain of latencies in either form, and the LDS form's is
+// longer.  From 8 MB of entries it is the faster one (lanes from the mean, FP32
+// row by row -> LDS: 800k entries in rows of 6, 34, 100 6.8 -> 7.6, 6.8 -> 7.2,
+// 4.6 -> 4.8 us, 1.6M 12.5 -> 13.1, 12.5 -> 11.8, 9.8 -> 8.6; FP64 400k 4.9 ->
+// 5.3, 5.5 -> 5.3, 3.7 -> 4.0, 800k 9.0 -> 8.4, 9.1 -> 8.0, 6.8 -> 5.6), and
+// earlier where lanes idle (FP32 rows of 6 by 64 lanes, 33k and 67k rows: 5.7 ->
+// 6.7, 11.0 -> 10.6 us) or a row is several waits of its lanes (rows of 34 by 4
+// lanes, 135k, 200k, 400k entries: 3.9 -> 4.0, 4.2 -> 4.0, 6.0 -> 4.4 us).
+static uint32_t csr_vector_rows(int dtype, uint32_t lanes, uint32_t rows, uint64_t nnz)
+{
+  if (rows == 0) return 0;
+  const uint32_t cap = dtype == MFP_F32 ? cvl<float>::CAP : cvl<double>::CAP;
+  const uint64_t vs = dtype_size(dtype);
+  const double mean = (double)nnz / rows;
+  if (mean > cap / 8 && mean < 2.0 * cap) return 0;
+  if (nnz * (4 + vs) < 8u << 20 && (uint64_t)rows * lanes * vs < 16u << 20 && !(nnz >= 1u << 18 && mean >= 4.0 * lanes))
+    return 0;
+  // rows that fill 85% of a chunk on average, fewer where that would leave
+  // a CU with less than two workgroups
+  const uint32_t fit = (uint32_t)std::min(256.0, std::max(1.0, 0.85 * cap / std::max(mean, 1.0)));
+  return std::max(1u, std::min(fit, ceil_div_u32(rows, 2u * (uint32_t)std::max(1, props().cu_count))));
+}
+
 template <typename T, int G>
 static int csr_vector_g(uint32_t rows, uint64_t nnz, const uint32_t *rp, const uint32_t *ci, const T *a, const T *x,
                         T *y, hipStream_t s)
 {
   const dim3 b(256);
   const uint32_t grid = ceil_div_u32((uint64_t)rows * G, 256);
-  // The LDS form for rows of up to CAP / 8 entries on average (256 FP32, 128
-  // FP64: enough rows per chunk for every group of lanes) and for rows of
-  // 2 CAP or more (whole chunks); between them a chunk holds one to seven
-  // rows and most groups idle: rows of about 1,200 took 25 us here against
-  // 27 to 301 from LDS, 64 to 2 lanes.  Below 131,072 entries both are a
-  // launch's latency (3,000 rows of 34: 3.9 us each).
-  const double mean = (double)nnz / rows;
-  const uint32_t cap = cvl<T>::CAP;
-  if (nnz >= (1u << 17) && (mean <= cap / 8 || mean >= 2.0 * cap)) {
-    // rows that fill 85% of a chunk on average, fewer where that would leave
-    // a CU with less than two workgroups
-    const uint32_t fit = (uint32_t)std::min(256.0, std::max(1.0, 0.85 * cap / std::max(mean, 1.0)));
-    const uint32_t rb = std::max(1u, std::min(fit, ceil_div_u32(rows, 2u * (uint32_t)std::max(1, props().cu_count))));
-    return launch_k(k_csr_vector_lds<T, G>, dim3(ceil_div_u32(rows, rb)), b, 0, s, rows, rb, rp, ci, a, x, y);
-  }
+  const uint32_t rb = csr_vector_rows(sizeof(T) == 4 ? MFP_F32 : MFP_F64, G, rows, nnz);
+  if (rb) return launch_k(k_csr_vector_lds<T, G>, dim3(ceil_div_u32(rows, rb)), b, 0, s, rows, rb, rp, ci, a, x, y);
   return launch_k(k_csr_vector<T, G>, dim3(grid), b, 0, s, rows, rp, ci, a, x, y);
 }
 
