@@ -31,7 +31,19 @@ uint32_t adaptive_vectors_per_lane(int dtype, uint32_t nnz_per_wg);
 
 int launch_csr_scalar(int dtype, uint32_t rows, const uint32_t *rp, const uint32_t *ci,
                       const void *a, const void *x, void *y, hipStream_t s);
-int launch_csr_vector(int dtype, uint32_t lanes, uint32_t rows, uint64_t nnz, const uint32_t *rp,
+// CSR-vector over FP32 / FP64: how the rows of one matrix are taken.
+struct csr_vector_layout {
+  uint32_t rb = 0;          // rows per workgroup of the LDS form; 0: row by row
+  uint32_t count = 0;       // blocks of rb rows that are summed row by row all the same
+  uint32_t *list = nullptr; // their numbers (mask owns the memory)
+  uint32_t *mask = nullptr; // a bit per block
+};
+uint32_t csr_vector_rows(int dtype, uint32_t lanes, uint32_t rows, uint64_t nnz); // rb
+// longest: entries of the longest row (of no use where rb <= 1); waits for the stream where blocks are looked at
+int csr_vector_layout_build(int dtype, uint32_t lanes, uint32_t rows, uint64_t nnz, uint32_t longest,
+                            const uint32_t *rp, csr_vector_layout *out, hipStream_t s);
+void csr_vector_layout_free(csr_vector_layout *l);
+int launch_csr_vector(int dtype, uint32_t lanes, uint32_t rows, const csr_vector_layout &l, const uint32_t *rp,
                       const uint32_t *ci, const void *a, const void *x, void *y, hipStream_t s);
 int launch_csr_adaptive(int dtype, const adaptive_args &g, const void *a, const void *x, void *y,
                         hipStream_t s);

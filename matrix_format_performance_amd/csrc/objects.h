@@ -27,6 +27,7 @@ struct mfp_plan_s {
   bool coo_owner = false; // COO: no row too long for the form without a zero fill
   uint32_t slices = 0, ss = 0, L = 0, scoo_threads = 512;
   uint32_t *sp = nullptr;
+  mfp::csr_vector_layout cv;
   mfp::adaptive_layout ad;
   // CSR-Adaptive plans over f32 / f64 values: row blocks of STREAM_W entries
   // as (first row, first entry) pairs for the CSR-stream SpMM (mfp_plan_spmm

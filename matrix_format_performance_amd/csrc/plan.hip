@@ -156,6 +156,7 @@ static int plan_free_arrays(mfp_plan p)
   dfree(p->pk_base);
   scoo_cs_free(&p->cs);
   lp_binned_free(&p->lpb);
+  csr_vector_layout_free(&p->cv);
   free_adaptive_layout(&p->ad);
   dfree(p->stream_meta);
   return MFP_OK;
@@ -560,6 +561,14 @@ int mfp_plan_create(mfp_plan *out, mfp_matrix m, int format, const mfp_tuning *t
       set_error("lanes must be a power of two in [2, 64]");
       return fail(MFP_ERR_ARG);
     }
+    {
+      mfp_row_stats rs{};
+      if (csr_vector_rows(m->dtype, t.lanes, m->rows, m->nnz) > 1) st = matrix_stats(m, &rs, s);
+      if (st == MFP_OK)
+        st = csr_vector_layout_build(m->dtype, t.lanes, m->rows, m->nnz, rs.max_elements_in_rows, m->row_ptr, &p->cv,
+                                     s);
+      if (st != MFP_OK) return fail(st);
+    }
     break;
   case MFP_CSR_ADAPTIVE:
     st = build_adaptive_layout(m->dtype, m->rows, m->row_ptr, t.nnz_per_wg, t.long_row, t.chunk,
@@ -702,7 +711,7 @@ static int plan_spmv(mfp_plan p, const void *x, void *y, hipStream_t s, void *pa
   case MFP_CSR_SCALAR:
     return launch_csr_scalar(dt, m->rows, m->row_ptr, m->columns, m->values, x, y, s);
   case MFP_CSR_VECTOR:
-    return launch_csr_vector(dt, p->t.lanes, m->rows, m->nnz, m->row_ptr, m->columns, m->values, x, y, s);
+    return launch_csr_vector(dt, p->t.lanes, m->rows, p->cv, m->row_ptr, m->columns, m->values, x, y, s);
   case MFP_CSR_ADAPTIVE: {
     adaptive_args g;
     g.rows = m->rows;

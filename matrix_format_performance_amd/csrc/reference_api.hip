@@ -239,13 +239,20 @@ int mfp_gpu_csr_vector_spmv(int dtype, const mfp_host_csr *A, mfp_buffer Ad, mfp
   MFP_ARG(out, "out is null");
   // y pre-filled with 24 so an unwritten row shows (gpu_matrix_multiplier.cu:403)
   MFP_CHECK(upload_csr(dtype, A, Ad, cd, rd, xd, yd, 24.0));
+  const uint32_t *rp = (const uint32_t *)mfp_buffer_ptr(rd);
+  mfp_row_stats rs{};
+  if (csr_vector_rows(dtype, REFERENCE_VECTOR_LANES, A->rows, A->nnz) > 1) MFP_CHECK(row_stats_device(A->rows, rp, &rs, nullptr));
+  csr_vector_layout l;
+  MFP_CHECK(csr_vector_layout_build(dtype, REFERENCE_VECTOR_LANES, A->rows, A->nnz, rs.max_elements_in_rows, rp, &l,
+                                    nullptr));
   double sec = 0;
-  MFP_CHECK(run_timed([&] {
-    return launch_csr_vector(dtype, REFERENCE_VECTOR_LANES, A->rows, A->nnz, (const uint32_t *)mfp_buffer_ptr(rd),
-                             (const uint32_t *)mfp_buffer_ptr(cd), mfp_buffer_ptr(Ad),
-                             mfp_buffer_ptr(xd), mfp_buffer_ptr(yd), nullptr);
-  }, &sec));
-  MFP_CHECK(finish(dtype, A->rows, mfp_buffer_ptr(yd), reusable_vector, reference_y));
+  int st = run_timed([&] {
+    return launch_csr_vector(dtype, REFERENCE_VECTOR_LANES, A->rows, l, rp, (const uint32_t *)mfp_buffer_ptr(cd),
+                             mfp_buffer_ptr(Ad), mfp_buffer_ptr(xd), mfp_buffer_ptr(yd), nullptr);
+  }, &sec);
+  if (st == MFP_OK) st = finish(dtype, A->rows, mfp_buffer_ptr(yd), reusable_vector, reference_y);
+  csr_vector_layout_free(&l);
+  MFP_CHECK(st);
   fill_measurement(out, "GPU CSR (vector)", sec, csr_bytes(dtype_size(dtype), A->rows, A->nnz),
                    2.0 * (double)A->nnz);
   return MFP_OK;

@@ -218,10 +218,10 @@ __global__ __launch_bounds__(256) void k_csr_vector(uint32_t rows, const uint32_
 // each after the last, and a row's 136 bytes are read in 4-byte loads.  Here
 // a workgroup's loads are independent of its row lengths: 16 bytes per lane,
 // two vectors of values and of columns, then their 8 (FP64: 4) gathers.
-// Eight workgroups share a CU (16 KB of LDS, 44 to 56 VGPRs).  Where the
+// Eight workgroups share a CU (16 KB of LDS, 48 to 60 VGPRs).  Where the
 // rows fit at once, their values and columns are on the way before the row
 // starts are staged, and the gathers go out together behind that barrier:
-// 300,007 rows of 4 to 64 random entries 58.7 -> 53.1 us (FP64 72.5 -> 61.5);
+// 300,007 rows of 4 to 64 random entries 58.7 -> 53.3 us (FP64 72.5 -> 61.5);
 // without the barrier between a wave's loads and its gathers 57 to 61 (71 to
 // 72).  FP32, lanes from the mean, row by row -> from LDS: 27-point stencil of
 // 100^3 121.7 -> 54.2 us, 5-point stencil of 1400^2 56.8 -> 22.5, those random
@@ -230,6 +230,10 @@ __global__ __launch_bounds__(256) void k_csr_vector(uint32_t rows, const uint32_
 // lane).  Larger chunks were slower: three vectors per lane 59.5 and four 70.6
 // us on the 27-point stencil, against 55.5.
 constexpr uint32_t CVL_K = 2, CVL_U = 2;
+// entries of a listed row in flight, and of a staged row read from LDS together
+constexpr uint32_t CVL_REST = 8;
+template <typename T>
+constexpr uint32_t CVL_STEP = sizeof(T) == 4 ? 8 : 4;
 template <typename T>
 struct cvl {
   static constexpr uint32_t N = vec16<T>::N, K = CVL_K, CAP = 256 * K * N;
@@ -275,8 +279,46 @@ __device__ __forceinline__ void cvl_stage(uint32_t base, uint32_t n, const uint3
   }
 }
 
+// One lane's sum of the row [b, e): its elements in k_csr_vector's order,
+// CVL_REST at a time.
 template <typename T, int G>
-__global__ __launch_bounds__(256, 8) void k_csr_vector_lds(uint32_t rows, uint32_t RB, const uint32_t *__restrict__ rp,
+__device__ __forceinline__ T csr_vector_row(uint32_t b, uint32_t e, uint32_t lane, const uint32_t *__restrict__ ci,
+                                            const T *__restrict__ a, const T *__restrict__ x)
+{
+  constexpr uint32_t U = CVL_REST;
+  uint32_t left = e - b > lane ? (e - b - lane - 1u) / G + 1u : 0u; // counted down: positions may end at 2^32
+  uint32_t i = b + lane;
+  T dot = 0;
+  if (left >= U) {
+    uint32_t next[U];
+#pragma unroll
+    for (uint32_t u = 0; u < U; u++) next[u] = ldg_stream(ci + i + u * G);
+    for (; left >= U; left -= U, i += U * G) {
+      // the gathers, this round's values and the next round's columns together
+      T v[U], xv[U];
+#pragma unroll
+      for (uint32_t u = 0; u < U; u++) xv[u] = x[next[u]];
+#pragma unroll
+      for (uint32_t u = 0; u < U; u++) {
+        v[u] = ldg_stream(a + i + u * G);
+        next[u] = ldg_stream(ci + min(i + (U + u) * G, e - 1u)); // past the row: not used
+      }
+#pragma unroll
+      for (uint32_t u = 0; u < U; u++) dot = fma_t(v[u], xv[u], dot);
+    }
+  }
+  for (; left; left--, i += G) dot = fma_t(ldg_stream(a + i), x[ldg_stream(ci + i)], dot);
+  return dot;
+}
+
+// The first `extra` workgroups (a multiple of 8) sum the nlist listed blocks of
+// rows as k_csr_vector does, `lists` lanes each; mask has a bit for each block
+// of the list (csr_vector_layout_build).
+template <typename T, int G>
+__global__ __launch_bounds__(256, 8) void k_csr_vector_lds(uint32_t rows, uint32_t RB, uint32_t extra, uint32_t lists,
+                                                        uint32_t nlist, const uint32_t *__restrict__ list,
+                                                        const uint32_t *__restrict__ mask,
+                                                        const uint32_t *__restrict__ rp,
                                                         const uint32_t *__restrict__ ci,
                                                         const T *__restrict__ a, const T *__restrict__ x,
                                                         T *__restrict__ y)
@@ -285,10 +327,22 @@ __global__ __launch_bounds__(256, 8) void k_csr_vector_lds(uint32_t rows, uint32
   __shared__ __align__(16) T sa[CAP];
   __shared__ __align__(16) T sx[CAP];
   __shared__ uint32_t rs[257];
-  const uint32_t r0 = xcd_block(blockIdx.x, gridDim.x) * RB; // RB <= 256
-  const uint32_t nr = min(RB, rows - r0), tid = threadIdx.x;
+  const uint32_t tid = threadIdx.x;
+  if (blockIdx.x < extra) {
+    const uint32_t per = (RB * G + lists - 1u) / lists, h = blockIdx.x / per;
+    if (h >= nlist || tid >= lists) return;
+    const uint32_t l0 = list[h] * RB, lr = (blockIdx.x % per * lists + tid) / G, row = l0 + lr;
+    const bool ok = lr < min(RB, rows - l0);
+    T dot = ok ? csr_vector_row<T, G>(rp[row], rp[row + 1], tid % G, ci, a, x) : (T)0;
+    dot = group_reduce<G>(dot);
+    if (ok && tid % G == 0) y[row] = dot;
+    return;
+  }
+  const uint32_t blk = xcd_block(blockIdx.x - extra, gridDim.x - extra), r0 = blk * RB; // RB <= 256
+  const uint32_t nr = min(RB, rows - r0);
   const uint32_t p = tid <= nr ? rp[r0 + tid] : 0u, first = rp[r0], last = rp[r0 + nr];
   const bool all = last - first <= CAP - first % N; // the usual case: every row fits at once
+  if (!all && nlist && ((mask[blk >> 5] >> (blk & 31u)) & 1u)) return; // listed
   auto row_starts = [&] {
     if (tid <= nr) rs[tid] = p;
     if (tid == 0 && nr == 256u) rs[256] = last;
@@ -362,8 +416,21 @@ __global__ __launch_bounds__(256, 8) void k_csr_vector_lds(uint32_t rows, uint32
 #pragma unroll
       for (uint32_t q = 0; q < U; q++) dot[q] = b[q] < e[q] ? fma_t(qa[q], qx[q], (T)0) : (T)0;
 #pragma unroll
-      for (uint32_t q = 0; q < U; q++)
-        for (uint32_t i = b[q] + G; i < e[q]; i += G) dot[q] = fma_t(sa[i], sx[i], dot[q]);
+      for (uint32_t q = 0; q < U; q++) {
+        constexpr uint32_t S = CVL_STEP<T>;
+        uint32_t i = b[q] + G;
+        for (; i + (S - 1u) * G < e[q]; i += S * G) { // not one LDS latency per element
+          T ra[S], rx[S];
+#pragma unroll
+          for (uint32_t k = 0; k < S; k++) {
+            ra[k] = sa[i + k * G];
+            rx[k] = sx[i + k * G];
+          }
+#pragma unroll
+          for (uint32_t k = 0; k < S; k++) dot[q] = fma_t(ra[k], rx[k], dot[q]);
+        }
+        for (; i < e[q]; i += G) dot[q] = fma_t(sa[i], sx[i], dot[q]);
+      }
 #pragma unroll
       for (uint32_t q = 0; q < U; q++) dot[q] = group_reduce<G>(dot[q]);
 #pragma unroll
@@ -1479,7 +1546,7 @@ static int launch_k(void (*kernel)(P...), dim3 grid, dim3 block, uint32_t lds, h
 // earlier where lanes idle (FP32 rows of 6 by 64 lanes, 33k and 67k rows: 5.7 ->
 // 6.7, 11.0 -> 10.6 us) or a row is several waits of its lanes (rows of 34 by 4
 // lanes, 135k, 200k, 400k entries: 3.9 -> 4.0, 4.2 -> 4.0, 6.0 -> 4.4 us).
-static uint32_t csr_vector_rows(int dtype, uint32_t lanes, uint32_t rows, uint64_t nnz)
+uint32_t csr_vector_rows(int dtype, uint32_t lanes, uint32_t rows, uint64_t nnz)
 {
   if (rows == 0) return 0;
   const uint32_t cap = dtype == MFP_F32 ? cvl<float>::CAP : cvl<double>::CAP;
@@ -1494,28 +1561,118 @@ static uint32_t csr_vector_rows(int dtype, uint32_t lanes, uint32_t rows, uint64
   return std::max(1u, std::min(fit, ceil_div_u32(rows, 2u * (uint32_t)std::max(1, props().cu_count))));
 }
 
+// Lists the blocks of RB rows whose rows would keep their one workgroup busy
+// for longer than `limit` and than their own lanes would take side by side.
+// Times in ns: a chunk waits 800, gathers at 0.85 per entry and then takes 8
+// per step of its longest row's lanes (a row that shares a chunk: its part of
+// all that); row by row, a row's lanes wait 570 per CVL_REST entries of each.
+// A wave per block.
+template <typename T>
+__global__ __launch_bounds__(256) void k_csr_vector_blocks(uint32_t rows, uint32_t RB, uint32_t nblocks, float lanes,
+                                                           float limit, const uint32_t *__restrict__ rp,
+                                                           uint32_t *__restrict__ list, uint32_t *__restrict__ mask,
+                                                           uint32_t *__restrict__ count)
+{
+  constexpr float CAP = cvl<T>::CAP, CHUNK = cvl<T>::CHUNK;
+  const uint32_t w = blockIdx.x * 4u + (threadIdx.x >> 6), lane = threadIdx.x & 63u;
+  if (w >= nblocks) return; // the whole wave
+  const uint32_t r0 = w * RB, nr = min(RB, rows - r0);
+  if (rp[r0 + nr] - rp[r0] <= cvl<T>::CAP - cvl<T>::N) return;
+  float chunks = 0, longest = 0;
+  for (uint32_t r = lane; r < nr; r += 64) {
+    const float len = (float)(rp[r0 + r + 1] - rp[r0 + r]);
+    longest = fmaxf(longest, len);
+    if (len > CAP)
+      chunks += ceilf(len / CHUNK) * (800.0f + 0.85f * CHUNK + 8.0f * CHUNK / lanes);
+    else
+      chunks += (960.0f / CAP + 0.85f) * len + 8.0f * fmaxf(len * len / (lanes * CAP), fmaxf(lanes, len) / 256.0f);
+  }
+  chunks = group_reduce<64>(chunks);
+#pragma unroll
+  for (int d = 32; d >= 1; d >>= 1) longest = fmaxf(longest, __shfl_xor(longest, d, 64));
+  chunks += 800.0f;
+  if (lane == 0 && chunks > limit && chunks > 2500.0f + 570.0f * longest / (CVL_REST * lanes)) {
+    atomicOr(&mask[w >> 5], 1u << (w & 31u));
+    list[atomicAdd(count, 1u)] = w;
+  }
+}
+
+// A workgroup sums its block's rows chunk after chunk.  Where long rows lie
+// side by side (rows sorted by length, a dense stretch) that is a chain of
+// hundreds of chunks on one CU, while their own lanes would work on all of them
+// at once: such blocks are listed and summed row by row, in the same launch, a
+// wave per workgroup while they are few.  300,007 rows of 6 with 256 rows of
+// 1,500 among them, FP32, 8 lanes: row by row 68 us, all from LDS 3,214,
+// listed 30 (4 lanes 157, 5,884, 59; FP64 77, 683, 32); 1M power-law rows
+// sorted by length 845, 6,610, 780 (FP64 1,170, 7,803, 560), unsorted 341, 175,
+// 176.  One row of 9,000 entries among 47,000 of 34, 64 lanes, is the case that
+// stays behind the row-by-row form: 15.6 against 18.6 us.
+int csr_vector_layout_build(int dtype, uint32_t lanes, uint32_t rows, uint64_t nnz, uint32_t longest,
+                            const uint32_t *rp, csr_vector_layout *out, hipStream_t s)
+{
+  *out = csr_vector_layout{};
+  out->rb = csr_vector_rows(dtype, lanes, rows, nnz);
+  const bool f32 = dtype == MFP_F32;
+  const uint32_t cap = f32 ? cvl<float>::CAP : cvl<double>::CAP;
+  if (out->rb <= 1 || (uint64_t)out->rb * longest <= 2 * cap) return MFP_OK; // no block is that long
+  // a quarter of what the whole product takes at least (1.5 TB/s, a launch)
+  const float limit = 0.25f * std::max(4000.0f, (float)nnz * (float)(4 + dtype_size(dtype)) / 1500.0f);
+  const uint32_t nb = ceil_div_u32(rows, out->rb), words = (nb + 31) / 32;
+  // mask, count, list
+  MFP_CHECK(dmalloc((void **)&out->mask, ((uint64_t)words + 1 + nb) * 4));
+  uint32_t *count = out->mask + words;
+  out->list = count + 1;
+  int st = fill_u32(out->mask, 0, (uint64_t)words + 1, s);
+  if (st == MFP_OK) {
+    const auto kern = f32 ? k_csr_vector_blocks<float> : k_csr_vector_blocks<double>;
+    kern<<<ceil_div_u32(nb, 4), 256, 0, s>>>(rows, out->rb, nb, (float)lanes, limit, rp, out->list, out->mask, count);
+    st = launched();
+  }
+  if (st == MFP_OK && (hipMemcpyAsync(&out->count, count, 4, hipMemcpyDeviceToHost, s) != hipSuccess ||
+                       hipStreamSynchronize(s) != hipSuccess)) {
+    set_error("CSR-vector: blocks of long rows");
+    st = MFP_ERR_HIP;
+  }
+  if (st != MFP_OK || out->count == 0) csr_vector_layout_free(out);
+  return st;
+}
+
+void csr_vector_layout_free(csr_vector_layout *l)
+{
+  dfree(l->mask);
+  l->mask = l->list = nullptr;
+  l->count = 0;
+}
+
 template <typename T, int G>
-static int csr_vector_g(uint32_t rows, uint64_t nnz, const uint32_t *rp, const uint32_t *ci, const T *a, const T *x,
-                        T *y, hipStream_t s)
+static int csr_vector_g(uint32_t rows, const csr_vector_layout &l, const uint32_t *rp, const uint32_t *ci, const T *a,
+                        const T *x, T *y, hipStream_t s)
 {
   const dim3 b(256);
+  if (l.rb) {
+    // few listed blocks spread over the CUs, a wave per workgroup
+    uint32_t lists = 64;
+    while (lists < 256 && l.count * ((l.rb * G + lists - 1) / lists) > 4u * (uint32_t)std::max(1, props().cu_count))
+      lists *= 2;
+    const uint32_t extra = (l.count * ((l.rb * G + lists - 1) / lists) + 7u) & ~7u;
+    return launch_k(k_csr_vector_lds<T, G>, dim3(extra + ceil_div_u32(rows, l.rb)), b, 0, s, rows, l.rb, extra, lists,
+                    l.count, l.list, l.mask, rp, ci, a, x, y);
+  }
   const uint32_t grid = ceil_div_u32((uint64_t)rows * G, 256);
-  const uint32_t rb = csr_vector_rows(sizeof(T) == 4 ? MFP_F32 : MFP_F64, G, rows, nnz);
-  if (rb) return launch_k(k_csr_vector_lds<T, G>, dim3(ceil_div_u32(rows, rb)), b, 0, s, rows, rb, rp, ci, a, x, y);
   return launch_k(k_csr_vector<T, G>, dim3(grid), b, 0, s, rows, rp, ci, a, x, y);
 }
 
 template <typename T>
-static int csr_vector_t(uint32_t lanes, uint32_t rows, uint64_t nnz, const uint32_t *rp, const uint32_t *ci,
-                        const T *a, const T *x, T *y, hipStream_t s)
+static int csr_vector_t(uint32_t lanes, uint32_t rows, const csr_vector_layout &l, const uint32_t *rp,
+                        const uint32_t *ci, const T *a, const T *x, T *y, hipStream_t s)
 {
   switch (lanes) {
-  case 2: return csr_vector_g<T, 2>(rows, nnz, rp, ci, a, x, y, s);
-  case 4: return csr_vector_g<T, 4>(rows, nnz, rp, ci, a, x, y, s);
-  case 8: return csr_vector_g<T, 8>(rows, nnz, rp, ci, a, x, y, s);
-  case 16: return csr_vector_g<T, 16>(rows, nnz, rp, ci, a, x, y, s);
-  case 32: return csr_vector_g<T, 32>(rows, nnz, rp, ci, a, x, y, s);
-  case 64: return csr_vector_g<T, 64>(rows, nnz, rp, ci, a, x, y, s);
+  case 2: return csr_vector_g<T, 2>(rows, l, rp, ci, a, x, y, s);
+  case 4: return csr_vector_g<T, 4>(rows, l, rp, ci, a, x, y, s);
+  case 8: return csr_vector_g<T, 8>(rows, l, rp, ci, a, x, y, s);
+  case 16: return csr_vector_g<T, 16>(rows, l, rp, ci, a, x, y, s);
+  case 32: return csr_vector_g<T, 32>(rows, l, rp, ci, a, x, y, s);
+  case 64: return csr_vector_g<T, 64>(rows, l, rp, ci, a, x, y, s);
   default: set_error("lanes must be a power of two in [2, 64]"); return MFP_ERR_ARG;
   }
 }
@@ -1532,13 +1689,13 @@ int launch_csr_scalar(int dtype, uint32_t rows, const uint32_t *rp, const uint32
                   (const double *)x, (double *)y);
 }
 
-int launch_csr_vector(int dtype, uint32_t lanes, uint32_t rows, uint64_t nnz, const uint32_t *rp,
+int launch_csr_vector(int dtype, uint32_t lanes, uint32_t rows, const csr_vector_layout &l, const uint32_t *rp,
                       const uint32_t *ci, const void *a, const void *x, void *y, hipStream_t s)
 {
   if (rows == 0) return MFP_OK;
   if (dtype == MFP_F32)
-    return csr_vector_t<float>(lanes, rows, nnz, rp, ci, (const float *)a, (const float *)x, (float *)y, s);
-  return csr_vector_t<double>(lanes, rows, nnz, rp, ci, (const double *)a, (const double *)x, (double *)y, s);
+    return csr_vector_t<float>(lanes, rows, l, rp, ci, (const float *)a, (const float *)x, (float *)y, s);
+  return csr_vector_t<double>(lanes, rows, l, rp, ci, (const double *)a, (const double *)x, (double *)y, s);
 }
 
 // Vectors a lane may need for a block of up to W elements at any alignment.
