@@ -25,6 +25,7 @@ struct mfp_plan_s {
   void *coo_val = nullptr;
   uint32_t *coo_col = nullptr, *coo_row = nullptr;
   bool coo_owner = false; // COO: no row too long for the form without a zero fill
+  uint32_t coo_longest = 0; // entries of the longest row, where coo_owner
   uint32_t slices = 0, ss = 0, L = 0, scoo_threads = 512;
   uint32_t *sp = nullptr;
   mfp::csr_vector_layout cv;

@@ -648,6 +648,7 @@ int mfp_plan_create(mfp_plan *out, mfp_matrix m, int format, const mfp_tuning *t
       st = matrix_stats(m, &rs, s);
       if (st != MFP_OK) return fail(st);
       p->coo_owner = coo_owner_fits(p->ncoo, rs.max_elements_in_rows);
+      p->coo_longest = rs.max_elements_in_rows;
     }
     if (format == MFP_SCOO) {
       p->ss = t.scoo_slice_size;
@@ -733,7 +734,7 @@ static int plan_spmv(mfp_plan p, const void *x, void *y, hipStream_t s, void *pa
     return launch_ell(dt, m->rows, p->ell_w, p->ell_col, p->ell_val, x, y, s);
   case MFP_COO:
     if (p->coo_owner)
-      return launch_coo_owner(dt, m->rows, p->ncoo, m->row_ptr, p->coo_row, p->coo_col, p->coo_val, x, y, s);
+      return launch_coo_owner(dt, m->rows, p->ncoo, p->coo_longest, m->row_ptr, p->coo_row, p->coo_col, p->coo_val, x, y, s);
     MFP_CHECK(fill_bytes_zero(y, (size_t)m->rows * dtype_size(dt), s));
     mark_kernel_end(); // the zero fill of y is its own interval under mfp_plan_kernel_times
     return launch_coo_add(dt, p->ncoo, p->coo_row, p->coo_col, p->coo_val, x, y, s);

@@ -910,20 +910,24 @@ __global__ __launch_bounds__(256) void k_vec_add(uint32_t n, const T *__restrict
 // result.
 //   atomic form  each run is added to y, which starts at zero
 //   owner form   (no row above COO_AHEAD entries) the wave that holds a row's
-//                first entry stores the row: it also reads the COO_AHEAD
-//                entries past its span.  Nothing is zeroed first and nothing
-//                is atomic, so an SpMV is one launch.  FP32, before -> now:
-//                65,536 rows of 5 7.4 -> 4.0 us (two launches of about 3.7),
-//                5-point stencil 1400^2 34.2 -> 28.2, 300,007 rows of 4 to 64
-//                74.9 -> 69.5.  With longer rows, walked on past the look-
-//                ahead, it lost: rows of up to 500, 72.5 against 57.2 us.
+//                first entry stores the row: it also reads the entries past
+//                its span that the longest row can have there.  Nothing is
+//                zeroed first and nothing is atomic, so an SpMV is one launch.
+//                FP32, before -> now: 65,536 rows of 5 7.4 -> 3.6 us (two
+//                launches of about 3.7), 5-point stencil 1400^2 34.3 -> 27.3,
+//                27-point 100^3 75.1 -> 65.8, 300,007 rows of 4 to 64 75.0 ->
+//                69.6; FP64 6.9 -> 3.6, 45.8 -> 38.4, 100.9 -> 98.8, 83.9 ->
+//                80.7 (27-point 100^3 with 64 entries read ahead: 104.1).
+//                With longer rows, walked on past the look-ahead, it lost:
+//                rows of up to 500, 72.5 against 57.2 us.
 // The atomic form was 64 entries per scan, four scans per wave: power-law 1M
 // rows 99.2 -> 86.9 us.
 // ---------------------------------------------------------------------------
 constexpr uint32_t COO_SPAN = 256, COO_AHEAD = 64, COO_NONE = 0xFFFFFFFFu;
 
+// ahead (owner form): entries that the longest row can have past its span
 template <typename T, bool OWNER>
-__device__ __forceinline__ void coo_span(uint64_t w0, uint64_t n, const uint32_t *__restrict__ cr,
+__device__ __forceinline__ void coo_span(uint64_t w0, uint64_t n, uint32_t ahead, const uint32_t *__restrict__ cr,
                                          const uint32_t *__restrict__ cc, const T *__restrict__ cv,
                                          const T *__restrict__ x, T *__restrict__ y)
 {
@@ -959,7 +963,7 @@ __device__ __forceinline__ void coo_span(uint64_t w0, uint64_t n, const uint32_t
       }
   }
   if constexpr (OWNER) {
-    if (ia < n) {
+    if (lane < ahead && ia < n) {
       ra = cr[ia];
       ca = cc[ia];
       va = cv[ia];
@@ -1048,24 +1052,27 @@ __global__ __launch_bounds__(256) void k_coo(uint64_t n, const uint32_t *__restr
 {
   const uint64_t waves = (uint64_t)gridDim.x * 4u;
   uint64_t w = (uint64_t)blockIdx.x * 4u + (threadIdx.x >> 6);
-  for (; w * COO_SPAN < n; w += waves) coo_span<T, false>(w * COO_SPAN, n, cr, cc, cv, x, y);
+  for (; w * COO_SPAN < n; w += waves) coo_span<T, false>(w * COO_SPAN, n, 0, cr, cc, cv, x, y);
 }
 
 // Owner form: workgroups [0, eblocks) take the entries, the others 256 rows
-// each and store the zeros of empty ones.
+// each and store the zeros of empty ones.  eblocks and ahead share a word (n is
+// below 2^32: 22 and 6 bits), which keeps the arguments in 64 bytes (past them
+// the smallest calls took 0.13 us more).
 template <typename T>
-__global__ __launch_bounds__(256) void k_coo_owner(uint64_t n, uint32_t rows, uint32_t eblocks,
+__global__ __launch_bounds__(256) void k_coo_owner(uint64_t n, uint32_t rows, uint32_t eblocks_ahead,
                                                    const uint32_t *__restrict__ rp, const uint32_t *__restrict__ cr,
                                                    const uint32_t *__restrict__ cc, const T *__restrict__ cv,
                                                    const T *__restrict__ x, T *__restrict__ y)
 {
+  const uint32_t eblocks = eblocks_ahead / COO_AHEAD, ahead = eblocks_ahead % COO_AHEAD;
   if (blockIdx.x >= eblocks) {
     const uint64_t r = (uint64_t)(blockIdx.x - eblocks) * 256u + threadIdx.x;
     if (r < rows && rp[r] == rp[r + 1]) y[r] = (T)0;
     return;
   }
   const uint64_t w = (uint64_t)xcd_block(blockIdx.x, eblocks) * 4u + (threadIdx.x >> 6);
-  if (w * COO_SPAN < n) coo_span<T, true>(w * COO_SPAN, n, cr, cc, cv, x, y);
+  if (w * COO_SPAN < n) coo_span<T, true>(w * COO_SPAN, n, ahead, cr, cc, cv, x, y);
 }
 
 // Fused hybrid (gpu_matrix_multiplier.cu:969-1002): workgroups [0, ell_blocks)
@@ -1088,7 +1095,7 @@ __global__ __launch_bounds__(256) void k_hyb_atomic(uint32_t rows, uint32_t w,
   }
   const uint64_t waves = (uint64_t)(gridDim.x - ell_blocks) * 4u;
   uint64_t wv = (uint64_t)(b - ell_blocks) * 4u + (threadIdx.x >> 6);
-  for (; wv * COO_SPAN < ncoo; wv += waves) coo_span<T, false>(wv * COO_SPAN, ncoo, cr, cc, cv, x, y);
+  for (; wv * COO_SPAN < ncoo; wv += waves) coo_span<T, false>(wv * COO_SPAN, ncoo, 0, cr, cc, cv, x, y);
 }
 
 // ---------------------------------------------------------------------------
@@ -1827,19 +1834,19 @@ int launch_coo_add(int dtype, uint64_t n, const uint32_t *cr, const uint32_t *cc
 
 bool coo_owner_fits(uint64_t n, uint32_t longest_row)
 {
-  // the entries' and the rows' workgroups are numbered in 32 bits
-  return longest_row <= COO_AHEAD && n <= (uint64_t)COO_SPAN * 4u * 0x7FFFFFu;
+  return longest_row <= COO_AHEAD && n < 1ull << 32; // k_coo_owner's word
 }
 
-int launch_coo_owner(int dtype, uint32_t rows, uint64_t n, const uint32_t *rp, const uint32_t *cr, const uint32_t *cc,
-                     const void *cv, const void *x, void *y, hipStream_t s)
+int launch_coo_owner(int dtype, uint32_t rows, uint64_t n, uint32_t longest_row, const uint32_t *rp, const uint32_t *cr,
+                     const uint32_t *cc, const void *cv, const void *x, void *y, hipStream_t s)
 {
   if (rows == 0) return MFP_OK;
   const uint32_t eb = ceil_div_u32(n, 4u * COO_SPAN), grid = eb + ceil_div_u32(rows, 256);
+  const uint32_t word = eb * COO_AHEAD + (longest_row ? longest_row - 1u : 0u);
   if (dtype == MFP_F32)
-    return launch_k(k_coo_owner<float>, dim3(grid), dim3(256), 0, s, n, rows, eb, rp, cr, cc, (const float *)cv,
+    return launch_k(k_coo_owner<float>, dim3(grid), dim3(256), 0, s, n, rows, word, rp, cr, cc, (const float *)cv,
                     (const float *)x, (float *)y);
-  return launch_k(k_coo_owner<double>, dim3(grid), dim3(256), 0, s, n, rows, eb, rp, cr, cc, (const double *)cv,
+  return launch_k(k_coo_owner<double>, dim3(grid), dim3(256), 0, s, n, rows, word, rp, cr, cc, (const double *)cv,
                   (const double *)x, (double *)y);
 }
 
