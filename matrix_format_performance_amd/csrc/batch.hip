@@ -264,12 +264,7 @@ static int spmm_bins_build(uint32_t rows, const uint32_t *rp_dev, spmm_bins_args
 // then a halving tree over the groups.  Every lane is
 // busy whatever the row lengths, and a group's gathers do not wait on one
 // another, where CSR-vector leaves lanes idle on short rows and each row is
-// one chain of dependent loads.  Of a batch, an XCD takes runs of 64
-// consecutive blocks: a batch of 64 in f32, one range per XCD -> runs: k = 8
-// 283 -> 243 us, k = 16 373 -> 328 us (f64 k = 2 248 -> 233, k = 16 568 ->
-// 554); runs of 8, 16, 32, 128 and 256 blocks are within 2% of 64.  One matrix
-// keeps a range per XCD (300k rows within a band of 1%, k = 16: 58.1 us, 60.7
-// in runs).
+// one chain of dependent loads.  (stream_run says which blocks an XCD takes.)
 constexpr uint32_t STREAM_T = 256; // STREAM_W (kernels.h): entries per row block
 static_assert(STREAM_W == 2 * STREAM_T, "the row scan gives each lane two entries");
 
@@ -321,13 +316,50 @@ __device__ __forceinline__ V stream_gather(const T *__restrict__ X, uint32_t c, 
 }
 
 // Workgroups per CU that the register budget is set for: 8 (the wave limit)
-// where the gathers in flight leave room.  f32 at KV = 16 holds 32 registers
-// of X: at 8 waves they spill (a batch of 64: 466 us), at 7 they do not
-// (373 us).  Wider f64 X rows hold more per gather.
+// for every f32 form and the narrow f64 ones; wider f64 X rows hold more
+// registers per gather.
 template <typename T, int KV>
 constexpr int stream_min_wg()
 {
-  return sizeof(T) == 4 && KV == 16 ? 7 : sizeof(T) == 4 || KV <= 4 ? 8 : (KV == 8 ? 5 : 4);
+  return sizeof(T) == 4 || KV <= 4 ? 8 : (KV == 8 ? 5 : 4);
+}
+
+// Whether a group's X rows are requested before the entries' rows are found.
+// A block spends its time on the latency of its phases one after another: a
+// batch of 64 in f32, gathers after the row scan -> before it: k = 4 256 -> 237
+// us, k = 8 310 -> 283 us; f64, k = 2, 4, 8, 16: 273 -> 247, 321 -> 299, 414 ->
+// 396, 572 -> 568 us.  f32 at KV = 16 holds 32 registers of X: with them over
+// the scan 8 waves spill (466 us) and 7 (373 us, 378 after) lose as much where
+// blocks are few: 7 matrices 12.3 -> 13.2 us.
+template <typename T, int KV>
+constexpr bool stream_early = !(sizeof(T) == 4 && KV == 16);
+
+// X rows of 64 bytes and more: gathers that miss the L2s are what the kernel
+// waits for, and the XCDs take their runs turned against one another, so that
+// they are not all in a matrix of random columns at once.
+template <typename T, int KV>
+constexpr bool stream_turned = KV * sizeof(T) >= 64;
+
+// Which blocks of a batch an XCD takes (log2 of a run).  One range per XCD
+// leaves the XCDs with the cheap matrices idle at the end, runs read the X of a
+// matrix into all L2s.  us, one range -> runs; start: gathers after the scan.
+//   narrow X rows, runs of 64: 64 matrices f32 k = 4, 8 236 -> 220, 282 -> 242
+//     (runs of 8 to 256 within 2%); 512 2,324 -> 2,078 at k = 4.  Up to 32 blocks
+//     per CU the runs are too few to be even: 7 matrices (2,841 blocks) k = 4
+//     12.7 -> 15.3, f64 k = 2 12.8 -> 15.4; 6 (7,211) 20.4 -> 23.3; 13 (8,354)
+//     43.9 -> 36.9.
+//   wide ones, turned runs of 16: f32 k = 16, 14, 22, 27, 52, 64 matrices 87 -> 78,
+//     245 -> 199, 274 -> 266, 213 -> 214, 379 -> 330 (not turned, runs of 64: 81,
+//     212, 277, 221, 328); f64 k = 8, 27 and 52 286 -> 282, 224 -> 230 (295, 238).
+//     With an X that is past the 256 MB Infinity Cache, one XCD after the other
+//     reads it from HBM: 512 matrices 3,413 -> 3,631 us, so they keep a range.
+// One matrix keeps a range too (300k rows within a band of 1%, k = 16: 58.1 us,
+// 60.7 in runs).
+static uint32_t stream_run(int dtype, uint32_t k, uint32_t cols, uint32_t nblocks)
+{
+  const uint64_t row = k * dtype_size(dtype);
+  if (row >= 64) return cols * row <= 256ull << 20 ? 4 : XCD_ONE_RUN;
+  return nblocks > 32u * (uint32_t)std::max(1, props().cu_count) ? BATCH_RUN : XCD_ONE_RUN;
 }
 
 template <typename T, int KV, bool OFF32>
@@ -345,7 +377,8 @@ __global__ __launch_bounds__(STREAM_T, (stream_min_wg<T, KV>())) void k_spmm_str
   __shared__ uint32_t s_rp[STREAM_W + 2];
   __shared__ V s_seg[STREAM_T];
   __shared__ uint32_t s_wmax[STREAM_T / 64];
-  const uint32_t bi = xcd_runs(blockIdx.x, gridDim.x, run);
+  const uint32_t bi = stream_turned<T, KV> ? xcd_runs_turned(blockIdx.x, gridDim.x, run)
+                                           : xcd_runs(blockIdx.x, gridDim.x, run);
   const uint2 m0 = meta[bi], m1 = meta[bi + 1];
   const uint32_t r0 = m0.x, r1 = m1.x, e0 = m0.y, e1 = m1.y;
   const uint32_t tid = threadIdx.x, g = tid / LPE, l = tid % LPE, lane = tid & 63, wv = tid >> 6;
@@ -441,20 +474,16 @@ __global__ __launch_bounds__(STREAM_T, (stream_min_wg<T, KV>())) void k_spmm_str
     s_row[i1] = 0;
   }
   __syncthreads();
-  // The group's X rows, in flight while the entries' rows are found (below):
-  // a block spends its time on the latency of its phases one after another.
-  // A batch of 64 in f32, gathers after the row scan -> before it: k = 4
-  // 256 -> 237 us, k = 8 310 -> 283 us, k = 16 378 -> 373 us; f64, k = 2, 4,
-  // 8, 16: 273 -> 247, 321 -> 299, 414 -> 396, 572 -> 568 us.
   const uint32_t base = g * EPG;
-  V xv[EPG];
-  {
+  V xv[EPG]; // the group's X rows
+  auto gather = [&] {
     uint32_t cc[EPG];
     lds_run<EPG>(&s_col[base], cc);
 #pragma unroll
     for (uint32_t j = 0; j < EPG; j++) // past the block: X row 0, never summed into a row
       xv[j] = stream_gather<V, LPE, OFF32>(X, base + j < n ? cc[j] : 0u, l);
-  }
+  };
+  if constexpr (stream_early<T, KV>) gather();
   for (uint32_t r = tid; r < nr; r += STREAM_T) {
     const uint32_t b = s_rp[r], z = s_rp[r + 1];
     if (b == z) {
@@ -482,6 +511,7 @@ __global__ __launch_bounds__(STREAM_T, (stream_min_wg<T, KV>())) void k_spmm_str
     *reinterpret_cast<uint2 *>(&s_row[2 * tid]) = make_uint2(max(ex, p.x), max(ex, hi));
   }
   __syncthreads();
+  if constexpr (!stream_early<T, KV>) gather();
   uint32_t rr[EPG];
   T v[EPG];
   lds_run<EPG>(&s_row[base], rr);
@@ -994,8 +1024,8 @@ static int batch_launch(mfp_batch b, uint32_t k, const void *X, void *Y, hipStre
     return launch_spmm_binned(m->dtype, k, b->bins, b->bin_list, m->rows, m->row_ptr, m->columns, m->values, X,
                               Y, s);
   if (b->lanes == MFP_BATCH_STREAM)
-    return launch_spmm_stream(m->dtype, k, m->cols, b->nstream, BATCH_RUN, b->stream_meta, m->row_ptr, m->columns, m->values, X, Y,
-                              s);
+    return launch_spmm_stream(m->dtype, k, m->cols, b->nstream, stream_run(m->dtype, k, m->cols, b->nstream),
+                              b->stream_meta, m->row_ptr, m->columns, m->values, X, Y, s);
   if (b->lanes == 1) {
     const uint32_t i = log2_k(k);
     if (i > 4 || !b->cs[i]) {

@@ -12,6 +12,8 @@
 // lane of the wave must call it (no divergence around the call).
 #pragma once
 
+#include "xcd_map.h"
+
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -84,27 +86,6 @@ __device__ __forceinline__ T group_reduce_rt(T v, uint32_t t)
   case 2: return group_reduce<2>(v);
   default: return v;
   }
-}
-
-// Workgroup ids are dispatched round-robin over the XCDs (each with its own
-// L2).  Remap so that XCD k works on one contiguous range of logical blocks:
-// neighbouring rows (and the x entries they share) stay in one L2.
-__device__ __forceinline__ uint32_t xcd_block(uint32_t b, uint32_t nb)
-{
-  constexpr uint32_t X = 8;
-  if (nb < X * 4) return b;
-  const uint32_t xcd = b % X, idx = b / X, q = nb / X, rem = nb % X;
-  return xcd < rem ? xcd * (q + 1) + idx : rem * (q + 1) + (xcd - rem) * q + idx;
-}
-
-// The same in runs of 1 << run logical blocks: XCD k takes runs k, k + 8, ...
-// Where the cost of a block differs along the range (a batch of matrices of
-// several kinds), one contiguous range per XCD leaves the XCDs with the cheap
-// ones idle at the end; a run still is long enough for its rows to share x.
-__device__ __forceinline__ uint32_t xcd_runs(uint32_t b, uint32_t nb, uint32_t run)
-{
-  const uint32_t w = 8u << run, at = b & ~(w - 1u);
-  return at + xcd_block(b - at, min(w, nb - at));
 }
 
 // A row of X (KV values, aligned to KV * sizeof(T)) with 16-byte loads where
