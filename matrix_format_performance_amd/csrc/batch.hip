@@ -653,11 +653,11 @@ int stream_meta_device(uint32_t rows, const uint32_t *rp, uint32_t **meta, uint3
 // register, in double as the slices do (exact for FP32 values).  The 16 rows
 // of a wave gather neighbouring X rows, so its gathers are two or three lines
 // each, mostly in L1.  64-matrix batch, k = 4, FP32: 20M entries of grids take
-// 64 us here and 99 there, the step 230 -> 190 us; k = 2 179 -> 156, k = 8
-// 417 -> 328, k = 16 875 -> 662 (with an XCD on one range; in runs of 64
-// workgroups 186, 148, 318 and 643).  Measured without gain: 2 or 4 columns
-// per lane with wider gathers (71 to 79 us), workgroups of 2, 4 or 8 row
-// groups with the next group's loads in flight (69 to 82).
+// 64 us here and 99 there, the step 236 -> 176 us; k = 8 414 -> 317, k = 16
+// 872 -> 642 (workgroups in runs of 64 per XCD; batch_split_aligned says where
+// it is used).  Measured without gain: 2 or 4 columns per lane with wider
+// gathers (71 to 79 us), workgroups of 2, 4 or 8 row groups with the next
+// group's loads in flight (69 to 82).
 constexpr uint32_t AL_T = 256, AL_CAP = 2048; // entries per chunk (FP64: half)
 constexpr uint32_t AL_U = 8;                  // gathers of a lane in flight
 constexpr uint32_t AL_MAX_ROW = 128;          // a lane walks its row alone
@@ -876,11 +876,24 @@ static int batch_order_items(scoo_cs_layout &l, uint32_t k, hipStream_t s)
 
 // Takes the slices with aligned rows out of the column-sorted plan's items
 // (those whose single item writes Y directly) and lists them for
-// k_spmm_aligned.
-static int batch_split_aligned(mfp_batch b, uint32_t i, hipStream_t s)
+// k_spmm_aligned, a launch of its own after the column-sorted one.  us, all
+// slices column-sorted -> split (FP32 unless said):
+//   narrow X rows gather too little per line: k = 2, 27, 52, 512 matrices 68 ->
+//     85, 73 -> 99, 932 -> 987, FP64 103 -> 132, 162 -> 197 (64), 1,357 -> 1,481;
+//     FP64 k = 4 19, 27, 512 matrices 80 -> 108, 159 -> 204, 1,987 -> 2,111.  So
+//     from k = 4 in FP32 and k = 8 in FP64;
+//   k = 4 with few items: they start together, and the second launch is added to
+//     the longest that stays (19, 23, 27 matrices 73 -> 87, 64 -> 82, 122 -> 153);
+//     1,076 items of 64 matrices 236 -> 176, 512 matrices 1,477 -> 1,423.  So above
+//     BATCH_FEW_ITEMS per CU;
+//   few entries: a tenth at least (7% of 5 matrices' entries, k = 8, 16 74 -> 81,
+//     127 -> 136).
+static int batch_split_aligned(mfp_batch b, uint32_t k, hipStream_t s)
 {
+  const uint32_t i = log2_k(k);
   scoo_cs_layout &l = b->cs[i]->cs;
-  if (l.S_reg == 0 || l.NI == 0 || l.R < AL_T) return MFP_OK;
+  if (l.S_reg == 0 || l.NI == 0 || l.R < AL_T || k < (b->big->dtype == MFP_F32 ? 4u : 8u)) return MFP_OK;
+  if (k == 4 && l.NI <= BATCH_FEW_ITEMS * (uint32_t)std::max(1, props().cu_count)) return MFP_OK;
   uint32_t *flag = nullptr, *list = nullptr;
   MFP_CHECK(dmalloc((void **)&flag, (uint64_t)l.S_reg * 4));
   k_aligned_slices<<<ceil_div_u32(l.S_reg, 4), 256, 0, s>>>(l.S_reg, l.R, b->big->rows, b->big->row_ptr,
@@ -897,15 +910,17 @@ static int batch_split_aligned(mfp_batch b, uint32_t i, hipStream_t s)
                : MFP_ERR_HIP;
   dfree(flag);
   if (st != MFP_OK) return st;
+  uint64_t taken = 0; // entries
   for (uint32_t q = 0; q < l.NI; q++) {
     if (items[q].w == CS_DIRECT && items[q].x < l.S_reg && hf[items[q].x]) {
       al.push_back(items[q].x);
+      taken += items[q].z - items[q].y;
     } else {
       keep.push_back(items[q]);
       keep_base.push_back(base[q]);
     }
   }
-  if (al.empty()) return MFP_OK;
+  if (al.empty() || taken < b->big->nnz / 10) return MFP_OK;
   std::sort(al.begin(), al.end());
   MFP_CHECK(dmalloc((void **)&list, al.size() * 4));
   if (hipMemcpyAsync(list, al.data(), al.size() * 4, hipMemcpyHostToDevice, s) != hipSuccess ||
@@ -938,8 +953,7 @@ static int launch_spmm_aligned(const mfp_batch_s *b, uint32_t i, const void *X, 
   if (b->naligned[i] == 0) return MFP_OK;
   const bool f32 = b->big->dtype == MFP_F32;
   switch (i) {
-  case 1: return f32 ? spmm_aligned_t<float, 2>(b, i, X, Y, s) : spmm_aligned_t<double, 2>(b, i, X, Y, s);
-  case 2: return f32 ? spmm_aligned_t<float, 4>(b, i, X, Y, s) : spmm_aligned_t<double, 4>(b, i, X, Y, s);
+  case 2: return spmm_aligned_t<float, 4>(b, i, X, Y, s); // batch_split_aligned: FP32 only
   case 3: return f32 ? spmm_aligned_t<float, 8>(b, i, X, Y, s) : spmm_aligned_t<double, 8>(b, i, X, Y, s);
   default: return f32 ? spmm_aligned_t<float, 16>(b, i, X, Y, s) : spmm_aligned_t<double, 16>(b, i, X, Y, s);
   }
@@ -967,12 +981,17 @@ static int batch_cs_plan(mfp_batch b, uint32_t k, mfp_stream sv)
   // 6,787 us).
   t.scoo_slice_size = 16384;
   while (t.scoo_slice_size > 1024 && (uint64_t)t.scoo_slice_size * k * 8 > 81920) t.scoo_slice_size /= 2;
-  // a slice per CU at least, as far as 256 rows: a slice is one workgroup, and
-  // a batch of few rows left most CUs without one.  407k rows (16 matrices),
-  // k = 2, 4: 72 -> 46, 82 -> 74 us (99, 199 -> 397 slices); 197k (6), k = 2, 4,
-  // 8: 65 -> 20, 64 -> 27, 74 -> 46.  Beyond it a smaller slice reads X more
-  // often: 1.3M rows, k = 4, 647 slices 112 us, 1,294 130, 2,588 163.
-  while (t.scoo_slice_size > 256 && b->big->rows / t.scoo_slice_size < (uint32_t)std::max(1, props().cu_count))
+  // a slice for nearly every CU, as far as 256 rows: a slice is one workgroup,
+  // and a batch of few rows left most CUs without one.  us, 16384 rows and half
+  // the LDS -> smaller slices: 197k rows (6 matrices), k = 2, 4, 8: 75 -> 13, 73
+  // -> 23, 95 -> 57; 343k (5) k = 2, 4 56 -> 34, 72 -> 64.  A smaller slice reads X
+  // more often: 195 to 250 slices of 2048 rows are better than twice as many of
+  // 1024 (399k rows, k = 2, 4: 39 and 47, 73 and 90 us, 420k 37 and 50, 60 and 82,
+  // 501k 41 and 43, 75 and 81; FP64 alike), 192 of 1024 are worse than twice as
+  // many of 512 (k = 2, 4, 8: 21 and 13, 38 and 23, 95 and 57).
+  const uint32_t cus = (uint32_t)std::max(1, props().cu_count);
+  while (t.scoo_slice_size > 256 &&
+         b->big->rows / t.scoo_slice_size < (t.scoo_slice_size >= 2048 ? cus * 3 / 4 : cus))
     t.scoo_slice_size /= 2;
   // one piece per slice: a slice of the block-diagonal batch seldom spans
   // more than one column band, so most slices write Y directly and skip the
@@ -985,11 +1004,14 @@ static int batch_cs_plan(mfp_batch b, uint32_t k, mfp_stream sv)
   if (k <= 4) t.flags |= MFP_TUNE_SCOO_WHOLE_SLICES;
   t.scoo_threads = 1024;
   MFP_CHECK(mfp_plan_create(&b->cs[i], b->big, MFP_SCOO, &t, sv));
-  int st = batch_split_aligned(b, i, as_stream(sv));
+  int st = batch_split_aligned(b, k, as_stream(sv));
   if (st == MFP_OK) st = batch_order_items(b->cs[i]->cs, k, as_stream(sv));
   if (st != MFP_OK) {
     mfp_plan_destroy(b->cs[i]);
     b->cs[i] = nullptr;
+    dfree(b->aligned[i]);
+    b->aligned[i] = nullptr;
+    b->naligned[i] = 0;
   }
   return st;
 }

@@ -57,3 +57,52 @@ def test_stream_narrow_rows_of_x(gpu, more, k, dtype):
     B.destroy()
     for m in mats:
         m.destroy()
+
+
+# Column-sorted batches.  Slices with aligned rows (bands) are summed row by row
+# from k = 4 in FP32 (there above four items per CU: 1,024 slices of 2,048 rows)
+# and k = 8 in FP64 (slices of 1,024 rows from 262,144 rows on; 64 to 16 rows per
+# workgroup), where they hold a tenth of the entries.  Members end inside
+# slices and inside workgroups.
+def _band(rows, width, seed):
+    lens = np.full(rows, width)
+    lens[5::1013] = 0
+    rp = np.concatenate([[0], np.cumsum(lens)]).astype(np.uint32)
+    r = np.repeat(np.arange(rows), lens)
+    ci = np.minimum(r, rows - width) + np.arange(rp[-1]) - rp[r]
+    return rp, ci.astype(np.uint32), np.random.default_rng(seed).integers(-3, 4, ci.size), rows
+
+
+@pytest.mark.parametrize("k,dtype,rows", [(4, "float32", 1100003), (8, "float32", 150001), (16, "float32", 150001),
+                                          (8, "float64", 150001), (16, "float64", 150001), (16, "float32", 9003),
+                                          (4, "float64", 150001), (2, "float32", 300007)])
+def test_column_sorted_with_aligned_members(gpu, k, dtype, rows):
+    announce(f"batch aligned members k={k} dtype={dtype} rows={rows}")
+    rng = np.random.default_rng(rows)
+    members = [_band(rows, 3, 1), _csr(rng.integers(0, 5, rows // 2 + 77), 5000, 2), _band(rows // 3 + 11, 9, 3),
+               _csr(rng.integers(0, 4, rows // 4 + 5), 70001, 4), _band(1037, 128, 5), _band(2053, 129, 6)]
+    mats = [gpu.DeviceMatrix.from_csr(rp, ci, va.astype(dtype), cols) for rp, ci, va, cols in members]
+    B = gpu.Batch(mats, lanes=1, flags=4, scoo_slice_size=8192, scoo_pieces=1)
+    _check(gpu, B, members, k, dtype)
+    B.destroy()
+    for m in mats:
+        m.destroy()
+
+
+# Slices shrink below 3/4 of a slice per CU (a slice per CU under 2,048 rows),
+# to 256 rows at the least.
+@pytest.mark.parametrize("dtype", ["float32", "float64"])
+@pytest.mark.parametrize("k", [2, 4, 8])
+@pytest.mark.parametrize("per_cu", [0.01, 0.74, 0.76, 1.01])
+def test_column_sorted_slices_of_few_rows(gpu, per_cu, k, dtype):
+    full = {2: 4096, 4: 2048, 8: 1024}[k]  # rows of a slice with half of the LDS
+    rows = int(per_cu * gpu.device_info()["cu_count"] * full) + 13
+    announce(f"batch few rows k={k} dtype={dtype} rows={rows}")
+    rng = np.random.default_rng(rows)
+    members = [_csr(rng.integers(0, 4, n), 3001, n) for n in (rows // 3, rows - rows // 3)]
+    mats = [gpu.DeviceMatrix.from_csr(rp, ci, va.astype(dtype), cols) for rp, ci, va, cols in members]
+    B = gpu.Batch(mats, lanes=1, flags=4, scoo_slice_size=8192, scoo_pieces=1)
+    _check(gpu, B, members, k, dtype)
+    B.destroy()
+    for m in mats:
+        m.destroy()
