@@ -894,6 +894,7 @@ static int batch_split_aligned(mfp_batch b, uint32_t k, hipStream_t s)
   scoo_cs_layout &l = b->cs[i]->cs;
   if (l.S_reg == 0 || l.NI == 0 || l.R < AL_T || k < (b->big->dtype == MFP_F32 ? 4u : 8u)) return MFP_OK;
   if (k == 4 && l.NI <= BATCH_FEW_ITEMS * (uint32_t)std::max(1, props().cu_count)) return MFP_OK;
+  if (!grid_fits((uint64_t)l.S_reg * (l.R / (AL_T / k)), AL_T)) return MFP_OK;
   uint32_t *flag = nullptr, *list = nullptr;
   MFP_CHECK(dmalloc((void **)&flag, (uint64_t)l.S_reg * 4));
   k_aligned_slices<<<ceil_div_u32(l.S_reg, 4), 256, 0, s>>>(l.S_reg, l.R, b->big->rows, b->big->row_ptr,

@@ -589,8 +589,10 @@ int row_stats_device(uint32_t rows, const uint32_t *rp, mfp_row_stats *out, hipS
 // ---------------------------------------------------------------------------
 // A workgroup turns 64 rows x 16 slots around in LDS: 16 lanes read a row's
 // 16 entries, then 64 lanes write one slot of 64 rows (5.1M entries, width
-// 64: 69 us with a lane per row reading along its own row).
-constexpr uint32_t ELLB_R = 64, ELLB_S = 16;
+// 64: 69 us with a lane per row reading along its own row).  Four lanes per row:
+// from 2^30 rows on a launch cannot hold them all, and the workgroups go on to
+// further tiles.
+constexpr uint32_t ELLB_R = 64, ELLB_S = 16, ELLB_GRID = 1u << 22;
 
 template <typename T>
 __global__ __launch_bounds__(256) void k_ell_build(uint32_t rows, const uint32_t *__restrict__ rp,
@@ -600,29 +602,31 @@ __global__ __launch_bounds__(256) void k_ell_build(uint32_t rows, const uint32_t
   __shared__ T sv[ELLB_R][ELLB_S + 1];
   __shared__ uint32_t sc[ELLB_R][ELLB_S + 1];
   __shared__ uint32_t srp[ELLB_R + 1];
-  const uint32_t r0 = blockIdx.x * ELLB_R, t = threadIdx.x;
-  if (t <= ELLB_R) srp[t] = rp[min((uint64_t)r0 + t, (uint64_t)rows)];
-  __syncthreads();
-  for (uint32_t k0 = blockIdx.y * ELLB_S; k0 < width; k0 += gridDim.y * ELLB_S) {
-#pragma unroll
-    for (uint32_t q = 0; q < ELLB_R * ELLB_S / 256; q++) {
-      const uint32_t lr = q * (256 / ELLB_S) + t / ELLB_S, k = k0 + t % ELLB_S;
-      const uint32_t s = srp[lr], len = srp[lr + 1] - s;
-      const bool in = k < len;
-      sv[lr][t % ELLB_S] = in ? a[s + k] : (T)0;
-      sc[lr][t % ELLB_S] = in ? ci[s + k] : 0u;
-    }
+  const uint32_t t = threadIdx.x;
+  for (uint64_t r0 = (uint64_t)blockIdx.x * ELLB_R; r0 < rows; r0 += (uint64_t)gridDim.x * ELLB_R) {
+    if (t <= ELLB_R) srp[t] = rp[min(r0 + t, (uint64_t)rows)];
     __syncthreads();
+    for (uint32_t k0 = blockIdx.y * ELLB_S; k0 < width; k0 += gridDim.y * ELLB_S) {
 #pragma unroll
-    for (uint32_t q = 0; q < ELLB_R * ELLB_S / 256; q++) {
-      const uint32_t lk = q * (256 / ELLB_R) + t / ELLB_R, lr = t % ELLB_R;
-      if (k0 + lk < width && r0 + lr < rows) {
-        const uint64_t o = (uint64_t)r0 + lr + (uint64_t)(k0 + lk) * rows;
-        ev[o] = sv[lr][lk];
-        ec[o] = sc[lr][lk];
+      for (uint32_t q = 0; q < ELLB_R * ELLB_S / 256; q++) {
+        const uint32_t lr = q * (256 / ELLB_S) + t / ELLB_S, k = k0 + t % ELLB_S;
+        const uint32_t s = srp[lr], len = srp[lr + 1] - s;
+        const bool in = k < len;
+        sv[lr][t % ELLB_S] = in ? a[s + k] : (T)0;
+        sc[lr][t % ELLB_S] = in ? ci[s + k] : 0u;
       }
+      __syncthreads();
+#pragma unroll
+      for (uint32_t q = 0; q < ELLB_R * ELLB_S / 256; q++) {
+        const uint32_t lk = q * (256 / ELLB_R) + t / ELLB_R, lr = t % ELLB_R;
+        if (k0 + lk < width && r0 + lr < rows) {
+          const uint64_t o = r0 + lr + (uint64_t)(k0 + lk) * rows;
+          ev[o] = sv[lr][lk];
+          ec[o] = sc[lr][lk];
+        }
+      }
+      __syncthreads(); // the tile and the row starts may be written again
     }
-    __syncthreads();
   }
 }
 
@@ -630,7 +634,7 @@ int ell_build_device(int dtype, uint32_t rows, const uint32_t *rp, const uint32_
                      const void *val, uint32_t width, void *ev, uint32_t *ec, hipStream_t s)
 {
   if (rows == 0 || width == 0) return MFP_OK;
-  const dim3 g(ceil_div_u32(rows, ELLB_R), std::min(ceil_div_u32(width, ELLB_S), 1024u));
+  const dim3 g(std::min(ceil_div_u32(rows, ELLB_R), ELLB_GRID), std::min(ceil_div_u32(width, ELLB_S), 1024u));
   if (dtype == MFP_F32)
     k_ell_build<float><<<g, 256, 0, s>>>(rows, rp, ci, (const float *)val, width, (float *)ev, ec);
   else

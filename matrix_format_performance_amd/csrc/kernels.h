@@ -60,7 +60,7 @@ int launch_coo_add(int dtype, uint64_t n, const uint32_t *cr, const uint32_t *cc
                    const void *x, void *y, hipStream_t s);
 // COO whose rows are at most coo_owner_fits' length: y is written once, without
 // a zero fill (rp: the matrix's row pointers, for the zeros of empty rows)
-bool coo_owner_fits(uint64_t n, uint32_t longest_row);
+bool coo_owner_fits(uint64_t n, uint32_t rows, uint32_t longest_row);
 int launch_coo_owner(int dtype, uint32_t rows, uint64_t n, uint32_t longest_row, const uint32_t *rp, const uint32_t *cr,
                      const uint32_t *cc, const void *cv, const void *x, void *y, hipStream_t s);
 int launch_vec_add(int dtype, uint32_t n, const void *t, void *y, hipStream_t s);

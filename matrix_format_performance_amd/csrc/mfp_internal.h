@@ -89,6 +89,9 @@ inline hipStream_t as_stream(mfp_stream s) { return reinterpret_cast<hipStream_t
 
 inline uint32_t ceil_div_u32(uint64_t a, uint64_t b) { return (uint32_t)((a + b - 1) / b); }
 
+// HIP takes fewer than 2^32 lanes along a dimension of a launch
+inline bool grid_fits(uint64_t blocks, uint32_t lanes) { return blocks * lanes < 1ull << 32; }
+
 // Device properties cached by mfp_init.
 struct device_props {
   int device = -1;

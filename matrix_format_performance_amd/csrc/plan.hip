@@ -647,7 +647,7 @@ int mfp_plan_create(mfp_plan *out, mfp_matrix m, int format, const mfp_tuning *t
       mfp_row_stats rs;
       st = matrix_stats(m, &rs, s);
       if (st != MFP_OK) return fail(st);
-      p->coo_owner = coo_owner_fits(p->ncoo, rs.max_elements_in_rows);
+      p->coo_owner = coo_owner_fits(p->ncoo, m->rows, rs.max_elements_in_rows);
       p->coo_longest = rs.max_elements_in_rows;
     }
     if (format == MFP_SCOO) {

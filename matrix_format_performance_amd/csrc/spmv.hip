@@ -1640,7 +1640,8 @@ int csr_vector_layout_build(int dtype, uint32_t lanes, uint32_t rows, uint64_t n
     set_error("CSR-vector: blocks of long rows");
     st = MFP_ERR_HIP;
   }
-  if (st != MFP_OK || out->count == 0) csr_vector_layout_free(out);
+  const uint64_t per = (out->rb * (uint64_t)lanes + 255) / 256;
+  if (st != MFP_OK || out->count == 0 || !grid_fits(out->count * per + nb + 8, 256)) csr_vector_layout_free(out);
   return st;
 }
 
@@ -1832,9 +1833,10 @@ int launch_coo_add(int dtype, uint64_t n, const uint32_t *cr, const uint32_t *cc
                   (double *)y);
 }
 
-bool coo_owner_fits(uint64_t n, uint32_t longest_row)
+bool coo_owner_fits(uint64_t n, uint32_t rows, uint32_t longest_row)
 {
-  return longest_row <= COO_AHEAD && n < 1ull << 32; // k_coo_owner's word
+  return longest_row <= COO_AHEAD && n < 1ull << 32 && // k_coo_owner's word
+         grid_fits((uint64_t)ceil_div_u32(n, 4u * COO_SPAN) + ceil_div_u32(rows, 256), 256);
 }
 
 int launch_coo_owner(int dtype, uint32_t rows, uint64_t n, uint32_t longest_row, const uint32_t *rp, const uint32_t *cr,

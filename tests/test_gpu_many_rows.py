@@ -1,0 +1,47 @@
+"""More rows than a launch has lanes for, at four lanes a row: 2^30 + 77 rows of
+at most one entry (17 GB of device memory)."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from gpu_cases import announce
+
+pytestmark = pytest.mark.gpu
+
+ROWS = (1 << 30) + 77
+
+
+def test_ell_of_2_30_rows(gpu):
+    from matrix_format_performance_amd import _lib as L
+    if gpu.device_info()["free_mem"] < 40 << 30:
+        pytest.skip("needs 40 GB of device memory")
+    announce(f"ell rows={ROWS}")
+    # rows around the tiles' and the grid's edges, and some at random
+    edge = np.array([0, 1, 63, 64, (1 << 22) * 64 - 1, (1 << 22) * 64, 1 << 29, (1 << 30) - 1, 1 << 30, ROWS - 1])
+    r = np.unique(np.concatenate([edge, np.random.default_rng(1).integers(0, ROWS, 5000)])).astype(np.uint32)
+    c = (r % 997).astype(np.uint32)
+    v = (r % 13 - 6.0) * 0.5
+    A = gpu.DeviceMatrix.from_triplets(ROWS, 997, r, c, v, np.dtype(np.float32))
+    plan = gpu.Plan(A, "ell")
+    x = np.arange(1, 998).astype(np.float32)
+    xd, yd = gpu.DeviceArray.from_host(x), gpu.DeviceArray(ROWS, np.dtype(np.float32))
+    yd.fill(np.nan)
+    plan.spmv(xd, yd)
+    gpu.synchronize()
+
+    def part(at, n):
+        out = np.empty(n, np.float32)
+        L.call("mfp_memcpy_d2h", out.ctypes.data_as(C.c_void_p), yd.ptr + 4 * int(at), out.nbytes)
+        return out
+
+    for lo in [0, (1 << 22) * 64 - 500, (1 << 29) - 500, (1 << 30) - 950, ROWS - 1000]:
+        want = np.zeros(1000, np.float32)
+        here = (r >= lo) & (r < lo + 1000)
+        want[r[here] - lo] = (v[here] * x[c[here]]).astype(np.float32)
+        assert np.array_equal(part(lo, 1000), want), lo
+    for i in range(0, r.size, 50):
+        assert part(r[i], 1)[0] == np.float32(v[i] * x[c[i]]), r[i]
+    plan.destroy()
+    A.destroy()
+    yd.free()
