@@ -2,9 +2,8 @@
 // only; the device calls come from Dev, so that the bookkeeping can be checked
 // without a GPU:
 //   static bool alloc(void **p, size_t bytes)  on the current device
-//   static void release(void *p)               a block of any device
+//   static bool release(void *p)               of any device; waits for the current one
 //   static int current()                       the current device, -1 unknown
-//   static bool idle()                         waits for the current device
 #pragma once
 
 #include <cstddef>
@@ -22,9 +21,13 @@ namespace mfp {
 // (nine formats of a 5M-entry matrix: 1.8 ms of kernels in 8.7 to 12.9 ms).
 // Freed blocks of 64 KB to 1 GB are therefore kept and handed out again, in
 // size classes an eighth of a power of two apart.
-//  * A block is kept only once its device is idle (put waits for it, as
-//    hipFree does), so whoever gets it next, on any stream or thread, finds
-//    nothing still running on it.
+//  * Every block that is taken from the cache or put there goes with a token, a
+//    small allocation of its own (1.4 us to allocate and free).  Allocating it
+//    is refused where hipMalloc is, in a stream capture; freeing it waits for the
+//    device as hipFree does, so that whoever gets the block next, on any stream
+//    or thread, finds nothing still running on it.  hipDeviceSynchronize (0.2 us
+//    on an idle device) would wait as well, but it ends every stream capture in
+//    the process, also those that another thread's hipFree leaves alone.
 //  * A block is filed under the device it was allocated on, whichever device
 //    the freeing thread uses, and handed out on that device only.
 //  * At most CACHE_BYTES are kept; an allocation that fails gives all of them
@@ -36,6 +39,11 @@ template <class Dev>
 class block_cache {
   using block = std::pair<int, size_t>; // device, size (0: not cacheable)
   using blocks = std::multimap<block, void *>;
+  struct held {
+    block b;
+    void *token;
+  };
+  static constexpr size_t TOKEN = 256;
 
 public:
   // a block of at least bytes on the current device, null when there is none
@@ -45,15 +53,15 @@ public:
     const bool cacheable = bytes >= CACHE_MIN && bytes <= CACHE_MAX && device >= 0;
     const size_t size = cacheable ? size_class(bytes) : bytes;
     if (cacheable) {
-      std::lock_guard<std::mutex> lock(mutex_);
-      const auto it = kept_.lower_bound({device, size});
-      if (it != kept_.end() && it->first.first == device && it->first.second <= size + size / 4) {
-        void *p = it->second;
-        const block b = it->first;
-        kept_bytes_ -= b.second;
-        kept_.erase(it);
-        taken(p, b);
-        return p;
+      block b{-1, 0};
+      if (void *p = take_kept(device, size, b)) {
+        void *token = nullptr;
+        if (Dev::alloc(&token, TOKEN)) {
+          std::lock_guard<std::mutex> lock(mutex_);
+          taken(p, b, token);
+          return p;
+        }
+        (void)Dev::release(p);
       }
     }
     void *p = nullptr;
@@ -63,7 +71,7 @@ public:
       if (size == bytes || !Dev::alloc(&p, bytes)) return nullptr; // without the rounding, then
     }
     std::lock_guard<std::mutex> lock(mutex_);
-    taken(p, b);
+    taken(p, b, nullptr);
     return p;
   }
 
@@ -71,18 +79,20 @@ public:
   void put(void *p)
   {
     if (!p) return;
-    block b{-1, 0};
+    held h{{-1, 0}, nullptr};
     {
       std::lock_guard<std::mutex> lock(mutex_);
       const auto it = sizes_.find(p);
       if (it != sizes_.end()) {
-        b = it->second;
+        h = it->second;
         sizes_.erase(it);
       }
     }
-    // idle() waits for the current device, so only its blocks are kept
-    const bool keep = b.second && Dev::current() == b.first && Dev::idle();
-    if (!(keep && add(b, p))) Dev::release(p);
+    // freeing waits for the current device, so only its blocks are kept
+    const bool own = h.b.second && Dev::current() == h.b.first;
+    if (own && !h.token && !Dev::alloc(&h.token, TOKEN)) h.token = nullptr;
+    const bool idle = h.token && Dev::release(h.token) && own;
+    if (!(idle && add(h.b, p))) (void)Dev::release(p);
     blocks out;
     {
       std::lock_guard<std::mutex> lock(mutex_);
@@ -128,13 +138,27 @@ private:
     return (bytes + step - 1) / step * step;
   }
 
+  // the smallest kept block that will do, null when there is none
+  void *take_kept(int device, size_t size, block &b)
+  {
+    std::lock_guard<std::mutex> lock(mutex_);
+    const auto it = kept_.lower_bound({device, size});
+    if (it == kept_.end() || it->first.first != device || it->first.second > size + size / 4) return nullptr;
+    void *p = it->second;
+    b = it->first;
+    kept_bytes_ -= b.second;
+    kept_.erase(it);
+    return p;
+  }
+
   // mutex_ held; without memory for the entry the block is not cacheable
-  void taken(void *p, const block &b)
+  void taken(void *p, const block &b, void *token)
   {
     in_use_++;
     try {
-      if (b.second) sizes_[p] = b;
+      if (b.second) sizes_[p] = held{b, token};
     } catch (const std::bad_alloc &) {
+      if (token) (void)Dev::release(token);
     }
   }
 
@@ -161,12 +185,12 @@ private:
   // without the mutex: giving memory back takes its time
   static void release(const blocks &out)
   {
-    for (const auto &b : out) Dev::release(b.second);
+    for (const auto &b : out) (void)Dev::release(b.second);
   }
 
   std::mutex mutex_;
   blocks kept_;
-  std::unordered_map<void *, block> sizes_; // cacheable blocks in use
+  std::unordered_map<void *, held> sizes_; // cacheable blocks in use
   size_t kept_bytes_ = 0;
   size_t in_use_ = 0; // blocks of any size
 };

@@ -80,7 +80,12 @@ struct hip_memory {
     }
     return e == hipSuccess;
   }
-  static void release(void *p) { (void)hipFree(p); }
+  static bool release(void *p)
+  {
+    if (hipFree(p) == hipSuccess) return true;
+    (void)hipGetLastError();
+    return false;
+  }
   static int current()
   {
     int d = -1;
@@ -89,12 +94,6 @@ struct hip_memory {
       return -1;
     }
     return d;
-  }
-  static bool idle()
-  {
-    if (hipDeviceSynchronize() == hipSuccess) return true;
-    (void)hipGetLastError();
-    return false;
   }
 };
 

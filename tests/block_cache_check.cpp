@@ -30,35 +30,31 @@ struct devices {
   static inline std::mutex mutex;
   static inline std::map<void *, block> live;
   static inline size_t bytes = 0, limit = ~size_t(0), next = 4096;
-  static inline bool sync_fails = false;
+  static inline bool refuse = false, free_fails = false; // a stream capture; a device in error
   static inline thread_local int now = 0; // a new thread's device is 0
 
   static bool alloc(void **p, size_t n)
   {
     std::lock_guard<std::mutex> lock(mutex);
-    if (bytes + n > limit) return false;
+    if (refuse || bytes + n > limit) return false;
     *p = reinterpret_cast<void *>(next);
     next += n + 4096;
     bytes += n;
     live[*p] = {now, n, false};
     return true;
   }
-  static void release(void *p)
+  static bool release(void *p)
   {
     std::lock_guard<std::mutex> lock(mutex);
     REQUIRE(live.count(p));
     bytes -= live[p].size;
     live.erase(p);
-  }
-  static int current() { return now; }
-  static bool idle()
-  {
-    std::lock_guard<std::mutex> lock(mutex);
-    if (sync_fails) return false;
+    if (free_fails) return false;
     for (auto &b : live)
       if (b.second.device == now) b.second.busy = false;
     return true;
   }
+  static int current() { return now; }
 };
 
 using cache_t = mfp::block_cache<devices>;
@@ -97,6 +93,31 @@ void reuse()
   c.put(q);
   c.put(hold);
   REQUIRE(devices::live.empty()); // the last block gives everything back
+}
+
+// Where allocations are refused, kept blocks are too, and a block that is freed
+// meanwhile is not kept
+void refused()
+{
+  cache_t c;
+  void *hold = take(c, 1000), *p = take(c, 20 * MB), *q = take(c, 30 * MB);
+  c.put(p);
+  devices::refuse = true;
+  REQUIRE(!c.get(20 * MB));
+  c.put(q);
+  REQUIRE(!devices::live.count(q));
+  devices::refuse = false;
+  REQUIRE(c.kept_bytes(0) == 0);
+  void *r = take(c, 20 * MB);
+  c.put(r);
+  r = take(c, 20 * MB); // with a token from here on
+  devices::refuse = true;
+  c.put(r); // its token is freed all the same
+  devices::refuse = false;
+  REQUIRE(take(c, 20 * MB) == r);
+  c.put(r);
+  c.put(hold);
+  REQUIRE(devices::live.empty());
 }
 
 // The object of one device is destroyed while the library works on another,
@@ -153,9 +174,9 @@ void limits()
   devices::limit = ~size_t(0);
   // a device that cannot be waited for keeps nothing
   void *p = take(c, 10 * MB);
-  devices::sync_fails = true;
+  devices::free_fails = true;
   c.put(p);
-  devices::sync_fails = false;
+  devices::free_fails = false;
   REQUIRE(c.kept_bytes(0) == 0 && !devices::live.count(p));
   c.put(hold);
   c.put(nullptr);
@@ -193,6 +214,7 @@ void threads()
 int main()
 {
   reuse();
+  refused();
   two_devices();
   limits();
   threads();

@@ -1,0 +1,78 @@
+"""Objects that come and go while another thread's stream is captured: what
+hipMalloc and hipFree leave alone, the library's block cache leaves alone too."""
+import ctypes as C
+import threading
+
+import numpy as np
+import pytest
+
+from gpu_cases import announce
+
+pytestmark = pytest.mark.gpu
+
+
+THREAD_LOCAL, RELAXED = 1, 2  # hipStreamCaptureMode
+
+
+@pytest.mark.parametrize("what", ["destroy", "create"])
+@pytest.mark.parametrize("mode,thread", [(THREAD_LOCAL, True), (RELAXED, True), (RELAXED, False)])
+def test_capture_survives_other_objects(gpu, mode, thread, what):
+    from matrix_format_performance_amd import _lib as L
+    lib = L.load()  # finds the HIP runtime's functions too
+
+    def hip(name, *args):
+        status = getattr(lib, name)(*args)
+        assert status == 0, (name, status)
+
+    announce(f"capture mode={mode} thread={thread} what={what}")
+    rng = np.random.default_rng(0)
+
+    def matrix():
+        rp = np.concatenate([[0], np.cumsum(rng.integers(1, 30, 40000))]).astype(np.uint32)
+        ci = rng.integers(0, 40000, rp[-1]).astype(np.uint32)
+        return gpu.DeviceMatrix.from_csr(rp, ci, rng.random(ci.size).astype(np.float32), 40000)
+
+    A, B = matrix(), matrix()
+    P, Q = gpu.Plan(A, "ell"), gpu.Plan(B, "ell")
+    gpu.Plan(B, "coo").destroy()  # blocks for the plan that is created
+    x = gpu.DeviceArray.from_host(rng.random(40000).astype(np.float32))
+    y = gpu.DeviceArray(40000, np.dtype(np.float32))
+    P.spmv(x, y)
+    gpu.synchronize()
+    want, made = y.to_host(), []
+
+    def act():
+        if what == "destroy":
+            Q.destroy()
+        else:
+            made.append(gpu.Plan(B, "coo"))
+
+    s, g, e = C.c_void_p(), C.c_void_p(), C.c_void_p()
+    hip("hipStreamCreateWithFlags", C.byref(s), C.c_uint(1))
+    hip("hipStreamBeginCapture", s, C.c_int(mode))
+    P.spmv(x, y, stream=s)
+    if thread:
+        t = threading.Thread(target=act)
+        t.start()
+        t.join()
+    else:
+        act()
+    P.spmv(x, y, stream=s)
+    hip("hipStreamEndCapture", s, C.byref(g))
+    hip("hipGraphInstantiate", C.byref(e), g, None, None, C.c_size_t(0))
+    for _ in range(3):
+        y.fill(np.nan)
+        gpu.synchronize()
+        hip("hipGraphLaunch", e, s)
+        hip("hipStreamSynchronize", s)
+        assert np.array_equal(y.to_host(), want)
+    hip("hipGraphExecDestroy", e)
+    hip("hipGraphDestroy", g)
+    hip("hipStreamDestroy", s)
+    if what == "create":
+        assert made
+        made[0].destroy()
+        Q.destroy()
+    P.destroy()
+    A.destroy()
+    B.destroy()
