@@ -54,7 +54,9 @@ typedef struct {
   int cu_count;           /* multiProcessorCount (sm_count at main.cpp:418) */
   int xcd_count;
   uint64_t lds_per_block; /* sharedMemPerBlock (main.cpp:419) */
-  uint64_t free_mem, total_mem;
+  uint64_t free_mem;      /* for this library: free on the device, and what
+                           * it keeps of freed objects (mfp_trim) */
+  uint64_t total_mem;
   char name[256];
   char arch[64];
 } mfp_device_info;
@@ -64,6 +66,11 @@ int mfp_device_query(mfp_device_info *out);
 const char *mfp_status_string(int status);
 const char *mfp_last_error(void);
 int mfp_synchronize(void);
+/* The arrays of destroyed matrices, plans and batches, and the scratch of
+ * building them, are kept for the next ones, up to 4 GB, while any object
+ * lives; the library's own allocations take them back when memory is short.
+ * mfp_trim gives them back to the device, for the program's other allocators. */
+int mfp_trim(void);
 int mfp_malloc(void **dev_ptr, size_t bytes);
 int mfp_free(void *dev_ptr);
 int mfp_memcpy_h2d(void *dst, const void *src, size_t bytes);

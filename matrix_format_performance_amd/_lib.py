@@ -124,6 +124,7 @@ SIGNATURES = {
     "mfp_status_string": (C.c_char_p, [i32]),
     "mfp_last_error": (C.c_char_p, []),
     "mfp_synchronize": (i32, []),
+    "mfp_trim": (i32, []),
     "mfp_malloc": (i32, [P(vp), sz]),
     "mfp_free": (i32, [vp]),
     "mfp_memcpy_h2d": (i32, [vp, vp, sz]),

@@ -7,6 +7,7 @@
 #pragma once
 
 #include <cstddef>
+#include <cstdint>
 #include <map>
 #include <mutex>
 #include <new>
@@ -30,15 +31,19 @@ namespace mfp {
 //    the process, also those that another thread's hipFree leaves alone.
 //  * A block is filed under the device it was allocated on, whichever device
 //    the freeing thread uses, and handed out on that device only.
-//  * At most CACHE_BYTES are kept; an allocation that fails gives all of them
-//    back and tries again, and they are given back when the library's last
-//    block is freed.
+//  * At most CACHE_BYTES are kept, the oldest make room; an allocation that
+//    fails gives all of them back and tries again, and they are given back by
+//    trim and when the library's last block is freed.
 constexpr size_t CACHE_MIN = 64u << 10, CACHE_MAX = 1u << 30, CACHE_BYTES = 4ull << 30;
 
 template <class Dev>
 class block_cache {
   using block = std::pair<int, size_t>; // device, size (0: not cacheable)
-  using blocks = std::multimap<block, void *>;
+  struct kept {
+    void *p;
+    uint64_t since; // counts the blocks that were put
+  };
+  using blocks = std::multimap<block, kept>;
   struct held {
     block b;
     void *token;
@@ -92,11 +97,14 @@ public:
     const bool own = h.b.second && Dev::current() == h.b.first;
     if (own && !h.token && !Dev::alloc(&h.token, TOKEN)) h.token = nullptr;
     const bool idle = h.token && Dev::release(h.token) && own;
-    if (!(idle && add(h.b, p))) (void)Dev::release(p);
     blocks out;
+    if (!(idle && add(h.b, p, out))) (void)Dev::release(p);
     {
       std::lock_guard<std::mutex> lock(mutex_);
-      if (--in_use_ == 0) take_all(out);
+      if (--in_use_ == 0) {
+        out.merge(kept_);
+        kept_bytes_ = 0;
+      }
     }
     release(out);
   }
@@ -115,7 +123,8 @@ public:
     blocks out;
     {
       std::lock_guard<std::mutex> lock(mutex_);
-      take_all(out);
+      out.swap(kept_);
+      kept_bytes_ = 0;
     }
     release(out);
   }
@@ -144,7 +153,7 @@ private:
     std::lock_guard<std::mutex> lock(mutex_);
     const auto it = kept_.lower_bound({device, size});
     if (it == kept_.end() || it->first.first != device || it->first.second > size + size / 4) return nullptr;
-    void *p = it->second;
+    void *p = it->second.p;
     b = it->first;
     kept_bytes_ -= b.second;
     kept_.erase(it);
@@ -162,36 +171,38 @@ private:
     }
   }
 
-  bool add(const block &b, void *p)
+  // the blocks that make room for it go to out
+  bool add(const block &b, void *p, blocks &out)
   {
     std::lock_guard<std::mutex> lock(mutex_);
-    if (kept_bytes_ + b.second > CACHE_BYTES) return false;
+    typename blocks::iterator at;
     try {
-      kept_.emplace(b, p);
+      at = kept_.emplace(b, kept{p, ++puts_});
     } catch (const std::bad_alloc &) {
       return false;
     }
     kept_bytes_ += b.second;
+    while (kept_bytes_ > CACHE_BYTES) { // CACHE_MAX is below it: not the new one
+      auto oldest = at;
+      for (auto it = kept_.begin(); it != kept_.end(); ++it)
+        if (it->second.since < oldest->second.since) oldest = it;
+      kept_bytes_ -= oldest->first.second;
+      out.insert(kept_.extract(oldest));
+    }
     return true;
-  }
-
-  // mutex_ held
-  void take_all(blocks &out)
-  {
-    out.swap(kept_);
-    kept_bytes_ = 0;
   }
 
   // without the mutex: giving memory back takes its time
   static void release(const blocks &out)
   {
-    for (const auto &b : out) (void)Dev::release(b.second);
+    for (const auto &b : out) (void)Dev::release(b.second.p);
   }
 
   std::mutex mutex_;
   blocks kept_;
   std::unordered_map<void *, held> sizes_; // cacheable blocks in use
   size_t kept_bytes_ = 0;
+  uint64_t puts_ = 0;
   size_t in_use_ = 0; // blocks of any size
 };
 

@@ -290,6 +290,12 @@ int mfp_malloc(void **p, size_t bytes)
   return cache().alloc(p, bytes + 256) ? MFP_OK : MFP_ERR_HIP; // the slack of dmalloc
 }
 
+int mfp_trim(void)
+{
+  cache().trim();
+  return MFP_OK;
+}
+
 int mfp_free(void *p)
 {
   if (!p) return MFP_OK;

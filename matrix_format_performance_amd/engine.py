@@ -73,6 +73,12 @@ def synchronize() -> None:
     L.call("mfp_synchronize")
 
 
+def trim() -> None:
+    """Gives the device memory of destroyed objects, which the library keeps for
+    the next ones, back to the program's other allocators."""
+    L.call("mfp_trim")
+
+
 def flush_cache(nbytes: int = 1 << 30, stream=None) -> None:
     L.call("mfp_flush_cache", nbytes, stream)
 

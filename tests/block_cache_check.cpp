@@ -156,13 +156,19 @@ void limits()
   for (void *p : many) c.put(p);
   REQUIRE(c.kept_bytes(0) <= mfp::CACHE_BYTES);
   REQUIRE(c.kept_bytes(0) >= mfp::CACHE_BYTES - 1024 * MB);
+  // the latest are kept, the first ones made room
+  REQUIRE(!devices::live.count(many[0]) && devices::live.count(many[11]));
+  std::vector<void *> small;
+  for (int i = 0; i < 100; i++) small.push_back(take(c, 50 * MB));
+  for (void *p : small) c.put(p);
+  REQUIRE(c.kept_bytes(0) <= mfp::CACHE_BYTES && !devices::live.count(many[11]) && devices::live.count(small[99]));
   // an allocation that fails takes back what is kept, the caller's own too
   devices::limit = devices::bytes + MB;
   void *big = take(c, 900 * MB);
   REQUIRE(c.kept_bytes(0) == 0);
   void *own = nullptr;
   c.put(big);
-  REQUIRE(c.alloc(&own, 3000 * MB));
+  REQUIRE(c.alloc(&own, 3800 * MB));
   REQUIRE(c.kept_bytes(0) == 0);
   devices::release(own);
   // exactly the last bytes: without the rounding to a class

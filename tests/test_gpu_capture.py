@@ -76,3 +76,24 @@ def test_capture_survives_other_objects(gpu, mode, thread, what):
     P.destroy()
     A.destroy()
     B.destroy()
+
+
+def test_trim_gives_kept_memory_to_other_allocators(gpu):
+    from matrix_format_performance_amd import _lib as L
+    lib = L.load()
+
+    def raw_free():
+        free, total = C.c_size_t(), C.c_size_t()
+        assert lib.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+        return free.value
+
+    n = 1 << 20  # 500 MB of ELL arrays, and the matrix lives on
+    rp = (np.arange(n + 1) * 8).astype(np.uint32)
+    A = gpu.DeviceMatrix.from_csr(rp, (np.arange(8 * n) % n).astype(np.uint32), np.ones(8 * n, np.float32), n)
+    gpu.trim()
+    before = raw_free()
+    gpu.Plan(A, "ell", ell_width=60).destroy()
+    assert gpu.device_info()["free_mem"] >= before - (8 << 20)  # what is kept counts as free
+    gpu.trim()
+    assert abs(raw_free() - before) < 64 << 20
+    A.destroy()
