@@ -78,19 +78,13 @@ __device__ __forceinline__ void spmm_row(uint32_t row, uint32_t rows, uint32_t l
   }
 }
 
-template <typename T, int G, int KV, bool PERSISTENT>
+template <typename T, int G, int KV>
 __global__ __launch_bounds__(256) void k_spmm_vector(uint32_t rows, const uint32_t *__restrict__ rp,
                                                      const uint32_t *__restrict__ ci,
                                                      const T *__restrict__ a, const T *__restrict__ X,
                                                      T *__restrict__ Y)
 {
-  const uint32_t lane = threadIdx.x % G;
-  const uint32_t rows_per_block = 256u / G;
-  const uint32_t nblk = (rows + rows_per_block - 1) / rows_per_block;
-  for (uint32_t blk = blockIdx.x; blk < nblk; blk += (PERSISTENT ? gridDim.x : nblk)) {
-    spmm_row<T, G, KV>(blk * rows_per_block + threadIdx.x / G, rows, lane, rp, ci, a, X, Y);
-    if (!PERSISTENT) break;
-  }
+  spmm_row<T, G, KV>(blockIdx.x * (256u / G) + threadIdx.x / G, rows, threadIdx.x % G, rp, ci, a, X, Y);
 }
 
 // Rows binned by length: bin b (G = 2 << b lanes per row) holds the rows
@@ -140,53 +134,48 @@ __global__ __launch_bounds__(256) void k_spmm_binned(spmm_bins_args bins, const 
   }
 }
 
-template <typename T, int KV, bool P>
+template <typename T, int KV>
 static int spmm_g(uint32_t lanes, uint32_t rows, const uint32_t *rp, const uint32_t *ci, const T *a,
                   const T *X, T *Y, uint32_t grid, hipStream_t s)
 {
   switch (lanes) {
-  case 2: k_spmm_vector<T, 2, KV, P><<<grid, 256, 0, s>>>(rows, rp, ci, a, X, Y); break;
-  case 4: k_spmm_vector<T, 4, KV, P><<<grid, 256, 0, s>>>(rows, rp, ci, a, X, Y); break;
-  case 8: k_spmm_vector<T, 8, KV, P><<<grid, 256, 0, s>>>(rows, rp, ci, a, X, Y); break;
-  case 16: k_spmm_vector<T, 16, KV, P><<<grid, 256, 0, s>>>(rows, rp, ci, a, X, Y); break;
-  case 32: k_spmm_vector<T, 32, KV, P><<<grid, 256, 0, s>>>(rows, rp, ci, a, X, Y); break;
-  case 64: k_spmm_vector<T, 64, KV, P><<<grid, 256, 0, s>>>(rows, rp, ci, a, X, Y); break;
+  case 2: k_spmm_vector<T, 2, KV><<<grid, 256, 0, s>>>(rows, rp, ci, a, X, Y); break;
+  case 4: k_spmm_vector<T, 4, KV><<<grid, 256, 0, s>>>(rows, rp, ci, a, X, Y); break;
+  case 8: k_spmm_vector<T, 8, KV><<<grid, 256, 0, s>>>(rows, rp, ci, a, X, Y); break;
+  case 16: k_spmm_vector<T, 16, KV><<<grid, 256, 0, s>>>(rows, rp, ci, a, X, Y); break;
+  case 32: k_spmm_vector<T, 32, KV><<<grid, 256, 0, s>>>(rows, rp, ci, a, X, Y); break;
+  case 64: k_spmm_vector<T, 64, KV><<<grid, 256, 0, s>>>(rows, rp, ci, a, X, Y); break;
   default: set_error("lanes must be a power of two in [2, 64]"); return MFP_ERR_ARG;
   }
   return hipGetLastError() == hipSuccess ? MFP_OK : (set_error("kernel launch failed"), MFP_ERR_HIP);
 }
 
-template <typename T, bool P>
+template <typename T>
 static int spmm_k(uint32_t k, uint32_t lanes, uint32_t rows, const uint32_t *rp, const uint32_t *ci,
                   const T *a, const T *X, T *Y, uint32_t grid, hipStream_t s)
 {
   switch (k) {
-  case 1: return spmm_g<T, 1, P>(lanes, rows, rp, ci, a, X, Y, grid, s);
-  case 2: return spmm_g<T, 2, P>(lanes, rows, rp, ci, a, X, Y, grid, s);
-  case 4: return spmm_g<T, 4, P>(lanes, rows, rp, ci, a, X, Y, grid, s);
-  case 8: return spmm_g<T, 8, P>(lanes, rows, rp, ci, a, X, Y, grid, s);
-  case 16: return spmm_g<T, 16, P>(lanes, rows, rp, ci, a, X, Y, grid, s);
+  case 1: return spmm_g<T, 1>(lanes, rows, rp, ci, a, X, Y, grid, s);
+  case 2: return spmm_g<T, 2>(lanes, rows, rp, ci, a, X, Y, grid, s);
+  case 4: return spmm_g<T, 4>(lanes, rows, rp, ci, a, X, Y, grid, s);
+  case 8: return spmm_g<T, 8>(lanes, rows, rp, ci, a, X, Y, grid, s);
+  case 16: return spmm_g<T, 16>(lanes, rows, rp, ci, a, X, Y, grid, s);
   default: set_error("k must be 1, 2, 4, 8 or 16"); return MFP_ERR_ARG;
   }
 }
 
 int launch_spmm_vector(int dtype, uint32_t k, uint32_t lanes, uint32_t rows, const uint32_t *rp,
-                       const uint32_t *ci, const void *a, const void *X, void *Y, bool persistent,
-                       hipStream_t s)
+                       const uint32_t *ci, const void *a, const void *X, void *Y, hipStream_t s)
 {
   if (rows == 0) return MFP_OK;
   if ((k * dtype_size(dtype)) % 16 == 0 && ((uintptr_t)X % 16) != 0) {
     set_error("X must be 16-byte aligned when its rows are a multiple of 16 bytes");
     return MFP_ERR_ARG;
   }
-  const uint32_t nblk = ceil_div_u32((uint64_t)rows * lanes, 256);
-  uint32_t grid = nblk;
-  if (persistent) grid = std::min<uint32_t>(nblk, (uint32_t)std::max(1, props().cu_count) * 8u);
+  const uint32_t grid = ceil_div_u32((uint64_t)rows * lanes, 256);
   if (dtype == MFP_F32)
-    return persistent ? spmm_k<float, true>(k, lanes, rows, rp, ci, (const float *)a, (const float *)X, (float *)Y, grid, s)
-                      : spmm_k<float, false>(k, lanes, rows, rp, ci, (const float *)a, (const float *)X, (float *)Y, grid, s);
-  return persistent ? spmm_k<double, true>(k, lanes, rows, rp, ci, (const double *)a, (const double *)X, (double *)Y, grid, s)
-                    : spmm_k<double, false>(k, lanes, rows, rp, ci, (const double *)a, (const double *)X, (double *)Y, grid, s);
+    return spmm_k<float>(k, lanes, rows, rp, ci, (const float *)a, (const float *)X, (float *)Y, grid, s);
+  return spmm_k<double>(k, lanes, rows, rp, ci, (const double *)a, (const double *)X, (double *)Y, grid, s);
 }
 
 template <typename T>
@@ -1058,8 +1047,7 @@ static int batch_launch(mfp_batch b, uint32_t k, const void *X, void *Y, hipStre
     MFP_CHECK(launch_scoo_cs_spmm(m->dtype, k, m->rows, b->cs[i]->cs, b->cs[i]->scoo_threads, X, Y, s));
     return launch_spmm_aligned(b, i, X, Y, s);
   }
-  return launch_spmm_vector(m->dtype, k, b->lanes, m->rows, m->row_ptr, m->columns, m->values, X, Y,
-                            false, s);
+  return launch_spmm_vector(m->dtype, k, b->lanes, m->rows, m->row_ptr, m->columns, m->values, X, Y, s);
 }
 
 extern "C" {
@@ -1084,8 +1072,7 @@ int mfp_plan_spmm(mfp_plan p, uint32_t k, const void *X, void *Y, mfp_stream sv)
           "SpMM with k > 1 runs on CSR-vector, CSR-Adaptive (f32 / f64) and column-sorted SCOO plans");
   MFP_ARG(p->dtype == MFP_F32 || p->dtype == MFP_F64, "SpMM values must be f32 or f64");
   const mfp_matrix m = p->m;
-  return launch_spmm_vector(p->dtype, k, p->t.lanes, m->rows, m->row_ptr, m->columns, m->values, X, Y,
-                            false, as_stream(sv));
+  return launch_spmm_vector(p->dtype, k, p->t.lanes, m->rows, m->row_ptr, m->columns, m->values, X, Y, as_stream(sv));
 }
 
 int mfp_batch_create(mfp_batch *out, const mfp_matrix *ms, uint32_t count, uint32_t lanes,

@@ -92,8 +92,7 @@ int build_adaptive_layout(int dtype, uint32_t rows, const uint32_t *rp, uint32_t
 void free_adaptive_layout(adaptive_layout *l);
 
 int launch_spmm_vector(int dtype, uint32_t k, uint32_t lanes, uint32_t rows, const uint32_t *rp,
-                       const uint32_t *ci, const void *a, const void *X, void *Y, bool persistent,
-                       hipStream_t s);
+                       const uint32_t *ci, const void *a, const void *X, void *Y, hipStream_t s);
 // CSR-stream SpMM over row blocks of STREAM_W entries (fill_row_blocks, batch.hip).
 // meta holds nblocks + 1 (first row, first entry) pairs from stream_meta_device.
 constexpr uint32_t STREAM_W = 512;
