@@ -272,10 +272,11 @@ typedef struct mfp_graph_s *mfp_graph;
  * summed in the CSR-vector order with its row's lane count); 1 for the
  * column-sorted SCOO SpMM over the assembled matrix (one plan per k, built by
  * the first mfp_batch_spmm or mfp_batch_graph_create with that k: the
- * largest power-of-two slice whose k doubles per row fit in 160 KB of LDS,
- * one work item per slice and column band, 1,024 threads;
- * slices whose neighbouring rows have nearly the same columns are summed row
- * by row, in double as well); MFP_BATCH_STREAM
+ * largest power-of-two slice whose k doubles per row fit in half of the LDS,
+ * 1,024 rows at least, halved down to 256 rows where fewer slices than CUs
+ * would be left; one work item per slice and column band, 1,024 threads; for
+ * k >= 4 (f64: 8) slices whose neighbouring rows have nearly the same columns
+ * may be summed row by row, in double as well); MFP_BATCH_STREAM
  * for the CSR-stream SpMM: row blocks of whole rows with at most 512 entries
  * (fill_row_blocks, a longer row alone), staged in LDS, each group of lanes
  * that covers one X row summing 512 / groups consecutive entries, rows that

@@ -139,8 +139,8 @@ __global__ __launch_bounds__(SCAN_T) void k_scan_tiles(const uint32_t *in, uint3
   if (!offs && t == 0) *total = all;
 }
 
-// In-place (in == out) is allowed.  total_out (host) gets in[0..n) summed;
-// the call waits for the stream only when it is given.
+// In-place (in == out) is allowed.  total_out (host, may be null) gets in[0..n)
+// summed.  Waits for the stream.
 int exclusive_scan_u32(const uint32_t *in, uint32_t *out, uint64_t n, hipStream_t s,
                        uint32_t *total_out)
 {

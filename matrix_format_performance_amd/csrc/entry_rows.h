@@ -46,8 +46,8 @@ __device__ __forceinline__ uint32_t block_row_of(const uint32_t *__restrict__ rp
 
 // row[k] = the row of entry t0 + ROWS_I threadIdx.x + k (entries at or past
 // t1: of some entry of the tile).  t0 < t1 <= t0 + ROWS_TILE; rp[first] <= t0,
-// and every row after first starts at t0 or later unless it is first's own
-// entry t0 that follows; sh_mark holds ROWS_TILE words and sh 4.
+// and every row after first starts at t0 or later; sh_mark holds ROWS_TILE
+// words and sh 4.
 __device__ __forceinline__ void tile_rows(const uint32_t *__restrict__ rp, uint32_t rows, uint32_t first, uint32_t t0,
                                           uint64_t t1, uint32_t *sh_mark, uint32_t *sh, uint32_t (&row)[ROWS_I])
 {

@@ -12,7 +12,9 @@
 //   CSR-vector  G-lane strided fma + halving tree (cpu_matrix_multiplier.cpp:170-227, G=32)
 //   ELL         sequential fma over the padded width
 //   CSR-Adaptive: see k_csr_adaptive.
-// COO, SCOO and the hybrids accumulate with atomics (order not fixed).
+//   COO without rows above 64 entries: see coo_span (owner form).
+// COO with longer rows, SCOO and the hybrids accumulate with atomics (order
+// not fixed).
 #include "kernels.h"
 #include "mfp_internal.h"
 #include "row_chunks.h"

@@ -43,7 +43,8 @@ def _spmv(mfp, rp, ci, va, x, fmt, **tuning):
 
 # A chunk holds 2,048 FP32 (1,024 FP64) elements, less up to 3 (1) where it
 # starts off a 16-byte boundary, and 1,984 (960) of a longer row; blocks take
-# at most 256 rows.
+# at most 256 rows.  The smaller of these matrices are summed row by row; from 8
+# MB of entries see test_gpu_csr_vector.py.
 VECTOR_ROWS = {
     "chunk edges": [1020, 1021, 1022, 1023, 1024, 1025, 2044, 2045, 2046, 2047, 2048, 2049, 0, 1, 2, 3, 959, 960, 961,
                     1983, 1984, 1985] * 2 + [0] * 300 + [90] * 1500,
@@ -100,8 +101,8 @@ def test_free_memory_counts_kept_blocks(gpu):
     A.destroy()
     assert abs(gpu.device_info()["free_mem"] - free) < 64 << 20
 # ---- converters ---------------------------------------------------------------
-# Tiles of the sort hold 2,048 entries below 4,194,304 of them, then 8,192
-# (FP64 4,096); digits have 1 to 8 bits; tiles of entry rows hold 2,048.
+# Tiles of the sort hold 2,048 entries below 2,097,152 of them, then 4,096;
+# digits have 1 to 8 bits; tiles of entry rows hold 2,048.
 
 def _triplets(rows, cols, n, seed, dup):
     rng = np.random.default_rng(seed)
@@ -188,8 +189,9 @@ def test_column_sorted_build(gpu, rows, values):
     A.destroy()
 
 
-# Segments of row blocks hold 16,384 rows; a block holds at most W entries (a
-# longer row alone) and W + 1 rows.
+# Segments of row blocks hold 4,096 rows (16,384 above 262,144 rows:
+# test_gpu_row_blocks.py); a block holds at most W entries (a longer row alone)
+# and W + 1 rows.
 BLOCK_ROWS = {
     "segment edges": [2] * 16384 * 3,
     "one short of a segment": [3] * 16383,
@@ -303,8 +305,10 @@ def test_coo_rows_of_any_length(gpu, rows, fmt, dtype):
 
 
 # ---- batch SpMM, slices with aligned rows -----------------------------------------
-# k = 4: 2,048-row slices, 64 rows per workgroup, chunks of 2,048 (FP64 1,024)
-# entries; rows above 128 entries keep a slice in the column-sorted form.
+# Batches of few rows: slices of 256 rows, whose aligned ones (k >= 8) go by 32 or
+# 16 rows per workgroup, in chunks of 2,048 (FP64 1,024) entries; rows above 128
+# entries keep a slice in the column-sorted form.  Larger slices, and k = 4:
+# test_gpu_batch_forms.py.
 
 def _band(rows, width, seed, cols=None, gaps=False):
     """Rows of `width` columns side by side along the diagonal."""
@@ -353,8 +357,9 @@ def test_batch_aligned_and_random_slices(gpu, k, dtype):
 
 # Blocks of a batch go to the XCDs in runs of 64 (512 blocks a round): one
 # block per row of 512 entries (stream, and CSR-Adaptive with 512 per
-# workgroup), one per 64 rows of a band (aligned slices, k = 4).  Whole
-# numbers, so every order gives the same sums.
+# workgroup; the stream up to 32 blocks per CU in one range: see
+# test_gpu_batch_forms.py), and 64 rows of a band for each (column-sorted, k =
+# 4).  Whole numbers, so every order gives the same sums.
 @pytest.mark.parametrize("blocks", [31, 511, 512, 513, 543, 544, 1061])
 @pytest.mark.parametrize("form", ["stream", "rows", "aligned"])
 def test_batch_blocks_over_the_xcds(gpu, form, blocks):
@@ -388,8 +393,9 @@ def test_batch_blocks_over_the_xcds(gpu, form, blocks):
         m.destroy()
 
 
-# Column-sorted items of a batch: largest first up to 4 per CU (256 threads a
-# workgroup rank them), in runs of 8 above.  Whole numbers, as above.
+# Column-sorted items of a batch, k = 1: the plan's order up to one per CU,
+# largest first up to 4 (256 threads a workgroup rank them), in runs of 8 above.
+# Whole numbers, as above.
 @pytest.mark.parametrize("slices", [1, 2, 3, 255, 256, 257, 1023, 1024, 1025, 1060])
 def test_batch_column_sorted_items(gpu, slices):
     announce(f"batch column-sorted items slices={slices}")
