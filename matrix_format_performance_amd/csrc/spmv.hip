@@ -509,18 +509,16 @@ __device__ __forceinline__ T wg_row_sum(const uint32_t *__restrict__ ci, const T
 }
 
 // Place of staged product e: lanes read runs of 8 (FP32) or 4 (FP64) side by
-// side, and a gap after each keeps their reads on different banks.
-template <typename T>
-__host__ __device__ constexpr uint32_t adaptive_slot(uint32_t e)
-{
-  return e + (sizeof(T) == 4 ? e >> 3 : e >> 2);
-}
+// side, and a gap after each keeps their reads on different banks.  gap is the
+// log2 of the run; ADAPTIVE_NO_GAP leaves the gaps out.
+constexpr uint32_t ADAPTIVE_NO_GAP = 31;
+__host__ __device__ constexpr uint32_t adaptive_slot(uint32_t e, uint32_t gap) { return e + (e >> gap); }
 
 // bytes of the staged products, a multiple of 16
 template <typename T>
-__host__ __device__ constexpr uint32_t adaptive_products(uint32_t W)
+__host__ __device__ constexpr uint32_t adaptive_products(uint32_t W, uint32_t gap)
 {
-  return (adaptive_slot<T>(W) * (uint32_t)sizeof(T) + 15u) & ~15u;
+  return (adaptive_slot(W, gap) * (uint32_t)sizeof(T) + 15u) & ~15u;
 }
 
 // A workgroup takes one item: the pieces of long rows first, then the row
@@ -535,14 +533,14 @@ __global__ __launch_bounds__(AD_T) void k_csr_adaptive(
     const uint32_t *__restrict__ rp, const uint32_t *__restrict__ ci, const T *__restrict__ a,
     const T *__restrict__ x, T *__restrict__ y, const uint32_t *__restrict__ blocks,
     uint32_t nnz_per_wg, uint32_t long_row, const uint4 *__restrict__ chunks, uint32_t nchunks,
-    uint32_t nchunks_pad, uint32_t chunk, T *__restrict__ partials)
+    uint32_t nchunks_pad, uint32_t chunk, uint32_t gap, T *__restrict__ partials)
 {
   using VT = vec16<T>;
   constexpr uint32_t N = VT::N;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   T *cache = reinterpret_cast<T *>(smem_raw); // staged products (nnz_per_wg, by adaptive_slot)
   // block-relative row starts (nnz_per_wg + 2)
-  uint32_t *rs = reinterpret_cast<uint32_t *>(smem_raw + adaptive_products<T>(nnz_per_wg));
+  uint32_t *rs = reinterpret_cast<uint32_t *>(smem_raw + adaptive_products<T>(nnz_per_wg, gap));
   __shared__ T wsum[4];
   __shared__ T sv[2 * AD_T];
   __shared__ uint32_t wsteps[4];
@@ -588,6 +586,32 @@ __global__ __launch_bounds__(AD_T) void k_csr_adaptive(
       vc[k] = ldg_stream(cv + v);
     }
   }
+  // EARLY: the products are finished before the row starts are staged.  With 16
+  // vectors per lane, x entries held over the search take 178 VGPRs in FP64 and
+  // leave a CU two workgroups of three (4,096 entries per workgroup, 27-point
+  // 100^3: 118 us, 98 so); the smaller forms gain from it.
+  constexpr bool EARLY = sizeof(T) == 8 && K >= 16;
+  T xv[K][N];
+  if constexpr (EARLY) {
+#pragma unroll
+    for (uint32_t k = 0; k < K; k++) {
+      const uint32_t v = v0 + tid + k * AD_T;
+#pragma unroll
+      for (uint32_t j = 0; j < N; j++) {
+        const uint32_t e = v * N + j;
+        xv[k][j] = (v < v1 && e >= base && e < base + n) ? x[vc[k][j]] : (T)0;
+      }
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < K; k++) {
+      const uint32_t v = v0 + tid + k * AD_T;
+#pragma unroll
+      for (uint32_t j = 0; j < N; j++) {
+        const uint32_t e = v * N + j;
+        if (v < v1 && e >= base && e < base + n) cache[adaptive_slot(e - base, gap)] = va[k][j] * xv[k][j];
+      }
+    }
+  }
   // the row starts are loaded beside the entries; the gathers go out together
   // behind their barrier and are in flight while the rows are searched
   const uint32_t nr = r1 - r0;
@@ -597,8 +621,7 @@ __global__ __launch_bounds__(AD_T) void k_csr_adaptive(
   if (tid + AD_T <= nr) rs[tid + AD_T] = p1 - base;
   for (uint32_t lr = tid + 2 * AD_T; lr <= nr; lr += AD_T) rs[lr] = rp[r0 + lr] - base;
   __syncthreads();
-  T xv[K][N];
-  if (n) { // without entries x may be empty
+  if (!EARLY && n) { // without entries x may be empty
 #pragma unroll
     for (uint32_t k = 0; k < K; k++) {
       const uint32_t v = v0 + tid + k * AD_T;
@@ -627,13 +650,15 @@ __global__ __launch_bounds__(AD_T) void k_csr_adaptive(
         hi = mid;
     }
   }
+  if constexpr (!EARLY) {
 #pragma unroll
-  for (uint32_t k = 0; k < K; k++) {
-    const uint32_t v = v0 + tid + k * AD_T;
+    for (uint32_t k = 0; k < K; k++) {
+      const uint32_t v = v0 + tid + k * AD_T;
 #pragma unroll
-    for (uint32_t j = 0; j < N; j++) {
-      const uint32_t e = v * N + j;
-      if (v < v1 && e >= base && e < base + n) cache[adaptive_slot<T>(e - base)] = va[k][j] * xv[k][j];
+      for (uint32_t j = 0; j < N; j++) {
+        const uint32_t e = v * N + j;
+        if (v < v1 && e >= base && e < base + n) cache[adaptive_slot(e - base, gap)] = va[k][j] * xv[k][j];
+      }
     }
   }
   __syncthreads();
@@ -661,7 +686,7 @@ __global__ __launch_bounds__(AD_T) void k_csr_adaptive(
         cur_start = cur_end;
         cur_end = rs[cur + 1];
       }
-      d = d + cache[adaptive_slot<T>(e)];
+      d = d + cache[adaptive_slot(e, gap)];
     }
     const bool starts = seg == cur_start;
     if (e1 == cur_end) {
@@ -1720,21 +1745,34 @@ uint32_t adaptive_vectors_per_lane(int dtype, uint32_t W)
 }
 
 template <typename T, uint32_t K>
-static int adaptive_launch_k(const adaptive_args &g, const T *a, const T *x, T *y, hipStream_t s,
+static int adaptive_launch_k(const adaptive_args &g, const T *a, const T *x, T *y, hipStream_t s, uint32_t gap,
                              size_t lds, uint32_t items, uint32_t nchunks_pad)
 {
   const auto fn = g.batch ? k_csr_adaptive<T, K, true> : k_csr_adaptive<T, K, false>;
   if (lds > 65536)
     MFP_HIP(hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   return launch_k(fn, dim3(items), dim3(AD_T), (uint32_t)lds, s, g.rp, g.ci, a, x, y, g.blocks, g.nnz_per_wg,
-                  g.long_row, g.chunks, g.nchunks, nchunks_pad, g.chunk, (T *)g.partials);
+                  g.long_row, g.chunks, g.nchunks, nchunks_pad, g.chunk, gap, (T *)g.partials);
 }
 
 // Dynamic LDS of k_csr_adaptive: the staged products, then the row starts.
 template <typename T>
-static size_t adaptive_lds_bytes(uint32_t W)
+static size_t adaptive_lds_bytes(uint32_t W, uint32_t gap)
 {
-  return adaptive_products<T>(W) + ((size_t)W + 2) * 4;
+  return adaptive_products<T>(W, gap) + ((size_t)W + 2) * 4;
+}
+
+// The gaps between the products, unless a CU would hold fewer workgroups with
+// them: us with and without, 27-point 100^3, FP64 W = 1,800, 2,800, 4,000 73.0 and
+// 68.3, 91.8 and 77.7, 107.5 and 81.3, FP32 W = 2,600, 4,700, 6,300 61.3 and 57.2,
+// 79.7 and 68.4, 100.2 and 73.8; where as many fit (FP32 W = 8,000) 92.7 and 104.8.
+template <typename T>
+static uint32_t adaptive_gap(uint32_t W)
+{
+  const size_t lds = 160u << 10, own = 2 * AD_T * sizeof(T) + 64; // sv, wsum, wsteps
+  constexpr uint32_t gap = sizeof(T) == 4 ? 3 : 2;
+  const auto groups = [&](uint32_t q) { return std::min<size_t>(8, lds / (adaptive_lds_bytes<T>(W, q) + own)); };
+  return groups(gap) < groups(ADAPTIVE_NO_GAP) ? ADAPTIVE_NO_GAP : gap;
 }
 
 template <typename T>
@@ -1743,16 +1781,17 @@ static int adaptive_t(const adaptive_args &g, const T *a, const T *x, T *y, hipS
   // chunk items first; padded to a multiple of 8 so block ids keep their XCD
   const uint32_t nchunks_pad = (g.nchunks + 7u) & ~7u;
   const uint32_t items = g.nblocks ? g.nblocks + nchunks_pad : nchunks_pad;
-  const size_t lds = adaptive_lds_bytes<T>(g.nnz_per_wg);
+  const uint32_t gap = adaptive_gap<T>(g.nnz_per_wg);
+  const size_t lds = adaptive_lds_bytes<T>(g.nnz_per_wg, gap);
   const uint32_t K = adaptive_vectors_per_lane(sizeof(T) == 4 ? MFP_F32 : MFP_F64, g.nnz_per_wg);
   if (items) {
     int st;
     switch (K) {
-    case 1: st = adaptive_launch_k<T, 1>(g, a, x, y, s, lds, items, nchunks_pad); break;
-    case 2: st = adaptive_launch_k<T, 2>(g, a, x, y, s, lds, items, nchunks_pad); break;
-    case 4: st = adaptive_launch_k<T, 4>(g, a, x, y, s, lds, items, nchunks_pad); break;
-    case 8: st = adaptive_launch_k<T, 8>(g, a, x, y, s, lds, items, nchunks_pad); break;
-    case 16: st = adaptive_launch_k<T, 16>(g, a, x, y, s, lds, items, nchunks_pad); break;
+    case 1: st = adaptive_launch_k<T, 1>(g, a, x, y, s, gap, lds, items, nchunks_pad); break;
+    case 2: st = adaptive_launch_k<T, 2>(g, a, x, y, s, gap, lds, items, nchunks_pad); break;
+    case 4: st = adaptive_launch_k<T, 4>(g, a, x, y, s, gap, lds, items, nchunks_pad); break;
+    case 8: st = adaptive_launch_k<T, 8>(g, a, x, y, s, gap, lds, items, nchunks_pad); break;
+    case 16: st = adaptive_launch_k<T, 16>(g, a, x, y, s, gap, lds, items, nchunks_pad); break;
     default: set_error("nnz_per_wg too large"); return MFP_ERR_ARG;
     }
     MFP_CHECK(st);
