@@ -622,6 +622,7 @@ int stream_meta_device(uint32_t rows, const uint32_t *rp, uint32_t **meta, uint3
       st = MFP_ERR_HIP;
     }
   }
+  const free_scope scope(st == MFP_OK);
   dfree(blocks);
   if (st != MFP_OK) {
     dfree(m);
@@ -858,6 +859,7 @@ static int batch_order_items(scoo_cs_layout &l, uint32_t k, hipStream_t s)
     std::swap(l.base, base);
     l.run = 0;
   }
+  const free_scope scope(st == MFP_OK);
   dfree(items);
   dfree(base);
   return st;
@@ -1242,6 +1244,7 @@ int mfp_graph_destroy(mfp_graph g)
 int mfp_batch_destroy(mfp_batch b)
 {
   if (!b) return MFP_OK;
+  const free_scope scope;
   mfp_plan_destroy(b->k1);
   for (mfp_plan p : b->cs) mfp_plan_destroy(p);
   for (uint32_t *p : b->aligned) dfree(p);

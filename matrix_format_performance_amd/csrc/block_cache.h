@@ -1,7 +1,8 @@
 // Freed device blocks, kept for the library's next allocations.  Host code
 // only; the device calls come from Dev, so that the bookkeeping can be checked
 // without a GPU:
-//   static bool alloc(void **p, size_t bytes)  on the current device
+//   static bool alloc(void **p, size_t bytes)  on the current device; of no
+//                                              bytes: whether it may be called
 //   static bool release(void *p)               of any device; waits for the current one
 //   static int current()                       the current device, -1 unknown
 #pragma once
@@ -22,13 +23,15 @@ namespace mfp {
 // (nine formats of a 5M-entry matrix: 1.8 ms of kernels in 8.7 to 12.9 ms).
 // Freed blocks of 64 KB to 1 GB are therefore kept and handed out again, in
 // size classes an eighth of a power of two apart.
-//  * Every block that is taken from the cache or put there goes with a token, a
-//    small allocation of its own (1.4 us to allocate and free).  Allocating it
-//    is refused where hipMalloc is, in a stream capture; freeing it waits for the
-//    device as hipFree does, so that whoever gets the block next, on any stream
-//    or thread, finds nothing still running on it.  hipDeviceSynchronize (0.2 us
-//    on an idle device) would wait as well, but it ends every stream capture in
-//    the process, also those that another thread's hipFree leaves alone.
+//  * A block is kept once its device is idle: by put, which waits as hipFree
+//    does, or by its caller's word (a stream that was waited for and alone used
+//    it). Whoever gets it next, on any stream or thread, finds nothing still
+//    running on it.  put waits by freeing a token, a small allocation that it
+//    makes for that: hipDeviceSynchronize would wait as well, but it ends every
+//    stream capture in the process, also those that another thread's hipFree
+//    leaves alone.
+//  * get is refused where hipMalloc is, in a stream capture, also when a kept
+//    block would do: an allocation of no bytes asks.
 //  * A block is filed under the device it was allocated on, whichever device
 //    the freeing thread uses, and handed out on that device only.
 //  * At most CACHE_BYTES are kept, the oldest make room; an allocation that
@@ -44,10 +47,6 @@ class block_cache {
     uint64_t since; // counts the blocks that were put
   };
   using blocks = std::multimap<block, kept>;
-  struct held {
-    block b;
-    void *token;
-  };
   static constexpr size_t TOKEN = 256;
 
 public:
@@ -60,10 +59,10 @@ public:
     if (cacheable) {
       block b{-1, 0};
       if (void *p = take_kept(device, size, b)) {
-        void *token = nullptr;
-        if (Dev::alloc(&token, TOKEN)) {
+        void *none = nullptr;
+        if (Dev::alloc(&none, 0)) {
           std::lock_guard<std::mutex> lock(mutex_);
-          taken(p, b, token);
+          taken(p, b);
           return p;
         }
         (void)Dev::release(p);
@@ -76,29 +75,32 @@ public:
       if (size == bytes || !Dev::alloc(&p, bytes)) return nullptr; // without the rounding, then
     }
     std::lock_guard<std::mutex> lock(mutex_);
-    taken(p, b, nullptr);
+    taken(p, b);
     return p;
   }
 
-  // gives back a block of get
-  void put(void *p)
+  // Gives back a block of get.  idle: nothing still uses it.  Returns idle, or
+  // that the current device was waited for.
+  bool put(void *p, bool idle)
   {
-    if (!p) return;
-    held h{{-1, 0}, nullptr};
+    if (!p) return idle;
+    block b{-1, 0};
     {
       std::lock_guard<std::mutex> lock(mutex_);
       const auto it = sizes_.find(p);
       if (it != sizes_.end()) {
-        h = it->second;
+        b = it->second;
         sizes_.erase(it);
       }
     }
-    // freeing waits for the current device, so only its blocks are kept
-    const bool own = h.b.second && Dev::current() == h.b.first;
-    if (own && !h.token && !Dev::alloc(&h.token, TOKEN)) h.token = nullptr;
-    const bool idle = h.token && Dev::release(h.token) && own;
+    // waiting is for the current device, so only its blocks are kept
+    const bool own = b.second && Dev::current() == b.first;
+    if (own && !idle) {
+      void *token = nullptr;
+      idle = Dev::alloc(&token, TOKEN) && Dev::release(token);
+    }
     blocks out;
-    if (!(idle && add(h.b, p, out))) (void)Dev::release(p);
+    if (!(own && idle && add(b, p, out))) (void)Dev::release(p);
     {
       std::lock_guard<std::mutex> lock(mutex_);
       if (--in_use_ == 0) {
@@ -107,6 +109,7 @@ public:
       }
     }
     release(out);
+    return idle;
   }
 
   // an allocation beside the cache's own that may take what it keeps
@@ -161,13 +164,12 @@ private:
   }
 
   // mutex_ held; without memory for the entry the block is not cacheable
-  void taken(void *p, const block &b, void *token)
+  void taken(void *p, const block &b)
   {
     in_use_++;
     try {
-      if (b.second) sizes_[p] = held{b, token};
+      if (b.second) sizes_[p] = b;
     } catch (const std::bad_alloc &) {
-      if (token) (void)Dev::release(token);
     }
   }
 
@@ -200,7 +202,7 @@ private:
 
   std::mutex mutex_;
   blocks kept_;
-  std::unordered_map<void *, held> sizes_; // cacheable blocks in use
+  std::unordered_map<void *, block> sizes_; // cacheable blocks in use
   size_t kept_bytes_ = 0;
   uint64_t puts_ = 0;
   size_t in_use_ = 0; // blocks of any size

@@ -18,9 +18,11 @@ namespace mfp {
 // Device allocations freed on every return path unless released.
 struct device_temps {
   std::vector<void *> held;
+  bool idle = false; // their one stream was waited for
   int alloc(void **p, size_t bytes)
   {
     const int st = dmalloc(p, bytes);
+    idle = false; // work on it follows
     if (st == MFP_OK) held.push_back(*p);
     return st;
   }
@@ -29,8 +31,16 @@ struct device_temps {
     for (void *&q : held)
       if (q == p) q = nullptr;
   }
+  // waits for the stream that alone uses them
+  int settle(hipStream_t s)
+  {
+    MFP_HIP(hipStreamSynchronize(s));
+    idle = true;
+    return MFP_OK;
+  }
   ~device_temps()
   {
+    const free_scope scope(idle);
     for (void *q : held) dfree(q);
   }
 };
@@ -159,7 +169,7 @@ int exclusive_scan_u32(const uint32_t *in, uint32_t *out, uint64_t n, hipStream_
   }
   MFP_HIP(hipGetLastError());
   if (total_out) MFP_HIP(hipMemcpyAsync(total_out, sums + tiles, 4, hipMemcpyDeviceToHost, s));
-  MFP_HIP(hipStreamSynchronize(s)); // sums is freed here
+  MFP_CHECK(tmp.settle(s)); // sums is freed here
   return MFP_OK;
 }
 
@@ -420,7 +430,7 @@ static int sort_entries_t(const uint32_t *row, const uint32_t *col, const VI *va
                                                              o.val);
     MFP_HIP(hipGetLastError());
   }
-  MFP_HIP(hipStreamSynchronize(s)); // hist is freed here
+  MFP_CHECK(tmp.settle(s)); // hist is freed here
   return MFP_OK;
 }
 
@@ -473,7 +483,7 @@ static int csr_from_triplets_t(uint32_t rows, uint32_t cols, uint64_t nnz, const
   MFP_HIP(hipGetLastError());
   uint32_t hbad = 0;
   MFP_HIP(hipMemcpyAsync(&hbad, bad, 4, hipMemcpyDeviceToHost, s));
-  MFP_HIP(hipStreamSynchronize(s));
+  MFP_CHECK(tmp.settle(s));
   if (hbad) {
     set_error("triplet row/col index out of range");
     return MFP_ERR_ARG;
@@ -566,7 +576,7 @@ int row_stats_device(uint32_t rows, const uint32_t *rp, mfp_row_stats *out, hipS
     MFP_HIP(hipGetLastError());
     std::vector<stats_acc> part(g);
     MFP_HIP(hipMemcpyAsync(part.data(), acc, g * sizeof(stats_acc), hipMemcpyDeviceToHost, s));
-    MFP_HIP(hipStreamSynchronize(s));
+    MFP_CHECK(tmp.settle(s));
     for (const stats_acc &p : part) {
       h.mn = std::min(h.mn, p.mn);
       h.mx = std::max(h.mx, p.mx);
@@ -728,7 +738,7 @@ int coo_tail_build_device(int dtype, uint32_t rows, uint64_t nnz, const uint32_t
                                                *cr);
     MFP_HIP(hipGetLastError());
   }
-  MFP_HIP(hipStreamSynchronize(s));
+  MFP_CHECK(tmp.settle(s));
   return MFP_OK;
 }
 
@@ -973,6 +983,7 @@ int scoo_cs_build_device(int dtype, uint32_t rows, uint32_t cols, uint64_t nnz, 
     return st;
   };
   auto done = [&](int st) {
+    const free_scope scope;
     for (void *p : tmp) dfree(p);
     if (st != MFP_OK) scoo_cs_free(out);
     return st;
@@ -1216,6 +1227,7 @@ int scoo_cs_build_device(int dtype, uint32_t rows, uint32_t cols, uint64_t nnz, 
 
 void scoo_cs_free(scoo_cs_layout *l)
 {
+  const free_scope scope;
   dfree(l->sp);
   dfree(l->long_rows);
   dfree(l->long_mask);
@@ -1428,12 +1440,12 @@ static int row_blocks_t(uint32_t rows, const uint32_t *rp, uint32_t W, uint32_t 
   MFP_HIP(hipGetLastError());
   uint32_t h[2] = {0, 0};
   MFP_HIP(hipMemcpyAsync(h, count + nseg, 8, hipMemcpyDeviceToHost, s));
-  MFP_HIP(hipStreamSynchronize(s));
+  MFP_CHECK(tmp.settle(s));
   const uint32_t total = h[0] + h[1];
   MFP_CHECK(tmp.alloc((void **)&out, ((uint64_t)total + 1) * 4));
   k_seg_write<SEG><<<nseg, SEG / 32, 0, s>>>(rows, nseg, bits, count, count + nseg + 1, out);
   MFP_HIP(hipGetLastError());
-  MFP_HIP(hipStreamSynchronize(s));
+  MFP_CHECK(tmp.settle(s));
   tmp.release(out);
   *blocks_out = out;
   *count_out = total;

@@ -286,7 +286,10 @@ extern "C" int mfp_matrix_features(mfp_matrix m, float *out)
     st = MFP_ERR_HIP;
   }
   if (st == MFP_OK) st = mfp_memcpy_d2h(&tot, dc, sizeof tot);
-  dfree(dc);
+  {
+    const free_scope scope(st == MFP_OK);
+    dfree(dc);
+  }
   MFP_CHECK(st);
   const feat_row_counters &h = tot.r;
   const feat_entry_counters &he = tot.e;

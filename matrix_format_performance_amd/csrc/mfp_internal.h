@@ -109,6 +109,21 @@ int ensure_init();
 // for the next ones (block_cache.h).  dfree waits for the device, as hipFree.
 int dmalloc(void **p, size_t bytes);
 void dfree(void *p);
+// While it lives, the thread's dfree calls wait for the device once, not each;
+// idle: not at all, since whatever used the blocks was waited for.  Nothing is
+// launched on the blocks meanwhile.
+class free_scope {
+public:
+  explicit free_scope(bool idle = false);
+  ~free_scope();
+  free_scope(const free_scope &) = delete;
+  free_scope &operator=(const free_scope &) = delete;
+
+private:
+  friend void dfree(void *p);
+  bool idle_;
+  free_scope *outer_;
+};
 // bytes kept that way now: free memory from the library's point of view
 size_t cached_device_bytes();
 

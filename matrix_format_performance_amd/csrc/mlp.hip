@@ -359,6 +359,7 @@ int mfp_mlp_create(mfp_mlp *out, uint64_t seed)
 int mfp_mlp_destroy(mfp_mlp m)
 {
   if (!m) return MFP_OK;
+  const free_scope scope;
   mlp_free_batch(m);
   dfree(m->params);
   dfree(m->grads);

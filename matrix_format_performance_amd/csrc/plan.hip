@@ -38,6 +38,7 @@ __global__ void k_chunk_fill(const uint32_t *__restrict__ blocks, uint32_t nb,
 
 void free_adaptive_layout(adaptive_layout *l)
 {
+  const free_scope scope;
   dfree(l->blocks);
   dfree(l->chunks);
   dfree(l->partials);
@@ -66,6 +67,7 @@ int build_adaptive_layout(int dtype, uint32_t rows, const uint32_t *rp, uint32_t
   if (st == MFP_OK && l.nchunks)
     k_chunk_fill<<<ceil_div_u32(l.nblocks, 256), 256, 0, s>>>(l.blocks, l.nblocks, cnt, base, l.chunks);
   if (st == MFP_OK && hipStreamSynchronize(s) != hipSuccess) st = MFP_ERR_HIP;
+  const free_scope scope(st == MFP_OK);
   dfree(cnt);
   dfree(base);
   if (st != MFP_OK) {
@@ -143,6 +145,7 @@ static void scoo_mi355x_geometry(int dtype, uint32_t rows, uint32_t *slices, uin
 
 static int plan_free_arrays(mfp_plan p)
 {
+  const free_scope scope;
   dfree(p->ell_val);
   dfree(p->ell_col);
   dfree(p->coo_val);
@@ -320,6 +323,7 @@ int mfp_matrix_from_triplets(mfp_matrix *out, int dtype, uint32_t rows, uint32_t
   const double *dv = tr_vals;
   void *tmp[3] = {nullptr, nullptr, nullptr};
   auto release = [&]() {
+    const free_scope scope;
     for (void *p : tmp) dfree(p);
   };
   if (!inputs_on_device && nnz) {
@@ -411,6 +415,7 @@ int mfp_matrix_convert(mfp_matrix src, int dtype, mfp_matrix *out)
 int mfp_matrix_destroy(mfp_matrix m)
 {
   if (!m) return MFP_OK;
+  const free_scope scope;
   dfree(m->row_ptr);
   dfree(m->columns);
   dfree(m->values);

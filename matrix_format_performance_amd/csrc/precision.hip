@@ -599,6 +599,7 @@ int lp_binned_build(uint32_t rows, const uint32_t *rp_dev, lp_binned_layout *out
 
 void lp_binned_free(lp_binned_layout *l)
 {
+  const free_scope scope;
   dfree(l->list);
   dfree(l->chunks);
   dfree(l->longs);

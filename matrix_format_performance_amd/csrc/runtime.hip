@@ -114,7 +114,17 @@ int dmalloc(void **p, size_t bytes)
   return *p ? MFP_OK : MFP_ERR_HIP;
 }
 
-void dfree(void *p) { cache().put(p); }
+static thread_local free_scope *g_free_scope = nullptr;
+
+free_scope::free_scope(bool idle) : idle_(idle), outer_(g_free_scope) { g_free_scope = this; }
+free_scope::~free_scope() { g_free_scope = outer_; }
+
+void dfree(void *p)
+{
+  free_scope *f = g_free_scope;
+  const bool idle = cache().put(p, f && f->idle_);
+  if (f) f->idle_ = idle;
+}
 
 // ---- fills ----------------------------------------------------------------
 

@@ -37,6 +37,10 @@ struct devices {
   {
     std::lock_guard<std::mutex> lock(mutex);
     if (refuse || bytes + n > limit) return false;
+    if (n == 0) {
+      *p = nullptr;
+      return true;
+    }
     *p = reinterpret_cast<void *>(next);
     next += n + 4096;
     bytes += n;
@@ -74,6 +78,9 @@ void *take(cache_t &c, size_t n)
   return p;
 }
 
+// gives it back as an object does that waited for nothing itself
+bool put(cache_t &c, void *p) { return c.put(p, false); }
+
 constexpr size_t MB = 1u << 20;
 
 void reuse()
@@ -81,17 +88,17 @@ void reuse()
   cache_t c;
   void *hold = take(c, 1000); // keeps the cache from emptying
   void *p = take(c, 20 * MB);
-  c.put(p);
+  put(c, p);
   REQUIRE(c.kept_bytes(0) >= 20 * MB && c.kept_bytes(1) == 0);
   REQUIRE(take(c, 19 * MB) == p);
   REQUIRE(c.kept_bytes(0) == 0);
-  c.put(p);
+  put(c, p);
   void *q = take(c, 5 * MB); // a far smaller one does not take it
   REQUIRE(q != p);
   c.trim();
   REQUIRE(c.kept_bytes(0) == 0 && devices::live.size() == 2);
-  c.put(q);
-  c.put(hold);
+  put(c, q);
+  put(c, hold);
   REQUIRE(devices::live.empty()); // the last block gives everything back
 }
 
@@ -101,22 +108,44 @@ void refused()
 {
   cache_t c;
   void *hold = take(c, 1000), *p = take(c, 20 * MB), *q = take(c, 30 * MB);
-  c.put(p);
+  put(c, p);
   devices::refuse = true;
   REQUIRE(!c.get(20 * MB));
-  c.put(q);
+  put(c, q);
   REQUIRE(!devices::live.count(q));
   devices::refuse = false;
   REQUIRE(c.kept_bytes(0) == 0);
   void *r = take(c, 20 * MB);
-  c.put(r);
-  r = take(c, 20 * MB); // with a token from here on
+  put(c, r);
   devices::refuse = true;
-  c.put(r); // its token is freed all the same
+  REQUIRE(!c.get(20 * MB) && !devices::live.count(r)); // the kept one is given back meanwhile
   devices::refuse = false;
-  REQUIRE(take(c, 20 * MB) == r);
-  c.put(r);
-  c.put(hold);
+  put(c, hold);
+  REQUIRE(devices::live.empty());
+}
+
+// An object's arrays: the first is waited for, which tells that the others are
+// idle too
+void together()
+{
+  cache_t c;
+  void *hold = take(c, 1000);
+  void *p = take(c, 20 * MB), *q = take(c, 30 * MB);
+  REQUIRE(put(c, p)); // waited
+  const size_t next = devices::next;
+  REQUIRE(c.put(q, true) && devices::next == next); // no token, no wait
+  REQUIRE(take(c, 30 * MB) == q && take(c, 20 * MB) == p);
+  // what is not known stays unknown: another device's block, a small one, a refused wait
+  devices::now = 1;
+  REQUIRE(!put(c, p) && !devices::live.count(p));
+  devices::now = 0;
+  void *small = take(c, 1000);
+  REQUIRE(!put(c, small));
+  devices::refuse = true;
+  REQUIRE(!put(c, q) && !devices::live.count(q));
+  devices::refuse = false;
+  REQUIRE(!c.put(nullptr, false) && c.put(nullptr, true));
+  put(c, hold);
   REQUIRE(devices::live.empty());
 }
 
@@ -131,17 +160,17 @@ void two_devices()
     devices::now = 1;
     void *b = take(c, 1000);
     devices::now = from;
-    c.put(a);
+    put(c, a);
     REQUIRE(c.kept_bytes(1) == 0);
     devices::now = 1;
     void *d = take(c, 20 * MB); // take checks its device
     REQUIRE(d != a);
     devices::now = 0;
     if (from == 0) REQUIRE(take(c, 20 * MB) == a); // kept where it belongs
-    if (from == 0) c.put(a);
+    if (from == 0) put(c, a);
     devices::now = 1;
-    c.put(d);
-    c.put(b);
+    put(c, d);
+    put(c, b);
     REQUIRE(devices::live.empty());
   }
   devices::now = 0;
@@ -153,21 +182,21 @@ void limits()
   void *hold = take(c, 1000);
   std::vector<void *> many;
   for (int i = 0; i < 12; i++) many.push_back(take(c, 700 * MB));
-  for (void *p : many) c.put(p);
+  for (void *p : many) put(c, p);
   REQUIRE(c.kept_bytes(0) <= mfp::CACHE_BYTES);
   REQUIRE(c.kept_bytes(0) >= mfp::CACHE_BYTES - 1024 * MB);
   // the latest are kept, the first ones made room
   REQUIRE(!devices::live.count(many[0]) && devices::live.count(many[11]));
   std::vector<void *> small;
   for (int i = 0; i < 100; i++) small.push_back(take(c, 50 * MB));
-  for (void *p : small) c.put(p);
+  for (void *p : small) put(c, p);
   REQUIRE(c.kept_bytes(0) <= mfp::CACHE_BYTES && !devices::live.count(many[11]) && devices::live.count(small[99]));
   // an allocation that fails takes back what is kept, the caller's own too
   devices::limit = devices::bytes + MB;
   void *big = take(c, 900 * MB);
   REQUIRE(c.kept_bytes(0) == 0);
   void *own = nullptr;
-  c.put(big);
+  put(c, big);
   REQUIRE(c.alloc(&own, 3800 * MB));
   REQUIRE(c.kept_bytes(0) == 0);
   devices::release(own);
@@ -176,16 +205,16 @@ void limits()
   void *tight = c.get(70001);
   REQUIRE(tight && devices::live[tight].size == 70001);
   REQUIRE(!c.get(70001));
-  c.put(tight);
+  put(c, tight);
   devices::limit = ~size_t(0);
   // a device that cannot be waited for keeps nothing
   void *p = take(c, 10 * MB);
   devices::free_fails = true;
-  c.put(p);
+  put(c, p);
   devices::free_fails = false;
   REQUIRE(c.kept_bytes(0) == 0 && !devices::live.count(p));
-  c.put(hold);
-  c.put(nullptr);
+  put(c, hold);
+  put(c, nullptr);
   REQUIRE(devices::live.empty());
 }
 
@@ -203,13 +232,13 @@ void threads()
           held.push_back(take(c, 1 + (size_t)(rng() % 4 ? rng() % (2 * MB) : rng() % (80 * MB))));
         } else if (!held.empty()) {
           const size_t k = rng() % held.size();
-          c.put(held[k]); // from either device
+          put(c, held[k]); // from either device
           held[k] = held.back();
           held.pop_back();
         }
         if (rng() % 500 == 0) c.trim();
       }
-      for (void *p : held) c.put(p);
+      for (void *p : held) put(c, p);
     });
   for (auto &t : ts) t.join();
   REQUIRE(devices::live.empty() && devices::bytes == 0);
@@ -221,6 +250,7 @@ int main()
 {
   reuse();
   refused();
+  together();
   two_devices();
   limits();
   threads();
