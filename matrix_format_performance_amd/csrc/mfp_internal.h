@@ -124,6 +124,22 @@ private:
   bool idle_;
   free_scope *outer_;
 };
+// While it lives, the thread may allocate, free and wait beside a stream capture
+// that would refuse it (on streams that are not captured).
+class beside_capture {
+public:
+  beside_capture() { ok_ = hipThreadExchangeStreamCaptureMode(&mode_) == hipSuccess; }
+  ~beside_capture()
+  {
+    if (ok_) (void)hipThreadExchangeStreamCaptureMode(&mode_);
+  }
+  beside_capture(const beside_capture &) = delete;
+  beside_capture &operator=(const beside_capture &) = delete;
+
+private:
+  hipStreamCaptureMode mode_ = hipStreamCaptureModeRelaxed;
+  bool ok_;
+};
 // bytes kept that way now: free memory from the library's point of view
 size_t cached_device_bytes();
 

@@ -110,6 +110,19 @@ static int matrix_stats(mfp_matrix m, mfp_row_stats *out, hipStream_t s)
   return MFP_OK;
 }
 
+// How a CSR-vector plan takes its rows is a matter of speed: it is made beside
+// a stream capture as well, and where no memory is left the rows go one by one.
+static void plan_csr_vector(mfp_plan p, mfp_matrix m, hipStream_t s)
+{
+  const beside_capture mode;
+  mfp_row_stats rs{};
+  int st = MFP_OK;
+  if (csr_vector_rows(m->dtype, p->t.lanes, m->rows, m->nnz) > 1) st = matrix_stats(m, &rs, s);
+  if (st == MFP_OK)
+    st = csr_vector_layout_build(m->dtype, p->t.lanes, m->rows, m->nnz, rs.max_elements_in_rows, m->row_ptr, &p->cv, s);
+  if (st != MFP_OK) p->cv.rb = 0;
+}
+
 static uint32_t next_pow2_u32(uint32_t v)
 {
   uint32_t p = 1;
@@ -566,14 +579,7 @@ int mfp_plan_create(mfp_plan *out, mfp_matrix m, int format, const mfp_tuning *t
       set_error("lanes must be a power of two in [2, 64]");
       return fail(MFP_ERR_ARG);
     }
-    {
-      mfp_row_stats rs{};
-      if (csr_vector_rows(m->dtype, t.lanes, m->rows, m->nnz) > 1) st = matrix_stats(m, &rs, s);
-      if (st == MFP_OK)
-        st = csr_vector_layout_build(m->dtype, t.lanes, m->rows, m->nnz, rs.max_elements_in_rows, m->row_ptr, &p->cv,
-                                     s);
-      if (st != MFP_OK) return fail(st);
-    }
+    plan_csr_vector(p, m, s);
     break;
   case MFP_CSR_ADAPTIVE:
     st = build_adaptive_layout(m->dtype, m->rows, m->row_ptr, t.nnz_per_wg, t.long_row, t.chunk,

@@ -1674,7 +1674,10 @@ int csr_vector_layout_build(int dtype, uint32_t lanes, uint32_t rows, uint64_t n
 
 void csr_vector_layout_free(csr_vector_layout *l)
 {
-  dfree(l->mask);
+  if (l->mask) {
+    const beside_capture mode;
+    dfree(l->mask);
+  }
   l->mask = l->list = nullptr;
   l->count = 0;
 }

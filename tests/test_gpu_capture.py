@@ -11,7 +11,7 @@ from gpu_cases import announce
 pytestmark = pytest.mark.gpu
 
 
-THREAD_LOCAL, RELAXED = 1, 2  # hipStreamCaptureMode
+GLOBAL, THREAD_LOCAL, RELAXED = 0, 1, 2  # hipStreamCaptureMode
 
 
 @pytest.mark.parametrize("what", ["destroy", "create"])
@@ -76,6 +76,65 @@ def test_capture_survives_other_objects(gpu, mode, thread, what):
     P.destroy()
     A.destroy()
     B.destroy()
+
+
+# CSR-vector plans are made and destroyed beside a capture in any mode (they need
+# no arrays).  Long rows side by side, so that the plan lists their blocks.
+@pytest.mark.parametrize("mode", [GLOBAL, THREAD_LOCAL, RELAXED])
+@pytest.mark.parametrize("thread", [False, True])
+def test_csr_vector_plans_within_a_capture(gpu, mode, thread):
+    from matrix_format_performance_amd import _lib as L
+    lib = L.load()
+
+    def hip(name, *args):
+        status = getattr(lib, name)(*args)
+        assert status == 0, (name, status)
+
+    announce(f"CSR-vector in a capture mode={mode} thread={thread}")
+    rng = np.random.default_rng(0)
+    lens = np.full(300007, 6)
+    lens[100000:100256] = 1500
+    rp = np.concatenate([[0], np.cumsum(lens)]).astype(np.uint32)
+    ci = np.sort(rng.integers(0, 300007, rp[-1])).astype(np.uint32)
+    va = rng.integers(-3, 4, ci.size).astype(np.float32)
+    A, B = (gpu.DeviceMatrix.from_csr(rp, ci, va, 300007) for _ in range(2))
+    xh = rng.integers(-5, 6, 300007).astype(np.float32)
+    x, y = gpu.DeviceArray.from_host(xh), gpu.DeviceArray(300007, np.dtype(np.float32))
+    sums = np.concatenate([[0], np.cumsum(va.astype(np.int64) * xh.astype(np.int64)[ci])])
+    want = (sums[rp[1:]] - sums[rp[:-1]]).astype(np.float32)
+    old, made = gpu.Plan(B, "csr_vector", lanes=8), []
+    s, g, e = C.c_void_p(), C.c_void_p(), C.c_void_p()
+    hip("hipStreamCreateWithFlags", C.byref(s), C.c_uint(1))
+
+    def act():
+        old.destroy()
+        made.append(gpu.Plan(A, "csr_vector", lanes=8))
+
+    gpu.synchronize()
+    hip("hipStreamBeginCapture", s, C.c_int(mode))
+    try:
+        if thread:
+            t = threading.Thread(target=act)
+            t.start()
+            t.join()
+        else:
+            act()
+        made[0].spmv(x, y, stream=s)
+    finally:
+        ended = lib.hipStreamEndCapture(s, C.byref(g))
+    assert ended == 0
+    hip("hipGraphInstantiate", C.byref(e), g, None, None, C.c_size_t(0))
+    for _ in range(3):
+        y.fill(np.nan)
+        gpu.synchronize()
+        hip("hipGraphLaunch", e, s)
+        hip("hipStreamSynchronize", s)
+        assert np.array_equal(y.to_host(), want)
+    hip("hipGraphExecDestroy", e)
+    hip("hipGraphDestroy", g)
+    hip("hipStreamDestroy", s)
+    for o in (made[0], A, B):
+        o.destroy()
 
 
 def test_trim_gives_kept_memory_to_other_allocators(gpu):
