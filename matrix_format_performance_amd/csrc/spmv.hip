@@ -1778,6 +1778,10 @@ static uint32_t adaptive_gap(uint32_t W)
   return groups(gap) < groups(ADAPTIVE_NO_GAP) ? ADAPTIVE_NO_GAP : gap;
 }
 
+// Workgroups of one launch: their lanes are numbered in 32 bits.  Blocks of one
+// entry are that many from 16.7M entries on.
+constexpr uint32_t ADAPTIVE_GRID = (1u << 24) - 8;
+
 template <typename T>
 static int adaptive_t(const adaptive_args &g, const T *a, const T *x, T *y, hipStream_t s)
 {
@@ -1787,17 +1791,23 @@ static int adaptive_t(const adaptive_args &g, const T *a, const T *x, T *y, hipS
   const uint32_t gap = adaptive_gap<T>(g.nnz_per_wg);
   const size_t lds = adaptive_lds_bytes<T>(g.nnz_per_wg, gap);
   const uint32_t K = adaptive_vectors_per_lane(sizeof(T) == 4 ? MFP_F32 : MFP_F64, g.nnz_per_wg);
-  if (items) {
+  adaptive_args part = g;
+  uint32_t pad = nchunks_pad;
+  for (uint32_t left = items; left;) {
+    const uint32_t n = pad < ADAPTIVE_GRID ? std::min(left, ADAPTIVE_GRID) : left;
     int st;
     switch (K) {
-    case 1: st = adaptive_launch_k<T, 1>(g, a, x, y, s, gap, lds, items, nchunks_pad); break;
-    case 2: st = adaptive_launch_k<T, 2>(g, a, x, y, s, gap, lds, items, nchunks_pad); break;
-    case 4: st = adaptive_launch_k<T, 4>(g, a, x, y, s, gap, lds, items, nchunks_pad); break;
-    case 8: st = adaptive_launch_k<T, 8>(g, a, x, y, s, gap, lds, items, nchunks_pad); break;
-    case 16: st = adaptive_launch_k<T, 16>(g, a, x, y, s, gap, lds, items, nchunks_pad); break;
+    case 1: st = adaptive_launch_k<T, 1>(part, a, x, y, s, gap, lds, n, pad); break;
+    case 2: st = adaptive_launch_k<T, 2>(part, a, x, y, s, gap, lds, n, pad); break;
+    case 4: st = adaptive_launch_k<T, 4>(part, a, x, y, s, gap, lds, n, pad); break;
+    case 8: st = adaptive_launch_k<T, 8>(part, a, x, y, s, gap, lds, n, pad); break;
+    case 16: st = adaptive_launch_k<T, 16>(part, a, x, y, s, gap, lds, n, pad); break;
     default: set_error("nnz_per_wg too large"); return MFP_ERR_ARG;
     }
     MFP_CHECK(st);
+    left -= n;
+    part.blocks += n - pad;
+    part.nchunks = pad = 0;
   }
   if (g.nchunks)
     MFP_CHECK(launch_k(k_adaptive_finish<T>, dim3(ceil_div_u32(g.nchunks, 256)), dim3(256), 0, s, g.chunks,

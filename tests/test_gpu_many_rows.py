@@ -1,5 +1,5 @@
-"""More rows than a launch has lanes for, at four lanes a row: 2^30 + 77 rows of
-at most one entry (17 GB of device memory)."""
+"""More than a launch has lanes for: 2^30 + 77 rows of at most one entry at four
+lanes a row (17 GB of device memory), 2^24 + 77 row blocks of a workgroup each."""
 import ctypes as C
 
 import numpy as np
@@ -45,3 +45,24 @@ def test_ell_of_2_30_rows(gpu):
     plan.destroy()
     A.destroy()
     yd.free()
+
+
+# blocks of one entry; the long row goes in pieces, before the blocks
+@pytest.mark.parametrize("dtype", ["float32", "float64"])
+def test_adaptive_batch_of_2_24_row_blocks(gpu, dtype):
+    announce(f"batch csr_adaptive nnz_per_wg=1 dtype={dtype}")
+    lens = np.ones((1 << 24) + 77, np.int64)
+    lens[5] = 9000
+    rp = np.concatenate([[0], np.cumsum(lens)]).astype(np.uint32)
+    e = np.arange(rp[-1])
+    ci, va = (e * 7 % 1009).astype(np.uint32), (e % 7 - 3).astype(dtype)
+    A = gpu.DeviceMatrix.from_csr(rp, ci, va, 1009)
+    B = gpu.Batch([A], nnz_per_wg=1)
+    x = (np.arange(1009) % 11 - 5).astype(dtype)
+    xd, yd = gpu.DeviceArray.from_host(x), gpu.DeviceArray(lens.size, np.dtype(dtype))
+    yd.fill(np.nan)
+    B.spmm(1, xd, yd)
+    gpu.synchronize()
+    assert np.array_equal(yd.to_host(), np.add.reduceat(va * x[ci], rp[:-1].astype(np.int64)))
+    B.destroy()
+    A.destroy()
